@@ -155,6 +155,43 @@ typedef struct {
     qgtl_c64_t M[4];
 } qgtl_inject_slot_t;
 
+/* ---- small circuits resident in LDS (4 <= n <= 13) ----
+ * One block of the circuit for qgtl_hip_resident_states: qubit q's matrix is
+ * diag(post) R diag(pre) with the rotation R = [[c, -s], [s, c]] and its
+ * larger entry taken out: R = c [[1, -t], [t, 1]] (swapped = 0, t = s / c) or
+ * R = s [[t, -1], [1, t]] (swapped = 1, t = c / s); a qubit without a gate has
+ * t = 0.  The post (pre) phases and the entries taken out come as two tables
+ * over qubits 0..6 (128 entries) and 7..12 (64), their product taken at a
+ * thread's bits, times reg_post (reg_pre): the products of the phase ratios over the
+ * register bits of the last group of four qubits, n-4 .. n-1 (of the first,
+ * 0 .. 3).  img[q]: image of basis bit q under the M-stage (GF(2)-linear). */
+#define QGTL_RES_MIN_QUBITS 4
+#define QGTL_RES_MAX_QUBITS 13
+#define QGTL_RES_TAB 192                       /* complex64 entries: post tables, then as many for pre */
+typedef struct {
+    float tan[QGTL_RES_MAX_QUBITS];
+    int32_t swapped[QGTL_RES_MAX_QUBITS];
+    uint32_t img[QGTL_RES_MAX_QUBITS];
+    int32_t has_pre, has_perm;
+    qgtl_c64_t reg_pre[16], reg_post[16];
+} qgtl_res_block_t;
+
+/* The injection of a D slot after block `block` (as qgtl_inject_slot_t). */
+typedef struct {
+    uint32_t v, w;
+    qgtl_c64_t M[4];
+    int32_t block;
+    int32_t pad;
+} qgtl_res_slot_t;
+
+/* The P derivative states at the end of the circuit (D, stride 2^n, slot
+ * order), the primal state (psi) and the FP64 injection sums (P x 4).  blocks:
+ * nblocks descriptors; tabs: 2 QGTL_RES_TAB complex64 per block; slots: P + 1
+ * in block order, the last one (the primal state) with block = nblocks.  All
+ * on the device. */
+int qgtl_hip_resident_states(int n, const void *blocks, int nblocks, const void *tabs, const void *slots, int P,
+                             void *D, void *psi, double *sums);
+
 /* ---- grouped launches ----
  * One launch runs the same kind of work for many independent instances.
  * Work item i covers the units [unit_begin_i, unit_begin_{i+1}) of the

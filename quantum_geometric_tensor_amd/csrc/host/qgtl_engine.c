@@ -259,6 +259,9 @@ static void plan_free_device(struct qgtl_plan *p)
     qgtl_hip_free(p->tabs_dev);
     p->tabs_dev = NULL;
     p->tabs_passes = 0;
+    qgtl_hip_free(p->res_dev);
+    qgtl_hip_host_free(p->res_host);
+    p->res_dev = p->res_host = NULL;
     qgtl_hip_free(p->inj_slots_dev);
     p->inj_slots_dev = NULL;
     qgtl_hip_free(p->inj_partials);
@@ -602,6 +605,48 @@ static int upload_tabs(struct qgtl_plan *p)
         }
         HIPCALL(qgtl_hip_h2d(p->inj_slots_dev, p->inj_slots_host, 2 * P * sizeof(qgtl_inject_slot_t)));
     }
+    p->tabs_dirty = 0;
+    return 0;
+}
+
+/* Circuits whose states one workgroup holds in LDS from start to end; the
+ * general-matrix sweep form and the one- to three-qubit circuits keep the
+ * breadth-first passes. */
+static int resident_ok(const struct qgtl_plan *p)
+{
+    return p->P > 0 && p->n >= QGTL_RES_MIN_QUBITS && p->n <= QGTL_RES_MAX_QUBITS && p->tune.sweep_form != 1;
+}
+
+/* Build and upload the resident kernel's blocks, phase tables and slots after
+ * the angles changed. */
+static int upload_resident(struct qgtl_plan *p)
+{
+    const size_t nb = (size_t)p->nblocks, P = (size_t)p->P;
+    if (!p->res_dev) {
+        p->res_tabs = nb * sizeof(qgtl_res_block_t);
+        p->res_slots = p->res_tabs + nb * 2 * QGTL_RES_TAB * sizeof(qgtl_c64_t);
+        p->res_bytes = p->res_slots + (P + 1) * sizeof(qgtl_res_slot_t);
+        if (!p->res_host) HIPCALL(qgtl_hip_host_alloc(&p->res_host, p->res_bytes));
+        HIPCALL(qgtl_hip_malloc(&p->res_dev, p->res_bytes));
+    } else if (!p->tabs_dirty) {
+        return 0;
+    }
+    char *h = (char *)p->res_host;
+    qgtl_res_slot_t *slots = (qgtl_res_slot_t *)(h + p->res_slots);
+    for (size_t b = 0; b < nb; b++)
+        qgtl_resident_block(&p->blocks[b], p->n, (qgtl_res_block_t *)h + b,
+                            (qgtl_c64_t *)(h + p->res_tabs) + b * 2 * QGTL_RES_TAB);
+    for (size_t s = 0; s < P; s++) {
+        const qgtl_param_t *pp = &p->params[p->slot_param[s]];
+        qgtl_inject_slot_t q;
+        q.v = pp->v;
+        q.w = pp->w;
+        slot_matrix(&q, &pp->A);
+        slots[s] = (qgtl_res_slot_t){q.v, q.w, {q.M[0], q.M[1], q.M[2], q.M[3]}, pp->block, 0};
+    }
+    memset(&slots[P], 0, sizeof slots[P]);
+    slots[P].block = p->nblocks;
+    HIPCALL(qgtl_hip_h2d(p->res_dev, p->res_host, p->res_bytes));
     p->tabs_dirty = 0;
     return 0;
 }
@@ -1051,7 +1096,8 @@ static int prepare_mixed(struct qgtl_plan *p)
 {
     int rc = alloc_mixed(p);
     if (rc) return rc;
-    rc = upload_tabs(p);
+    p->resident = resident_ok(p);
+    rc = p->resident ? upload_resident(p) : upload_tabs(p);
     if (rc) return rc;
     const int depth_first = any_flip(p);
     p->meet = choose_meet(p, depth_first);
@@ -1074,11 +1120,27 @@ static int prepare_mixed(struct qgtl_plan *p)
     return 0;
 }
 
+/* Every derivative state, the primal state and the injection sums of a small
+ * circuit in one launch. */
+static int run_resident(struct qgtl_plan *p, qgtl_stats_t *st)
+{
+    const char *d = (const char *)p->res_dev;
+    LAUNCH(K_SWEEP, qgtl_hip_resident_states(p->n, d, p->nblocks, d + p->res_tabs, d + p->res_slots, p->P, p->D,
+                                             p->psi[0], p->inj_sums));
+    p->psi_final = p->psi[0];
+    if (st) {
+        st->sweep_launches++;
+        st->sweep_state_passes += p->P + 1;
+        st->sweep_bytes += (double)p->N * 8.0 * (p->P + 1);
+    }
+    return 0;
+}
+
 /* The launches of a mixed execute (prepare_mixed done). */
 static int run_mixed(struct qgtl_plan *p, qgtl_stats_t *st)
 {
     const int lanes = any_flip(p) && !g_profiling;
-    int rc = run_mixed_lanes(p, st, lanes);
+    int rc = p->resident ? run_resident(p, st) : run_mixed_lanes(p, st, lanes);
     if (lanes) qgtl_hip_set_lane(0);
     if (rc) return rc;
     if (p->P == 0) return 0;

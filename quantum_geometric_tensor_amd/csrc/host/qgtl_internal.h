@@ -124,6 +124,12 @@ struct qgtl_plan {
      * and backward (P..2P-1), rebuilt with the tables */
     qgtl_inject_slot_t *inj_slots_host;
     void *inj_slots_dev;
+    /* small circuits evolved in LDS by one launch (qgtl_hip_resident_states): the
+     * blocks' descriptors, their phase tables and the injection slots, in one
+     * buffer rebuilt with the tables (pinned host copy beside it) */
+    int resident;
+    void *res_dev, *res_host;
+    size_t res_tabs, res_slots, res_bytes;   /* byte offsets of the tables and the slots; size */
     /* Hamiltonian for energy / gradient */
     int nterms;
     void *terms_dev;
@@ -184,6 +190,7 @@ int qgtl_init_if_needed(void);
 /* learned preconditioner (qgtl_mlp.c) */
 void qgtl_mlp_shape(const qgtl_mlp_t *m, int *in_dim, int *P, int *rank);
 void qgtl_pass_phase_tables(const qgtl_pass_desc_t *p, float *out);
+void qgtl_resident_block(const qgtl_block_t *b, int n, qgtl_res_block_t *out, qgtl_c64_t *tabs);
 int qgtl_carry_to_meet(struct qgtl_plan *p, void **state, void **scratch);
 
 /* file container of qgtl_io.c (prefix, kind header, payload, FNV-1a 64 checksum) */

@@ -879,6 +879,60 @@ void qgtl_pass_phase_tables(const qgtl_pass_desc_t *p, float *out)
     }
 }
 
+/* Phase table of the qubits q0 .. q0 + bits - 1: entry i is the product of
+ * ph[q][bit q - q0 of i], from f, each entry one FP64 product of an earlier
+ * one, rounded once. */
+static void doubling_table(qgtl_cd (*ph)[2], int q0, int bits, qgtl_cd f, qgtl_c64_t *out)
+{
+    qgtl_cd t[128];
+    for (int i = 0; i < bits; i++) f = cmul(f, ph[q0 + i][0]);
+    t[0] = f;
+    for (int i = 0; i < bits; i++) {
+        const qgtl_cd rel = cmul(ph[q0 + i][1], cconj(ph[q0 + i][0]));
+        for (int k = 0; k < 1 << i; k++) t[(1 << i) + k] = cmul(t[k], rel);
+    }
+    for (int k = 0; k < 1 << bits; k++) out[k] = c64(t[k]);
+}
+
+/* Block b for the resident kernel (see qgtl_res_block_t), 4 <= n <= 13. */
+void qgtl_resident_block(const qgtl_block_t *b, int n, qgtl_res_block_t *out, qgtl_c64_t *tabs)
+{
+    qgtl_cd pre[QGTL_RES_MAX_QUBITS][2], post[QGTL_RES_MAX_QUBITS][2];
+    double scale = 1.0;
+    out->has_pre = 0;
+    out->has_perm = b->nperm > 0;
+    for (int q = 0; q < QGTL_RES_MAX_QUBITS; q++) {
+        pre[q][0] = pre[q][1] = post[q][0] = post[q][1] = cd(1.0, 0.0);
+        out->tan[q] = 0.f;
+        out->swapped[q] = 0;
+        out->img[q] = q < n ? perm_apply(b, 1u << q) : 0u;
+        if (q >= n || !b->has_u[q]) continue;
+        double c, s;
+        factor_rotation(&b->u[q], &c, &s, pre[q], post[q]);
+        out->swapped[q] = fabs(c) < fabs(s);
+        out->tan[q] = (float)(out->swapped[q] ? c / s : s / c);
+        scale *= out->swapped[q] ? s : c;
+        if (pre[q][0].re != 1.0 || pre[q][0].im != 0.0 || pre[q][1].re != 1.0 || pre[q][1].im != 0.0) out->has_pre = 1;
+    }
+    const int lo = n < 7 ? n : 7, hi = n - lo;
+    doubling_table(post, 0, lo, cd(scale, 0.0), tabs);
+    doubling_table(post, 7, hi, cd(1.0, 0.0), tabs + 128);
+    if (out->has_pre) {
+        doubling_table(pre, 0, lo, cd(1.0, 0.0), tabs + QGTL_RES_TAB);
+        doubling_table(pre, 7, hi, cd(1.0, 0.0), tabs + QGTL_RES_TAB + 128);
+    }
+    for (int r = 0; r < 16; r++) {
+        qgtl_cd a = cd(1.0, 0.0), p = cd(1.0, 0.0);
+        for (int i = 0; i < 4; i++) {
+            if (!((r >> i) & 1)) continue;
+            a = cmul(a, cmul(post[n - 4 + i][1], cconj(post[n - 4 + i][0])));
+            p = cmul(p, cmul(pre[i][1], cconj(pre[i][0])));
+        }
+        out->reg_post[r] = c64(a);
+        out->reg_pre[r] = c64(p);
+    }
+}
+
 /* Diagnostics: max |diag(post) R diag(pre) - U| over every gate of every pass
  * (FP32 descriptor values, FP64 arithmetic) and the number of passes that
  * need a pre-phase layer. */
