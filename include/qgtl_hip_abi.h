@@ -445,6 +445,10 @@ int qgtl_hip_kaporin(int P, int r, int B, const float *Y, const float *As_all, c
 /* ---- FP64 natural-gradient solves, one workgroup per system ---- */
 int qgtl_hip_lu_solve_c128(void *A, const void *b, void *x, int *piv, int P, int batch, int *status);
 int qgtl_hip_herm_eig_c128(void *A, void *V, double *ev, int P, int batch, int max_sweeps, int *sweeps);
+/* out4 (device): smallest, largest, smallest positive (+inf: none) and largest
+ * negative (-inf: none) eigenvalue of the Hermitian A (upper triangle read);
+ * W: P x P complex128 scratch */
+int qgtl_hip_herm_extremes_c128(const void *A, void *W, int P, double *out4);
 int qgtl_hip_cholesky_solve_f64(double *A, const double *b, double *x, int P, int batch, double lambda, int *status);
 int qgtl_hip_pcg_f64(const double *A, const double *b, double *x, int P, int batch, double lambda, const double *d,
                      const double *U, int r, double tol, int maxit, int *iters, double *relres);

@@ -509,6 +509,245 @@ __global__ __launch_bounds__(kT) void pcg_f64_kernel(const double *Aall, const d
     if (i == 0) { iters[blockIdx.x] = it; relres[blockIdx.x] = rel; }
 }
 
+// ------------------------------------------- extreme Hermitian eigenvalues
+// The eigenvalues a condition number needs -- the smallest, the largest and
+// the two next to zero -- of a Hermitian matrix (its upper triangle), without
+// eigenvectors: Householder reduction to a real tridiagonal, then
+// multisection on the Sturm counts, 256 points at a time for each of the four.
+//
+// One workgroup; thread t owns column t % n and the rows t / n (mod nseg), in
+// registers (ROWS per thread) where they fit, else in W (global, in L2).  A
+// step of the reduction applies the previous step's rank-2 update and forms the
+// next matrix-vector product in one pass over the owned entries, with three
+// barriers.  What bounds it: the latency of those steps (at P = 96 about 2 us
+// each); the cyclic Jacobi iteration it replaces here runs 8 to 10 sweeps of
+// P - 1 steps, each two passes over A and one over V in global memory.
+//
+// Indices whose row is zero off the diagonal are set aside first: their
+// diagonal entries are exact eigenvalues (a parameter without effect leaves a
+// zero row, and its exact zero is no part of the condition number).
+constexpr int kExtRows = 16;      // register rows per thread (64 VGPRs of the 128 at 16 waves; 20 spill): n <= 128
+
+// number of eigenvalues of the tridiagonal (d, e2 = squared off-diagonals) below x
+__device__ __forceinline__ int sturm_count(const double *d, const double *e2, int n, double x, double pivmin) {
+    int c = 0;
+    double q = 1.0, prev = 0.0;
+    for (int i = 0; i < n; i++) {
+        double r = __builtin_amdgcn_rcp(q);
+        r = fma(r, fma(-q, r, 1.0), r);
+        r = fma(r, fma(-q, r, 1.0), r);
+        q = (d[i] - x) - prev * r;
+        if (fabs(q) < pivmin) q = -pivmin;
+        c += q < 0.0;
+        prev = e2[i];
+    }
+    return c;
+}
+
+// out: smallest, largest, smallest positive (+inf: none), largest negative (-inf: none)
+template <bool REG>
+__global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__restrict__ A, int P, double2 *W,
+                                                           double *out) {
+    __shared__ double2 su[kT], sq[kT], sx[kT], part[kT];
+    __shared__ double sd[kT], se2[kT], swv[kT / 64][4];
+    __shared__ int map[kT];
+    __shared__ unsigned long long bal[kT / 64];
+    __shared__ int cnt[kT / 64];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    // isolated indices
+    bool iso = false;
+    double isov = 0.0;
+    if (t < P) {
+        iso = true;
+        for (int i = 0; i < P; i++) {
+            if (i == t) continue;
+            const double2 a = i < t ? A[(size_t)i * P + t] : A[(size_t)t * P + i];
+            if (a.x != 0.0 || a.y != 0.0) iso = false;
+        }
+        isov = A[(size_t)t * P + t].x;
+    }
+    const bool live = t < P && !iso;
+    const unsigned long long b = __ballot(live);
+    if (lane == 0) bal[wave] = b;
+    su[t] = sq[t] = make_double2(0.0, 0.0);
+    __syncthreads();
+    int rank = 0, n = 0;
+    for (int w = 0; w < kT / 64; w++) {
+        const int c = __popcll(bal[w]);
+        if (w < wave) rank += c;
+        n += c;
+    }
+    rank += __popcll(b & ((1ull << lane) - 1ull));
+    if (live) map[rank] = t;
+    __syncthreads();
+    const double inf = __builtin_inf();
+    double lo_all = iso ? isov : inf, hi_all = iso ? isov : -inf;
+    double pos_all = iso && isov > 0.0 ? isov : inf, neg_all = iso && isov < 0.0 ? isov : -inf;
+    if (n > 0) {                                             // n >= 2: an index is live with another
+        const int nseg = kT / n, seg = t / n, j = t % n;
+        const int rows = (n + nseg - 1) / nseg;
+        double2 a[REG ? kExtRows : 1];
+        const int oj = map[j];
+        auto entry = [&](int i) -> double2 {
+            const int oi = map[i];
+            if (oi <= oj) { double2 v = A[(size_t)oi * P + oj]; if (oi == oj) v.y = 0.0; return v; }
+            const double2 v = A[(size_t)oj * P + oi];
+            return make_double2(v.x, -v.y);
+        };
+        if constexpr (REG) {
+#pragma unroll
+            for (int r = 0; r < kExtRows; r++) {
+                const int i = seg + nseg * r;
+                a[r] = (seg < nseg && i < n) ? entry(i) : make_double2(0.0, 0.0);
+            }
+        } else {
+            if (seg < nseg)
+                for (int i = seg; i < n; i += nseg) W[(size_t)i * n + j] = entry(i);
+        }
+        // x_i of column k for this thread's rows (it owns column k): the entry with the pending update
+        auto pend = [&](double2 v, int i, double2 uk, double2 qk) -> double2 {
+            const double2 ui = su[i], qi = sq[i];
+            v.x -= ui.x * qk.x + ui.y * qk.y + qi.x * uk.x + qi.y * uk.y;
+            v.y -= ui.y * qk.x - ui.x * qk.y + qi.y * uk.x - qi.x * uk.y;
+            return v;
+        };
+        for (int k = 0; k < n; k++) {
+            const double2 uj = su[j], qj = sq[j];
+            if (j == k && seg < nseg) {
+                if constexpr (REG) {
+#pragma unroll
+                    for (int r = 0; r < kExtRows; r++) {
+                        const int i = seg + nseg * r;
+                        if (i >= k && i < n) sx[i] = pend(a[r], i, uj, qj);
+                    }
+                } else {
+                    for (int r = 0; r < rows; r++) {
+                        const int i = seg + nseg * r;
+                        if (i >= k && i < n) sx[i] = pend(W[(size_t)i * n + j], i, uj, qj);
+                    }
+                }
+            }
+            __syncthreads();
+            if (t == 0) sd[k] = sx[k].x;
+            if (k == n - 1) break;
+            double tail = 0.0;
+            for (int i = k + 2 + lane; i < n; i += 64) tail += sx[i].x * sx[i].x + sx[i].y * sx[i].y;
+            tail = wave_sum_f64(tail);
+            double2 u0 = sx[k + 1];
+            const double x0 = u0.x * u0.x + u0.y * u0.y;
+            double tau = 0.0, e2 = x0;
+            if (tail > 0.0) {
+                e2 = tail + x0;
+                const double s = sqrt(e2), m = sqrt(x0);
+                tau = 1.0 / (s * (s + m));                   // 2 / |u|^2
+                if (m > 0.0) { u0.x += u0.x * (s / m); u0.y += u0.y * (s / m); }
+                else u0.x = s;
+            }
+            if (t == 0) se2[k] = e2;
+            double pr = 0.0, pi = 0.0;
+            if (j > k && seg < nseg) {
+                auto one = [&](double2 v, int i) -> double2 {
+                    v = pend(v, i, uj, qj);
+                    const double2 ui = i == k + 1 ? u0 : sx[i];
+                    pr += v.x * ui.x + v.y * ui.y;           // conj(a_ij) u_i
+                    pi += v.x * ui.y - v.y * ui.x;
+                    return v;
+                };
+                if constexpr (REG) {
+#pragma unroll
+                    for (int r = 0; r < kExtRows; r++) {
+                        const int i = seg + nseg * r;
+                        if (i > k && i < n) a[r] = one(a[r], i);
+                    }
+                } else {
+                    for (int r = 0; r < rows; r++) {
+                        const int i = seg + nseg * r;
+                        if (i > k && i < n) W[(size_t)i * n + j] = one(W[(size_t)i * n + j], i);
+                    }
+                }
+            }
+            part[t] = make_double2(pr, pi);
+            __syncthreads();
+            // p = tau A u; K = tau / 2 u^H p; q = p - K u (every wave forms u^H p for itself)
+            double up = 0.0;
+            for (int i = k + 1 + lane; i < n; i += 64) {
+                double2 s = part[i];
+                for (int g = 1; g < nseg; g++) { s.x += part[g * n + i].x; s.y += part[g * n + i].y; }
+                const double2 ui = i == k + 1 ? u0 : sx[i];
+                up += ui.x * s.x + ui.y * s.y;
+            }
+            up = wave_sum_f64(up);
+            if (t < n) {
+                double2 ut = make_double2(0.0, 0.0), qt = make_double2(0.0, 0.0);
+                if (t > k && tau > 0.0) {
+                    double2 s = part[t];
+                    for (int g = 1; g < nseg; g++) { s.x += part[g * n + t].x; s.y += part[g * n + t].y; }
+                    ut = t == k + 1 ? u0 : sx[t];
+                    const double kk = 0.5 * tau * tau * up;
+                    qt = make_double2(tau * s.x - kk * ut.x, tau * s.y - kk * ut.y);
+                }
+                su[t] = ut;
+                sq[t] = qt;
+            }
+            __syncthreads();
+        }
+        __syncthreads();
+        // Gershgorin bound
+        double bd = 0.0;
+        if (t < n)
+            bd = fabs(sd[t]) + (t > 0 ? sqrt(se2[t - 1]) : 0.0) + (t + 1 < n ? sqrt(se2[t]) : 0.0);
+        for (int o = 32; o > 0; o >>= 1) bd = fmax(bd, __shfl_xor(bd, o, 64));
+        if (lane == 0) swv[wave][0] = bd;
+        __syncthreads();
+        bd = 0.0;
+        for (int w = 0; w < kT / 64; w++) bd = fmax(bd, swv[w][0]);
+        // eigenvalues within 1e-30 of the bound of zero are exact zeros: rounding is at 1e-16 of it
+        const double B = bd * (1.0 + 1e-10), tiny = 1e-30 * bd, pivmin = 1e-40 * bd;
+        const int grp = t >> 8, m = t & 255;
+        const int cz = bd > 0.0 ? sturm_count(sd, se2, n, (t & 1) ? tiny : -tiny, pivmin) : 0;
+        const int n_neg = __shfl(cz, 0, 64), n_pos = __shfl(cz, 1, 64);   // below -tiny, below +tiny
+        const int idx = grp == 0 ? 0 : grp == 1 ? n - 1 : grp == 2 ? n_pos : n_neg - 1;
+        const bool want = bd > 0.0 && idx >= 0 && idx < n;
+        double lo = grp == 2 ? 0.0 : -B, hi = grp == 3 ? 0.0 : B;
+        for (int round = 0; round < 9; round++) {
+            const double h = (hi - lo) * (1.0 / 257.0);
+            int c = 0;
+            if (want) c = sturm_count(sd, se2, n, lo + h * (m + 1), pivmin) <= idx;
+            const int below = __popcll(__ballot(c != 0));
+            if (lane == 0) cnt[wave] = below;
+            __syncthreads();
+            const int k = cnt[4 * grp] + cnt[4 * grp + 1] + cnt[4 * grp + 2] + cnt[4 * grp + 3];
+            const double nl = k == 0 ? lo : lo + h * k, nh = k == 256 ? hi : lo + h * (k + 1);
+            lo = nl;
+            hi = nh;
+            __syncthreads();
+        }
+        const double v = bd > 0.0 ? 0.5 * (lo + hi) : 0.0;
+        if (grp == 0 && (want || bd == 0.0)) lo_all = fmin(lo_all, v);
+        if (grp == 1 && (want || bd == 0.0)) hi_all = fmax(hi_all, v);
+        if (grp == 2 && want) pos_all = fmin(pos_all, v);
+        if (grp == 3 && want) neg_all = fmax(neg_all, v);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        lo_all = fmin(lo_all, __shfl_xor(lo_all, o, 64));
+        hi_all = fmax(hi_all, __shfl_xor(hi_all, o, 64));
+        pos_all = fmin(pos_all, __shfl_xor(pos_all, o, 64));
+        neg_all = fmax(neg_all, __shfl_xor(neg_all, o, 64));
+    }
+    __syncthreads();
+    if (lane == 0) { swv[wave][0] = lo_all; swv[wave][1] = hi_all; swv[wave][2] = pos_all; swv[wave][3] = neg_all; }
+    __syncthreads();
+    if (t == 0) {
+        for (int w = 1; w < kT / 64; w++) {
+            lo_all = fmin(lo_all, swv[w][0]);
+            hi_all = fmax(hi_all, swv[w][1]);
+            pos_all = fmin(pos_all, swv[w][2]);
+            neg_all = fmax(neg_all, swv[w][3]);
+        }
+        out[0] = lo_all; out[1] = hi_all; out[2] = pos_all; out[3] = neg_all;
+    }
+}
+
 // B = M^H M for the singular values of a general complex matrix
 __global__ void gram_small_c128_kernel(const double2 *M, double2 *B, int P) {
     for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < P * P; e += gridDim.x * blockDim.x) {
@@ -651,6 +890,21 @@ int qgtl_hip_herm_eig_c128(void *A, void *V, double *ev, int P, int batch, int m
     hipLaunchKernelGGL(herm_eig_c128_kernel, dim3(batch), dim3(kT), 0, qgtl::stream(), (double2 *)A, (double2 *)V,
                        ev, P, max_sweeps, sweeps);
     QGTL_LAUNCH_CHECK("herm_eig_c128");
+    return 0;
+}
+
+int qgtl_hip_herm_extremes_c128(const void *A, void *W, int P, double *out4) {
+    if (P < 1 || P > kT) return qgtl::set_error_msg(-118, "herm_extremes: needs 1 <= P <= 1024");
+    // every matrix of the kernel's order n <= P fits the register rows when that of order P does
+    // (n^2 entries over kT threads: rows(n) = ceil(n / floor(kT / n)) grows with n)
+    const int nseg = kT / P, rows = (P + nseg - 1) / nseg;
+    if (rows <= kExtRows)
+        hipLaunchKernelGGL(herm_extremes_kernel<true>, dim3(1), dim3(kT), 0, qgtl::stream(), (const double2 *)A, P,
+                           (double2 *)W, out4);
+    else
+        hipLaunchKernelGGL(herm_extremes_kernel<false>, dim3(1), dim3(kT), 0, qgtl::stream(), (const double2 *)A, P,
+                           (double2 *)W, out4);
+    QGTL_LAUNCH_CHECK("herm_extremes_c128");
     return 0;
 }
 

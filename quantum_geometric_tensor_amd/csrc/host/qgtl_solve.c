@@ -264,15 +264,16 @@ static double *to_c128(const ComplexFloat *m, size_t count)
 
 static int is_hermitian(const double *M, size_t P)
 {
+    /* squared magnitudes of float-range values: no overflow in FP64 */
     double mx = 0.0, dev = 0.0;
     for (size_t i = 0; i < P; i++)
-        for (size_t j = 0; j < P; j++) {
+        for (size_t j = i; j < P; j++) {
             const double ar = M[2 * (i * P + j)], ai = M[2 * (i * P + j) + 1];
             const double br = M[2 * (j * P + i)], bi = M[2 * (j * P + i) + 1];
-            mx = fmax(mx, hypot(ar, ai));
-            dev = fmax(dev, hypot(ar - br, ai + bi));
+            mx = fmax(mx, fmax(ar * ar + ai * ai, br * br + bi * bi));
+            dev = fmax(dev, (ar - br) * (ar - br) + (ai + bi) * (ai + bi));
         }
-    return dev <= 1e-6 * (mx > 0 ? mx : 1.0);
+    return dev <= 1e-12 * (mx > 0 ? mx : 1.0);
 }
 
 /* Singular values of M (FP64 on the GPU): |eigenvalues| when Hermitian,
@@ -300,23 +301,63 @@ static int singular_values(const double *M, size_t P, double *sv, int *hermitian
     return 0;
 }
 
+/* The largest and the smallest nonzero singular value of M (smallest: +inf when
+ * M has none), as singular_values would list them, without the eigenvectors. */
+static int extreme_singular_values(const double *M, size_t P, double *smax, double *smin)
+{
+    const size_t PP = P * P;
+    int finite = 1;
+    for (size_t i = 0; i < 2 * PP; i++) finite &= isfinite(M[i]) != 0;
+    if (!finite) {                             /* infinities and NaN: whatever the full decomposition lists */
+        double *sv = (double *)malloc(P * sizeof(double));
+        int h = 0;
+        if (!sv) return QGT_ERROR_NO_MEMORY;
+        const int rc = singular_values(M, P, sv, &h);
+        *smax = 0.0;
+        *smin = INFINITY;
+        for (size_t i = 0; !rc && i < P; i++) {
+            if (sv[i] > *smax) *smax = sv[i];
+            if (sv[i] > 0.0 && sv[i] < *smin) *smin = sv[i];
+        }
+        free(sv);
+        return rc;
+    }
+    void *dA, *dV, *dev, *dB;
+    double e[4];
+    TRY(scratch(S_A, PP * 16, &dA));
+    TRY(scratch(S_V, PP * 16, &dV));
+    TRY(scratch(S_EV, P * 8 > sizeof e ? P * 8 : sizeof e, &dev));
+    const int herm = is_hermitian(M, P);
+    if (herm) {
+        TRY(qgtl_hip_h2d(dA, M, PP * 16));
+    } else {
+        TRY(scratch(S_B, PP * 16, &dB));
+        TRY(qgtl_hip_h2d(dB, M, PP * 16));
+        TRY(qgtl_hip_gram_small_c128(dB, dA, (int)P));
+    }
+    TRY(qgtl_hip_herm_extremes_c128(dA, dV, (int)P, (double *)dev));
+    TRY(qgtl_hip_d2h(e, dev, sizeof e));
+    TRY(qgtl_hip_sync());
+    if (herm) {
+        *smax = fmax(fabs(e[0]), fabs(e[1]));
+        *smin = fmin(e[2], -e[3]);
+    } else {                                   /* eigenvalues of M^H M: rounding below zero counts as zero */
+        *smax = sqrt(fmax(e[1], 0.0));
+        *smin = sqrt(e[2]);
+    }
+    return 0;
+}
+
 bool compute_complex_matrix_condition_number(const ComplexFloat *matrix, size_t dimension, float *condition_number)
 {
     QGTL_LOCKED();
     if (!matrix || !condition_number || dimension == 0 || dimension > 1024) return false;
     if (qgtl_init_if_needed()) return false;
     double *M = to_c128(matrix, dimension * dimension);
-    double *sv = (double *)malloc(dimension * sizeof(double));
-    int herm = 0;
-    if (!M || !sv || singular_values(M, dimension, sv, &herm)) { free(M); free(sv); return false; }
     double smax = 0.0, smin = INFINITY;
-    for (size_t i = 0; i < dimension; i++) {
-        if (sv[i] > smax) smax = sv[i];
-        if (sv[i] > 0.0 && sv[i] < smin) smin = sv[i];
-    }
+    if (!M || extreme_singular_values(M, dimension, &smax, &smin)) { free(M); return false; }
     *condition_number = (smin > 1e-15) ? (float)(smax / smin) : INFINITY;
     free(M);
-    free(sv);
     return true;
 }
 

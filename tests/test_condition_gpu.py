@@ -1,0 +1,66 @@
+"""Condition numbers of the drop-in API (Householder tridiagonalisation and multisection on the
+GPU) against numpy's singular values, at the sizes where the kernel's row split changes.  Bar:
+a backward-stable eigenvalue is off by at most P eps ||A||, i.e. kappa by P eps kappa relative
+(kappa^2 for a general matrix, whose singular values come from M^H M), plus float rounding."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import quantum_geometric_tensor_amd as Q
+
+pytestmark = pytest.mark.gpu
+
+
+def _kappa(M):
+    L = Q.lib()
+    f = L.compute_complex_matrix_condition_number
+    f.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.POINTER(ctypes.c_float)]
+    f.restype = ctypes.c_bool
+    M = np.ascontiguousarray(M, np.complex64)
+    k = ctypes.c_float()
+    assert f(M.ctypes.data, len(M), ctypes.byref(k))
+    return k.value
+
+
+def _hermitian(P, ev, seed):
+    rng = np.random.default_rng(seed)
+    V, _ = np.linalg.qr(rng.normal(size=(P, P)) + 1j * rng.normal(size=(P, P)))
+    M = ((V * ev) @ V.conj().T).astype(np.complex64)
+    return np.tril(M, -1) + np.tril(M, -1).conj().T + np.diag(M.diagonal().real)
+
+
+def _check(M, general=False):
+    sv = np.linalg.svd(M.astype(np.complex128), compute_uv=False)
+    ref = sv.max() / sv.min()
+    eps = np.finfo(np.float64).eps
+    assert abs(_kappa(M) - ref) <= ref * (1e-6 + len(M) * eps * ref ** (2 if general else 1))
+
+
+@pytest.mark.parametrize("P", [2, 3, 31, 64, 65, 96, 128, 129, 171, 342, 513])
+def test_condition_number_hermitian(P):
+    _check(_hermitian(P, 0.25 * np.logspace(-4, 0, P), P))
+    ev = np.linspace(-1.0, 1.0, P) + 0.3 / P               # both signs, the smallest either side of zero
+    _check(_hermitian(P, ev, P + 1))
+    _check(_hermitian(P, -ev, P + 2))
+
+
+@pytest.mark.parametrize("P", [2, 5, 66, 130])
+def test_condition_number_general(P):
+    rng = np.random.default_rng(P)
+    U, _ = np.linalg.qr(rng.normal(size=(P, P)) + 1j * rng.normal(size=(P, P)))
+    V, _ = np.linalg.qr(rng.normal(size=(P, P)) + 1j * rng.normal(size=(P, P)))
+    _check(((U * np.logspace(-2, 0, P)) @ V).astype(np.complex64), general=True)
+
+
+def test_condition_number_zero_rows_and_diagonals():
+    assert _kappa(np.eye(1)) == 1.0
+    assert _kappa(np.diag([4.0, 0.0, -2.0, 0.5])) == 8.0    # exact zeros are not counted
+    assert _kappa(np.zeros((3, 3))) == 0.0                  # no nonzero value at all: 0 / inf
+    M = np.zeros((70, 70), np.complex64)                     # a parameter without effect: an exact zero row
+    keep = [i for i in range(70) if i not in (0, 13, 64)]
+    B = _hermitian(67, 0.25 * np.logspace(-3, 0, 67), 5)
+    M[np.ix_(keep, keep)] = B
+    sv = np.abs(np.linalg.eigvalsh(B.astype(np.complex128)))
+    assert abs(_kappa(M) - sv.max() / sv.min()) <= 1e-6 * sv.max() / sv.min()
+    assert np.isinf(_kappa(np.ones((40, 40)))) or _kappa(np.ones((40, 40))) > 1e13   # rank one
