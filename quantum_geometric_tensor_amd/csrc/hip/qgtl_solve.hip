@@ -516,12 +516,13 @@ __global__ __launch_bounds__(kT) void pcg_f64_kernel(const double *Aall, const d
 // multisection on the Sturm counts, 256 points at a time for each of the four.
 //
 // One workgroup; thread t owns column t % n and the rows t / n (mod nseg), in
-// registers (ROWS per thread) where they fit, else in W (global, in L2).  A
+// registers (kExtRows per thread) where they fit, else in W (global, in L2).  A
 // step of the reduction applies the previous step's rank-2 update and forms the
 // next matrix-vector product in one pass over the owned entries, with three
-// barriers.  What bounds it: the latency of those steps (at P = 96 about 2 us
-// each); the cyclic Jacobi iteration it replaces here runs 8 to 10 sweeps of
-// P - 1 steps, each two passes over A and one over V in global memory.
+// barriers.  What bounds it: the latency of those steps, about 6 us each.  At
+// P = 96 the condition number takes 667 us; the cyclic Jacobi iteration, which
+// did this before and still gives the eigenvectors elsewhere, 29.5 ms (8 to 10
+// sweeps of P - 1 steps, each two passes over A and one over V in global memory).
 //
 // Indices whose row is zero off the diagonal are set aside first: their
 // diagonal entries are exact eigenvalues (a parameter without effect leaves a
@@ -613,11 +614,15 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
         };
         for (int k = 0; k < n; k++) {
             const double2 uj = su[j], qj = sq[j];
+            // the row numbers formed anew at every step: hoisted out of the loop, the rows' LDS
+            // addresses take the registers the rows need (192 bytes of spills a thread: 710 against 667 us)
+            int s0 = seg;
+            __asm__ volatile("" : "+v"(s0));
             if (j == k && seg < nseg) {
                 if constexpr (REG) {
 #pragma unroll
                     for (int r = 0; r < kExtRows; r++) {
-                        const int i = seg + nseg * r;
+                        const int i = s0 + nseg * r;
                         if (i >= k && i < n) sx[i] = pend(a[r], i, uj, qj);
                     }
                 } else {
@@ -656,7 +661,7 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
                 if constexpr (REG) {
 #pragma unroll
                     for (int r = 0; r < kExtRows; r++) {
-                        const int i = seg + nseg * r;
+                        const int i = s0 + nseg * r;
                         if (i > k && i < n) a[r] = one(a[r], i);
                     }
                 } else {
