@@ -264,65 +264,183 @@ __global__ __launch_bounds__(kT) void herm_eig_c128_kernel(double2 *Aall, double
 }
 
 // ------------------------------------------------------------- Cholesky (real)
-__global__ __launch_bounds__(kT) void cholesky_f64_kernel(double *Lall, const double *ball, double *xall, int P,
+// Blocked right-looking factorisation of A + lambda I, one workgroup per
+// system, NB columns a step: the diagonal block by one wave (a row per lane, in
+// registers), the rows below it one per thread from LDS, the trailing update on
+// v_mfma_f64_16x16x4_f64 (16 x 16 tiles of the lower triangle, the panel in
+// LDS).  b is carried as one more row, so the forward substitution comes with
+// the factorisation; the back substitution runs block by block on L.  What
+// bounds it: the serial chain of the diagonal blocks (square root, reciprocal
+// and a row of multiply-adds per column).  P = 192: CHOL_NOW, from 1220 us with a
+// rank-1 update of the whole trailing matrix per column in global memory and
+// one reduction over a wave per row of the substitutions.
+//
+// NB = 32 while the panel fits LDS beside the rest (P <= 512), 16 above;
+// up to 256 the panel buffer is sized so that two workgroups share a CU.
+constexpr int kCT = 512;          // 8 waves: the register rows of 32 doubles need more than 128 VGPRs
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ double readlane_f64(double v, int lane);
+
+template <int NB, int ROWS>
+__global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const double *ball, double *xall, int P,
                                                           double lambda, int *status) {
-    double *L = Lall + (size_t)blockIdx.x * P * P;    // holds A on entry (row-major, symmetric)
+    constexpr int LD = ROWS + 1;                     // odd: the transposing writes hit all banks
+    __shared__ double lp[NB * LD];                   // panel, column c of row i at c * LD + i
+    __shared__ double dg[NB][NB + 1];                // diagonal block, then its factor by rows
+    __shared__ double y[1024], inv[NB];
+    __shared__ int s_fail;
+    double *L = Lall + (size_t)blockIdx.x * P * P;   // holds A on entry (row-major, symmetric)
     const double *b = ball + (size_t)blockIdx.x * P;
     double *x = xall + (size_t)blockIdx.x * P;
-    __shared__ int s_fail;
-    if (threadIdx.x == 0) s_fail = 0;
-    for (int i = threadIdx.x; i < P; i += kT) L[(size_t)i * P + i] += lambda;
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    if (t == 0) s_fail = 0;
+    for (int i = t; i < P; i += kCT) {
+        y[i] = b[i];
+        L[(size_t)i * P + i] += lambda;
+    }
     __syncthreads();
-    for (int j = 0; j < P; j++) {
-        const double d = L[(size_t)j * P + j];
-        if (!(d > 0.0)) {
-            if (threadIdx.x == 0) s_fail = 1;
-            break;
+    for (int kb = 0; kb < P; kb += NB) {
+        const int nb = min(NB, P - kb);
+        const int m = P - kb - nb + 1;               // rows below the block and the row of b
+        const int m16 = (m + 15) / 16 * 16;
+        for (int e = t; e < NB * NB; e += kCT) {
+            const int r = e / NB, c = e % NB;
+            dg[r][c] = (r < nb && c <= r) ? L[(size_t)(kb + r) * P + kb + c] : (r == c ? 1.0 : 0.0);
         }
-        const double ljj = sqrt(d);
+        for (int e = t; e < m16 * NB; e += kCT) {
+            const int r = e / NB, c = e % NB;
+            double v = 0.0;
+            if (c < nb) {
+                if (r < m - 1) v = L[(size_t)(kb + nb + r) * P + kb + c];
+                else if (r == m - 1) v = y[kb + c];
+            }
+            lp[c * LD + r] = v;
+        }
         __syncthreads();
-        for (int i = j + 1 + threadIdx.x; i < P; i += kT) L[(size_t)i * P + j] /= ljj;
-        if (threadIdx.x == 0) L[(size_t)j * P + j] = ljj;
+        if (w == 0) {
+            const int row = lane < NB ? lane : NB - 1;   // lanes past the block repeat its last row
+            double a[NB];
+#pragma unroll
+            for (int c = 0; c < NB; c++) a[c] = dg[row][c];
+            int bad = 0;
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                const double d = readlane_f64(a[j], j);
+                bad |= !(d > 0.0);
+                // l_jj and its reciprocal from one reciprocal square root, two Newton steps
+                double r = __builtin_amdgcn_rsq(d);
+                if (d < __builtin_inf()) {           // an infinite pivot keeps its reciprocal, 0
+                    r = fma(r * 0.5, fma(-d * r, r, 1.0), r);
+                    r = fma(r * 0.5, fma(-d * r, r, 1.0), r);
+                }
+                const double l = a[j] * r;           // lane j: d / sqrt(d)
+                a[j] = l;
+                if (lane == 0) inv[j] = r;
+#pragma unroll
+                for (int k = j + 1; k < NB; k++) a[k] = fma(-l, readlane_f64(l, k), a[k]);
+            }
+            if (lane < NB)
+#pragma unroll
+                for (int c = 0; c < NB; c++) dg[lane][c] = a[c];
+            if (bad && lane == 0) s_fail = 1;
+        }
         __syncthreads();
-        const int m = P - j - 1;
-        for (int e = threadIdx.x; e < m * (m + 1) / 2; e += kT) {
-            // lower triangle of the trailing block: (i, k) with k <= i
-            int i = (int)((sqrt(8.0 * e + 1.0) - 1.0) / 2.0);
-            while ((i + 1) * (i + 2) / 2 <= e) i++;
-            while (i * (i + 1) / 2 > e) i--;
-            const int k = e - i * (i + 1) / 2;
-            const int ii = j + 1 + i, kk = j + 1 + k;
-            L[(size_t)ii * P + kk] -= L[(size_t)ii * P + j] * L[(size_t)kk * P + j];
+        if (s_fail) break;                           // uniform
+        for (int r = t; r < m; r += kCT) {
+            double v[NB];
+#pragma unroll
+            for (int c = 0; c < NB; c++) v[c] = lp[c * LD + r];
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                v[j] *= inv[j];
+#pragma unroll
+                for (int k = j + 1; k < NB; k++) v[k] = fma(-v[j], dg[k][j], v[k]);
+                lp[j * LD + r] = v[j];
+            }
+        }
+        __syncthreads();
+        // the factor's columns, for the back substitution (b's row: y)
+        for (int e = t; e < nb * nb; e += kCT) {
+            const int r = e / nb, c = e % nb;
+            if (c <= r) L[(size_t)(kb + r) * P + kb + c] = c == r ? inv[r] : dg[r][c];   // the diagonal inverted
+        }
+        for (int e = t; e < m * nb; e += kCT) {
+            const int r = e / nb, c = e % nb;
+            if (r < m - 1) L[(size_t)(kb + nb + r) * P + kb + c] = lp[c * LD + r];
+            else y[kb + c] = lp[c * LD + r];
+        }
+        // trailing tiles (ti >= tj) of 16 x 16, one wave each: C -= L21 L21^T.  Lane l holds
+        // A[l % 16][k0 + l / 16], B alike, and D[4 e + l / 16][l % 16] in register e.
+        const int nt = m16 / 16, base = kb + nb;
+        for (int u = w; u < nt * (nt + 1) / 2; u += kCT / 64) {
+            int ti = 0, tj = u;
+            while (tj > ti) { ti++; tj -= ti; }
+            const int col = tj * 16 + (lane & 15);
+            f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+            double c[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int r = ti * 16 + 4 * e + (lane >> 4);
+                c[e] = 0.0;
+                if (col < m - 1) {
+                    if (r < m - 1) c[e] = L[(size_t)(base + r) * P + base + col];
+                    else if (r == m - 1) c[e] = y[base + col];
+                }
+            }
+#pragma unroll
+            for (int k0 = 0; k0 < NB; k0 += 4) {
+                const double av = lp[(k0 + (lane >> 4)) * LD + ti * 16 + (lane & 15)];
+                const double bv = lp[(k0 + (lane >> 4)) * LD + tj * 16 + (lane & 15)];
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc, 0, 0, 0);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int r = ti * 16 + 4 * e + (lane >> 4);
+                if (col < m - 1) {
+                    if (r < m - 1) L[(size_t)(base + r) * P + base + col] = c[e] - acc[e];
+                    else if (r == m - 1) y[base + col] = c[e] - acc[e];
+                }
+            }
         }
         __syncthreads();
     }
-    __syncthreads();
     if (s_fail) {
-        if (threadIdx.x == 0) status[blockIdx.x] = -1;
+        if (t == 0) status[blockIdx.x] = -1;
         return;
     }
-    __shared__ double sx[1024];
-    if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        for (int i = 0; i < P; i++) {
-            double s = 0.0;
-            for (int k = lane; k < i; k += 64) s += L[(size_t)i * P + k] * sx[k];
-            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-            if (lane == 0) sx[i] = (b[i] - s) / L[(size_t)i * P + i];
-            __builtin_amdgcn_s_waitcnt(0);
-            __builtin_amdgcn_wave_barrier();
+    // L^T x = y, blocks from the last: the block by one wave (lane i: unknown i), then its
+    // columns taken out of the unknowns above
+    for (int kb = (P - 1) / NB * NB; kb >= 0; kb -= NB) {
+        const int nb = min(NB, P - kb);
+        if (w == 0) {
+            double row[NB];
+#pragma unroll
+            for (int j = 0; j < NB; j++) row[j] = (j < nb && lane <= j) ? L[(size_t)(kb + j) * P + kb + lane] : 0.0;
+            double v = lane < nb ? y[kb + lane] : 0.0;
+#pragma unroll
+            for (int j = NB - 1; j >= 0; j--) {
+                if (j >= nb) continue;
+                const double xj = readlane_f64(v, j) * readlane_f64(row[j], j);
+                if (lane == j) v = xj;
+                else if (lane < j) v = fma(-row[j], xj, v);
+            }
+            if (lane < nb) {
+                y[kb + lane] = v;
+                x[kb + lane] = v;
+            }
         }
-        for (int i = P - 1; i >= 0; i--) {
-            double s = 0.0;
-            for (int k = i + 1 + lane; k < P; k += 64) s += L[(size_t)k * P + i] * sx[k];
-            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-            if (lane == 0) sx[i] = (sx[i] - s) / L[(size_t)i * P + i];
-            __builtin_amdgcn_s_waitcnt(0);
-            __builtin_amdgcn_wave_barrier();
+        __syncthreads();
+        for (int i = t; i < kb; i += kCT) {
+            double s = y[i];
+#pragma unroll 8
+            for (int j = 0; j < nb; j++) s = fma(-L[(size_t)(kb + j) * P + i], y[kb + j], s);
+            y[i] = s;
         }
-        for (int i = lane; i < P; i += 64) x[i] = sx[i];
-        if (lane == 0) status[blockIdx.x] = 0;
+        __syncthreads();
     }
+    if (t == 0) status[blockIdx.x] = 0;
 }
 
 // ------------------------------------------------------------------- PCG
@@ -914,7 +1032,14 @@ int qgtl_hip_herm_extremes_c128(const void *A, void *W, int P, double *out4) {
 }
 
 int qgtl_hip_cholesky_solve_f64(double *A, const double *b, double *x, int P, int batch, double lambda, int *status) {
-    hipLaunchKernelGGL(cholesky_f64_kernel, dim3(batch), dim3(kT), 0, qgtl::stream(), A, b, x, P, lambda, status);
+    if (P < 1 || P > 1024) return qgtl::set_error_msg(-118, "cholesky: needs 1 <= P <= 1024");
+#define QGTL_CHOL(NB, ROWS)                                                                                       \
+    hipLaunchKernelGGL((cholesky_f64_kernel<NB, ROWS>), dim3(batch), dim3(kCT), 0, qgtl::stream(), A, b, x, P, lambda, \
+                       status)
+    if (P <= 256) QGTL_CHOL(32, 240);                // ROWS >= round16(P - NB + 1)
+    else if (P <= 512) QGTL_CHOL(32, 496);
+    else QGTL_CHOL(16, 1024);
+#undef QGTL_CHOL
     QGTL_LAUNCH_CHECK("cholesky_f64");
     return 0;
 }
