@@ -271,7 +271,9 @@ __global__ __launch_bounds__(kT) void herm_eig_c128_kernel(double2 *Aall, double
 // LDS).  b is carried as one more row, so the forward substitution comes with
 // the factorisation; the back substitution runs block by block on L.  What
 // bounds it: the serial chain of the diagonal blocks (square root, reciprocal
-// and a row of multiply-adds per column).  P = 192: CHOL_NOW, from 1220 us with a
+// and a row of multiply-adds per column), the first of which nothing hides; the
+// others run beside the trailing updates.  P = 192: 140 us (263 us without that
+// overlap and with the panel rows reading the diagonal block by columns), from 1220 us with a
 // rank-1 update of the whole trailing matrix per column in global memory and
 // one reduction over a wave per row of the substitutions.
 //
@@ -282,13 +284,47 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ double readlane_f64(double v, int lane);
 
+// Factor of the diagonal block in dg (by rows; the lower triangle is read) by one
+// wave, a row per lane in registers: dg receives it by columns (dg[j][i] = l_ij,
+// i > j), inv the reciprocals of its diagonal.  Returns nonzero when a pivot is
+// not positive.
+template <int NB>
+__device__ __forceinline__ int factor_diag(double (*dg)[NB + 2], double *inv, int lane) {
+    const int row = lane < NB ? lane : NB - 1;       // lanes past the block repeat its last row
+    double a[NB];
+#pragma unroll
+    for (int c = 0; c < NB; c++) a[c] = dg[row][c];
+    int bad = 0;
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+        const double d = readlane_f64(a[j], j);
+        bad |= !(d > 0.0);
+        // 1 / l_jj from one reciprocal square root and two Newton steps
+        double r = __builtin_amdgcn_rsq(d);
+        if (d < __builtin_inf()) {                   // an infinite pivot keeps its reciprocal, 0
+            r = fma(r * 0.5, fma(-d * r, r, 1.0), r);
+            r = fma(r * 0.5, fma(-d * r, r, 1.0), r);
+        }
+        const double l = a[j] * r;
+        a[j] = l;
+        if (lane == 0) inv[j] = r;
+#pragma unroll
+        for (int k = j + 1; k < NB; k++) a[k] = fma(-l, readlane_f64(l, k), a[k]);
+    }
+    if (lane < NB)
+#pragma unroll
+        for (int c = 0; c < NB; c++) dg[c][lane] = a[c];
+    return bad;
+}
+
 template <int NB, int ROWS>
 __global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const double *ball, double *xall, int P,
                                                           double lambda, int *status) {
     constexpr int LD = ROWS + 1;                     // odd: the transposing writes hit all banks
+    constexpr int kOwn = NB == 32 ? 3 : 1;           // 16 x 16 tiles of a diagonal block
     __shared__ double lp[NB * LD];                   // panel, column c of row i at c * LD + i
-    __shared__ double dg[NB][NB + 1];                // diagonal block, then its factor by rows
-    __shared__ double y[1024], inv[NB];
+    __shared__ __attribute__((aligned(16))) double dgs[2][NB][NB + 2];
+    __shared__ double y[1024], invs[2][NB];
     __shared__ int s_fail;
     double *L = Lall + (size_t)blockIdx.x * P * P;   // holds A on entry (row-major, symmetric)
     const double *b = ball + (size_t)blockIdx.x * P;
@@ -301,50 +337,26 @@ __global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const d
         L[(size_t)i * P + i] += lambda;
     }
     __syncthreads();
-    for (int kb = 0; kb < P; kb += NB) {
+    for (int e = t; e < NB * NB; e += kCT) {
+        const int r = e / NB, c = e % NB;
+        dgs[0][r][c] = (r < P && c <= r) ? L[(size_t)r * P + c] : (r == c ? 1.0 : 0.0);
+    }
+    __syncthreads();
+    if (w == 0 && factor_diag<NB>(dgs[0], invs[0], lane) && lane == 0) s_fail = 1;
+    int cur = 0;
+    for (int kb = 0; kb < P; kb += NB, cur ^= 1) {
+        double (*dg)[NB + 2] = dgs[cur];
+        const double *inv = invs[cur];
         const int nb = min(NB, P - kb);
         const int m = P - kb - nb + 1;               // rows below the block and the row of b
         const int m16 = (m + 15) / 16 * 16;
-        for (int e = t; e < NB * NB; e += kCT) {
-            const int r = e / NB, c = e % NB;
-            dg[r][c] = (r < nb && c <= r) ? L[(size_t)(kb + r) * P + kb + c] : (r == c ? 1.0 : 0.0);
-        }
+#pragma unroll 4
         for (int e = t; e < m16 * NB; e += kCT) {
             const int r = e / NB, c = e % NB;
-            double v = 0.0;
-            if (c < nb) {
-                if (r < m - 1) v = L[(size_t)(kb + nb + r) * P + kb + c];
-                else if (r == m - 1) v = y[kb + c];
-            }
+            const bool in = c < nb && r < m - 1;
+            double v = L[in ? (size_t)(kb + nb + r) * P + kb + c : (size_t)0];
+            if (!in) v = (c < nb && r == m - 1) ? y[kb + c] : 0.0;
             lp[c * LD + r] = v;
-        }
-        __syncthreads();
-        if (w == 0) {
-            const int row = lane < NB ? lane : NB - 1;   // lanes past the block repeat its last row
-            double a[NB];
-#pragma unroll
-            for (int c = 0; c < NB; c++) a[c] = dg[row][c];
-            int bad = 0;
-#pragma unroll
-            for (int j = 0; j < NB; j++) {
-                const double d = readlane_f64(a[j], j);
-                bad |= !(d > 0.0);
-                // l_jj and its reciprocal from one reciprocal square root, two Newton steps
-                double r = __builtin_amdgcn_rsq(d);
-                if (d < __builtin_inf()) {           // an infinite pivot keeps its reciprocal, 0
-                    r = fma(r * 0.5, fma(-d * r, r, 1.0), r);
-                    r = fma(r * 0.5, fma(-d * r, r, 1.0), r);
-                }
-                const double l = a[j] * r;           // lane j: d / sqrt(d)
-                a[j] = l;
-                if (lane == 0) inv[j] = r;
-#pragma unroll
-                for (int k = j + 1; k < NB; k++) a[k] = fma(-l, readlane_f64(l, k), a[k]);
-            }
-            if (lane < NB)
-#pragma unroll
-                for (int c = 0; c < NB; c++) dg[lane][c] = a[c];
-            if (bad && lane == 0) s_fail = 1;
         }
         __syncthreads();
         if (s_fail) break;                           // uniform
@@ -355,26 +367,27 @@ __global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const d
 #pragma unroll
             for (int j = 0; j < NB; j++) {
                 v[j] *= inv[j];
+                if (((j + 1) & 1) && j + 1 < NB) v[j + 1] = fma(-v[j], dg[j][j + 1], v[j + 1]);
 #pragma unroll
-                for (int k = j + 1; k < NB; k++) v[k] = fma(-v[j], dg[k][j], v[k]);
-                lp[j * LD + r] = v[j];
+                for (int k = (j + 2) & ~1; k < NB; k += 2) {
+                    const double2 q = *reinterpret_cast<const double2 *>(&dg[j][k]);
+                    v[k] = fma(-v[j], q.x, v[k]);
+                    v[k + 1] = fma(-v[j], q.y, v[k + 1]);
+                }
+                // a few columns' reads in flight at a time: all of them hoisted would spill
+                if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
             }
+#pragma unroll
+            for (int c = 0; c < NB; c++) lp[c * LD + r] = v[c];
         }
         __syncthreads();
-        // the factor's columns, for the back substitution (b's row: y)
-        for (int e = t; e < nb * nb; e += kCT) {
-            const int r = e / nb, c = e % nb;
-            if (c <= r) L[(size_t)(kb + r) * P + kb + c] = c == r ? inv[r] : dg[r][c];   // the diagonal inverted
-        }
-        for (int e = t; e < m * nb; e += kCT) {
-            const int r = e / nb, c = e % nb;
-            if (r < m - 1) L[(size_t)(kb + nb + r) * P + kb + c] = lp[c * LD + r];
-            else y[kb + c] = lp[c * LD + r];
-        }
         // trailing tiles (ti >= tj) of 16 x 16, one wave each: C -= L21 L21^T.  Lane l holds
-        // A[l % 16][k0 + l / 16], B alike, and D[4 e + l / 16][l % 16] in register e.
+        // A[l % 16][k0 + l / 16], B alike, and D[4 e + l / 16][l % 16] in register e.  Wave 0
+        // takes the tiles of the next diagonal block and factors it while the other waves
+        // update the rest, so its serial chain overlaps their work.
         const int nt = m16 / 16, base = kb + nb;
-        for (int u = w; u < nt * (nt + 1) / 2; u += kCT / 64) {
+        const int nn = min(NB, P - base);            // the next block's size (<= 0: none)
+        auto tile = [&](int u, bool next) {
             int ti = 0, tj = u;
             while (tj > ti) { ti++; tj -= ti; }
             const int col = tj * 16 + (lane & 15);
@@ -383,11 +396,9 @@ __global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const d
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int r = ti * 16 + 4 * e + (lane >> 4);
-                c[e] = 0.0;
-                if (col < m - 1) {
-                    if (r < m - 1) c[e] = L[(size_t)(base + r) * P + base + col];
-                    else if (r == m - 1) c[e] = y[base + col];
-                }
+                const bool in = col < m - 1 && r < m - 1;
+                c[e] = L[in ? (size_t)(base + r) * P + base + col : (size_t)0];
+                if (!in && col < m - 1 && r == m - 1) c[e] = y[base + col];
             }
 #pragma unroll
             for (int k0 = 0; k0 < NB; k0 += 4) {
@@ -398,10 +409,31 @@ __global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const d
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int r = ti * 16 + 4 * e + (lane >> 4);
-                if (col < m - 1) {
-                    if (r < m - 1) L[(size_t)(base + r) * P + base + col] = c[e] - acc[e];
-                    else if (r == m - 1) y[base + col] = c[e] - acc[e];
-                }
+                if (col >= m - 1) continue;
+                if (r == m - 1) y[base + col] = c[e] - acc[e];
+                else if (r < m - 1 && next && col <= r) dgs[cur ^ 1][r][col] = c[e] - acc[e];
+                else if (r < m - 1 && !next) L[(size_t)(base + r) * P + base + col] = c[e] - acc[e];
+            }
+        };
+        if (w == 0) {
+            if (nn > 0) {
+                for (int e = lane; e < NB * NB; e += 64)         // identity past a short last block
+                    if (e / NB >= nn) dgs[cur ^ 1][e / NB][e % NB] = e / NB == e % NB ? 1.0 : 0.0;
+                for (int u = 0; u < kOwn && u < nt * (nt + 1) / 2; u++) tile(u, true);
+                if (factor_diag<NB>(dgs[cur ^ 1], invs[cur ^ 1], lane) && lane == 0) s_fail = 1;
+            }
+        } else {
+            for (int u = kOwn + w - 1; u < nt * (nt + 1) / 2; u += kCT / 64 - 1) tile(u, false);
+            // the factor's columns, for the back substitution (the diagonal inverted; b's row: y)
+            for (int e = t - 64; e < NB * NB; e += kCT - 64) {
+                const int r = e / NB, c = e % NB;
+                if (c <= r && r < nb) L[(size_t)(kb + r) * P + kb + c] = c == r ? inv[r] : dg[c][r];
+            }
+            for (int e = t - 64; e < m * NB; e += kCT - 64) {
+                const int r = e / NB, c = e % NB;
+                if (c >= nb) continue;
+                if (r < m - 1) L[(size_t)(kb + nb + r) * P + kb + c] = lp[c * LD + r];
+                else y[kb + c] = lp[c * LD + r];
             }
         }
         __syncthreads();
@@ -411,18 +443,26 @@ __global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const d
         return;
     }
     // L^T x = y, blocks from the last: the block by one wave (lane i: unknown i), then its
-    // columns taken out of the unknowns above
-    for (int kb = (P - 1) / NB * NB; kb >= 0; kb -= NB) {
-        const int nb = min(NB, P - kb);
-        if (w == 0) {
-            double row[NB];
+    // columns taken out of the unknowns above; the next block's rows are fetched meanwhile
+    double row[NB];
+    auto fetch = [&](int kb) {
 #pragma unroll
-            for (int j = 0; j < NB; j++) row[j] = (j < nb && lane <= j) ? L[(size_t)(kb + j) * P + kb + lane] : 0.0;
+        for (int j = 0; j < NB; j++) {
+            const bool in = kb >= 0 && kb + j < P && lane <= j;
+            row[j] = L[in ? (size_t)(kb + j) * P + kb + lane : (size_t)0];
+            if (!in) row[j] = 0.0;
+        }
+    };
+    const int kl = (P - 1) / NB * NB;
+    if (w == 0) fetch(kl);
+    for (int kb = kl; kb >= 0; kb -= NB) {
+        const int nb = min(NB, P - kb);
+        double lc[NB];
+        if (w == 0) {
             double v = lane < nb ? y[kb + lane] : 0.0;
 #pragma unroll
             for (int j = NB - 1; j >= 0; j--) {
-                if (j >= nb) continue;
-                const double xj = readlane_f64(v, j) * readlane_f64(row[j], j);
+                const double xj = readlane_f64(v, j) * readlane_f64(row[j], j);   // 0 past the block
                 if (lane == j) v = xj;
                 else if (lane < j) v = fma(-row[j], xj, v);
             }
@@ -430,13 +470,25 @@ __global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const d
                 y[kb + lane] = v;
                 x[kb + lane] = v;
             }
+            fetch(kb - NB);
+        } else if (t - 64 < kb) {
+#pragma unroll
+            for (int j = 0; j < NB; j++) lc[j] = L[(size_t)(kb + min(j, nb - 1)) * P + t - 64];
         }
         __syncthreads();
-        for (int i = t; i < kb; i += kCT) {
-            double s = y[i];
-#pragma unroll 8
-            for (int j = 0; j < nb; j++) s = fma(-L[(size_t)(kb + j) * P + i], y[kb + j], s);
-            y[i] = s;
+        if (w != 0) {
+            if (t - 64 < kb) {
+                double s = y[t - 64];
+#pragma unroll
+                for (int j = 0; j < NB; j++) s = fma(-lc[j], j < nb ? y[kb + j] : 0.0, s);
+                y[t - 64] = s;
+            }
+            for (int i = t - 64 + kCT - 64; i < kb; i += kCT - 64) {
+                double s = y[i];
+#pragma unroll 4
+                for (int j = 0; j < nb; j++) s = fma(-L[(size_t)(kb + j) * P + i], y[kb + j], s);
+                y[i] = s;
+            }
         }
         __syncthreads();
     }
