@@ -427,13 +427,26 @@ int qgtl_hip_dotc_c128(const void *D, int P, size_t N, const void *psi, double *
 int qgtl_hip_qgt_finalize_plain(const double *G, const double *a, int P, double *Q);
 
 /* ---- learned preconditioner: dense layers (bf16 MFMA, fp32 accumulate) ---- */
-/* C (M x N fp32) = op(A) op(B) [+ bias] [+ C]; op(A)[m][k] = ta ? A[k][m] : A[m][k] (lda
- * columns), op(B)[k][n] = tb ? B[n][k] : B[k][n] (ldb columns); *_bf16: operand stored as bf16 */
-int qgtl_hip_mlp_gemm(int M, int N, int K, const void *A, int a_bf16, int ta, int lda, const void *B, int b_bf16,
-                      int tb, int ldb, float *C, int ldc, const float *bias, int accumulate);
-int qgtl_hip_gelu_fwd(const float *z, float *a, size_t n);
-int qgtl_hip_gelu_bwd(const float *z, float *da, size_t n);           /* da *= g'(z) */
-int qgtl_hip_colsum(const float *X, int rows, int cols, float *out);
+/* One product of a dense layer, C (M x N fp32, rows of N) from K products per
+ * entry, operands rounded to bf16, fp32 accumulation:
+ *   forward: C[m][n] = sum_k A[m][k] W[k][n] + bias[n], act (if given) = GELU(C)
+ *     (A fp32 rows of lda; W bf16 rows of ldb);
+ *   weight gradient: C[m][n] = sum_k A[k][m] B[k][n], colsum[n] = sum_k B[k][n]
+ *     (A, B fp32 rows of lda, ldb);
+ *   input gradient: C[m][n] = GELU'(pre[m][n]) sum_k A[m][k] W[n][k]
+ *     (A fp32 rows of lda; W bf16 rows of ldb; pre: rows of N).
+ * avec, bvec are set by the launcher. */
+typedef struct {
+    const void *A, *B;
+    float *C;
+    const float *bias, *pre;
+    float *act, *colsum;
+    int32_t M, N, K, lda, ldb;
+    int32_t avec, bvec;
+} qgtl_mlp_product_t;
+int qgtl_hip_mlp_forward(const qgtl_mlp_product_t *desc);
+/* input may be NULL (the first layer) */
+int qgtl_hip_mlp_backward(const qgtl_mlp_product_t *weight, const qgtl_mlp_product_t *input);
 int qgtl_hip_gather_rows(const float *src, const int *idx, int rows, int cols, float *dst);
 int qgtl_hip_adam(float *w, uint16_t *w_bf16, float *m, float *v, const float *g, size_t n, float lr, float b1,
                   float b2, float eps, int step);

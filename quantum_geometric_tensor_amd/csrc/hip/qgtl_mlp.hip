@@ -18,99 +18,244 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kThreads = 256;
-constexpr int kTM = 64, kTN = 64, kTK = 32;
-constexpr int kLdsRow = kTK + 8;                 // bf16 per LDS row: 80 B, 16-B aligned
 
 __device__ __forceinline__ uint16_t bf16_rn(float x) {
     const uint32_t u = __float_as_uint(x);
     return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
 }
 
-__device__ __forceinline__ float load_op(const void *p, int bf16, size_t i) {
-    if (bf16) return __uint_as_float((uint32_t)reinterpret_cast<const uint16_t *>(p)[i] << 16);
-    return reinterpret_cast<const float *>(p)[i];
+// ---- dense layers ----
+// C (M x N, fp32) = op(A) op(B): operands rounded to bf16 when staged into LDS,
+// fp32 accumulation, one 32 x 32 tile per workgroup.  The layers are small (the
+// preconditioner's: 256 x 256 .. 1728 outputs, K = 256 .. 1728), so a product is
+// a few memory latencies long and what counts is how many are in a row: a stage
+// covers 256 of K (64 KB of fp32 in flight per workgroup), its 16-byte loads go
+// out before the previous stage's MFMAs, the four waves take a quarter of the
+// stage's K each and add their accumulators at the end, and the small tiles
+// give 64 .. 432 workgroups.  The activation, its derivative, the bias and the
+// bias gradient (column sums) ride on the products instead of reading and
+// writing the layer again, and a layer's weight gradient and the gradient handed
+// down are one launch.  Loss and gradient at P = 192, rank 8, 256 samples: 21
+// launches of 880 us in all before, 8 of 53 us now; the call 1402 -> 584 us.
+constexpr int kTile = 32, kK = 256;
+constexpr int kLdsRow = kK + 8;                  // bf16 per LDS row: 528 B (16-B aligned, rows 4 banks apart)
+constexpr float kGeluC = 0.7978845608028654f;    // sqrt(2 / pi)
+
+__device__ __forceinline__ float gelu(float x) {
+    return 0.5f * x * (1.f + tanhf(kGeluC * (x + 0.044715f * x * x * x)));
 }
 
-// C (M x N, fp32, row-major) = op(A) op(B) [+ bias] [+ C]:
-//   op(A)[m][k] = ta ? A[k][m] : A[m][k]  (A row-major with lda columns)
-//   op(B)[k][n] = tb ? B[n][k] : B[k][n]
-// Operands are rounded to bf16 when staged into LDS.  One 64 x 64 tile per
-// workgroup, one 32 x 32 MFMA block per wave.
-__global__ __launch_bounds__(kThreads) void gemm_bf16_kernel(int M, int N, int K, const void *__restrict__ A, int a_bf16,
-                                                             int ta, int lda, const void *__restrict__ B, int b_bf16,
-                                                             int tb, int ldb, float *C, int ldc,
-                                                             const float *__restrict__ bias, int accumulate) {
-    __shared__ uint16_t As[kTM * kLdsRow];   // [m][k]
-    __shared__ uint16_t Bs[kTN * kLdsRow];   // [n][k]
-    const int m0 = blockIdx.y * kTM, n0 = blockIdx.x * kTN;
+__device__ __forceinline__ float gelu_grad(float x) {
+    const float t = tanhf(kGeluC * (x + 0.044715f * x * x * x));
+    return 0.5f * (1.f + t) + 0.5f * x * (1.f - t * t) * kGeluC * (1.f + 3.f * 0.044715f * x * x);
+}
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+    const f32x2 v = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+
+// An operand tile: 32 rows (of M or N) x 256 of K.  kContig: a row's K values are
+// adjacent (element (r, k) at r * ld + k); else its rows are (k * ld + r).
+// vec: 16-byte (fp32) or 8-byte (bf16, strided) loads are aligned; without it, and
+// at the edges, elements are read one by one.
+template <bool BF16, bool CONTIG>
+struct Operand;
+
+// n adjacent elements of a row, n = min(COUNT, left) of them real, the rest zero
+template <int COUNT, typename Vec, typename Elem>
+__device__ __forceinline__ Vec load_run(const Elem *q, int left, bool vec) {
+    if (vec && left >= COUNT) return *reinterpret_cast<const Vec *>(q);
+    Vec v;
+#pragma unroll
+    for (int c = 0; c < COUNT; c++) v[c] = c < left ? q[c] : Elem(0);
+    return v;
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+
+template <>
+struct Operand<false, true> {                    // fp32, K adjacent: 8 lanes per row, 8 loads
+    f32x4 v[8];
+    __device__ __forceinline__ void load(const void *p, int ld, int r0, int R, int k0, int K, bool vec) {
+        const int r = r0 + (int)(threadIdx.x >> 3);
+        const float *q = reinterpret_cast<const float *>(p) + (size_t)(r < R ? r : 0) * ld;
+        const int lim = r < R ? K : 0;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int k = k0 + 4 * (int)(threadIdx.x & 7) + 32 * i;
+            v[i] = load_run<4, f32x4>(q + k, lim - k, vec);
+        }
+    }
+    __device__ __forceinline__ void store(uint16_t *lds) const {
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            *reinterpret_cast<uint2 *>(lds + (threadIdx.x >> 3) * kLdsRow + 4 * (threadIdx.x & 7) + 32 * i) =
+                make_uint2(pack_bf16(v[i][0], v[i][1]), pack_bf16(v[i][2], v[i][3]));
+    }
+};
+
+template <>
+struct Operand<false, false> {                   // fp32, rows adjacent: 4 rows x 2 of K per thread, 4 times
+    f32x4 v[8];
+    __device__ __forceinline__ void load(const void *p, int ld, int r0, int R, int k0, int K, bool vec) {
+        const int r = r0 + 4 * (int)(threadIdx.x & 7);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int k = k0 + 2 * (int)(threadIdx.x >> 3) + 64 * (i >> 1) + (i & 1);
+            const float *q = reinterpret_cast<const float *>(p) + (size_t)(k < K ? k : 0) * ld + r;
+            v[i] = load_run<4, f32x4>(q, k < K ? R - r : 0, vec);
+        }
+    }
+    __device__ __forceinline__ void store(uint16_t *lds) const {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                *reinterpret_cast<uint32_t *>(lds + (4 * (threadIdx.x & 7) + c) * kLdsRow + 2 * (threadIdx.x >> 3) +
+                                              64 * i) = pack_bf16(v[2 * i][c], v[2 * i + 1][c]);
+    }
+};
+
+template <>
+struct Operand<true, true> {                     // bf16, K adjacent
+    u16x8 v[4];
+    __device__ __forceinline__ void load(const void *p, int ld, int r0, int R, int k0, int K, bool vec) {
+        const int r = r0 + (int)(threadIdx.x >> 3);
+        const uint16_t *q = reinterpret_cast<const uint16_t *>(p) + (size_t)(r < R ? r : 0) * ld;
+        const int lim = r < R ? K : 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int k = k0 + 8 * (int)(threadIdx.x & 7) + 64 * i;
+            v[i] = load_run<8, u16x8>(q + k, lim - k, vec);
+        }
+    }
+    __device__ __forceinline__ void store(uint16_t *lds) const {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            *reinterpret_cast<u16x8 *>(lds + (threadIdx.x >> 3) * kLdsRow + 8 * (threadIdx.x & 7) + 64 * i) = v[i];
+    }
+};
+
+template <>
+struct Operand<true, false> {                    // bf16, rows adjacent
+    u16x4 v[8];
+    __device__ __forceinline__ void load(const void *p, int ld, int r0, int R, int k0, int K, bool vec) {
+        const int r = r0 + 4 * (int)(threadIdx.x & 7);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int k = k0 + 2 * (int)(threadIdx.x >> 3) + 64 * (i >> 1) + (i & 1);
+            const uint16_t *q = reinterpret_cast<const uint16_t *>(p) + (size_t)(k < K ? k : 0) * ld + r;
+            v[i] = load_run<4, u16x4>(q, k < K ? R - r : 0, vec);
+        }
+    }
+    __device__ __forceinline__ void store(uint16_t *lds) const {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                *reinterpret_cast<uint32_t *>(lds + (4 * (threadIdx.x & 7) + c) * kLdsRow + 2 * (threadIdx.x >> 3) +
+                                              64 * i) = (uint32_t)v[2 * i][c] | ((uint32_t)v[2 * i + 1][c] << 16);
+    }
+};
+
+struct Lds {
+    uint16_t a[kTile * kLdsRow], b[kTile * kLdsRow];
+};
+
+enum { kForward, kWeightGrad, kInputGrad };      // what a product is (see qgtl_mlp_product_t)
+
+template <int KIND>
+__device__ __forceinline__ void product(const qgtl_mlp_product_t &g, int tile, Lds &sm) {
+    constexpr bool A_CONTIG = KIND != kWeightGrad, B_BF16 = KIND != kWeightGrad, B_CONTIG = KIND == kInputGrad;
+    const int tn = (g.N + kTile - 1) / kTile;
+    const int m0 = tile / tn * kTile, n0 = tile % tn * kTile;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
     f32x16 acc;
 #pragma unroll
     for (int e = 0; e < 16; e++) acc[e] = 0.f;
+    f32x4 cs = {0.f, 0.f, 0.f, 0.f};               // weight gradient: column sums of B (the bias gradient)
+    const bool sums = KIND == kWeightGrad && m0 == 0;
 
-    for (int k0 = 0; k0 < K; k0 += kTK) {
-        for (int i = threadIdx.x; i < kTM * kTK; i += kThreads) {
-            const int mm = i / kTK, kk = i % kTK;
-            const int m = m0 + mm, k = k0 + kk;
-            float v = 0.f;
-            if (m < M && k < K) v = load_op(A, a_bf16, ta ? (size_t)k * lda + m : (size_t)m * lda + k);
-            As[mm * kLdsRow + kk] = bf16_rn(v);
-            const int nn = i / kTK;
-            const int n = n0 + nn;
-            float w = 0.f;
-            if (n < N && k < K) w = load_op(B, b_bf16, tb ? (size_t)n * ldb + k : (size_t)k * ldb + n);
-            Bs[nn * kLdsRow + kk] = bf16_rn(w);
+    Operand<false, A_CONTIG> oa;
+    Operand<B_BF16, B_CONTIG> ob;
+    oa.load(g.A, g.lda, m0, g.M, 0, g.K, g.avec);
+    ob.load(g.B, g.ldb, n0, g.N, 0, g.K, g.bvec);
+    for (int k0 = 0; k0 < g.K; k0 += kK) {
+        oa.store(sm.a);
+        ob.store(sm.b);
+        if constexpr (KIND == kWeightGrad) {
+            if (sums)
+#pragma unroll
+                for (int i = 0; i < 8; i++) cs += ob.v[i];
         }
         __syncthreads();
+        if (k0 + kK < g.K) {
+            oa.load(g.A, g.lda, m0, g.M, k0 + kK, g.K, g.avec);
+            ob.load(g.B, g.ldb, n0, g.N, k0 + kK, g.K, g.bvec);
+        }
 #pragma unroll
-        for (int kk = 0; kk < kTK; kk += 16) {
-            const int koff = kk + 8 * (lane >> 5);
-            const bf16x8 fa = *reinterpret_cast<const bf16x8 *>(&As[(wm * 32 + (lane & 31)) * kLdsRow + koff]);
-            const bf16x8 fb = *reinterpret_cast<const bf16x8 *>(&Bs[(wn * 32 + (lane & 31)) * kLdsRow + koff]);
+        for (int s = 0; s < 4; s++) {
+            const int koff = 64 * wave + 16 * s + 8 * (lane >> 5);
+            const bf16x8 fa = *reinterpret_cast<const bf16x8 *>(&sm.a[(lane & 31) * kLdsRow + koff]);
+            const bf16x8 fb = *reinterpret_cast<const bf16x8 *>(&sm.b[(lane & 31) * kLdsRow + koff]);
             acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa, fb, acc, 0, 0, 0);
         }
         __syncthreads();
     }
+    // the four waves' accumulators, added in wave order; wave w finishes elements 4 w .. 4 w + 3
+    float *red = reinterpret_cast<float *>(sm.a);                // 4 x 16 x 64 floats (16 KB of the 16.5 KB tile)
+    static_assert(sizeof(sm.a) >= 4 * 16 * 64 * sizeof(float), "accumulators fit the A tile");
 #pragma unroll
-    for (int e = 0; e < 16; e++) {
-        const int row = m0 + wm * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-        const int col = n0 + wn * 32 + (lane & 31);
-        if (row < M && col < N) {
-            float v = acc[e];
-            if (bias) v += bias[col];
-            float *c = C + (size_t)row * ldc + col;
-            *c = accumulate ? *c + v : v;
+    for (int e = 0; e < 16; e++) red[(wave * 16 + e) * 64 + lane] = acc[e];
+    f32x4 *cred = reinterpret_cast<f32x4 *>(sm.b);               // 32 x 8
+    if (sums) cred[threadIdx.x] = cs;
+    __syncthreads();
+    const int col = n0 + (lane & 31);
+#pragma unroll
+    for (int e2 = 0; e2 < 4; e2++) {
+        const int e = 4 * wave + e2;
+        float v = red[e * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < 4; w++) v += red[(w * 16 + e) * 64 + lane];
+        const int row = m0 + wave * 8 + (lane >> 5) * 4 + e2;
+        if (row >= g.M || col >= g.N) continue;
+        const size_t at = (size_t)row * g.N + col;
+        if constexpr (KIND == kForward) {
+            v += g.bias[col];
+            if (g.act) g.act[at] = gelu(v);
         }
+        if constexpr (KIND == kInputGrad) v *= gelu_grad(g.pre[at]);
+        g.C[at] = v;
+    }
+    if (sums && threadIdx.x < 32) {
+        const int n = n0 + (int)threadIdx.x;
+        const float *c = reinterpret_cast<const float *>(cred) + threadIdx.x;   // (thread kp * 8 + n / 4, n % 4)
+        float v = 0.f;
+        for (int kp = 0; kp < 32; kp++) v += c[kp * 32];
+        if (n < g.N) g.colsum[n] = v;
     }
 }
 
-constexpr float kGeluC = 0.7978845608028654f;   // sqrt(2 / pi)
-
-__global__ void gelu_fwd_kernel(const float *__restrict__ z, float *a, size_t n) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const float x = z[i];
-        a[i] = 0.5f * x * (1.f + tanhf(kGeluC * (x + 0.044715f * x * x * x)));
-    }
+__device__ __forceinline__ int product_tiles(const qgtl_mlp_product_t &g) {
+    return ((g.M + kTile - 1) / kTile) * ((g.N + kTile - 1) / kTile);
 }
 
-// dz = da * g'(z), in place on da
-__global__ void gelu_bwd_kernel(const float *__restrict__ z, float *da, size_t n) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const float x = z[i];
-        const float t = tanhf(kGeluC * (x + 0.044715f * x * x * x));
-        const float g = 0.5f * (1.f + t) + 0.5f * x * (1.f - t * t) * kGeluC * (1.f + 3.f * 0.044715f * x * x);
-        da[i] *= g;
-    }
+__global__ __launch_bounds__(kThreads) void mlp_forward_kernel(const qgtl_mlp_product_t g) {
+    __shared__ __attribute__((aligned(16))) Lds sm;
+    product<kForward>(g, blockIdx.x, sm);
 }
 
-// out[j] = sum_i X[i][j] (rows in a fixed order)
-__global__ void colsum_kernel(const float *__restrict__ X, int rows, int cols, float *out) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= cols) return;
-    float s = 0.f;
-    for (int i = 0; i < rows; i++) s += X[(size_t)i * cols + j];
-    out[j] = s;
+// a layer's weight gradient w (its tiles first) and, in the same launch, the gradient x of its input
+__global__ __launch_bounds__(kThreads) void mlp_backward_kernel(const qgtl_mlp_product_t w, const qgtl_mlp_product_t x) {
+    __shared__ __attribute__((aligned(16))) Lds sm;
+    const int tw = product_tiles(w);
+    if ((int)blockIdx.x < tw) product<kWeightGrad>(w, blockIdx.x, sm);
+    else product<kInputGrad>(x, (int)blockIdx.x - tw, sm);
 }
 
 __global__ void gather_rows_kernel(const float *__restrict__ src, const int *__restrict__ idx, int rows, int cols,
@@ -296,32 +441,44 @@ unsigned grid_1d(size_t n) {
 
 extern "C" {
 
-int qgtl_hip_mlp_gemm(int M, int N, int K, const void *A, int a_bf16, int ta, int lda, const void *B, int b_bf16,
-                      int tb, int ldb, float *C, int ldc, const float *bias, int accumulate) {
-    if (M < 1 || N < 1 || K < 1) return qgtl::set_error_msg(-118, "mlp_gemm: empty shape");
-    const dim3 grid((unsigned)((N + kTN - 1) / kTN), (unsigned)((M + kTM - 1) / kTM));
-    hipLaunchKernelGGL(gemm_bf16_kernel, grid, dim3(kThreads), 0, qgtl::stream(), M, N, K, A, a_bf16, ta, lda, B,
-                       b_bf16, tb, ldb, C, ldc, bias, accumulate);
-    QGTL_LAUNCH_CHECK("mlp_gemm");
+static int product_ok(const qgtl_mlp_product_t *g) {
+    return g && g->M >= 1 && g->N >= 1 && g->K >= 1 && g->A && g->B && g->C;
+}
+
+static unsigned product_grid(const qgtl_mlp_product_t *g) {
+    return (unsigned)(((g->M + kTile - 1) / kTile) * ((g->N + kTile - 1) / kTile));
+}
+
+// whether the operand's vector loads (size bytes of a row start, every elems-th element) are aligned
+static int vec_ok(const void *p, int ld, int bytes_per_elem, int bytes) {
+    return (uintptr_t)p % (uintptr_t)bytes == 0 && ((size_t)ld * bytes_per_elem) % (size_t)bytes == 0;
+}
+
+int qgtl_hip_mlp_forward(const qgtl_mlp_product_t *desc) {
+    if (!product_ok(desc) || !desc->bias) return qgtl::set_error_msg(-118, "mlp_forward: empty product");
+    qgtl_mlp_product_t g = *desc;
+    g.avec = vec_ok(g.A, g.lda, 4, 16);
+    g.bvec = vec_ok(g.B, g.ldb, 2, 8);
+    hipLaunchKernelGGL(mlp_forward_kernel, dim3(product_grid(&g)), dim3(kThreads), 0, qgtl::stream(), g);
+    QGTL_LAUNCH_CHECK("mlp_forward");
     return 0;
 }
 
-int qgtl_hip_gelu_fwd(const float *z, float *a, size_t n) {
-    hipLaunchKernelGGL(gelu_fwd_kernel, dim3(grid_1d(n)), dim3(256), 0, qgtl::stream(), z, a, n);
-    QGTL_LAUNCH_CHECK("gelu_fwd");
-    return 0;
-}
-
-int qgtl_hip_gelu_bwd(const float *z, float *da, size_t n) {
-    hipLaunchKernelGGL(gelu_bwd_kernel, dim3(grid_1d(n)), dim3(256), 0, qgtl::stream(), z, da, n);
-    QGTL_LAUNCH_CHECK("gelu_bwd");
-    return 0;
-}
-
-int qgtl_hip_colsum(const float *X, int rows, int cols, float *out) {
-    hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, qgtl::stream(), X, rows,
-                       cols, out);
-    QGTL_LAUNCH_CHECK("colsum");
+int qgtl_hip_mlp_backward(const qgtl_mlp_product_t *weight, const qgtl_mlp_product_t *input) {
+    if (!product_ok(weight) || !weight->colsum || (input && (!product_ok(input) || !input->pre)))
+        return qgtl::set_error_msg(-118, "mlp_backward: empty product");
+    qgtl_mlp_product_t w = *weight, x;
+    w.avec = vec_ok(w.A, w.lda, 4, 16);
+    w.bvec = vec_ok(w.B, w.ldb, 4, 16);
+    x = input ? *input : w;
+    unsigned grid = product_grid(&w);
+    if (input) {
+        x.avec = vec_ok(x.A, x.lda, 4, 16);
+        x.bvec = vec_ok(x.B, x.ldb, 2, 16);
+        grid += product_grid(&x);
+    }
+    hipLaunchKernelGGL(mlp_backward_kernel, dim3(grid), dim3(kThreads), 0, qgtl::stream(), w, x);
+    QGTL_LAUNCH_CHECK("mlp_backward");
     return 0;
 }
 

@@ -47,7 +47,7 @@ struct qgtl_mlp {
     float *x;                            /* cap x F */
     float *pre[MLP_MAX_LAYERS + 1];      /* cap x out_i */
     float *act[MLP_MAX_LAYERS + 1];
-    float *dact[MLP_MAX_LAYERS + 1];     /* gradient w.r.t. act (reused as dz) */
+    float *dact[MLP_MAX_LAYERS + 1];     /* gradient w.r.t. pre */
     double *loss;                        /* cap */
     int *idx;                            /* cap */
     /* training data on the device */
@@ -215,9 +215,9 @@ static int forward_dev(struct qgtl_mlp *m, int B)
     for (int i = 0; i <= m->nh; i++) {
         const uint16_t *W = m->wb + m->off[i];
         const float *b = m->w + m->off[i] + (size_t)m->in[i] * m->out[i];
-        MTRY(qgtl_hip_mlp_gemm(B, m->out[i], m->in[i], in, 0, 0, m->in[i], W, 1, 0, m->out[i], m->pre[i],
-                               m->out[i], b, 0));
-        if (i < m->nh) MTRY(qgtl_hip_gelu_fwd(m->pre[i], m->act[i], (size_t)B * m->out[i]));
+        const qgtl_mlp_product_t g = {.A = in, .B = W, .C = m->pre[i], .bias = b, .act = i < m->nh ? m->act[i] : NULL,
+                                      .M = B, .N = m->out[i], .K = m->in[i], .lda = m->in[i], .ldb = m->out[i]};
+        MTRY(qgtl_hip_mlp_forward(&g));
         in = (i < m->nh) ? m->act[i] : m->pre[i];
     }
     return 0;
@@ -240,16 +240,17 @@ static int loss_grad_dev(struct qgtl_mlp *m, int B, const int *idx, double *loss
     /* output layer is linear: y = pre[L]; dact[L] = dL/dy / B */
     MTRY(qgtl_hip_kaporin(m->P, m->r, B, m->pre[L], m->As_all, m->idx, m->loss, m->dact[L], 1.0f / (float)B));
     for (int i = L; i >= 0; i--) {
-        float *dz = m->dact[i];
-        if (i < L) MTRY(qgtl_hip_gelu_bwd(m->pre[i], dz, (size_t)B * m->out[i]));
+        const float *dz = m->dact[i];          /* dL/dpre_i: dact[i] times GELU' where it was formed */
         const float *in = (i == 0) ? m->x : m->act[i - 1];
         float *gW = m->g + m->off[i], *gb = gW + (size_t)m->in[i] * m->out[i];
-        /* gW (in x out) = in^T (in x B) dz (B x out) */
-        MTRY(qgtl_hip_mlp_gemm(m->in[i], m->out[i], B, in, 0, 1, m->in[i], dz, 0, 0, m->out[i], gW, m->out[i], NULL, 0));
-        MTRY(qgtl_hip_colsum(dz, B, m->out[i], gb));
-        if (i > 0)   /* dact[i-1] (B x in) = dz (B x out) W^T */
-            MTRY(qgtl_hip_mlp_gemm(B, m->in[i], m->out[i], dz, 0, 0, m->out[i], m->wb + m->off[i], 1, 1, m->out[i],
-                                   m->dact[i - 1], m->in[i], NULL, 0));
+        /* gW (in x out) = in^T (in x B) dz (B x out), gb its column sums */
+        const qgtl_mlp_product_t w = {.A = in, .B = dz, .C = gW, .colsum = gb, .M = m->in[i], .N = m->out[i], .K = B,
+                                      .lda = m->in[i], .ldb = m->out[i]};
+        /* dz of the layer below (B x in) = dz (B x out) W^T, times GELU' */
+        const qgtl_mlp_product_t x = {.A = dz, .B = m->wb + m->off[i], .C = i > 0 ? m->dact[i - 1] : NULL,
+                                      .pre = i > 0 ? m->pre[i - 1] : NULL, .M = B, .N = m->in[i], .K = m->out[i],
+                                      .lda = m->out[i], .ldb = m->out[i]};
+        MTRY(qgtl_hip_mlp_backward(&w, i > 0 ? &x : NULL));
     }
     if (loss_mean) {
         double *h = (double *)malloc(sizeof(double) * (size_t)B);
