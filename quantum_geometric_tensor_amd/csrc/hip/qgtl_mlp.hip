@@ -291,6 +291,8 @@ constexpr int kMaxRank = 32;
 constexpr int kMaxP = 1024;
 constexpr int kMaxPR = 8192;    // P * r: the low-rank factor held in LDS as the network's fp32 outputs (32 KB)
 
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
 __device__ double block_sum(double v, double *red) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -302,131 +304,199 @@ __device__ double block_sum(double v, double *red) {
     return s;
 }
 
-// Columns jb .. jb + 7 of the low-rank factor are handled together, in registers (compile-time indices).
-constexpr int kJB = 8;
-
-// (A_s u)_k,j for row k and the column block j = jb + i, i < kJB (zero past r), FP64; u_lj = yu[l r + j] / sqrt(P)
-__device__ __forceinline__ void row_times_u(const float *__restrict__ As, const float *yu, int P, int r, int k, int jb,
-                                            double us, double (&acc)[kJB]) {
-#pragma unroll
-    for (int i = 0; i < kJB; i++) acc[i] = 0.0;
-    for (int l = 0; l < P; l++) {
-        const double a = As[(size_t)k * P + l];
-#pragma unroll
-        for (int i = 0; i < kJB; i++)
-            if (jb + i < r) acc[i] += a * ((double)yu[l * r + jb + i] * us);
-    }
-}
-
-// (u W^-1)_k,j for the same column block
-__device__ __forceinline__ void row_times_winv(const float *yu, const double *Wi, int r, int k, int jb, double us,
-                                               double (&uw)[kJB]) {
-#pragma unroll
-    for (int i = 0; i < kJB; i++) uw[i] = 0.0;
-    for (int a = 0; a < r; a++) {
-        const double ua = (double)yu[k * r + a] * us;
-#pragma unroll
-        for (int i = 0; i < kJB; i++)
-            if (jb + i < r) uw[i] += ua * Wi[a * r + jb + i];
-    }
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
 // Kaporin loss of sample b and dL/dy (scaled by `scale`), FP64.
 //   s_k = y[k(1+r)], u_kj = y[k(1+r)+1+j] / sqrt(P), Mt = diag(e^s) + u u^T,
 //   L = P log(tr(Mt As)/P) - sum s - log det(I + u^T e^-s u).
-// The low-rank outputs stay fp32 in LDS (each use scales them by 1/sqrt(P) in FP64, the value an FP64 copy
-// of u would hold).  A_s u is formed twice, for the trace and again for the gradient, eight columns at a
-// time in registers, rather than held (P r doubles do not fit beside u at rank 32).
+//
+// One workgroup per sample.  A_s u, the bulk of the work, and the r x r matrix
+// W = I + u^T e^-s u run on v_mfma_f64_16x16x4_f64 (A_s read once, a float4 per
+// lane, exact in FP64; u scaled by 1/sqrt(P) in FP64 as it is read from LDS),
+// A_s u kept in LDS for the trace and the gradient; W is factored by one wave
+// (a row per lane) and inverted a column per lane.  What bounds it: the latency
+// of the sample's serial steps (W's factor) and of reading A_s.  P = 192, r = 8,
+// 256 samples: 42 us, from 278 us with a row of A_s per thread (uncoalesced),
+// twice, an exponential per term of W and one thread factoring and inverting it.
+//
+// RT: 16-column tiles of the rank (1: r <= 16, 2: r <= 32); PR: bound on P r.
+template <int RT, int PR>
 __global__ __launch_bounds__(kThreads) void kaporin_kernel(int P, int r, const float *__restrict__ Y,
                                                            const float *__restrict__ As_all, const int *__restrict__ idx,
-                                                           double *loss, float *dY, float scale) {
+                                                           double *loss, float *dY, float scale, int vec) {
+    constexpr int R = 16 * RT, MP = RT == 1 ? kMaxP : 512;   // r > 16: P <= 8192 / 17
     const int b = blockIdx.x;
     const float *y = Y + (size_t)b * P * (1 + r);
     const float *As = As_all + (size_t)idx[b] * P * P;
     float *dy = dY + (size_t)b * P * (1 + r);
-    __shared__ float yu[kMaxPR];
-    __shared__ double W[kMaxRank * kMaxRank], Wi[kMaxRank * kMaxRank];
+    __shared__ float yu[PR];                      // u sqrt(P), row k at k * r
+    __shared__ double au[PR];                     // A_s u, likewise
+    __shared__ double es[MP], ems[MP];            // e^s, e^-s
+    __shared__ double inv[R];                     // reciprocal diagonal of W's factor
+    __shared__ double W[R * (R + 1)], Wi[R * (R + 1)], part[4][RT * RT][256];
     __shared__ double red[kThreads / 64];
     __shared__ double sh_logdet;
     const double us = 1.0 / sqrt((double)P);
     const int st = 1 + r;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int l16 = lane & 15, q4 = lane >> 4;
     for (int e = threadIdx.x; e < P * r; e += kThreads) yu[e] = y[(size_t)(e / r) * st + 1 + e % r];
-    __syncthreads();
     double trp = 0.0, ssum = 0.0;
     for (int k = threadIdx.x; k < P; k += kThreads) {
-        const double s = y[(size_t)k * st];
+        const double s = y[(size_t)k * st], ek = exp(s);
+        es[k] = ek;
+        ems[k] = exp(-s);
         ssum += s;
-        trp += exp(s) * (double)As[(size_t)k * P + k];
-        for (int jb = 0; jb < r; jb += kJB) {
-            double acc[kJB];
-            row_times_u(As, yu, P, r, k, jb, us, acc);
-#pragma unroll
-            for (int i = 0; i < kJB; i++)
-                if (jb + i < r) trp += ((double)yu[k * r + jb + i] * us) * acc[i];
-        }
-    }
-    const double tr = block_sum(trp, red);
-    const double S = block_sum(ssum, red);
-    for (int e = threadIdx.x; e < r * r; e += kThreads) {
-        const int a = e / r, c = e % r;
-        double v = (a == c) ? 1.0 : 0.0;
-        for (int k = 0; k < P; k++)
-            v += exp(-(double)y[(size_t)k * st]) * ((double)yu[k * r + a] * us) * ((double)yu[k * r + c] * us);
-        W[e] = v;
+        trp += ek * (double)As[(size_t)k * P + k];
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double ld = 0.0;
-        for (int j = 0; j < r; j++) {   // Cholesky, lower, in place
-            double d = W[j * r + j];
-            for (int k = 0; k < j; k++) d -= W[j * r + k] * W[j * r + k];
-            d = sqrt(d);
-            W[j * r + j] = d;
-            ld += 2.0 * log(d);
-            for (int i = j + 1; i < r; i++) {
-                double v = W[i * r + j];
-                for (int k = 0; k < j; k++) v -= W[i * r + k] * W[j * r + k];
-                W[i * r + j] = v / d;
-            }
+    auto u_at = [&](int k, int j) -> double { return k < P && j < r ? (double)yu[k * r + j] * us : 0.0; };
+    // A_s u: 16 rows a wave.  Lane l takes A_s[row l % 16][k .. k + 3], k = k0 + 4 (l / 16); product e
+    // of a group of four sums over k0 + e, k0 + 4 + e, k0 + 8 + e, k0 + 12 + e, A and B alike.
+    for (int r0 = 16 * wave; r0 < P && r > 0; r0 += 16 * (kThreads / 64)) {
+        f64x4 acc[RT];
+#pragma unroll
+        for (int c = 0; c < RT; c++) acc[c] = f64x4{0.0, 0.0, 0.0, 0.0};
+        const bool row_ok = r0 + l16 < P;
+        const float *row = As + (size_t)(row_ok ? r0 + l16 : 0) * P;
+        const int lim = row_ok ? P : 0;
+        f32x4 a = load_run<4, f32x4>(row + 4 * q4, lim - 4 * q4, vec);
+        for (int k0 = 0; k0 < P; k0 += 16) {
+            const int kn = k0 + 16 + 4 * q4;
+            const f32x4 an = load_run<4, f32x4>(row + kn, lim - kn, vec);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int c = 0; c < RT; c++)
+                    acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[e], u_at(k0 + 4 * q4 + e, 16 * c + l16), acc[c], 0, 0, 0);
+            a = an;
         }
-        for (int c = 0; c < r; c++) {    // W^-1 column c (symmetric, stored as row c)
-            double *x = Wi + c * r;
-            for (int i = 0; i < r; i++) {
-                double v = (i == c) ? 1.0 : 0.0;
-                for (int k = 0; k < i; k++) v -= W[i * r + k] * x[k];
-                x[i] = v / W[i * r + i];
+#pragma unroll
+        for (int c = 0; c < RT; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int k = r0 + 4 * e + q4, j = 16 * c + l16;
+                if (k < P && j < r) au[k * r + j] = acc[c][e];
             }
-            for (int i = r - 1; i >= 0; i--) {
-                double v = x[i];
-                for (int k = i + 1; k < r; k++) v -= W[k * r + i] * x[k];
-                x[i] = v / W[i * r + i];
-            }
-        }
-        sh_logdet = ld;
     }
+    // W - I: each wave a quarter of the rows
+    if (r > 0) {
+        f64x4 acc[RT * RT];
+#pragma unroll
+        for (int c = 0; c < RT * RT; c++) acc[c] = f64x4{0.0, 0.0, 0.0, 0.0};
+        for (int k0 = 4 * wave; k0 < P; k0 += 4 * (kThreads / 64)) {
+            const int k = k0 + q4;
+            double uj[RT];
+#pragma unroll
+            for (int c = 0; c < RT; c++) uj[c] = u_at(k, 16 * c + l16);
+            const double ek = k < P ? ems[k] : 0.0;
+#pragma unroll
+            for (int c = 0; c < RT; c++)
+#pragma unroll
+                for (int d = 0; d < RT; d++)
+                    acc[c * RT + d] = __builtin_amdgcn_mfma_f64_16x16x4f64(ek * uj[c], uj[d], acc[c * RT + d], 0, 0, 0);
+        }
+#pragma unroll
+        for (int c = 0; c < RT * RT; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) part[wave][c][(4 * e + q4) * 16 + l16] = acc[c][e];
+    }
+    __syncthreads();
+    if (r > 0) {
+        for (int e = threadIdx.x; e < P * r; e += kThreads) trp += ((double)yu[e] * us) * au[e];
+        for (int e = threadIdx.x; e < R * R; e += kThreads) {
+            const int i = e / R, j = e % R, c = (i / 16) * RT + j / 16, o = (i % 16) * 16 + j % 16;
+            const double v = ((part[0][c][o] + part[1][c][o]) + part[2][c][o]) + part[3][c][o];
+            W[i * (R + 1) + j] = v + (i == j ? 1.0 : 0.0);     // past r: the identity
+        }
+    }
+    const double tr = block_sum(trp, red);                     // (barriers: W is complete after them)
+    const double S = block_sum(ssum, red);
+    if (wave == 0 && r > 0) {
+        // Cholesky of W, a row per lane; then W^-1, a column per lane
+        const int row = lane < R ? lane : R - 1;
+        double ld = 0.0;
+        {
+            double a[R];
+#pragma unroll
+            for (int c = 0; c < R; c++) a[c] = W[row * (R + 1) + c];
+#pragma unroll
+            for (int j = 0; j < R; j++) {
+                const double d = lane_value(a[j], j);
+                if (lane == j) ld = log(d);
+                const double ri = 1.0 / sqrt(d);
+                if (lane == 0) inv[j] = ri;
+                const double l = a[j] * ri;
+                a[j] = l;
+#pragma unroll
+                for (int k = j + 1; k < R; k++) a[k] = fma(-l, lane_value(l, k), a[k]);
+            }
+            if (lane < R)
+#pragma unroll
+                for (int c = 0; c < R; c++) W[lane * (R + 1) + c] = a[c];
+        }
+        ld = lane < R ? ld : 0.0;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) ld += __shfl_xor(ld, o, 64);
+        if (lane == 0) sh_logdet = ld;
+        __builtin_amdgcn_wave_barrier();
+        if constexpr (RT == 1) {
+            double x[R];
+#pragma unroll
+            for (int i = 0; i < R; i++) {
+                double v = i == row ? 1.0 : 0.0;
+#pragma unroll
+                for (int k = 0; k < i; k++) v = fma(-W[i * (R + 1) + k], x[k], v);
+                x[i] = v * inv[i];
+            }
+            // the same elements of W, read again: kept from above they would spill
+            __asm__ volatile("" ::: "memory");
+#pragma unroll
+            for (int i = R - 1; i >= 0; i--) {
+                double v = x[i];
+#pragma unroll
+                for (int k = i + 1; k < R; k++) v = fma(-W[k * (R + 1) + i], x[k], v);
+                x[i] = v * inv[i];
+            }
+            if (lane < R)
+#pragma unroll
+                for (int i = 0; i < R; i++) Wi[lane * (R + 1) + i] = x[i];
+        } else {
+            // 32 unknowns and their rows do not fit the registers: the column lives in LDS
+            double *x = Wi + row * (R + 1);
+            for (int i = 0; i < R; i++) {
+                double v = i == row ? 1.0 : 0.0;
+#pragma unroll 4
+                for (int k = 0; k < i; k++) v = fma(-W[i * (R + 1) + k], x[k], v);
+                x[i] = v * inv[i];
+            }
+            for (int i = R - 1; i >= 0; i--) {
+                double v = x[i];
+#pragma unroll 4
+                for (int k = i + 1; k < R; k++) v = fma(-W[k * (R + 1) + i], x[k], v);
+                x[i] = v * inv[i];
+            }
+        }
+    }
+    if (threadIdx.x == 0 && r == 0) sh_logdet = 0.0;
     __syncthreads();
     if (threadIdx.x == 0) loss[b] = (double)P * log(tr / P) - S - sh_logdet;
     const double g = (double)P / tr;
     for (int k = threadIdx.x; k < P; k += kThreads) {
-        const double s = y[(size_t)k * st], ems = exp(-s);
         double q = 0.0;
-        for (int jb = 0; jb < r; jb += kJB) {
-            double uw[kJB];
-            row_times_winv(yu, Wi, r, k, jb, us, uw);
-#pragma unroll
-            for (int i = 0; i < kJB; i++)
-                if (jb + i < r) q += uw[i] * ((double)yu[k * r + jb + i] * us);
+        for (int j = 0; j < r; j++) {
+            double uw = 0.0;                                   // (u W^-1)_kj
+            for (int c = 0; c < r; c++) uw += ((double)yu[k * r + c] * us) * Wi[c * (R + 1) + j];
+            q += uw * ((double)yu[k * r + j] * us);
+            dy[(size_t)k * st + 1 + j] = (float)(scale * (2.0 * g * au[k * r + j] - 2.0 * ems[k] * uw) * us);
         }
-        dy[(size_t)k * st] = (float)(scale * (g * exp(s) * (double)As[(size_t)k * P + k] - 1.0 + ems * q));
-        for (int jb = 0; jb < r; jb += kJB) {
-            double acc[kJB], uw[kJB];
-            row_times_u(As, yu, P, r, k, jb, us, acc);
-            row_times_winv(yu, Wi, r, k, jb, us, uw);
-#pragma unroll
-            for (int i = 0; i < kJB; i++)
-                if (jb + i < r)
-                    dy[(size_t)k * st + 1 + jb + i] = (float)(scale * (2.0 * g * acc[i] - 2.0 * ems * uw[i]) * us);
-        }
+        dy[(size_t)k * st] = (float)(scale * (g * es[k] * (double)As[(size_t)k * P + k] - 1.0 + ems[k] * q));
     }
 }
 
@@ -508,8 +578,15 @@ int qgtl_hip_kaporin(int P, int r, int B, const float *Y, const float *As_all, c
                      float *dY, float scale) {
     if (P < 1 || P > kMaxP || r < 0 || r > kMaxRank || P * r > kMaxPR || B < 1)
         return qgtl::set_error_msg(-118, "kaporin: needs P <= 1024, r <= 32, P r <= 8192");
-    hipLaunchKernelGGL(kaporin_kernel, dim3((unsigned)B), dim3(kThreads), 0, qgtl::stream(), P, r, Y, As_all, idx,
-                       loss, dY, scale);
+    const int vec = vec_ok(As_all, P, 4, 16);
+#define QGTL_KAPORIN(RT, PR)                                                                                      \
+    hipLaunchKernelGGL((kaporin_kernel<RT, PR>), dim3((unsigned)B), dim3(kThreads), 0, qgtl::stream(), P, r, Y,    \
+                       As_all, idx, loss, dY, scale, vec)
+    // up to P r = 2048 two workgroups share a CU's LDS
+    if (r <= 16 && P * r <= 2048) QGTL_KAPORIN(1, 2048);
+    else if (r <= 16) QGTL_KAPORIN(1, kMaxPR);
+    else QGTL_KAPORIN(2, kMaxPR);
+#undef QGTL_KAPORIN
     QGTL_LAUNCH_CHECK("kaporin");
     return 0;
 }

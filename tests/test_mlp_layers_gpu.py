@@ -36,3 +36,29 @@ def test_layers_match_oracle(F, H, nh, P, r, B):
     assert abs(loss - lo) <= 1e-2 * max(1.0, abs(lo))
     assert np.max(np.abs(g - go)) <= 1e-2 * np.max(np.abs(go)) and cos >= 0.9999
     m.close()
+
+
+@pytest.mark.parametrize("P,r", [(3, 1), (17, 16), (31, 17), (200, 10), (255, 32), (481, 17), (1023, 8)])
+def test_loss_kernel_sizes(P, r):
+    """(P = 1 is left out: its loss is zero whatever y is.)  The loss kernel's forms (rank up to 16 and up to 32, both LDS sizes, odd P without vector
+    loads).  A network of one narrow layer, so the gradient of the output bias is the kernel's
+    own dL/dy summed over the samples.  Loss: FP64 but for the network's bf16 output error (bar as
+    above); the output bias' gradient: 3.5e-2 normwise, the rank-32 bar of tests/test_mlp_gpu.py."""
+    F, H, nh, B = 4, 8, 1, 3
+    m = Q.MLP(F, H, nh, P, r, seed=P)
+    p = m.get_params()
+    p *= 6.0
+    m.set_params(p)
+    rng = np.random.default_rng(P)
+    X = rng.normal(size=(B, F)).astype(np.float32)
+    As = np.stack([spd_unit_diag(P, 50 + s) for s in range(B)]).astype(np.float32)
+    m.set_data(X, As)
+    idx = np.arange(B, dtype=np.int32)
+    loss, g = m.loss_grad(idx)
+    lo, go = O.mlp_loss_grad(F, H, nh, P, r, oracle_params(m), bf16(X), As.astype(np.float64))
+    gb, gob = g[-m.out_dim:], go[-m.out_dim:]
+    err = np.max(np.abs(gb - gob)) / np.max(np.abs(gob))
+    print(f"P={P} r={r}: loss {loss:.6f} oracle {lo:.6f} bias gradient err {err:.2e}")
+    assert abs(loss - lo) <= 1e-2 * max(1.0, abs(lo))
+    assert err <= 3.5e-2
+    m.close()
