@@ -256,14 +256,15 @@ static void plan_free_device(struct qgtl_plan *p)
     qgtl_hip_free(p->psi[1]);
     qgtl_hip_free(p->D);
     qgtl_hip_free(p->tmp);
-    qgtl_hip_free(p->tabs_dev);
-    p->tabs_dev = NULL;
+    qgtl_hip_free(p->tabs_dev);                          /* the injection slots are part of it */
+    qgtl_hip_host_free(p->tabs_host);
+    p->tabs_dev = p->inj_slots_dev = NULL;
+    p->tabs_host = NULL;
+    p->inj_slots_host = NULL;
     p->tabs_passes = 0;
     qgtl_hip_free(p->res_dev);
     qgtl_hip_host_free(p->res_host);
     p->res_dev = p->res_host = NULL;
-    qgtl_hip_free(p->inj_slots_dev);
-    p->inj_slots_dev = NULL;
     qgtl_hip_free(p->inj_partials);
     qgtl_hip_free(p->inj_sums);
     qgtl_hip_free(p->gram_partials);
@@ -319,7 +320,7 @@ qgtl_plan_t *qgtl_plan_create(int n, int nops, const qgtl_op_t *ops, int mode, c
     if (nops) memcpy(p->ops, ops, sizeof(qgtl_op_t) * (size_t)nops);
     if (tune) p->tune = *tune;
     if (qgtl_plan_build(p) != 0) {
-        free(p->ops); free(p->blocks); free(p->params); free(p->slot_param); free(p);
+        free(p->ops); free(p->blocks); free(p->params); free(p->slot_param); free(p->gates1); free(p->u_at); free(p);
         return NULL;
     }
     p->N = (size_t)1 << n;
@@ -333,7 +334,8 @@ int qgtl_plan_set_angles_nolock(qgtl_plan_t *p, int nops, const double *angles)
 {
     if (!p || !angles || nops != p->nops) return qgtl_set_error(QGT_ERROR_INVALID_ARGUMENT, "angle count mismatch");
     for (int i = 0; i < nops; i++) p->ops[i].angle = angles[i];
-    return qgtl_plan_build(p);
+    qgtl_plan_new_angles(p);
+    return 0;
 }
 
 int qgtl_plan_set_angles(qgtl_plan_t *p, int nops, const double *angles)
@@ -348,16 +350,16 @@ void qgtl_plan_destroy(qgtl_plan_t *p)
     if (!p) return;
     qgtl_hip_graph_destroy(p->graph);
     plan_free_device(p);
-    free(p->inj_slots_host);
     qgtl_hip_event_destroy(p->ev_psi);
     qgtl_hip_event_destroy(p->ev_inj);
     for (int k = 0; k < p->nev_chain; k++) qgtl_hip_event_destroy(p->ev_chain[k]);
     free(p->ev_chain);
-    free(p->tabs_host);
     free(p->ops);
     free(p->blocks);
     free(p->params);
     free(p->slot_param);
+    free(p->gates1);
+    free(p->u_at);
     free(p);
 }
 
@@ -569,13 +571,20 @@ static int upload_tabs(struct qgtl_plan *p)
     }
     if (total == 0) { p->tabs_dirty = 0; return 0; }
     const size_t per = 2 * QGTL_PHASE_TAB * 2;                /* floats per pass */
+    const size_t P = (size_t)p->P;
+    /* tables and slots in one pinned buffer: one asynchronous copy */
+    const size_t tab_bytes = sizeof(float) * per * (size_t)total;
+    const size_t bytes = tab_bytes + 2 * P * sizeof(qgtl_inject_slot_t);
     if (total != p->tabs_passes) {
         qgtl_hip_free(p->tabs_dev);
-        p->tabs_dev = NULL;
-        free(p->tabs_host);
-        p->tabs_host = (float *)malloc(sizeof(float) * per * (size_t)total);
-        if (!p->tabs_host) return qgtl_set_error(QGT_ERROR_NO_MEMORY, "out of host memory");
-        HIPCALL(qgtl_hip_malloc(&p->tabs_dev, sizeof(float) * per * (size_t)total));
+        qgtl_hip_host_free(p->tabs_host);
+        p->tabs_dev = p->inj_slots_dev = NULL;
+        p->tabs_host = NULL;
+        p->tabs_passes = 0;
+        HIPCALL(qgtl_hip_host_alloc((void **)&p->tabs_host, bytes));
+        HIPCALL(qgtl_hip_malloc(&p->tabs_dev, bytes));
+        p->inj_slots_host = (qgtl_inject_slot_t *)((char *)p->tabs_host + tab_bytes);
+        p->inj_slots_dev = P > 0 ? (char *)p->tabs_dev + tab_bytes : NULL;
         p->tabs_passes = total;
     }
     int k = 0;
@@ -585,26 +594,16 @@ static int upload_tabs(struct qgtl_plan *p)
         for (int i = 0; i < p->blocks[bi].ninv; i++, k++)
             qgtl_pass_phase_tables(&p->blocks[bi].ipass[i], p->tabs_host + per * (size_t)k);
     }
-    HIPCALL(qgtl_hip_h2d(p->tabs_dev, p->tabs_host, sizeof(float) * per * (size_t)total));
-    if (p->P > 0) {
-        const size_t P = (size_t)p->P;
-        if (!p->inj_slots_dev) {
-            free(p->inj_slots_host);
-            p->inj_slots_host = (qgtl_inject_slot_t *)malloc(2 * P * sizeof(qgtl_inject_slot_t));
-            if (!p->inj_slots_host) return qgtl_set_error(QGT_ERROR_NO_MEMORY, "out of host memory");
-            HIPCALL(qgtl_hip_malloc(&p->inj_slots_dev, 2 * P * sizeof(qgtl_inject_slot_t)));
-        }
-        for (size_t s = 0; s < P; s++) {
-            const qgtl_param_t *pp = &p->params[p->slot_param[s]];
-            qgtl_inject_slot_t *f = &p->inj_slots_host[s], *bk = &p->inj_slots_host[P + s];
-            f->v = pp->v;
-            f->w = pp->w;
-            bk->v = bk->w = 1u << pp->qubit;
-            slot_matrix(f, &pp->A);
-            slot_matrix(bk, &pp->B);
-        }
-        HIPCALL(qgtl_hip_h2d(p->inj_slots_dev, p->inj_slots_host, 2 * P * sizeof(qgtl_inject_slot_t)));
+    for (size_t s = 0; s < P; s++) {
+        const qgtl_param_t *pp = &p->params[p->slot_param[s]];
+        qgtl_inject_slot_t *f = &p->inj_slots_host[s], *bk = &p->inj_slots_host[P + s];
+        f->v = pp->v;
+        f->w = pp->w;
+        bk->v = bk->w = 1u << pp->qubit;
+        slot_matrix(f, &pp->A);
+        slot_matrix(bk, &pp->B);
     }
+    HIPCALL(qgtl_hip_h2d(p->tabs_dev, p->tabs_host, bytes));
     p->tabs_dirty = 0;
     return 0;
 }

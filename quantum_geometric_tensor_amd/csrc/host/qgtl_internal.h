@@ -66,6 +66,9 @@ typedef struct {
                                             the parameter's qubit acting on the block's input state */
 } qgtl_param_t;
 
+/* a single-qubit gate of the expanded gate list (CZ and CY rewritten) */
+typedef struct { int type, q, param, op_index, block; } qgtl_gate1_t;
+
 struct qgtl_plan {
     int n;
     int mode;
@@ -77,6 +80,9 @@ struct qgtl_plan {
     int blocks_cap;
     qgtl_param_t *params;                /* indexed by parameter number */
     int *slot_param;                     /* D slot -> parameter number */
+    qgtl_gate1_t *gates1;                /* single-qubit gates in order */
+    int ngates1;
+    qgtl_mat2 *u_at;                     /* the block's matrix on the parameter's qubit up to its gate */
     qgtl_tune_t tune;
     /* device buffers */
     size_t N;
@@ -118,7 +124,7 @@ struct qgtl_plan {
     /* rotation-form phase tables of every pass (block order), built on the host */
     int tabs_dirty;                      /* angles changed since the last upload */
     int tabs_passes;
-    float *tabs_host;                    /* tabs_passes x 2 x QGTL_PHASE_TAB complex64 */
+    float *tabs_host;                    /* tabs_passes x 2 x QGTL_PHASE_TAB complex64, then the slots; pinned */
     void *tabs_dev;
     /* per D slot: the injection as a load-time formula, forward (slots 0..P-1)
      * and backward (P..2P-1), rebuilt with the tables */
@@ -152,6 +158,7 @@ struct qgtl_plan {
 
 /* plan construction (qgtl_plan.c) */
 int qgtl_plan_build(struct qgtl_plan *plan);
+void qgtl_plan_new_angles(struct qgtl_plan *plan);
 int qgtl_gate_matrix(const qgtl_op_t *op, qgtl_mat2 *m);
 int qgtl_is_param_gate(int type);
 uint64_t qgtl_structure_hash(int n, int nops, const qgtl_op_t *ops, int mode);

@@ -213,40 +213,50 @@ static void factor_rotation(const qgtl_mat2 *U, double *c, double *s, qgtl_cd pr
     }
 }
 
-/* matrix g of pass p: general form always, rotation form alongside */
-static void set_gate(qgtl_pass_desc_t *p, int g, const qgtl_mat2 *U)
-{
-    to_c64(U, p->mat[g]);
+/* diag(post) [[c, -s], [s, c]] diag(pre) of one qubit's matrix */
+typedef struct {
     double c, s;
     qgtl_cd pre[2], post[2];
-    factor_rotation(U, &c, &s, pre, post);
-    p->rot[g].re = (float)c;
-    p->rot[g].im = (float)s;
-    for (int b = 0; b < 2; b++) {
-        p->pre[g][b] = c64(pre[b]);
-        p->post[g][b] = c64(post[b]);
-    }
-}
+} rot_factor_t;
 
-/* switch a finished pass to the rotation form */
-static void finish_form(qgtl_pass_desc_t *p, int general)
+/* qubit of gate g of pass p */
+static int gate_qubit(const qgtl_pass_desc_t *p, int g)
 {
-    p->form = 0;
-    p->has_pre = 0;
-    if (general) return;
-    for (int g = 0; g < p->ngates; g++) {
-        if (p->pre[g][0].re != 1.f || p->pre[g][0].im != 0.f || p->pre[g][1].re != 1.f || p->pre[g][1].im != 0.f)
-            p->has_pre = 1;
-    }
-    p->form = 1;
+    const int tb = p->gate_bit[g];
+    return tb < p->nlow ? tb : p->hi_pos[tb - p->nlow];
 }
 
-/* Register-kernel form of a finished rotation-form pass (see
+/* Matrices of a finished pass layout (gates in phase order) from the block's
+ * matrices u and their factors f: the general form always, the rotation form
+ * alongside (general != 0: only the general form is used). */
+static void set_gates(qgtl_pass_desc_t *p, const qgtl_mat2 *u, const rot_factor_t *f, int general)
+{
+    p->has_pre = 0;
+    p->form = general ? 0 : 1;
+    for (int g = 0; g < p->ngates; g++) {
+        const int q = gate_qubit(p, g);
+        to_c64(&u[q], p->mat[g]);
+        p->rot[g].re = (float)f[q].c;
+        p->rot[g].im = (float)f[q].s;
+        for (int b = 0; b < 2; b++) {
+            p->pre[g][b] = c64(f[q].pre[b]);
+            p->post[g][b] = c64(f[q].post[b]);
+            if (!general && (p->pre[g][b].re != 1.f || p->pre[g][b].im != 0.f)) p->has_pre = 1;
+        }
+    }
+    for (int ph = 0; ph < p->nphase; ph++)
+        for (int g = p->ph_first[ph]; g < p->ph_first[ph + 1]; g++) {
+            p->ph_rot[ph][p->ph_greg[g]] = p->rot[g];
+            memcpy(p->ph_mat[ph][p->ph_greg[g]], p->mat[g], sizeof(qgtl_c64_t) * 4);
+        }
+}
+
+/* Register-kernel form of a rotation-form pass with its gates set (see
  * qgtl_pass_desc_t): per gate the scaled-out rotation coefficient and the
  * factor taken out, the pair swaps left to the store (xmask) and where their
  * signs go (xfold), and the register parts of the phase layers, from the
- * block's matrices u (FP64, rounded once). */
-static void finish_rotation(qgtl_pass_desc_t *p, const qgtl_mat2 *u)
+ * factors f of the block's matrices (FP64, rounded once). */
+static void finish_rotation(qgtl_pass_desc_t *p, const rot_factor_t *f)
 {
     p->has_post = 0;
     p->scale = 1.f;
@@ -254,29 +264,26 @@ static void finish_rotation(qgtl_pass_desc_t *p, const qgtl_mat2 *u)
     p->xfold = 0;
     p->nolayer = 0;
     p->tf_n = 0;
-    for (int ph = 0; ph < QGTL_MAX_PHASES; ph++)
-        for (int j = 0; j < 5; j++) p->ph_tan[ph][j] = 0.f;
+    memset(p->tf_bit, 0, sizeof p->tf_bit);
+    memset(p->tf, 0, sizeof p->tf);
+    memset(p->ph_tan, 0, sizeof p->ph_tan);
     for (int r = 0; r < 32; r++) p->reg_post[r] = p->reg_pre[r] = c64(cd(1.0, 0.0));
     if (p->form != 1) return;
-    double cs[QGTL_TILE_BITS_MAX], sns[QGTL_TILE_BITS_MAX], coef[QGTL_TILE_BITS_MAX], scale = 1.0;
+    double coef[QGTL_TILE_BITS_MAX], scale = 1.0;
     int swap[QGTL_TILE_BITS_MAX], gate_of_bit[QGTL_TILE_BITS_MAX];
-    qgtl_cd rel_pre[QGTL_TILE_BITS_MAX], rel_post[QGTL_TILE_BITS_MAX];
+    const rot_factor_t *gf[QGTL_TILE_BITS_MAX];
     for (int b = 0; b < QGTL_TILE_BITS_MAX; b++) gate_of_bit[b] = -1;
     for (int g = 0; g < p->ngates; g++) {
-        const int tb = p->gate_bit[g];
-        const int q = tb < p->nlow ? tb : p->hi_pos[tb - p->nlow];
-        qgtl_cd pre[2], post[2];
-        factor_rotation(&u[q], &cs[g], &sns[g], pre, post);
-        rel_pre[g] = cmul(pre[1], cconj(pre[0]));
-        rel_post[g] = cmul(post[1], cconj(post[0]));
+        gf[g] = &f[gate_qubit(p, g)];
+        const qgtl_cd *post = gf[g]->post;
         if (post[0].re != 1.0 || post[0].im != 0.0 || post[1].re != 1.0 || post[1].im != 0.0) p->has_post = 1;
-        gate_of_bit[tb] = g;
+        gate_of_bit[p->gate_bit[g]] = g;
     }
     /* the sign of a swapped gate goes into the layer the kernel applies:
      * the post layer unless the pass has a pre layer and no post layer */
     p->xfold = (p->has_pre && !p->has_post) ? 1 : 0;
     for (int g = 0; g < p->ngates; g++) {
-        const double c = cs[g], sn = sns[g];
+        const double c = gf[g]->c, sn = gf[g]->s;
         swap[g] = fabs(c) < fabs(sn);
         if (swap[g]) {
             p->xmask |= 1u << p->gate_bit[g];
@@ -292,25 +299,30 @@ static void finish_rotation(qgtl_pass_desc_t *p, const qgtl_mat2 *u)
     for (int ph = 0; ph < p->nphase; ph++)
         for (int g = p->ph_first[ph]; g < p->ph_first[ph + 1]; g++) p->ph_tan[ph][p->ph_greg[g]] = (float)coef[g];
     const int last = p->nphase - 1;
-    for (int r = 0; r < 32; r++) {
-        qgtl_cd a = cd(1.0, 0.0), b = cd(1.0, 0.0);
-        for (int i = 0; i < 5; i++) {
-            if (!((r >> i) & 1)) continue;
-            const int gl = gate_of_bit[p->ph_rbits[last][i]], g0 = gate_of_bit[p->ph_rbits[0][i]];
-            if (gl >= 0) {
-                /* post layer: a swapped bit reads the other phase, signed under xfold = 0 */
-                qgtl_cd f = swap[gl] ? cconj(rel_post[gl]) : rel_post[gl];
-                if (swap[gl] && !p->xfold) f = cd(-f.re, -f.im);
-                a = cmul(a, f);
-            }
-            if (g0 >= 0) {
-                qgtl_cd f = rel_pre[g0];
-                if (swap[g0] && p->xfold) f = cd(-f.re, -f.im);
-                b = cmul(b, f);
-            }
+    /* entry r is entry r without its highest bit times that bit's ratio */
+    qgtl_cd a[32], b[32];
+    a[0] = b[0] = cd(1.0, 0.0);
+    for (int i = 0; i < 5; i++) {
+        const int gl = gate_of_bit[p->ph_rbits[last][i]], g0 = gate_of_bit[p->ph_rbits[0][i]];
+        qgtl_cd fa = cd(1.0, 0.0), fb = fa;
+        if (gl >= 0) {
+            /* post layer: a swapped bit reads the other phase, signed under xfold = 0 */
+            const qgtl_cd rel = cmul(gf[gl]->post[1], cconj(gf[gl]->post[0]));
+            fa = swap[gl] ? cconj(rel) : rel;
+            if (swap[gl] && !p->xfold) fa = cd(-fa.re, -fa.im);
         }
-        p->reg_post[r] = c64(a);
-        p->reg_pre[r] = c64(b);
+        if (g0 >= 0) {
+            fb = cmul(gf[g0]->pre[1], cconj(gf[g0]->pre[0]));
+            if (swap[g0] && p->xfold) fb = cd(-fb.re, -fb.im);
+        }
+        for (int k = 0; k < 1 << i; k++) {
+            a[(1 << i) + k] = cmul(a[k], fa);
+            b[(1 << i) + k] = cmul(b[k], fb);
+        }
+    }
+    for (int r = 0; r < 32; r++) {
+        p->reg_post[r] = c64(a[r]);
+        p->reg_pre[r] = c64(b[r]);
     }
 }
 
@@ -329,9 +341,9 @@ static int reg_pass_ok(const qgtl_pass_desc_t *p)
  * bit, c diag(p0, p1) or, for a swapped gate, s diag(-p0, p1) (the post layer
  * read at y with the sign of y ^ xmask).  fwd = 0: d runs just after r and
  * applies a pre layer only (xfold = 1); its layer in d's input index is
- * c diag(q0, q1), or s diag(q0, -q1) for a swapped gate.  u: the matrices d
- * was finished with. */
-static void fold_layer(qgtl_pass_desc_t *d, qgtl_pass_desc_t *r, const qgtl_mat2 *u, int fwd)
+ * c diag(q0, q1), or s diag(q0, -q1) for a swapped gate.  f: the factors d was
+ * finished with. */
+static void fold_layer(qgtl_pass_desc_t *d, qgtl_pass_desc_t *r, const rot_factor_t *f, int fwd)
 {
     if (!reg_pass_ok(d) || !reg_pass_ok(r) || r->nlow != QGTL_TILE_BITS_MAX || r->tf_n || r->nolayer || d->tf_n)
         return;
@@ -341,23 +353,18 @@ static void fold_layer(qgtl_pass_desc_t *d, qgtl_pass_desc_t *r, const qgtl_mat2
     if (d->ngates < 1 || d->ngates > QGTL_TILE_BITS_MAX) return;
     int bit[QGTL_TILE_BITS_MAX];
     for (int g = 0; g < d->ngates; g++) {
-        const int tb = d->gate_bit[g];
-        const int q = tb < d->nlow ? tb : d->hi_pos[tb - d->nlow];
+        const int q = gate_qubit(d, g);
         bit[g] = -1;
         for (int i = 0; i < r->nrest; i++)
             if (r->rest_pos[i] == q) bit[g] = i;
         if (bit[g] < 0) return;                 /* a gate inside r's tile: no fold */
     }
     for (int g = 0; g < d->ngates; g++) {
-        const int tb = d->gate_bit[g];
-        const int q = tb < d->nlow ? tb : d->hi_pos[tb - d->nlow];
-        double c, sn;
-        qgtl_cd pre[2], post[2];
-        factor_rotation(&u[q], &c, &sn, pre, post);
-        const int swapped = fabs(c) < fabs(sn);
-        const double f = swapped ? sn : c;
-        const qgtl_cd *ph = fwd ? post : pre;
-        qgtl_cd f0 = cd(f * ph[0].re, f * ph[0].im), f1 = cd(f * ph[1].re, f * ph[1].im);
+        const rot_factor_t *x = &f[gate_qubit(d, g)];
+        const int swapped = fabs(x->c) < fabs(x->s);
+        const double e = swapped ? x->s : x->c;
+        const qgtl_cd *ph = fwd ? x->post : x->pre;
+        qgtl_cd f0 = cd(e * ph[0].re, e * ph[0].im), f1 = cd(e * ph[1].re, e * ph[1].im);
         if (swapped && fwd) f0 = cd(-f0.re, -f0.im);
         if (swapped && !fwd) f1 = cd(-f1.re, -f1.im);
         r->tf_bit[g] = bit[g];
@@ -479,21 +486,9 @@ static void plan_phases(qgtl_pass_desc_t *p)
     }
     p->ph_first[nph] = (int8_t)cnt;
     p->nphase = nph;
-    /* reorder matrices and their tile bits into phase order */
-    qgtl_c64_t mats[QGTL_TILE_BITS_MAX][4], rot[QGTL_TILE_BITS_MAX], pre[QGTL_TILE_BITS_MAX][2],
-        post[QGTL_TILE_BITS_MAX][2];
+    /* tile bits in phase order */
     int32_t bits[QGTL_TILE_BITS_MAX];
-    for (int i = 0; i < cnt; i++) {
-        memcpy(mats[i], p->mat[order[i]], sizeof mats[i]);
-        rot[i] = p->rot[order[i]];
-        memcpy(pre[i], p->pre[order[i]], sizeof pre[i]);
-        memcpy(post[i], p->post[order[i]], sizeof post[i]);
-        bits[i] = p->gate_bit[order[i]];
-    }
-    memcpy(p->mat, mats, sizeof(qgtl_c64_t) * 4 * (size_t)cnt);
-    memcpy(p->rot, rot, sizeof(qgtl_c64_t) * (size_t)cnt);
-    memcpy(p->pre, pre, sizeof(qgtl_c64_t) * 2 * (size_t)cnt);
-    memcpy(p->post, post, sizeof(qgtl_c64_t) * 2 * (size_t)cnt);
+    for (int i = 0; i < cnt; i++) bits[i] = p->gate_bit[order[i]];
     memcpy(p->gate_bit, bits, sizeof(int32_t) * (size_t)cnt);
     /* thread-bit orders (the last layout also writes the ring store) */
     for (int ph = 0; ph < nph; ph++)
@@ -501,20 +496,14 @@ static void plan_phases(qgtl_pass_desc_t *p)
     /* by register bit, for the kernels */
     for (int ph = 0; ph < nph; ph++) {
         p->ph_mask[ph] = 0;
-        for (int g = p->ph_first[ph]; g < p->ph_first[ph + 1]; g++) {
-            const int j = p->ph_greg[g];
-            p->ph_mask[ph] |= 1 << j;
-            p->ph_rot[ph][j] = p->rot[g];
-            memcpy(p->ph_mat[ph][j], p->mat[g], sizeof(qgtl_c64_t) * 4);
-        }
+        for (int g = p->ph_first[ph]; g < p->ph_first[ph + 1]; g++) p->ph_mask[ph] |= 1 << p->ph_greg[g];
     }
 }
 
-/* High-qubit passes of a block with n > 13 (matrices u[q]): the qubits >= 13
+/* High-qubit passes of a block with n > 13: the qubits >= 13
  * that carry a gate, in groups that leave CMIN_LOW_BITS contiguous low bits
  * in the tile; in place. */
-static void high_passes(const qgtl_block_t *b, int n, const qgtl_mat2 *u, qgtl_pass_desc_t *out, int *flips,
-                        int *count)
+static void high_passes(const qgtl_block_t *b, int n, qgtl_pass_desc_t *out, int *flips, int *count)
 {
     const int TB = QGTL_TILE_BITS_MAX;
     int hq[QGTL_MAX_QUBITS], nh = 0;
@@ -533,7 +522,6 @@ static void high_passes(const qgtl_block_t *b, int n, const qgtl_mat2 *u, qgtl_p
             p->hi_pos[i] = (int8_t)hq[g0 + i];
             in_tile[hq[g0 + i]] = 1;
             p->gate_bit[i] = (int8_t)(c + i);
-            set_gate(p, i, &u[hq[g0 + i]]);
         }
         p->ngates = len;
         for (int q = 0; q < n; q++)
@@ -544,9 +532,9 @@ static void high_passes(const qgtl_block_t *b, int n, const qgtl_mat2 *u, qgtl_p
     }
 }
 
-/* The pass over tile bits 0..12 (matrices u[q], q < 13) with the given load
+/* The pass over tile bits 0..12 with the given load
  * and store; returns 0 when it has nothing to do. */
-static int low_pass(const qgtl_block_t *b, int n, const qgtl_mat2 *u, qgtl_pass_desc_t *p, int store, int load)
+static int low_pass(const qgtl_block_t *b, int n, qgtl_pass_desc_t *p, int store, int load)
 {
     const int TB = QGTL_TILE_BITS_MAX;
     memset(p, 0, sizeof *p);
@@ -554,15 +542,14 @@ static int low_pass(const qgtl_block_t *b, int n, const qgtl_mat2 *u, qgtl_pass_
     for (int q = TB; q < n; q++) p->rest_pos[p->nrest++] = (int8_t)q;
     for (int q = 0; q < TB; q++)
         if (b->has_u[q]) {
-            p->gate_bit[p->ngates] = (int8_t)q;
-            set_gate(p, p->ngates, &u[q]);
-            p->ngates++;
+            p->gate_bit[p->ngates++] = (int8_t)q;
         }
     p->store = store;
     p->load = load;
     return p->ngates > 0 || store != QGTL_STORE_INPLACE || load != QGTL_LOAD_NATURAL;
 }
 
+/* The layouts of block b's passes (their matrices are set for given angles). */
 static void build_passes(qgtl_block_t *b, int n)
 {
     const int TB = QGTL_TILE_BITS_MAX;
@@ -574,9 +561,7 @@ static void build_passes(qgtl_block_t *b, int n)
         p->n = n; p->m = n; p->nlow = n; p->nrest = 0;
         for (int q = 0; q < n; q++)
             if (b->has_u[q]) {
-                p->gate_bit[p->ngates] = (int8_t)q;
-                set_gate(p, p->ngates, &b->u[q]);
-                p->ngates++;
+                p->gate_bit[p->ngates++] = (int8_t)q;
             }
         p->store = QGTL_STORE_INPLACE;
         if (b->nperm > 0) {
@@ -598,8 +583,8 @@ static void build_passes(qgtl_block_t *b, int n)
         }
         return;
     }
-    high_passes(b, n, b->u, b->pass, b->pass_flips, &b->npasses);
-    if (low_pass(b, n, b->u, &b->pass[b->npasses], b->is_ring ? QGTL_STORE_RING : QGTL_STORE_INPLACE,
+    high_passes(b, n, b->pass, b->pass_flips, &b->npasses);
+    if (low_pass(b, n, &b->pass[b->npasses], b->is_ring ? QGTL_STORE_RING : QGTL_STORE_INPLACE,
                  QGTL_LOAD_NATURAL)) {
         b->pass_flips[b->npasses] = b->is_ring;
         b->npasses++;
@@ -616,14 +601,12 @@ static void build_inverse_passes(qgtl_block_t *b, int n)
     b->ninv = 0;
     b->inv_ok = 0;
     if (n <= QGTL_TILE_BITS_MAX || (!b->is_ring && b->nperm > 0)) return;
-    qgtl_mat2 uadj[QGTL_MAX_QUBITS];
-    for (int q = 0; q < n; q++) uadj[q] = mat_adj(&b->u[q]);
-    if (low_pass(b, n, uadj, &b->ipass[0], QGTL_STORE_INPLACE, b->is_ring ? QGTL_LOAD_RING : QGTL_LOAD_NATURAL)) {
+    if (low_pass(b, n, &b->ipass[0], QGTL_STORE_INPLACE, b->is_ring ? QGTL_LOAD_RING : QGTL_LOAD_NATURAL)) {
         b->ipass_flips[0] = b->is_ring;
         b->ninv = 1;
     }
     int nh = 0;
-    high_passes(b, n, uadj, &b->ipass[b->ninv], &b->ipass_flips[b->ninv], &nh);
+    high_passes(b, n, &b->ipass[b->ninv], &b->ipass_flips[b->ninv], &nh);
     b->ninv += nh;
     for (int i = 0; i < b->ninv; i++) {
         qgtl_pass_desc_t *p = &b->ipass[i];
@@ -680,6 +663,74 @@ static qgtl_block_t *open_block(qgtl_block_t *blocks, int i, int n)
     return b;
 }
 
+/* The angle-dependent half of a plan: every matrix, rotation factor, phase and
+ * injection operator, for the angles in plan->ops, into the layouts that
+ * build_structure made. */
+static void set_matrices(struct qgtl_plan *plan)
+{
+    const int n = plan->n, general = plan->tune.sweep_form == 1;
+    for (int bi = 0; bi < plan->nblocks; bi++)
+        for (int q = 0; q < n; q++) plan->blocks[bi].u[q] = mat_identity();
+    for (int i = 0; i < plan->ngates1; i++) {
+        const qgtl_gate1_t *g = &plan->gates1[i];
+        const qgtl_op_t op = {g->type, g->q, -1, -1, plan->ops[g->op_index].angle};
+        qgtl_mat2 *u = &plan->blocks[g->block].u[g->q], m;
+        qgtl_gate_matrix(&op, &m);
+        *u = mat_mul(&m, u);
+        if (g->param >= 0) {
+            plan->u_at[g->param] = *u;
+            plan->params[g->param].A = generator(g->type);
+        }
+    }
+    for (int bi = 0; bi < plan->nblocks; bi++) {
+        qgtl_block_t *b = &plan->blocks[bi];
+        rot_factor_t f[QGTL_MAX_QUBITS];
+        for (int q = 0; q < n; q++)
+            if (b->has_u[q]) factor_rotation(&b->u[q], &f[q].c, &f[q].s, f[q].pre, f[q].post);
+        for (int i = 0; i < b->npasses; i++) {
+            set_gates(&b->pass[i], b->u, f, general);
+            finish_rotation(&b->pass[i], f);
+        }
+        if (b->npasses == 2) fold_layer(&b->pass[0], &b->pass[1], f, 1);
+        if (b->ninv > 0) {
+            qgtl_mat2 uadj[QGTL_MAX_QUBITS];
+            rot_factor_t fa[QGTL_MAX_QUBITS];
+            for (int q = 0; q < n; q++) {
+                if (!b->has_u[q]) continue;
+                uadj[q] = mat_adj(&b->u[q]);
+                factor_rotation(&uadj[q], &fa[q].c, &fa[q].s, fa[q].pre, fa[q].post);
+            }
+            for (int i = 0; i < b->ninv; i++) {
+                set_gates(&b->ipass[i], uadj, fa, general);
+                finish_rotation(&b->ipass[i], fa);
+            }
+            if (b->ninv == 2) fold_layer(&b->ipass[1], &b->ipass[0], fa, 0);
+        }
+        for (int j = b->param_begin; j < b->param_end; j++) {
+            const int k = plan->slot_param[j];
+            qgtl_param_t *pp = &plan->params[k];
+            const int q = pp->qubit;
+            qgtl_mat2 at_adj = mat_adj(&plan->u_at[k]);
+            qgtl_mat2 S = mat_mul(&b->u[q], &at_adj);           /* gates after the parameter */
+            qgtl_mat2 Sadj = mat_adj(&S);
+            qgtl_mat2 t = mat_mul(&S, &pp->A);
+            pp->A = mat_mul(&t, &Sadj);
+            const qgtl_mat2 ub = mat_adj(&b->u[q]);
+            t = mat_mul(&ub, &pp->A);
+            pp->B = mat_mul(&t, &b->u[q]);
+        }
+    }
+    plan->tabs_dirty = 1;                                     /* new angles: phase tables to rebuild */
+}
+
+/* New angles for a built plan: the structure (blocks, pass layouts, injection
+ * masks) depends on the gate list alone and is kept. */
+void qgtl_plan_new_angles(struct qgtl_plan *plan)
+{
+    plan->build_gen++;                   /* any captured launch sequence is stale */
+    set_matrices(plan);
+}
+
 int qgtl_plan_build(struct qgtl_plan *plan)
 {
     const int n = plan->n;
@@ -723,19 +774,23 @@ int qgtl_plan_build(struct qgtl_plan *plan)
     int rc = expand(plan, &g, &ng);
     if (rc) return rc;
 
-    /* the block array is kept across rebuilds (set_angles): each block is
-     * cleared when it is opened, so only the blocks in use are touched */
+    /* the block array is kept across rebuilds: each block is cleared when it is
+     * opened, so only the blocks in use are touched */
     if (!plan->blocks || plan->blocks_cap < ng + 1) {
         free(plan->blocks);
         plan->blocks = (qgtl_block_t *)malloc((size_t)(ng + 1) * sizeof(qgtl_block_t));
         plan->blocks_cap = plan->blocks ? ng + 1 : 0;
     }
     free(plan->params);
+    free(plan->gates1);
+    free(plan->u_at);
     plan->params = (qgtl_param_t *)calloc((size_t)(P > 0 ? P : 1), sizeof(qgtl_param_t));
-    qgtl_mat2 *u_at = (qgtl_mat2 *)calloc((size_t)(P > 0 ? P : 1), sizeof(qgtl_mat2));
+    plan->u_at = (qgtl_mat2 *)calloc((size_t)(P > 0 ? P : 1), sizeof(qgtl_mat2));
+    plan->gates1 = (qgtl_gate1_t *)malloc((size_t)(ng > 0 ? ng : 1) * sizeof(qgtl_gate1_t));
+    plan->ngates1 = 0;
     int *order = (int *)calloc((size_t)(P > 0 ? P : 1), sizeof(int));   /* params in creation order */
-    if (!plan->blocks || !plan->params || !u_at || !order) {
-        free(g); free(u_at); free(order);
+    if (!plan->blocks || !plan->params || !plan->u_at || !plan->gates1 || !order) {
+        free(g); free(order);
         return QGT_ERROR_NO_MEMORY;
     }
     int nb = 0, npar = 0;
@@ -773,19 +828,14 @@ int qgtl_plan_build(struct qgtl_plan *plan)
             cur->nperm++;
             touched[op->q0] = touched[op->q1] = 1;
         } else {
-            qgtl_op_t tmp = {op->type, op->q0, -1, -1, op->angle};
-            qgtl_mat2 m;
-            qgtl_gate_matrix(&tmp, &m);
-            cur->u[op->q0] = mat_mul(&m, &cur->u[op->q0]);
+            plan->gates1[plan->ngates1++] =
+                (qgtl_gate1_t){op->type, op->q0, op->param, op->op_index, nb};
             cur->has_u[op->q0] = 1;
             if (op->param >= 0) {
                 qgtl_param_t *pp = &plan->params[op->param];
                 pp->block = nb;
                 pp->qubit = op->q0;
                 pp->op_index = op->op_index;
-                u_at[op->param] = cur->u[op->q0];
-                /* remember the generator through A (finished at block close) */
-                pp->A = generator(op->type);
                 order[npar++] = op->param;
             }
         }
@@ -796,45 +846,22 @@ int qgtl_plan_build(struct qgtl_plan *plan)
     }
     plan->nblocks = nb;
 
-    /* finish blocks: ring detection, passes, injection operators */
+    /* finish blocks: ring detection, pass layouts, injection masks */
     for (int bi = 0; bi < nb; bi++) {
         qgtl_block_t *b = &plan->blocks[bi];
         detect_ring(b, n);
         build_passes(b, n);
         if (plan->mode == QGTL_MODE_MIXED && plan->tune.sweep_schedule != 1) build_inverse_passes(b, n);
-        for (int i = 0; i < b->npasses; i++) {
-            finish_form(&b->pass[i], plan->tune.sweep_form == 1);
-            finish_rotation(&b->pass[i], b->u);
-        }
-        if (b->npasses == 2) fold_layer(&b->pass[0], &b->pass[1], b->u, 1);
-        if (b->ninv > 0) {
-            qgtl_mat2 uadj[QGTL_MAX_QUBITS];
-            for (int q = 0; q < n; q++) uadj[q] = mat_adj(&b->u[q]);
-            for (int i = 0; i < b->ninv; i++) {
-                finish_form(&b->ipass[i], plan->tune.sweep_form == 1);
-                finish_rotation(&b->ipass[i], uadj);
-            }
-            if (b->ninv == 2) fold_layer(&b->ipass[1], &b->ipass[0], uadj, 0);
-        }
         /* images of the basis vectors under the inverse M-stage (the Z-frame masks below) */
         uint32_t inv_img[QGTL_MAX_QUBITS];
         if (b->param_end > b->param_begin)
             for (int j2 = 0; j2 < n; j2++) inv_img[j2] = perm_apply_inverse(b, 1u << j2);
         for (int j = b->param_begin; j < b->param_end; j++) {
             qgtl_param_t *pp = &plan->params[order[j]];
-            const int q = pp->qubit;
-            qgtl_mat2 at_adj = mat_adj(&u_at[order[j]]);
-            qgtl_mat2 S = mat_mul(&b->u[q], &at_adj);           /* gates after the parameter */
-            qgtl_mat2 Sadj = mat_adj(&S);
-            qgtl_mat2 t = mat_mul(&S, &pp->A);
-            pp->A = mat_mul(&t, &Sadj);
-            const qgtl_mat2 uadj = mat_adj(&b->u[q]);
-            t = mat_mul(&uadj, &pp->A);
-            pp->B = mat_mul(&t, &b->u[q]);
-            pp->v = perm_apply(b, 1u << q);
+            pp->v = perm_apply(b, 1u << pp->qubit);
             uint32_t w = 0;
             for (int j2 = 0; j2 < n; j2++)
-                if ((inv_img[j2] >> q) & 1u) w |= 1u << j2;
+                if ((inv_img[j2] >> pp->qubit) & 1u) w |= 1u << j2;
             pp->w = w;
         }
     }
@@ -842,12 +869,9 @@ int qgtl_plan_build(struct qgtl_plan *plan)
      * slots back to the caller's parameter numbers. */
     free(plan->slot_param);
     plan->slot_param = order;
-    order = NULL;
-    free(order);
-    free(u_at);
     free(g);
-    plan->tabs_dirty = 1;                                     /* new angles: phase tables to rebuild */
     plan->meet = nb - 1;
+    set_matrices(plan);
     return 0;
 }
 
@@ -856,26 +880,39 @@ int qgtl_plan_build(struct qgtl_plan *plan)
  * out[QGTL_PHASE_TAB + t] the pre phases, as interleaved float pairs. */
 void qgtl_pass_phase_tables(const qgtl_pass_desc_t *p, float *out)
 {
-    for (int t = 0; t < QGTL_PHASE_TAB; t++) {
-        const int lo = t < 128;
-        const int i = lo ? t : t - 128;
-        double ar = 1.0, ai = 0.0, br = 1.0, bi = 0.0;
-        for (int g = 0; g < p->ngates; g++) {
-            const int bit = p->gate_bit[g];
-            if (lo ? bit >= 7 : bit < 7) continue;
-            const int v = (i >> (lo ? bit : bit - 7)) & 1;
-            const double pr = p->post[g][v].re, pi = p->post[g][v].im;
-            const double qr = p->pre[g][v].re, qi = p->pre[g][v].im;
-            const double a2 = ar * pr - ai * pi, b2 = br * qr - bi * qi;
-            ai = ar * pi + ai * pr;
-            ar = a2;
-            bi = br * qi + bi * qr;
-            br = b2;
+    int gate_of_bit[QGTL_TILE_BITS_MAX];
+    for (int b = 0; b < QGTL_TILE_BITS_MAX; b++) gate_of_bit[b] = -1;
+    for (int g = 0; g < p->ngates; g++) gate_of_bit[p->gate_bit[g]] = g;
+    for (int layer = 0; layer < 2; layer++) {
+        float *o = out + 2 * layer * QGTL_PHASE_TAB;
+        if (layer == 1 && !p->has_pre) {        /* every pre phase is 1 */
+            for (int t = 0; t < QGTL_PHASE_TAB; t++) { o[2 * t] = 1.f; o[2 * t + 1] = 0.f; }
+            continue;
         }
-        out[2 * t] = (float)ar;
-        out[2 * t + 1] = (float)ai;
-        out[2 * (QGTL_PHASE_TAB + t)] = (float)br;
-        out[2 * (QGTL_PHASE_TAB + t) + 1] = (float)bi;
+        for (int half = 0; half < 2; half++) {
+            /* entry i: the product over the half's tile bits, doubled bit by bit */
+            const int first = half ? 7 : 0, bits = half ? QGTL_TILE_BITS_MAX - 7 : 7;
+            qgtl_cd t[128];
+            t[0] = cd(1.0, 0.0);
+            for (int i = 0; i < bits; i++) {
+                const int g = gate_of_bit[first + i];
+                qgtl_cd p0 = cd(1.0, 0.0), p1 = p0;
+                if (g >= 0) {
+                    const qgtl_c64_t *ph = layer ? p->pre[g] : p->post[g];
+                    p0 = cd(ph[0].re, ph[0].im);
+                    p1 = cd(ph[1].re, ph[1].im);
+                }
+                for (int k = 0; k < 1 << i; k++) {
+                    const qgtl_cd v = t[k];
+                    t[k] = cmul(v, p0);
+                    t[(1 << i) + k] = cmul(v, p1);
+                }
+            }
+            for (int k = 0; k < 1 << bits; k++) {
+                o[2 * (128 * half + k)] = (float)t[k].re;
+                o[2 * (128 * half + k) + 1] = (float)t[k].im;
+            }
+        }
     }
 }
 
