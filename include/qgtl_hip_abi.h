@@ -246,7 +246,7 @@ typedef struct {
     uint64_t C;             /* (nt * 128)^2 FP64 */
     int32_t nt, nchunks;
     uint32_t unit_begin;    /* units: T * 64 (256 elements each) */
-    uint32_t pad;
+    uint32_t states;        /* complex form: rows and columns of G that are formed */
 } qgtl_gram_reduce_item_t;
 
 typedef struct {

@@ -365,41 +365,42 @@ __global__ __launch_bounds__(kThreads, 1) void gram_cplx_kernel(const uint8_t *_
 // accumulator that grows over the chunk, whatever the instruction's K), so the
 // chunks are kept at 1024 amplitudes: normwise error 3.4e-7 at n = 20, L = 6
 // against 1.4e-7 with the 256-amplitude outer sums of the per-tile-pair form.
+// With fewer than eight blocks of states (up to 224) the blocks past the last are
+// neither loaded nor multiplied: 15, 21 or 28 block pairs instead of 36, spread
+// over the twelve waves so that the SIMDs' sums differ by at most one pair
+// (found by a randomised search over orientations and splits).  P = 170 (six
+// blocks), N = 2^17, with a chunk per CU: n = 17, L = 5 as a whole 473 -> 430 us.
 constexpr int kThreads256 = 768;
 constexpr int kWaves256 = kThreads256 / 64;
 
+// B block, number of pairs, A blocks (a diagonal pair comes first)
 struct Role3 {
-    int a0, a1, a2, b;
+    int b, count, a0, a1, a2;
 };
 
-__device__ __forceinline__ Role3 wave_role3(int w) {
-    switch (w) {
-    case 0: return Role3{0, 1, 2, 0};
-    case 1: return Role3{1, 2, 3, 1};
-    case 2: return Role3{2, 3, 4, 2};
-    case 3: return Role3{3, 0, 4, 3};
-    case 4: return Role3{4, 0, 1, 4};
-    case 5: return Role3{5, 6, 7, 4};
-    case 6: return Role3{5, 0, 1, 5};
-    case 7: return Role3{2, 3, 6, 5};
-    case 8: return Role3{2, 3, 7, 6};
-    case 9: return Role3{6, 0, 1, 6};
-    case 10: return Role3{2, 3, 5, 7};
-    default: return Role3{7, 0, 1, 7};
-    }
-}
+__device__ constexpr Role3 kRoles256[4][kWaves256] = {
+    {{3, 2, 3, 0, 0}, {4, 1, 3, 3, 3}, {1, 2, 1, 0, 0}, {2, 2, 2, 1, 1}, {0, 1, 2, 2, 2}, {2, 1, 3, 3, 3},
+     {0, 1, 4, 4, 4}, {3, 1, 1, 1, 1}, {0, 1, 0, 0, 0}, {1, 1, 4, 4, 4}, {4, 1, 4, 4, 4}, {4, 1, 2, 2, 2}},
+    {{5, 2, 5, 4, 4}, {4, 2, 1, 3, 3}, {3, 2, 5, 1, 1}, {5, 2, 0, 2, 2}, {0, 2, 0, 4, 4}, {1, 2, 1, 5, 5},
+     {3, 2, 3, 0, 0}, {4, 2, 4, 2, 2}, {2, 2, 2, 3, 3}, {2, 1, 0, 0, 0}, {1, 1, 2, 2, 2}, {0, 1, 1, 1, 1}},
+    {{0, 3, 0, 6, 1}, {6, 3, 6, 4, 1}, {2, 3, 2, 6, 4}, {4, 3, 4, 0, 3}, {3, 2, 6, 2, 2}, {0, 2, 3, 5, 5},
+     {2, 2, 0, 5, 5}, {5, 2, 1, 6, 6}, {1, 2, 1, 4, 4}, {1, 2, 2, 3, 3}, {5, 2, 5, 4, 4}, {3, 2, 3, 5, 5}},
+    {{0, 3, 0, 1, 2}, {1, 3, 1, 2, 3}, {2, 3, 2, 3, 4}, {3, 3, 3, 0, 4}, {4, 3, 4, 0, 1}, {4, 3, 5, 6, 7},
+     {5, 3, 5, 0, 1}, {5, 3, 2, 3, 6}, {6, 3, 2, 3, 7}, {6, 3, 6, 0, 1}, {7, 3, 2, 3, 5}, {7, 3, 7, 0, 1}},
+};
 
 // Direct-to-LDS loads of one stage (amplitudes k0 .. k0 + 31) of states 0..255:
-// 64 wave-loads of 1 KB (four 256-byte rows each), wave-load g = 12 i + w.
-// States past P read state P - 1 (their rows feed only G entries >= P).
-__device__ __forceinline__ void issue_stage256(const uint8_t *__restrict__ D, size_t SB, int P, size_t k0,
+// 8 wave-loads of 1 KB (four 256-byte rows each) per block of 32, wave-load
+// g = 12 i + w.  States past P read state P - 1 (their rows feed only G entries
+// >= P).
+__device__ __forceinline__ void issue_stage256(const uint8_t *__restrict__ D, size_t SB, int P, int nb, size_t k0,
                                                uint8_t *buf, int w, uint32_t lane) {
     typedef Geo<32> G;
     const size_t ko = (k0 >> 6) * 512 + (k0 & 63) * 4;
 #pragma unroll
     for (int i = 0; i < 6; i++) {
         const int g = i * kWaves256 + w;
-        if (g >= 64) break;                                  // uniform: waves 4..11 issue five
+        if (g >= 8 * nb) break;                              // uniform
         int row = 4 * g + (int)(lane / G::kSlots);
         __asm__ volatile("" : "+v"(row));
         const uint32_t lgc = (lane % G::kSlots) ^ G::swz((uint32_t)row);
@@ -435,9 +436,9 @@ __device__ __forceinline__ u32x4 frag16(const uint8_t *buf, int blk, int sub, in
 
 // acc[i][2 sa + sb]: pair i, sub-block (sa, sb); Re and Im.  DIAG: pair 0 is a
 // diagonal pair and its sub-block (1, 0), below the diagonal, is not computed.
-template <int PT, bool DIAG>
-__device__ __forceinline__ void stage_mfma3_16(const uint8_t *buf, const Role3 &ro, f32x4 (&re)[3][4],
-                                               f32x4 (&im)[3][4], uint32_t lane) {
+template <int PT, bool DIAG, int COUNT>
+__device__ __forceinline__ void stage_mfma3_16(const uint8_t *buf, const Role3 &ro, f32x4 (&re)[COUNT][4],
+                                               f32x4 (&im)[COUNT][4], uint32_t lane) {
     const int ab[3] = {ro.a0, ro.a1, ro.a2};
 #pragma unroll 1
     for (int t = 0; t < 2; t++) {
@@ -454,16 +455,16 @@ __device__ __forceinline__ void stage_mfma3_16(const uint8_t *buf, const Role3 &
         }
 #pragma unroll
         for (int sa = 0; sa < 2; sa++) {
-            u32x4 ah[3], al[3];
+            u32x4 ah[COUNT], al[COUNT];
 #pragma unroll
-            for (int i = 0; i < 3; i++) {
+            for (int i = 0; i < COUNT; i++) {
                 ah[i] = frag16(buf, ab[i], sa, 0, t, lane);
                 al[i] = frag16(buf, ab[i], sa, 1, t, lane);
             }
             // smallest terms first; the accumulators interleaved
             if constexpr (PT == 4) {
 #pragma unroll
-                for (int i = 0; i < 3; i++)
+                for (int i = 0; i < COUNT; i++)
 #pragma unroll
                     for (int sb = 0; sb < 2; sb++) {
                         if (DIAG && i == 0 && sa == 1 && sb == 0) continue;
@@ -472,7 +473,7 @@ __device__ __forceinline__ void stage_mfma3_16(const uint8_t *buf, const Role3 &
                     }
             }
 #pragma unroll
-            for (int i = 0; i < 3; i++)
+            for (int i = 0; i < COUNT; i++)
 #pragma unroll
                 for (int sb = 0; sb < 2; sb++) {
                     if (DIAG && i == 0 && sa == 1 && sb == 0) continue;
@@ -480,7 +481,7 @@ __device__ __forceinline__ void stage_mfma3_16(const uint8_t *buf, const Role3 &
                     im[i][2 * sa + sb] = mma16(al[i], yh[sb], im[i][2 * sa + sb]);
                 }
 #pragma unroll
-            for (int i = 0; i < 3; i++)
+            for (int i = 0; i < COUNT; i++)
 #pragma unroll
                 for (int sb = 0; sb < 2; sb++) {
                     if (DIAG && i == 0 && sa == 1 && sb == 0) continue;
@@ -488,7 +489,7 @@ __device__ __forceinline__ void stage_mfma3_16(const uint8_t *buf, const Role3 &
                     im[i][2 * sa + sb] = mma16(ah[i], yl[sb], im[i][2 * sa + sb]);
                 }
 #pragma unroll
-            for (int i = 0; i < 3; i++)
+            for (int i = 0; i < COUNT; i++)
 #pragma unroll
                 for (int sb = 0; sb < 2; sb++) {
                     if (DIAG && i == 0 && sa == 1 && sb == 0) continue;
@@ -524,7 +525,7 @@ __device__ __forceinline__ void store_pair256_16(float *__restrict__ out, int a,
 
 // One split-K chunk of a two-tile Gram: stages of 32 amplitudes through the two
 // LDS buffers, the chunk's fp32 partials of the three tile pairs at the end.
-template <int PT, bool DIAG>
+template <int PT, bool DIAG, int COUNT>
 __device__ __forceinline__ void gram_cplx256_chunk(const uint8_t *__restrict__ D, int P, size_t N, size_t chunk_len,
                                                    int chunk, float *__restrict__ partials, uint8_t *lds,
                                                    const Role3 &ro, int w, uint32_t lane) {
@@ -535,10 +536,11 @@ __device__ __forceinline__ void gram_cplx256_chunk(const uint8_t *__restrict__ D
     const size_t kbeg = (size_t)chunk * chunk_len;
     const size_t kend = (kbeg + chunk_len < N) ? kbeg + chunk_len : N;
     const int nst = kend > kbeg ? (int)((kend - kbeg) / 32) : 0;
+    const int nb = (P + 31) >> 5;                            // blocks of 32 states
 
-    f32x4 re4[3][4], im4[3][4];
+    f32x4 re4[COUNT][4], im4[COUNT][4];
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
+    for (int i = 0; i < COUNT; i++) {
 #pragma unroll
         for (int q = 0; q < 4; q++)
 #pragma unroll
@@ -547,32 +549,37 @@ __device__ __forceinline__ void gram_cplx256_chunk(const uint8_t *__restrict__ D
                 im4[i][q][e] = 0.f;
             }
     }
-    if (nst > 0) issue_stage256(D, SB, P, kbeg, lds, w, lane);
+    if (nst > 0) issue_stage256(D, SB, P, nb, kbeg, lds, w, lane);
     for (int st = 0; st < nst; st++) {
         // this wave's loads of stage st have landed; after the barrier every wave's
         // have, and every wave is done with stage st - 1's buffer, which stage st + 1 refills
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (st + 1 < nst) issue_stage256(D, SB, P, kbeg + (size_t)(st + 1) * 32, lds + ((st + 1) & 1) * kBuf, w, lane);
-        stage_mfma3_16<PT, DIAG>(lds + (st & 1) * kBuf, ro, re4, im4, lane);
+        if (st + 1 < nst) issue_stage256(D, SB, P, nb, kbeg + (size_t)(st + 1) * 32, lds + ((st + 1) & 1) * kBuf, w, lane);
+        stage_mfma3_16<PT, DIAG, COUNT>(lds + (st & 1) * kBuf, ro, re4, im4, lane);
     }
     float *out = partials + (size_t)chunk * 3 * 2 * kTileElems;
     store_pair256_16(out, ro.a0, ro.b, re4[0], im4[0], lane);
-    store_pair256_16(out, ro.a1, ro.b, re4[1], im4[1], lane);
-    store_pair256_16(out, ro.a2, ro.b, re4[2], im4[2], lane);
+    if constexpr (COUNT > 1) store_pair256_16(out, ro.a1, ro.b, re4[1], im4[1], lane);
+    if constexpr (COUNT > 2) store_pair256_16(out, ro.a2, ro.b, re4[2], im4[2], lane);
 }
 
-// The wave's role decides the form once per chunk (a diagonal pair's waves
-// skip one sub-block), so each form keeps its own accumulator allocation.
+// The wave's role decides the form once per chunk (its pairs, and a diagonal
+// pair's skipped sub-block), so each form keeps its own accumulator allocation.
 template <int PT>
 __device__ __forceinline__ void gram_cplx256_unit(const uint8_t *__restrict__ D, int P, size_t N, size_t chunk_len,
                                                   int chunk, float *__restrict__ partials, uint8_t *lds) {
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t lane = threadIdx.x & 63;
-    const Role3 ro = wave_role3(w);
-    if (ro.a0 == ro.b) gram_cplx256_chunk<PT, true>(D, P, N, chunk_len, chunk, partials, lds, ro, w, lane);
-    else gram_cplx256_chunk<PT, false>(D, P, N, chunk_len, chunk, partials, lds, ro, w, lane);
+    const Role3 ro = kRoles256[((P + 31) >> 5) - 5][w];      // 129 <= P <= 256
+    const bool diag = ro.a0 == ro.b;
+#define QGTL_CHUNK(DIAG, COUNT) \
+    gram_cplx256_chunk<PT, DIAG, COUNT>(D, P, N, chunk_len, chunk, partials, lds, ro, w, lane)
+    if (ro.count == 3) { if (diag) QGTL_CHUNK(true, 3); else QGTL_CHUNK(false, 3); }
+    else if (ro.count == 2) { if (diag) QGTL_CHUNK(true, 2); else QGTL_CHUNK(false, 2); }
+    else { if (diag) QGTL_CHUNK(true, 1); else QGTL_CHUNK(false, 1); }
+#undef QGTL_CHUNK
 }
 
 template <int PT>
@@ -625,7 +632,7 @@ __global__ void mfma16_layout_probe_kernel(float *out) {
 // order with eight loads in flight, and wave 0 adds the eight sums in wave
 // order.
 // Group grp (64 adjacent entries of the tile-pair partials) of one reduction.
-__device__ __forceinline__ void gram_cplx_reduce_group(const float *__restrict__ partials, int nt, int nchunks,
+__device__ __forceinline__ void gram_cplx_reduce_group(const float *__restrict__ partials, int P, int nt, int nchunks,
                                                        double2 *__restrict__ G, size_t grp, double2 (*part)[64]) {
     constexpr int kGroups = kThreads / 64;                   // waves per entry, chunk stride
     const int T = nt * (nt + 1) / 2;
@@ -637,7 +644,8 @@ __device__ __forceinline__ void gram_cplx_reduce_group(const float *__restrict__
     const int r = e / kTileStates, c = e % kTileStates;
     int ti, tj;
     tile_coords(tile, nt, ti, tj);
-    const bool skip = ti == tj && (r >> 5) > (c >> 5);       // never written
+    // never written: below the diagonal blocks, past the last state's block
+    const bool skip = (ti == tj && (r >> 5) > (c >> 5)) || ti * kTileStates + r >= P || tj * kTileStates + c >= P;
     double sr = 0.0, si = 0.0;
     if (!skip) {
         const float *q = partials + (size_t)tile * 2 * kTileElems + e;
@@ -675,11 +683,11 @@ __device__ __forceinline__ void gram_cplx_reduce_group(const float *__restrict__
     __syncthreads();
 }
 
-__global__ __launch_bounds__(kThreads) void gram_cplx_reduce_kernel(const float *__restrict__ partials, int nt,
+__global__ __launch_bounds__(kThreads) void gram_cplx_reduce_kernel(const float *__restrict__ partials, int P, int nt,
                                                                     int nchunks, double2 *__restrict__ G) {
     __shared__ double2 part[kThreads / 64][64];
     const size_t ngrp = (size_t)(nt * (nt + 1) / 2) * kTileElems / 64;
-    for (size_t grp = blockIdx.x; grp < ngrp; grp += gridDim.x) gram_cplx_reduce_group(partials, nt, nchunks, G, grp, part);
+    for (size_t grp = blockIdx.x; grp < ngrp; grp += gridDim.x) gram_cplx_reduce_group(partials, P, nt, nchunks, G, grp, part);
 }
 
 // grouped: unit = one 64-entry group of an item (units per item: T * 256)
@@ -688,7 +696,8 @@ __global__ __launch_bounds__(kThreads) void gram_cplx_reduce_grouped_kernel(
     __shared__ double2 part[kThreads / 64][64];
     for (uint32_t u = blockIdx.x; u < units; u += gridDim.x) {
         const qgtl_gram_reduce_item_t it = items[qgtl::find_item(items, nitems, u)];
-        gram_cplx_reduce_group(qgtl::global_ptr<const float>(qgtl::uniform(it.partials)), qgtl::uniform(it.nt),
+        gram_cplx_reduce_group(qgtl::global_ptr<const float>(qgtl::uniform(it.partials)), (int)qgtl::uniform(it.states),
+                               qgtl::uniform(it.nt),
                                qgtl::uniform(it.nchunks), qgtl::global_ptr<double2>(qgtl::uniform(it.C)),
                                (size_t)(u - qgtl::uniform(it.unit_begin)), part);
     }
@@ -787,8 +796,8 @@ int qgtl_hip_gram_cplx_reduce(const float *partials, int P, int nchunks, double 
     const int nt = (P + kTileStates - 1) / kTileStates;
     const size_t total = (size_t)(nt * (nt + 1) / 2) * kTileElems;
     const unsigned grid = (unsigned)(total / 64);            // one 64-entry group per workgroup
-    hipLaunchKernelGGL(gram_cplx_reduce_kernel, dim3(grid), dim3(kThreads), 0, qgtl::stream(), partials, nt, nchunks,
-                       reinterpret_cast<double2 *>(G));
+    hipLaunchKernelGGL(gram_cplx_reduce_kernel, dim3(grid), dim3(kThreads), 0, qgtl::stream(), partials, P, nt,
+                       nchunks, reinterpret_cast<double2 *>(G));
     QGTL_LAUNCH_CHECK("gram_cplx_reduce");
     return 0;
 }

@@ -571,7 +571,7 @@ static int build_schedule(struct qgtl_batch *B)
             it[k].nt = in->nt;
             it[k].nchunks = in->nchunks;
             it[k].unit_begin = (uint32_t)u;
-            it[k].pad = 0;
+            it[k].states = (uint32_t)in->P + 1u;
             /* units: 256-element groups (real form), 64-entry groups (complex form) */
             u += (uint64_t)in->T * (form ? GRAM_TILE * GRAM_TILE / 64 : GRAM_TILE * GRAM_TILE / 256);
             k++;

@@ -422,7 +422,9 @@ static int gram_chunks_cplx(const struct qgtl_plan *p, size_t free_bytes)
     /* 129..256 states run one workgroup per chunk whose MFMA accumulators hold the whole
      * chunk (no outer fp32 sums): chunks of 1024 amplitudes bound the accumulation's rounding */
     size_t want = T == 3 ? p->N / 1024 : p->N / 2048;
-    const size_t minw = (512 + T - 1) / T;
+    /* at least one workgroup per CU: there is one per chunk then (at n = 17 it was 176 of 256), one
+     * per chunk and tile pair otherwise */
+    const size_t minw = T == 3 ? 256 : (512 + T - 1) / T;
     if (want < minw) want = minw;
     size_t budget = ((size_t)p->P + 1) * p->N * 8 / 16;
     if (budget > free_bytes / 2) budget = free_bytes / 2;
