@@ -96,27 +96,28 @@ __device__ __forceinline__ f32x16 mma(u32x4 a, u32x4 b, f32x16 c) {
 }
 
 // The blocks (of 32 states, within the tile) a wave multiplies: A blocks a0, a1
-// against B block b; which of the two pairs (a0, b), (a1, b) it computes (bits 0,
-// 1) is the template argument MASK of the code the wave runs.  Waves w and w + 4
-// share SIMD w % 4.  Off-diagonal tile pairs: A blocks 2 (w / 4), 2 (w / 4) + 1
-// against B block w % 4 (four pairs per SIMD).  Diagonal tile pairs: the 10
-// pairs (a, b), a <= b, as 2 + 1, 2 + 1, 2 + 0, 2 + 0 per SIMD.
+// against B block b, and which of the two pairs (a0, b), (a1, b) it computes
+// (mask bits 0, 1, the template argument MASK of the code the wave runs).  Waves
+// w and w + 4 share SIMD w % 4.  nb: blocks of the B tile that hold states (the
+// last tile may have fewer than four; the A tile of an off-diagonal pair is
+// full).  Off-diagonal tile pairs: 4 nb block pairs, equal per SIMD; diagonal
+// ones: the nb (nb + 1) / 2 pairs (a, b), a <= b, at most 3, 2, 1 or 1 per SIMD.
 struct Role {
-    int a0, a1, b;
+    int a0, a1, b, mask;
 };
 
-__device__ __forceinline__ Role wave_role(bool diag, int w) {
-    if (!diag) return Role{2 * (w >> 2), 2 * (w >> 2) + 1, w & 3};
-    switch (w) {
-    case 0: return Role{0, 1, 3};        // MASK 3: (0,3) (1,3)
-    case 1: return Role{2, 3, 3};        // MASK 3: (2,3) (3,3)
-    case 2: return Role{0, 1, 2};        // MASK 3: (0,2) (1,2)
-    case 3: return Role{0, 1, 1};        // MASK 3: (0,1) (1,1)
-    case 4: return Role{0, 0, 0};        // MASK 1: (0,0)
-    case 5: return Role{2, 2, 2};        // MASK 1: (2,2)
-    default: return Role{0, 0, 0};       // MASK 0: loads and barriers only
-    }
-}
+__device__ constexpr Role kRolesOff[4][8] = {
+    {{0, 0, 0, 1}, {1, 1, 0, 1}, {2, 2, 0, 1}, {3, 3, 0, 1}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}},
+    {{0, 0, 0, 1}, {1, 1, 0, 1}, {2, 2, 0, 1}, {3, 3, 0, 1}, {0, 0, 1, 1}, {1, 1, 1, 1}, {2, 2, 1, 1}, {3, 3, 1, 1}},
+    {{0, 1, 0, 3}, {0, 1, 1, 3}, {0, 1, 2, 3}, {2, 3, 0, 3}, {2, 2, 1, 1}, {3, 3, 1, 1}, {2, 2, 2, 1}, {3, 3, 2, 1}},
+    {{0, 1, 0, 3}, {0, 1, 1, 3}, {0, 1, 2, 3}, {0, 1, 3, 3}, {2, 3, 0, 3}, {2, 3, 1, 3}, {2, 3, 2, 3}, {2, 3, 3, 3}},
+};
+__device__ constexpr Role kRolesDiag[4][8] = {
+    {{0, 0, 0, 1}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}},
+    {{0, 0, 1, 1}, {1, 1, 1, 1}, {0, 0, 0, 1}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}},
+    {{0, 1, 2, 3}, {0, 1, 1, 3}, {2, 2, 2, 1}, {0, 0, 0, 1}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}},
+    {{0, 1, 3, 3}, {2, 3, 3, 3}, {0, 1, 2, 3}, {0, 1, 1, 3}, {0, 0, 0, 1}, {2, 2, 2, 1}, {0, 0, 0, 0}, {0, 0, 0, 0}},
+};
 
 // fragment of block blk, piece p (0 hi, 1 lo), K-step t: lane l reads row
 // 32 blk + l % 32, logical slot S/2 p + 2 t + l / 32
@@ -204,12 +205,15 @@ __device__ __forceinline__ void flush(Acc &acc, Acc &outer) {
 // asm so that the addresses are formed at every stage instead of being hoisted
 // out of the loop (where they would hold registers the accumulators need).
 template <int SA>
-__device__ __forceinline__ void issue_tile(const uint8_t *__restrict__ D, size_t SB, int P, int s0, size_t k0,
+__device__ __forceinline__ void issue_tile(const uint8_t *__restrict__ D, size_t SB, int P, int s0, int nb, size_t k0,
                                            uint8_t *lds, int w, int rr, uint32_t in_blk) {
     typedef Geo<SA> G;
     const size_t ko = (k0 >> 6) * 512 + (k0 & 63) * 4 + in_blk;
 #pragma unroll
     for (int i = 0; i < G::kLoads; i++) {
+        // with stages of 32 amplitudes load i is block i; blocks without states are left out
+        // (stages of 16 count the loads in flight, so they issue them all)
+        if (SA == 32 && i >= nb) break;
         int st = s0 + rr + 8 * G::kRowsPerLoad * i;
         __asm__ volatile("" : "+v"(st));
         st = st < P ? st : P - 1;
@@ -244,12 +248,12 @@ __device__ __forceinline__ void wait_stage(int ahead) {
 template <int SA, int PT, bool DIAG, int MASK>
 __device__ __forceinline__ void gram_cplx_unit(const uint8_t *__restrict__ D, int P, size_t N, int T, int tile,
                                                int chunk, int ti, int tj, size_t chunk_len, int w,
-                                               float *__restrict__ partials, uint8_t *lds) {
+                                               int nb, const Role &ro, float *__restrict__ partials,
+                                               uint8_t *lds) {
     typedef Geo<SA> G;
     constexpr int BUFS = G::kBufs;
     constexpr int LW = DIAG ? G::kLoads : 2 * G::kLoads;   // loads per wave and stage
     const uint32_t lane = threadIdx.x & 63;
-    const Role ro = wave_role(DIAG, w);
     // load constants: row rr of each load's row group and the logical slot its stored slot holds
     const int rr = G::kRowsPerLoad * w + (int)(lane / G::kSlots);
     const uint32_t lgc = (lane % G::kSlots) ^ G::swz((uint32_t)rr);
@@ -276,8 +280,8 @@ __device__ __forceinline__ void gram_cplx_unit(const uint8_t *__restrict__ D, in
     auto bufB = [&](int b) { return lds + (size_t)b * 2 * G::kTileBytes + G::kTileBytes; };
     auto issue = [&](int st, int b) {
         const size_t k0 = kbeg + (size_t)st * SA;
-        issue_tile<SA>(D, SB, P, sa, k0, bufA(b), w, rr, in_blk);
-        if (!DIAG) issue_tile<SA>(D, SB, P, sb, k0, bufB(b), w, rr, in_blk);
+        issue_tile<SA>(D, SB, P, sa, DIAG ? nb : 4, k0, bufA(b), w, rr, in_blk);
+        if (!DIAG) issue_tile<SA>(D, SB, P, sb, nb, k0, bufB(b), w, rr, in_blk);
     };
     // stage st in buffer B: wait for it, release the buffer of stage st - 1 for
     // stage st + BUFS - 1, multiply
@@ -332,14 +336,21 @@ __global__ __launch_bounds__(kThreads, 1) void gram_cplx_kernel(const uint8_t *_
     int ti, tj;
     tile_coords(tile, nt, ti, tj);
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    if (ti != tj)
-        gram_cplx_unit<SA, PT, false, 3>(D, P, N, T, tile, chunk, ti, tj, chunk_len, w, partials, lds);
-    else if (w < 4)
-        gram_cplx_unit<SA, PT, true, 3>(D, P, N, T, tile, chunk, ti, tj, chunk_len, w, partials, lds);
-    else if (w < 6)
-        gram_cplx_unit<SA, PT, true, 1>(D, P, N, T, tile, chunk, ti, tj, chunk_len, w, partials, lds);
-    else
-        gram_cplx_unit<SA, PT, true, 0>(D, P, N, T, tile, chunk, ti, tj, chunk_len, w, partials, lds);
+    const int left = P - tj * kTileStates, nb = left >= kTileStates ? 4 : (left + 31) >> 5;
+    const bool diag = ti == tj;
+    const Role ro = diag ? kRolesDiag[nb - 1][w] : kRolesOff[nb - 1][w];
+#define QGTL_UNIT(DIAG, MASK) \
+    gram_cplx_unit<SA, PT, DIAG, MASK>(D, P, N, T, tile, chunk, ti, tj, chunk_len, w, nb, ro, partials, lds)
+    if (diag) {
+        if (ro.mask == 3) QGTL_UNIT(true, 3);
+        else if (ro.mask == 1) QGTL_UNIT(true, 1);
+        else QGTL_UNIT(true, 0);
+    } else {
+        if (ro.mask == 3) QGTL_UNIT(false, 3);
+        else if (ro.mask == 1) QGTL_UNIT(false, 1);
+        else QGTL_UNIT(false, 0);
+    }
+#undef QGTL_UNIT
 }
 
 // ---------------------------------------------------------------------------
