@@ -23,7 +23,12 @@
 
 #include "qgtl_internal.h"
 
-#define CMIN_LOW_BITS 5   /* contiguous low bits kept in every high-qubit pass (256-B runs) */
+/* Contiguous low bits of a high-qubit pass: five (256-byte runs), or CMIN_LOW_BITS
+ * (128 bytes, a cache line) where that saves a second such pass.  At n = 22, L = 6 the sweep takes
+ * 7.5 ms with one pass over nine qubits and 9.7 ms with two; runs shorter than a line lose more than
+ * the pass (n = 23 with 64 bytes 25 ms against 20.6, n = 24 with 32 bytes 122 against 45). */
+#define CLOW_BITS 5
+#define CMIN_LOW_BITS 4
 
 static qgtl_cd cd(double re, double im) { qgtl_cd z = {re, im}; return z; }
 static qgtl_cd cmul(qgtl_cd a, qgtl_cd b) { return cd(a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re); }
@@ -501,15 +506,15 @@ static void plan_phases(qgtl_pass_desc_t *p)
 }
 
 /* High-qubit passes of a block with n > 13: the qubits >= 13
- * that carry a gate, in groups that leave CMIN_LOW_BITS contiguous low bits
- * in the tile; in place. */
+ * that carry a gate, in groups that leave CLOW_BITS contiguous low bits in the
+ * tile (one group where CMIN_LOW_BITS do); in place. */
 static void high_passes(const qgtl_block_t *b, int n, qgtl_pass_desc_t *out, int *flips, int *count)
 {
     const int TB = QGTL_TILE_BITS_MAX;
     int hq[QGTL_MAX_QUBITS], nh = 0;
     for (int q = TB; q < n; q++)
         if (b->has_u[q]) hq[nh++] = q;
-    const int group = TB - CMIN_LOW_BITS;
+    const int group = nh == TB - CMIN_LOW_BITS ? nh : TB - CLOW_BITS;
     for (int g0 = 0; g0 < nh; g0 += group) {
         const int len = (nh - g0 < group) ? nh - g0 : group;
         const int c = TB - len;
