@@ -29,7 +29,8 @@ typedef struct { float re, im; } qgtl_c64_t;
 enum {
     QGTL_STORE_INPLACE = 0,   /* write the tile back where it was read */
     QGTL_STORE_RING = 1,      /* tile = bits 0..m-1; apply CNOT(i->i+1 mod n), i ascending, while storing */
-    QGTL_STORE_PERM = 2       /* whole state in one tile; apply perm_* (CNOT/SWAP list) while storing */
+    QGTL_STORE_PERM = 2,      /* whole state in one tile; apply perm_* (CNOT/SWAP/CZ list) while storing */
+    QGTL_STORE_LINEAR = 3     /* tile = bits 0..m-1; apply the index map mstage (register pass only) while storing */
 };
 
 enum {
@@ -38,6 +39,25 @@ enum {
                                  store would have written it to (the inverse ring), register pass only,
                                  not in place, natural store */
 };
+
+/* An M-stage of a register pass over bits 0..12 of a wider state: CNOT, SWAP
+ * and CZ gates as out[M x] = (-1)^{q(x)} in[x], M a GF(2)-linear map and q a
+ * quadratic form of the index.  With x = (x_l, r), r the tile index: y_l = a x_l
+ * + b r is a bijection within the tile, and the output's high bits are e y_l + f r.
+ * a, b, e, f: columns (the image of one bit).  e is zero but for the bits 4, 5,
+ * 6, 11 and 12 (thread bits of the coalesced layout, a cache line and more
+ * contiguous).  reg: the images under a of the register bits of the last
+ * phase's layout.  q(x) = sum over i of x_i
+ * parity(sgn[i] & x), sgn[i] within bits i..n-1; sgn_reg (bit R: q of register
+ * index R) and sgn_bil (rows of q's polar form at the register bits) are its
+ * register part. */
+typedef struct {
+    uint32_t a[QGTL_TILE_BITS_MAX], b[QGTL_MAX_QUBITS - QGTL_TILE_BITS_MAX];
+    uint32_t e[QGTL_TILE_BITS_MAX], f[QGTL_MAX_QUBITS - QGTL_TILE_BITS_MAX];
+    uint32_t reg[5];
+    uint32_t sgn[QGTL_MAX_QUBITS];
+    uint32_t sgn_reg, sgn_bil[5];
+} qgtl_mstage_t;
 
 /* One LDS-tiled sweep pass: a set of commuting 2x2 matrices on tile bits,
  * followed by an optional index permutation on store. */
@@ -54,9 +74,15 @@ typedef struct {
     int32_t hi_pos[QGTL_TILE_BITS_MAX];        /* physical bit of tile bit nlow+i */
     int32_t rest_pos[QGTL_MAX_QUBITS];         /* physical bit of tile-index bit i */
     int32_t gate_bit[QGTL_TILE_BITS_MAX];      /* tile bit of matrix g */
-    int32_t perm_type[QGTL_PERM_MAX];          /* 0 = CNOT(a -> b), 1 = SWAP(a, b) */
-    int32_t perm_a[QGTL_PERM_MAX];
-    int32_t perm_b[QGTL_PERM_MAX];
+    int32_t sign;                              /* mstage's sign, applied before the store */
+    union {
+        struct {                               /* QGTL_STORE_PERM */
+            int32_t perm_type[QGTL_PERM_MAX];  /* 0 = CNOT(a -> b), 1 = SWAP(a, b), 2 = CZ(a, b) */
+            int32_t perm_a[QGTL_PERM_MAX];
+            int32_t perm_b[QGTL_PERM_MAX];
+        };
+        qgtl_mstage_t mstage;                  /* QGTL_STORE_LINEAR, sign != 0 */
+    };
     qgtl_c64_t mat[QGTL_TILE_BITS_MAX][4];     /* row-major 2x2 */
     /* Register-phase plan (full 2^13 tiles): 32 amplitudes per thread; in
      * phase p the tile bits ph_rbits[p][0..4] index a thread's registers and
@@ -138,20 +164,23 @@ typedef struct {
 } qgtl_pass_desc_t;
 
 /* Derivative-state injection in the frame after a block:
- * d_k[y] = A_k[s][s] psi[y] + A_k[s][1-s] psi[y ^ v_k], s = parity(y & w_k). */
+ * d_k[y] = A_k[s][s] psi[y] + (-1)^{parity(y & z_k)} A_k[s][1-s] psi[y ^ v_k],
+ * s = parity(y & w_k); z_k = 0 unless the block's M-stage has CZ gates on the
+ * parameter's qubit. */
 typedef struct {
     int32_t n;
     int32_t K;
     uint32_t v[QGTL_INJECT_MAX];
     uint32_t w[QGTL_INJECT_MAX];
+    uint32_t z[QGTL_INJECT_MAX];
     qgtl_c64_t A[QGTL_INJECT_MAX][4];
 } qgtl_inject_desc_t;
 
 /* One derivative state for a pass that forms it while loading (see
- * qgtl_hip_pass_c64_inject): element y is M[s][s] psi[y] + M[s][1-s]
- * psi[y ^ v], s = parity(y & w), M row-major. */
+ * qgtl_hip_pass_c64_inject): element y is M[s][s] psi[y] + (-1)^{parity(y & z)}
+ * M[s][1-s] psi[y ^ v], s = parity(y & w), M row-major. */
 typedef struct {
-    uint32_t v, w;
+    uint32_t v, w, z, pad;
     qgtl_c64_t M[4];
 } qgtl_inject_slot_t;
 
@@ -164,7 +193,9 @@ typedef struct {
  * over qubits 0..6 (128 entries) and 7..12 (64), their product taken at a
  * thread's bits, times reg_post (reg_pre): the products of the phase ratios over the
  * register bits of the last group of four qubits, n-4 .. n-1 (of the first,
- * 0 .. 3).  img[q]: image of basis bit q under the M-stage (GF(2)-linear). */
+ * 0 .. 3).  img[q]: image of basis bit q under the M-stage (GF(2)-linear); sgn,
+ * sgn_reg, sgn_bil: its sign, as in qgtl_mstage_t, for the register bits of
+ * the last group. */
 #define QGTL_RES_MIN_QUBITS 4
 #define QGTL_RES_MAX_QUBITS 13
 #define QGTL_RES_TAB 192                       /* complex64 entries: post tables, then as many for pre */
@@ -172,7 +203,8 @@ typedef struct {
     float tan[QGTL_RES_MAX_QUBITS];
     int32_t swapped[QGTL_RES_MAX_QUBITS];
     uint32_t img[QGTL_RES_MAX_QUBITS];
-    int32_t has_pre, has_perm;
+    int32_t has_pre, has_perm, has_sign;
+    uint32_t sgn[QGTL_RES_MAX_QUBITS], sgn_reg, sgn_bil[4];
     qgtl_c64_t reg_pre[16], reg_post[16];
 } qgtl_res_block_t;
 
@@ -181,16 +213,16 @@ typedef struct {
     uint32_t v, w;
     qgtl_c64_t M[4];
     int32_t block;
-    int32_t pad;
+    uint32_t z;
 } qgtl_res_slot_t;
 
 /* The P derivative states at the end of the circuit (D, stride 2^n, slot
  * order), the primal state (psi) and the FP64 injection sums (P x 4).  blocks:
  * nblocks descriptors; tabs: 2 QGTL_RES_TAB complex64 per block; slots: P + 1
- * in block order, the last one (the primal state) with block = nblocks.  All
- * on the device. */
+ * in block order, the last one (the primal state) with block = nblocks; signs:
+ * some block has has_sign.  All on the device. */
 int qgtl_hip_resident_states(int n, const void *blocks, int nblocks, const void *tabs, const void *slots, int P,
-                             void *D, void *psi, double *sums);
+                             int signs, void *D, void *psi, double *sums);
 
 /* ---- grouped launches ----
  * One launch runs the same kind of work for many independent instances.
@@ -356,13 +388,15 @@ int qgtl_hip_inject_c64(const qgtl_inject_desc_t *desc, const void *psi, void *d
 /* the FP64 sums of qgtl_hip_inject_c64 only (the states are not written) */
 int qgtl_hip_inject_sums_c64(const qgtl_inject_desc_t *desc, const void *psi, double *partials, int *tiles_out);
 /* qgtl_hip_pass_c64 on nstates derivative states formed while loading from the
- * one state psi: state s uses slots[s] (device array); register passes only */
+ * one state psi: state s uses slots[s] (device array), signs: some slot has
+ * z != 0; register passes only */
 int qgtl_hip_pass_c64_inject(const qgtl_pass_desc_t *desc, const void *psi, const void *slots, void *dst,
-                             size_t stride, int nstates, int split_out, const void *tabs);
+                             size_t stride, int nstates, int split_out, int signs, const void *tabs);
 /* out[k*4 + c] = sum over t of partials[(k*tiles + t)*4 + c], fixed order, FP64 */
 int qgtl_hip_reduce_partials_f64(const double *partials, int K, int tiles, double *out);
 int qgtl_hip_cnot_c64(void *base, size_t stride, int nstates, int n, int c, int t);
 int qgtl_hip_swap_c64(void *base, size_t stride, int nstates, int n, int a, int b);
+int qgtl_hip_cz_c64(void *base, size_t stride, int nstates, int n, int a, int b);
 int qgtl_hip_c64_to_c128(const void *src, void *dst, size_t count);
 int qgtl_hip_fill_f32(void *dst, size_t count, float value);
 int qgtl_hip_copy_f32x4(void *dst, const void *src, size_t count16);    /* count16 units of 16 bytes */

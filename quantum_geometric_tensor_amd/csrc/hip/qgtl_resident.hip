@@ -49,6 +49,12 @@ __device__ __forceinline__ float2 cmadd(float2 acc, float2 a, float2 b) {
     return acc;
 }
 
+// z with the sign (-1)^n
+__device__ __forceinline__ float2 flip_sign(float2 z, uint32_t n) {
+    const uint32_t m = n << 31;
+    return make_float2(__uint_as_float(__float_as_uint(z.x) ^ m), __uint_as_float(__float_as_uint(z.y) ^ m));
+}
+
 // A rotation [[c, -s], [s, c]] on register bit I with its larger entry taken
 // out (the block's phase table carries it): |t| <= 1, one multiply-add per
 // component and no copies in either branch.
@@ -94,7 +100,7 @@ struct Shape {
 };
 
 // Gates of group G (bits max(base, 4 G) .. base + 3), and on.
-template <int NQ, int G>
+template <int NQ, int G, bool SIGN>
 __device__ __forceinline__ void groups(const qgtl_res_block_t &b, float2 *tile, uint32_t t, float2 pre, float2 post) {
     typedef Shape<NQ> S;
     if constexpr (G < S::kGroups) {
@@ -115,6 +121,18 @@ __device__ __forceinline__ void groups(const qgtl_res_block_t &b, float2 *tile, 
         if constexpr (G + 1 == S::kGroups) {
 #pragma unroll
             for (int r = 0; r < 16; r++) v[r] = cmul(v[r], cmul(post, make_float2(b.reg_post[r].re, b.reg_post[r].im)));
+            if (SIGN && b.has_sign) {
+                // (-1)^{q(j)}: q(j0 + r) = q(j0) + q(r) + the polar form of both
+                uint32_t acc = 0;
+#pragma unroll
+                for (int i = 0; i < NQ; i++) acc ^= (0u - ((j0 >> i) & 1u)) & b.sgn[i];
+                constexpr uint32_t kBit[4] = {0xaaaau, 0xccccu, 0xf0f0u, 0xff00u};
+                uint32_t neg = b.sgn_reg ^ (0u - ((uint32_t)__popc(acc & j0) & 1u));
+#pragma unroll
+                for (int i = 0; i < 4; i++) neg ^= (0u - ((uint32_t)__popc(b.sgn_bil[i] & j0) & 1u)) & kBit[i];
+#pragma unroll
+                for (int r = 0; r < 16; r++) v[r] = flip_sign(v[r], neg >> r);
+            }
             if (b.has_perm) {
                 // element j goes to pi(j), the XOR of the images of its bits
                 uint32_t p = j0 & ~((1u << NQ) - 1u);        // the state's number in the tile
@@ -138,14 +156,15 @@ __device__ __forceinline__ void groups(const qgtl_res_block_t &b, float2 *tile, 
 #pragma unroll
         for (int r = 0; r < 16; r++) tile[l0 ^ rpad((uint32_t)r << B)] = v[r];
         __syncthreads();
-        groups<NQ, G + 1>(b, tile, t, pre, post);
+        groups<NQ, G + 1, SIGN>(b, tile, t, pre, post);
     }
 }
 
 // States blockIdx.x * kStates .. of the P derivative states (slot order) and
 // the primal state (number P): D receives the former, psi the latter, sums
-// (4 doubles per slot) the FP64 injection sums.
-template <int NQ>
+// (4 doubles per slot) the FP64 injection sums.  SIGN: some block's M-stage has
+// CZ gates (a variant of its own: it costs 16 registers, and n = 13 has 12 left).
+template <int NQ, bool SIGN>
 __global__ __launch_bounds__(Shape<NQ>::kThreads) void resident_states_kernel(
     const qgtl_res_block_t *__restrict__ blocks, int nblocks, const float2 *__restrict__ tabs,
     const qgtl_res_slot_t *__restrict__ slots, int P, float2 *__restrict__ D, float2 *__restrict__ psi,
@@ -176,9 +195,9 @@ __global__ __launch_bounds__(Shape<NQ>::kThreads) void resident_states_kernel(
         const float2 post = cmul(tb[yl & 127u], tb[128u + (yl >> 7)]);
         float2 pre = make_float2(1.f, 0.f);
         if (b.has_pre) pre = cmul(tb[QGTL_RES_TAB + (y0 & 127u)], tb[QGTL_RES_TAB + 128u + (y0 >> 7)]);
-        groups<NQ, 0>(b, tile, t, pre, post);
+        groups<NQ, 0, SIGN>(b, tile, t, pre, post);
         if (bi < blk_first || bi > blk_last) continue;        // uniform: slots are in block order
-        // d[y] = M[s][s] psi[y] + M[s][1 - s] psi[y ^ v], s = parity(y & w)
+        // d[y] = M[s][s] psi[y] + (-1)^parity(y & z) M[s][1 - s] psi[y ^ v], s = parity(y & w)
         const bool mine = q.block == bi;
         double sr = 0.0, si = 0.0, sd = 0.0, sp = 0.0;
         float2 o[16];
@@ -188,11 +207,13 @@ __global__ __launch_bounds__(Shape<NQ>::kThreads) void resident_states_kernel(
             const float2 m00 = make_float2(q.M[0].re, q.M[0].im), m01 = make_float2(q.M[1].re, q.M[1].im);
             const float2 m10 = make_float2(q.M[2].re, q.M[2].im), m11 = make_float2(q.M[3].re, q.M[3].im);
             const uint32_t lv = l0 ^ rpad(q.v);
-            const uint32_t s0 = (uint32_t)__popc(y0 & q.w);
+            const uint32_t s0 = (uint32_t)__popc(y0 & q.w), z0 = (uint32_t)__popc(y0 & q.z);
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const bool sg = ((s0 + (uint32_t)__popc((uint32_t)r & q.w)) & 1u) != 0;
-                const float2 a = o[r], p = tile[lv ^ (uint32_t)r];
+                const float2 a = o[r];
+                float2 p = tile[lv ^ (uint32_t)r];
+                if constexpr (SIGN) p = flip_sign(p, z0 + (uint32_t)__popc((uint32_t)r & q.z));
                 const float2 d = cmadd(cmadd(make_float2(0.f, 0.f), sg ? m11 : m00, a), sg ? m10 : m01, p);
                 const double dr = d.x, di = d.y, pr = a.x, pi = a.y;
                 sr += dr * pr + di * pi;
@@ -238,12 +259,12 @@ __global__ __launch_bounds__(Shape<NQ>::kThreads) void resident_states_kernel(
     }
 }
 
-template <int NQ>
+template <int NQ, bool SIGN>
 int launch(const void *blocks, int nblocks, const void *tabs, const void *slots, int P, void *D, void *psi,
            double *sums) {
     typedef Shape<NQ> S;
     const unsigned grid = (unsigned)((P + 1 + S::kStates - 1) / S::kStates);
-    hipLaunchKernelGGL(resident_states_kernel<NQ>, dim3(grid), dim3(S::kThreads), 0, qgtl::stream(),
+    hipLaunchKernelGGL((resident_states_kernel<NQ, SIGN>), dim3(grid), dim3(S::kThreads), 0, qgtl::stream(),
                        (const qgtl_res_block_t *)blocks, nblocks, (const float2 *)tabs,
                        (const qgtl_res_slot_t *)slots, P, (float2 *)D, (float2 *)psi, sums);
     QGTL_LAUNCH_CHECK("resident_states");
@@ -255,22 +276,27 @@ int launch(const void *blocks, int nblocks, const void *tabs, const void *slots,
 extern "C" {
 
 int qgtl_hip_resident_states(int n, const void *blocks, int nblocks, const void *tabs, const void *slots, int P,
-                             void *D, void *psi, double *sums) {
+                             int signs, void *D, void *psi, double *sums) {
     if (!blocks || !tabs || !slots || !D || !psi || !sums || nblocks < 1 || P < 1)
         return qgtl::set_error_msg(-118, "qgtl_hip_resident_states: bad arguments");
+#define QGTL_RES_CASE(N)                                                                                     \
+    case N:                                                                                                  \
+        return signs ? launch<N, true>(blocks, nblocks, tabs, slots, P, D, psi, sums)                        \
+                     : launch<N, false>(blocks, nblocks, tabs, slots, P, D, psi, sums)
     switch (n) {
-    case 4: return launch<4>(blocks, nblocks, tabs, slots, P, D, psi, sums);
-    case 5: return launch<5>(blocks, nblocks, tabs, slots, P, D, psi, sums);
-    case 6: return launch<6>(blocks, nblocks, tabs, slots, P, D, psi, sums);
-    case 7: return launch<7>(blocks, nblocks, tabs, slots, P, D, psi, sums);
-    case 8: return launch<8>(blocks, nblocks, tabs, slots, P, D, psi, sums);
-    case 9: return launch<9>(blocks, nblocks, tabs, slots, P, D, psi, sums);
-    case 10: return launch<10>(blocks, nblocks, tabs, slots, P, D, psi, sums);
-    case 11: return launch<11>(blocks, nblocks, tabs, slots, P, D, psi, sums);
-    case 12: return launch<12>(blocks, nblocks, tabs, slots, P, D, psi, sums);
-    case 13: return launch<13>(blocks, nblocks, tabs, slots, P, D, psi, sums);
+    QGTL_RES_CASE(4);
+    QGTL_RES_CASE(5);
+    QGTL_RES_CASE(6);
+    QGTL_RES_CASE(7);
+    QGTL_RES_CASE(8);
+    QGTL_RES_CASE(9);
+    QGTL_RES_CASE(10);
+    QGTL_RES_CASE(11);
+    QGTL_RES_CASE(12);
+    QGTL_RES_CASE(13);
     default: return qgtl::set_error_msg(-118, "qgtl_hip_resident_states: needs 4 <= n <= 13");
     }
+#undef QGTL_RES_CASE
 }
 
 }  // extern "C"

@@ -5,8 +5,9 @@
 // matrices on tile bits (three at a time from registers, so one LDS round
 // trip serves three gates), and stores the tile, optionally through an index
 // permutation: the CNOT ring of the hardware-efficient ansatz
-// (CNOT(i -> i+1 mod n), i ascending) or, when the whole state is one tile,
-// any CNOT/SWAP list.  Counterparts in QGTL: the per-gate loops
+// (CNOT(i -> i+1 mod n), i ascending), another CNOT/SWAP stage whose map is a
+// bijection within the tiles (the linear store, with the CZ gates' sign) or, when the whole
+// state is one tile, any CNOT/SWAP/CZ list.  Counterparts in QGTL: the per-gate loops
 // apply_rotation_y/z and apply_controlled_x
 // (src/quantum_geometric/core/quantum_circuit_operations.c:171-265) and
 // apply_single_qubit_gate / apply_cnot_gate
@@ -17,6 +18,14 @@
 // (bits m..n-1), the low output bits depend on the tile only, and the output
 // high bits are prefix_xor(r), complemented when y_{m-1} = 1.  The tile thus
 // lands in two contiguous half tiles: every store is coalesced.
+//
+// Linear store: the tile's output index and sign come from the descriptor's
+// columns, thread part once per thread, register part uniform, so a whole
+// entangling stage costs a pass about 100 instructions a thread and no memory
+// traffic, where one kernel per gate read and wrote half of every state.  A CZ is a sign
+// of the index and ends no block; as H CNOT H it started a new block of two passes for every gate
+// of a line.  Four layers of random gates with CNOT and CZ lines, n = 15, P = 120: 196 launches
+// and 1.41 ms, now 32 and 0.35 ms.
 #include "qgtl_hip_common.h"
 
 namespace {
@@ -290,13 +299,15 @@ __device__ __forceinline__ void pass_lds_body(const qgtl_pass_desc_t &d, const f
             float2 o[2];
 #pragma unroll
             for (int e = 0; e < 2; e++) {
-                uint32_t x = 2u * (uint32_t)p + (uint32_t)e;
+                uint32_t x = 2u * (uint32_t)p + (uint32_t)e, neg = 0;
                 for (int i = d.nperm - 1; i >= 0; i--) {
                     const uint32_t ab = (x >> d.perm_a[i]) & 1u, bb = (x >> d.perm_b[i]) & 1u;
                     if (d.perm_type[i] == 0) x ^= ab << d.perm_b[i];              // CNOT a -> b
-                    else x ^= (ab ^ bb) * ((1u << d.perm_a[i]) | (1u << d.perm_b[i]));  // SWAP
+                    else if (d.perm_type[i] == 1) x ^= (ab ^ bb) * ((1u << d.perm_a[i]) | (1u << d.perm_b[i]));  // SWAP
+                    else neg ^= ab & bb;                                          // CZ
                 }
                 o[e] = tile[lds_pad((int)x)];
+                if (neg) o[e] = make_float2(-o[e].x, -o[e].y);
                 if (rotf) o[e] = cmul(o[e], phase_at(post_tab, x));
             }
             *reinterpret_cast<float4 *>(dst + 2 * p) = make_float4(o[0].x, o[0].y, o[1].x, o[1].y);
@@ -409,6 +420,23 @@ __device__ __forceinline__ RingLds ring_lds(const RegLayout &L, uint32_t par_r, 
     return q;
 }
 
+// word where bit is 1, else 0
+__device__ __forceinline__ uint32_t pick(uint32_t bit, uint32_t word) { return (0u - bit) & word; }
+
+// The same for the linear map d.mstage, con the tile's constant.
+__device__ __forceinline__ RingLds linear_lds(const qgtl_pass_desc_t &d, const RegLayout &L, uint32_t con,
+                                              uint32_t xm = 0) {
+    const uint32_t x = L.tdep ^ xm;
+    uint32_t y = con;
+#pragma unroll
+    for (int i = 0; i < kRT; i++) y ^= pick((x >> i) & 1u, d.mstage.a[i]);
+    RingLds q;
+    q.base = (uint32_t)rpad(y) << 3;
+#pragma unroll
+    for (int i = 0; i < 5; i++) q.bit[i] = (uint32_t)rpad(d.mstage.reg[i]) << 3;
+    return q;
+}
+
 template <int R>
 __device__ __forceinline__ uint32_t ring_index(const RingLds &q) {
     uint32_t u = 0;
@@ -468,6 +496,20 @@ __device__ __forceinline__ GlobalMap natural_map(const RegLayout &L, uint32_t ba
 __device__ __forceinline__ GlobalMap ring_map(const RegLayout &L, uint32_t pre, uint32_t ones) {
     GlobalMap g;
     const uint32_t yhi = ((L.tdep >> (kRT - 1)) & 1u) ? (pre ^ ones) : pre;
+    g.lane = ((size_t)yhi << kRT) | L.tdep;
+#pragma unroll
+    for (int i = 0; i < 5; i++) g.bit[i] = L.rb[i];
+    return g;
+}
+
+// linear placement of tile r: the high part of y is pre (f r) plus the images
+// of the thread bits the map allows
+__device__ __forceinline__ GlobalMap linear_map(const qgtl_pass_desc_t &d, const RegLayout &L, uint32_t pre) {
+    uint32_t yhi = pre;
+    constexpr int kMay[5] = {4, 5, 6, 11, 12};
+#pragma unroll
+    for (int i = 0; i < 5; i++) yhi ^= pick((L.tdep >> kMay[i]) & 1u, d.mstage.e[kMay[i]]);
+    GlobalMap g;
     g.lane = ((size_t)yhi << kRT) | L.tdep;
 #pragma unroll
     for (int i = 0; i < 5; i++) g.bit[i] = L.rb[i];
@@ -568,6 +610,12 @@ __device__ __forceinline__ void apply_phase_mat(float2 (&v)[kRegs], const qgtl_p
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
+// z with the sign (-1)^n
+__device__ __forceinline__ float2 flip_sign(float2 z, uint32_t n) {
+    const uint32_t m = n << 31;
+    return make_float2(__uint_as_float(__float_as_uint(z.x) ^ m), __uint_as_float(__float_as_uint(z.y) ^ m));
+}
+
 // 16-byte global load / store of two amplitudes; NT: non-temporal (streamed
 // through the caches: each state is read and written once per pass)
 template <bool NT>
@@ -649,16 +697,22 @@ struct RegLoop {
     // derivative state formed while loading: element y of the state is
     // M[s][s] psi[y] + M[s][1-s] psi[y ^ v], s = parity(y & w), the same
     // arithmetic as the injection kernel (psi is shared by every state of the
-    // launch and read through the caches)
+    // launch and read through the caches).  SIGN: the partner with the sign (-1)^parity(y & z)
+    template <bool SIGN = false>
     __device__ __forceinline__ static void load_global_inject(const float2 *psi, const GlobalMap &g,
                                                               const qgtl_inject_slot_t &q, float2 (&v)[kRegs]) {
-        RegLoop<R - 2>::load_global_inject(psi, g, q, v);
+        RegLoop<R - 2>::template load_global_inject<SIGN>(psi, g, q, v);
         const size_t a = global_index<R - 2>(g);
         const float4 qa = *reinterpret_cast<const float4 *>(psi + a);
         const float4 qb = *reinterpret_cast<const float4 *>(psi + ((a ^ (size_t)q.v) & ~(size_t)1));
         const bool odd = (q.v & 1u) != 0;
-        const float2 b0 = odd ? make_float2(qb.z, qb.w) : make_float2(qb.x, qb.y);
-        const float2 b1 = odd ? make_float2(qb.x, qb.y) : make_float2(qb.z, qb.w);
+        float2 b0 = odd ? make_float2(qb.z, qb.w) : make_float2(qb.x, qb.y);
+        float2 b1 = odd ? make_float2(qb.x, qb.y) : make_float2(qb.z, qb.w);
+        if constexpr (SIGN) {
+            const uint32_t n0 = (uint32_t)__popc((uint32_t)a & q.z);
+            b0 = flip_sign(b0, n0);
+            b1 = flip_sign(b1, n0 + (q.z & 1u));
+        }
         const bool s0 = (__popc((uint32_t)a & q.w) & 1) != 0, s1 = s0 != ((q.w & 1u) != 0);
         const float2 m00 = make_float2(q.M[0].re, q.M[0].im), m01 = make_float2(q.M[1].re, q.M[1].im);
         const float2 m10 = make_float2(q.M[2].re, q.M[2].im), m11 = make_float2(q.M[3].re, q.M[3].im);
@@ -711,6 +765,7 @@ struct RegLoop<0> {
     __device__ __forceinline__ static void phase_split(float2, const qgtl_pass_desc_t &, float2 (&)[kRegs]) {}
     template <bool NT = false>
     __device__ __forceinline__ static void load_global(const float2 *, const GlobalMap &, float2 (&)[kRegs]) {}
+    template <bool SIGN = false>
     __device__ __forceinline__ static void load_global_inject(const float2 *, const GlobalMap &,
                                                               const qgtl_inject_slot_t &, float2 (&)[kRegs]) {}
     __device__ __forceinline__ static void load_global_inject_diag(const float2 *, const GlobalMap &,
@@ -783,6 +838,35 @@ __device__ __forceinline__ RingFrame ring_frame(int n, uint32_t r) {
     return RingFrame{pre & ones, ones, (uint32_t)__popc(r) & 1u};
 }
 
+// The same for the linear map d.mstage: pre = f r, par_r = b r (the tile's
+// constant within the tile).
+__device__ __forceinline__ RingFrame linear_frame(const qgtl_pass_desc_t &d, uint32_t r) {
+    uint32_t pre = 0, con = 0;
+#pragma unroll
+    for (int i = 0; i < QGTL_MAX_QUBITS - kRT; i++) {
+        pre ^= pick((r >> i) & 1u, d.mstage.f[i]);
+        con ^= pick((r >> i) & 1u, d.mstage.b[i]);
+    }
+    return RingFrame{pre, 0u, con};
+}
+
+// The sign of d.mstage on the amplitudes of tile r, x the tile index of
+// register 0: q(x + reg) = q(x) + q(reg) + the polar form of both.
+__device__ __forceinline__ void apply_signs(const qgtl_pass_desc_t &d, uint32_t r, uint32_t x, float2 (&v)[kRegs]) {
+    uint32_t acc = 0;
+#pragma unroll
+    for (int i = 0; i < QGTL_MAX_QUBITS - kRT; i++) acc ^= pick((r >> i) & 1u, d.mstage.sgn[kRT + i]);
+#pragma unroll
+    for (int i = 0; i < kRT; i++) acc ^= pick((x >> i) & 1u, d.mstage.sgn[i]);
+    const uint32_t full = x | (r << kRT);
+    constexpr uint32_t kBit[5] = {0xaaaaaaaau, 0xccccccccu, 0xf0f0f0f0u, 0xff00ff00u, 0xffff0000u};
+    uint32_t neg = d.mstage.sgn_reg ^ (0u - ((uint32_t)__popc(acc & full) & 1u));
+#pragma unroll
+    for (int i = 0; i < 5; i++) neg ^= (0u - ((uint32_t)__popc(d.mstage.sgn_bil[i] & full) & 1u)) & kBit[i];
+#pragma unroll
+    for (int i = 0; i < kRegs; i++) v[i] = flip_sign(v[i], neg >> i);
+}
+
 // Per-workgroup set-up of a register pass: the phase tables.  The host-built
 // tables (2 kPhaseTab complex64, post then pre) are fetched as one 16-byte
 // word per thread before the tile's global loads are issued and written to
@@ -814,12 +898,14 @@ __device__ __forceinline__ void pass_setup(const qgtl_pass_desc_t &d, float2 *po
 
 // Where tile r of a state is read from and written to, in the load/store
 // layout L0: gin for the load (the ring map for a gathering load), gout for
-// the store (the ring map for a ring store).
+// the store (the ring or linear map for such a store).
 struct TileMaps {
+    uint32_t r;
     RingFrame f;
     GlobalMap gin, gout;
 };
 
+template <bool MST>
 __device__ __forceinline__ TileMaps tile_maps(const qgtl_pass_desc_t &d, uint32_t r, const RegLayout &L0) {
     // state offset of the tile index (fixed trip count, as deposit_hi)
     uint32_t base = 0;
@@ -831,12 +917,19 @@ __device__ __forceinline__ TileMaps tile_maps(const qgtl_pass_desc_t &d, uint32_
     }
     const bool ring_load = d.load == QGTL_LOAD_RING, ring_store = d.store == QGTL_STORE_RING;
     TileMaps m;
+    m.r = r;
     m.f = RingFrame{0u, 0u, 0u};
-    if (ring_load || ring_store) m.f = ring_frame(d.n, r);
     const GlobalMap gnat = natural_map(L0, base, d);
+    if (ring_load || ring_store) m.f = ring_frame(d.n, r);
     const GlobalMap gring = (ring_load || ring_store) ? ring_map(L0, m.f.pre, m.f.ones) : gnat;
     m.gin = ring_load ? gring : gnat;
     m.gout = ring_store ? gring : gnat;
+    if constexpr (MST) {
+        if (d.store == QGTL_STORE_LINEAR) {
+            m.f = linear_frame(d, r);
+            m.gout = linear_map(d, L0, m.f.pre);
+        }
+    }
     return m;
 }
 
@@ -897,7 +990,7 @@ __device__ __forceinline__ void run_phases(const qgtl_pass_desc_t &d, float2 (&v
     }
 }
 
-template <bool SPLIT, bool NT = false, uint32_t SHAPE = 0>
+template <bool SPLIT, bool NT = false, uint32_t SHAPE = 0, bool MST = false>
 __device__ __forceinline__ void pass_compute_store(const qgtl_pass_desc_t &d, float2 (&v)[kRegs], const TileMaps &m,
                                                    const RegLayout &L0, float2 tfac, float2 *dst, float2 *tile,
                                                    const float2 *post_tab, const float2 *pre_tab) {
@@ -908,7 +1001,7 @@ __device__ __forceinline__ void pass_compute_store(const qgtl_pass_desc_t &d, fl
     // is one, else with the pre layer
     const bool layers = rotf && d.nolayer == 0;
     const bool post_on = layers && (d.has_post || !d.has_pre), pre_on = layers && d.has_pre;
-    const bool ring_load = d.load == QGTL_LOAD_RING, ring_store = d.store == QGTL_STORE_RING;
+    const bool ring_load = d.load == QGTL_LOAD_RING;
     RegLayout Lc = L0;
     if (ring_load) {
         // inverse ring: tile r of the output was gathered from the two half
@@ -934,8 +1027,13 @@ __device__ __forceinline__ void pass_compute_store(const qgtl_pass_desc_t &d, fl
     // swaps of the rotation form); without one (a single natural phase) a
     // swap adds it
     const uint32_t xm = rotf ? (uint32_t)d.xmask : 0u;
-    if (ring_store) {
-        RegLoop<kRegs>::store_lds_ring(tile, ring_lds(Lc, m.f.par_r, xm), v);
+    if constexpr (MST)
+        if (d.sign) apply_signs(d, m.r, Lc.tdep ^ xm, v);
+    if (d.store == QGTL_STORE_RING || (MST && d.store == QGTL_STORE_LINEAR)) {
+        RingLds q = ring_lds(Lc, m.f.par_r, xm);
+        if constexpr (MST)
+            if (d.store == QGTL_STORE_LINEAR) q = linear_lds(d, Lc, m.f.par_r, xm);
+        RegLoop<kRegs>::store_lds_ring(tile, q, v);
         __syncthreads();
         RegLoop<kRegs>::load_lds(tile, L0, v);
     } else if (d.nphase > 1 || ring_load || xm) {
@@ -954,32 +1052,35 @@ __device__ __forceinline__ void pass_compute_store(const qgtl_pass_desc_t &d, fl
 // One tile r of one state.  inj != nullptr: src is the primal state the
 // derivative state *inj is injected from while loading.  The global loads go
 // out first; the phase tables are set up while they are in flight.
-template <bool SPLIT = false, bool NT = false, uint32_t SHAPE = 0>
+// MST: the pass has a linear M-stage or its sign (a variant of its own: the
+// maps cost the other passes 25 to 40 registers).
+template <bool SPLIT = false, bool NT = false, uint32_t SHAPE = 0, bool MST = false>
 __device__ __forceinline__ void pass_regs_body(const qgtl_pass_desc_t &d, const float2 *__restrict__ src,
                                                float2 *dst, uint32_t r, float2 *tile, float2 *post_tab,
                                                float2 *pre_tab, const float2 *gtabs = nullptr,
                                                const qgtl_inject_slot_t *inj = nullptr) {
     const float4 tq = fetch_tables(d, gtabs);
     const RegLayout L0 = make_layout(d.ph_rbits[0], d.ph_tbits[0], threadIdx.x);
-    const TileMaps m = tile_maps(d, r, L0);
+    const TileMaps m = tile_maps<MST>(d, r, L0);
     float2 v[kRegs];
     if (inj && inj->v == 0) RegLoop<kRegs>::load_global_inject_diag(src, m.gin, *inj, v);
+    else if (MST && inj && inj->z) RegLoop<kRegs>::template load_global_inject<true>(src, m.gin, *inj, v);
     else if (inj && inject_anti(*inj)) RegLoop<kRegs>::load_global_inject_anti(src, m.gin, *inj, v);
-    else if (inj) RegLoop<kRegs>::load_global_inject(src, m.gin, *inj, v);
+    else if (inj) RegLoop<kRegs>::template load_global_inject<false>(src, m.gin, *inj, v);
     else RegLoop<kRegs>::template load_global<NT>(src, m.gin, v);
     const float2 tfac = tile_factor(d, r);
     pass_setup(d, post_tab, pre_tab, gtabs, tq);
-    pass_compute_store<SPLIT, NT, SHAPE>(d, v, m, L0, tfac, dst, tile, post_tab, pre_tab);
+    pass_compute_store<SPLIT, NT, SHAPE, MST>(d, v, m, L0, tfac, dst, tile, post_tab, pre_tab);
 }
 
-template <bool SPLIT, bool NT = false, uint32_t SHAPE = 0>
+template <bool SPLIT, bool NT = false, uint32_t SHAPE = 0, bool MST = false>
 __global__ __launch_bounds__(kThreads) void pass_c64_regs_kernel(const qgtl_pass_desc_t d,
                                                                  const float2 *__restrict__ src_all,
                                                                  float2 *dst_all, size_t stride,
                                                                  const float2 *__restrict__ gtabs) {
     __shared__ float2 tile[kRegTileElems];
     __shared__ float2 tabs[2 * kPhaseTab];
-    pass_regs_body<SPLIT, NT, SHAPE>(d, src_all + (size_t)blockIdx.y * stride, dst_all + (size_t)blockIdx.y * stride,
+    pass_regs_body<SPLIT, NT, SHAPE, MST>(d, src_all + (size_t)blockIdx.y * stride, dst_all + (size_t)blockIdx.y * stride,
                               blockIdx.x, tile, tabs, tabs + kPhaseTab, gtabs);
 }
 
@@ -988,7 +1089,7 @@ __global__ __launch_bounds__(kThreads) void pass_c64_regs_kernel(const qgtl_pass
 // shared), so the injected states are never written to or read from HBM.
 constexpr uint32_t kXcd = 8;   // XCDs; workgroups are dispatched to them round-robin
 
-template <bool SPLIT, uint32_t SHAPE = 0>
+template <bool SPLIT, uint32_t SHAPE = 0, bool MST = false>
 __global__ __launch_bounds__(kThreads) void pass_c64_inject_kernel(const qgtl_pass_desc_t d,
                                                                    const float2 *__restrict__ psi,
                                                                    const qgtl_inject_slot_t *__restrict__ inj,
@@ -1013,7 +1114,7 @@ __global__ __launch_bounds__(kThreads) void pass_c64_inject_kernel(const qgtl_pa
         t = b / nstates;
     }
     const qgtl_inject_slot_t q = inj[s];
-    pass_regs_body<SPLIT, true, SHAPE>(d, psi, dst_all + (size_t)s * stride, t, tile, tabs, tabs + kPhaseTab, gtabs,
+    pass_regs_body<SPLIT, true, SHAPE, MST>(d, psi, dst_all + (size_t)s * stride, t, tile, tabs, tabs + kPhaseTab, gtabs,
                                        &q);
 }
 
@@ -1034,7 +1135,7 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 // Tile `tile` of derivative state k; its four sums go to out[0..3].  SPLIT:
 // dst receives the split-plane form (four fp16 planes of N values).
-template <bool SPLIT = false, bool STORE = true, int PER = kInjectPerThread, bool SUMS = true>
+template <bool SPLIT = false, bool STORE = true, int PER = kInjectPerThread, bool SUMS = true, bool SIGN = false>
 __device__ __forceinline__ void inject_body(const qgtl_inject_desc_t &d, const float2 *__restrict__ psi,
                                             float2 *dst, int k, uint32_t tile, double *out,
                                             double (*red)[4]) {
@@ -1055,8 +1156,13 @@ __device__ __forceinline__ void inject_body(const qgtl_inject_desc_t &d, const f
             const float4 qa = *reinterpret_cast<const float4 *>(psi + y);
             const float4 qb = *reinterpret_cast<const float4 *>(psi + ((y ^ v) & ~1u));
             const float2 a0 = make_float2(qa.x, qa.y), a1 = make_float2(qa.z, qa.w);
-            const float2 b0 = odd ? make_float2(qb.z, qb.w) : make_float2(qb.x, qb.y);
-            const float2 b1 = odd ? make_float2(qb.x, qb.y) : make_float2(qb.z, qb.w);
+            float2 b0 = odd ? make_float2(qb.z, qb.w) : make_float2(qb.x, qb.y);
+            float2 b1 = odd ? make_float2(qb.x, qb.y) : make_float2(qb.z, qb.w);
+            if constexpr (SIGN) {
+                const uint32_t z = d.z[k], n0 = (uint32_t)__popc(y & z);
+                b0 = flip_sign(b0, n0);
+                b1 = flip_sign(b1, n0 + (z & 1u));
+            }
             const bool s0 = (__popc(y & w) & 1) != 0, s1 = s0 != wodd;
             const float2 o0 = cmadd(cmadd(make_float2(0.f, 0.f), s0 ? a11 : a00, a0), s0 ? a10 : a01, b0);
             const float2 o1 = cmadd(cmadd(make_float2(0.f, 0.f), s1 ? a11 : a00, a1), s1 ? a10 : a01, b1);
@@ -1102,9 +1208,12 @@ __global__ __launch_bounds__(kThreads) void inject_c64_kernel(const qgtl_inject_
                                                               double *partials) {
     __shared__ double red[kThreads / 64][4];
     const int k = blockIdx.y;
-    inject_body<SPLIT, STORE, kInjectPerThreadPlan, SUMS>(
-        d, psi, STORE ? dst_all + (size_t)k * stride : nullptr, k, blockIdx.x,
-        SUMS ? partials + ((size_t)k * gridDim.x + blockIdx.x) * 4 : nullptr, red);
+    float2 *dst = STORE ? dst_all + (size_t)k * stride : nullptr;
+    double *out = SUMS ? partials + ((size_t)k * gridDim.x + blockIdx.x) * 4 : nullptr;
+    if (d.z[k] == 0)
+        inject_body<SPLIT, STORE, kInjectPerThreadPlan, SUMS>(d, psi, dst, k, blockIdx.x, out, red);
+    else
+        inject_body<SPLIT, STORE, kInjectPerThreadPlan, SUMS, true>(d, psi, dst, k, blockIdx.x, out, red);
 }
 
 // One complex64 state in split-plane form (the Gram's operand form).
@@ -1257,6 +1366,15 @@ __global__ void swap_c64_kernel(float2 *base, size_t stride, uint32_t quarter, i
     }
 }
 
+__global__ void cz_c64_kernel(float2 *base, size_t stride, uint32_t quarter, int qa, int qb) {
+    float2 *psi = base + (size_t)blockIdx.y * stride;
+    const int lo = min(qa, qb), hi = max(qa, qb);
+    for (uint32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < quarter; x += gridDim.x * blockDim.x) {
+        const uint32_t i = insert_zero(insert_zero(x, lo), hi) | (1u << qa) | (1u << qb);
+        psi[i] = make_float2(-psi[i].x, -psi[i].y);
+    }
+}
+
 __global__ void c64_to_c128_kernel(const float2 *src, double2 *dst, size_t count) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x)
         dst[i] = make_double2(src[i].x, src[i].y);
@@ -1334,15 +1452,21 @@ __global__ __launch_bounds__(kThreads) void inject_grouped_kernel(const qgtl_inj
         __syncthreads();
         const qgtl_inject_desc_t &d = *reinterpret_cast<const qgtl_inject_desc_t *>(it.desc);
         float2 *dst = reinterpret_cast<float2 *>(it.dst) + (size_t)k * it.stride;
-        if (it.partials)        // FP64 sums of <d|psi>, |d|^2, |psi|^2 per tile as well
-            inject_body(d, reinterpret_cast<const float2 *>(it.psi), dst, k, t,
-                        reinterpret_cast<double *>(it.partials) + ((size_t)k * it.tiles + t) * 4, red);
-        else if (it.pad & QGTL_INJECT_ITEM_SPLIT)   // the state in split-plane form
-            inject_body<true, true, kInjectPerThread, false>(d, reinterpret_cast<const float2 *>(it.psi), dst, k, t,
-                                                             nullptr, red);
+        const float2 *psi = reinterpret_cast<const float2 *>(it.psi);
+        double *out = it.partials ? reinterpret_cast<double *>(it.partials) + ((size_t)k * it.tiles + t) * 4 : nullptr;
+        const bool sign = d.z[k] != 0;
+        if (it.partials && sign)        // FP64 sums of <d|psi>, |d|^2, |psi|^2 per tile as well
+            inject_body<false, true, kInjectPerThread, true, true>(d, psi, dst, k, t, out, red);
+        else if (it.partials)
+            inject_body(d, psi, dst, k, t, out, red);
+        else if ((it.pad & QGTL_INJECT_ITEM_SPLIT) && sign)   // the state in split-plane form
+            inject_body<true, true, kInjectPerThread, false, true>(d, psi, dst, k, t, nullptr, red);
+        else if (it.pad & QGTL_INJECT_ITEM_SPLIT)
+            inject_body<true, true, kInjectPerThread, false>(d, psi, dst, k, t, nullptr, red);
+        else if (sign)
+            inject_body<false, true, kInjectPerThread, false, true>(d, psi, dst, k, t, nullptr, red);
         else
-            inject_body<false, true, kInjectPerThread, false>(d, reinterpret_cast<const float2 *>(it.psi), dst, k, t,
-                                                              nullptr, red);
+            inject_body<false, true, kInjectPerThread, false>(d, psi, dst, k, t, nullptr, red);
     }
 }
 
@@ -1482,6 +1606,10 @@ int qgtl_hip_pass_c64(const qgtl_pass_desc_t *desc, const void *src, void *dst, 
         return qgtl::set_error_msg(-118, "qgtl_hip_pass_c64: inconsistent pass descriptor");
     if (desc->store == QGTL_STORE_RING && (desc->nlow != desc->m || desc->m < 2 || desc->n <= desc->m))
         return qgtl::set_error_msg(-118, "qgtl_hip_pass_c64: ring store needs the low tile of a wider state");
+    const bool lin = desc->store == QGTL_STORE_LINEAR, mst = lin || desc->sign;
+    if (mst && (!regs_pass(desc, tile_variant) || desc->nlow != kRT || desc->n <= kRT || (lin && src == dst) || split_out))
+        return qgtl::set_error_msg(-118, "qgtl_hip_pass_c64: a linear M-stage needs a register pass over bits 0..12 "
+                                         "of a wider state, separate buffers and complex64 output");
     if (desc->store == QGTL_STORE_PERM && desc->m != desc->n)
         return qgtl::set_error_msg(-118, "qgtl_hip_pass_c64: permutation store needs the whole state in one tile");
     if ((desc->store == QGTL_STORE_RING || desc->store == QGTL_STORE_PERM) && src == dst && desc->store == QGTL_STORE_RING)
@@ -1498,15 +1626,17 @@ int qgtl_hip_pass_c64(const qgtl_pass_desc_t *desc, const void *src, void *dst, 
     const float2 *gt = (const float2 *)tabs;
     // non-temporal loads and stores: every tile is read once and written once per pass
     const uint32_t shape = regs ? pass_shape(desc) : 0;
-#define QGTL_REGS_LAUNCH(SPLIT, SHAPE)                                                                         \
-    hipLaunchKernelGGL((pass_c64_regs_kernel<SPLIT, true, SHAPE>), grid, dim3(kThreads), 0, qgtl::stream(), *desc, \
+#define QGTL_REGS_LAUNCH(SPLIT, SHAPE, MST)                                                                    \
+    hipLaunchKernelGGL((pass_c64_regs_kernel<SPLIT, true, SHAPE, MST>), grid, dim3(kThreads), 0, qgtl::stream(), *desc, \
                        (const float2 *)src, (float2 *)dst, stride, gt)
-    if (regs && split_out && shape == kShape3Full) QGTL_REGS_LAUNCH(true, kShape3Full);
-    else if (regs && split_out && shape == kShape2Hi7) QGTL_REGS_LAUNCH(true, kShape2Hi7);
-    else if (regs && split_out) QGTL_REGS_LAUNCH(true, 0);
-    else if (regs && shape == kShape3Full) QGTL_REGS_LAUNCH(false, kShape3Full);
-    else if (regs && shape == kShape2Hi7) QGTL_REGS_LAUNCH(false, kShape2Hi7);
-    else if (regs) QGTL_REGS_LAUNCH(false, 0);
+    if (mst && shape == kShape3Full) QGTL_REGS_LAUNCH(false, kShape3Full, true);
+    else if (mst) QGTL_REGS_LAUNCH(false, 0, true);
+    else if (regs && split_out && shape == kShape3Full) QGTL_REGS_LAUNCH(true, kShape3Full, false);
+    else if (regs && split_out && shape == kShape2Hi7) QGTL_REGS_LAUNCH(true, kShape2Hi7, false);
+    else if (regs && split_out) QGTL_REGS_LAUNCH(true, 0, false);
+    else if (regs && shape == kShape3Full) QGTL_REGS_LAUNCH(false, kShape3Full, false);
+    else if (regs && shape == kShape2Hi7) QGTL_REGS_LAUNCH(false, kShape2Hi7, false);
+    else if (regs) QGTL_REGS_LAUNCH(false, 0, false);
 #undef QGTL_REGS_LAUNCH
     else
         hipLaunchKernelGGL(pass_c64_kernel, grid, dim3(kThreads), 0, qgtl::stream(), *desc,
@@ -1539,7 +1669,7 @@ int qgtl_hip_inject_sums_c64(const qgtl_inject_desc_t *desc, const void *psi, do
 }
 
 int qgtl_hip_pass_c64_inject(const qgtl_pass_desc_t *desc, const void *psi, const void *slots, void *dst,
-                             size_t stride, int nstates, int split_out, const void *tabs) {
+                             size_t stride, int nstates, int split_out, int signs, const void *tabs) {
     if (desc->m != kRT || desc->nlow < 1 || desc->nlow > kRT || kRT - desc->nlow > kHiTableBits ||
         desc->ngates > kRT || desc->m + desc->nrest != desc->n || nstates < 1 || !regs_pass(desc, 0) ||
         stride < ((size_t)1 << desc->n))
@@ -1554,20 +1684,29 @@ int qgtl_hip_pass_c64_inject(const qgtl_pass_desc_t *desc, const void *psi, cons
         (desc->load != QGTL_LOAD_RING || desc->nlow != kRT || desc->n <= kRT || desc->store != QGTL_STORE_INPLACE ||
          !tbits_ok(desc, desc->gather_tbits)))
         return qgtl::set_error_msg(-118, "qgtl_hip_pass_c64_inject: bad ring gather");
+    if ((desc->store == QGTL_STORE_LINEAR || desc->sign) && (desc->nlow != desc->m || desc->n <= desc->m))
+        return qgtl::set_error_msg(-118, "qgtl_hip_pass_c64_inject: a linear M-stage needs the low tile of a wider state");
     const uint32_t ntiles = 1u << desc->nrest;
     const dim3 grid((unsigned)nstates * ntiles);   // <= 65535 * 2^15 workgroups
     const float2 *gt = (const float2 *)tabs;
     const qgtl_inject_slot_t *sl = (const qgtl_inject_slot_t *)slots;
     const uint32_t shape = pass_shape(desc);
-#define QGTL_INJECT_LAUNCH(SPLIT, SHAPE)                                                                          \
-    hipLaunchKernelGGL((pass_c64_inject_kernel<SPLIT, SHAPE>), grid, dim3(kThreads), 0, qgtl::stream(), *desc,    \
+    /* signs: some slot has z != 0 */
+    const bool mst = desc->store == QGTL_STORE_LINEAR || desc->sign || signs;
+    if (split_out && (desc->store == QGTL_STORE_LINEAR || desc->sign))
+        return qgtl::set_error_msg(-118, "qgtl_hip_pass_c64_inject: a linear M-stage needs complex64 output");
+#define QGTL_INJECT_LAUNCH(SPLIT, SHAPE, MST)                                                                     \
+    hipLaunchKernelGGL((pass_c64_inject_kernel<SPLIT, SHAPE, MST>), grid, dim3(kThreads), 0, qgtl::stream(), *desc,    \
                        (const float2 *)psi, sl, (float2 *)dst, stride, gt, (uint32_t)nstates, ntiles)
-    if (split_out && shape == kShape3Full) QGTL_INJECT_LAUNCH(true, kShape3Full);
-    else if (split_out && shape == kShape2Hi7) QGTL_INJECT_LAUNCH(true, kShape2Hi7);
-    else if (split_out) QGTL_INJECT_LAUNCH(true, 0);
-    else if (shape == kShape3Full) QGTL_INJECT_LAUNCH(false, kShape3Full);
-    else if (shape == kShape2Hi7) QGTL_INJECT_LAUNCH(false, kShape2Hi7);
-    else QGTL_INJECT_LAUNCH(false, 0);
+    if (mst && split_out) QGTL_INJECT_LAUNCH(true, 0, true);
+    else if (mst && shape == kShape3Full) QGTL_INJECT_LAUNCH(false, kShape3Full, true);
+    else if (mst) QGTL_INJECT_LAUNCH(false, 0, true);
+    else if (split_out && shape == kShape3Full) QGTL_INJECT_LAUNCH(true, kShape3Full, false);
+    else if (split_out && shape == kShape2Hi7) QGTL_INJECT_LAUNCH(true, kShape2Hi7, false);
+    else if (split_out) QGTL_INJECT_LAUNCH(true, 0, false);
+    else if (shape == kShape3Full) QGTL_INJECT_LAUNCH(false, kShape3Full, false);
+    else if (shape == kShape2Hi7) QGTL_INJECT_LAUNCH(false, kShape2Hi7, false);
+    else QGTL_INJECT_LAUNCH(false, 0, false);
 #undef QGTL_INJECT_LAUNCH
     QGTL_LAUNCH_CHECK("pass_c64_inject");
     return 0;
@@ -1622,6 +1761,15 @@ int qgtl_hip_swap_c64(void *base, size_t stride, int nstates, int n, int a, int 
     hipLaunchKernelGGL(swap_c64_kernel, dim3(grid_for(quarter), (unsigned)nstates), dim3(256), 0,
                        qgtl::stream(), (float2 *)base, stride, quarter, a, b);
     QGTL_LAUNCH_CHECK("swap_c64");
+    return 0;
+}
+
+int qgtl_hip_cz_c64(void *base, size_t stride, int nstates, int n, int a, int b) {
+    if (n < 2) return qgtl::set_error_msg(-118, "cz needs two qubits");
+    const uint32_t quarter = 1u << (n - 2);
+    hipLaunchKernelGGL(cz_c64_kernel, dim3(grid_for(quarter), (unsigned)nstates), dim3(256), 0,
+                       qgtl::stream(), (float2 *)base, stride, quarter, a, b);
+    QGTL_LAUNCH_CHECK("cz_c64");
     return 0;
 }
 

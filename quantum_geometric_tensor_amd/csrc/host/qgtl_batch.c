@@ -183,6 +183,7 @@ static void fill_inst_descs(struct qgtl_batch *B, int i)
                 const qgtl_mat2 *M = backward ? &pp->B : &pp->A;
                 d->v[j] = backward ? 1u << pp->qubit : pp->v;
                 d->w[j] = backward ? 1u << pp->qubit : pp->w;
+                d->z[j] = backward ? 0 : pp->z;
                 for (int e = 0; e < 4; e++) {
                     d->A[j][e].re = (float)M->m[e].re;
                     d->A[j][e].im = (float)M->m[e].im;
@@ -770,7 +771,7 @@ qgtl_batch_t *qgtl_batch_create(int count, const int *n, const int *nops, const 
         }
         in->flips = 0;
         for (int b = 0; b < p->nblocks; b++) {
-            if (p->blocks[b].mstage_kernels) {
+            if (n[i] > QGTL_TILE_BITS_MAX && p->blocks[b].nperm > 0 && !p->blocks[b].is_ring) {
                 qgtl_set_error(QGT_ERROR_NOT_IMPLEMENTED,
                                "instance %d: a CNOT/SWAP stage that is not a ring on more than 13 qubits "
                                "(batched sweeps fold M-stages into passes)", i);

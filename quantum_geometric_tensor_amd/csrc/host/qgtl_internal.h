@@ -3,7 +3,7 @@
  *
  * A circuit is compiled into blocks.  A block is a U-layer (one 2x2 matrix
  * per qubit, the product of that qubit's single-qubit gates, FP64) followed
- * by an M-stage (a list of CNOT/SWAP gates, a GF(2)-linear permutation of
+ * by an M-stage (a list of CNOT/SWAP/CZ gates, a GF(2)-linear permutation of
  * basis indices).  Derivative states of the block's parameters are created
  * after the block from the block's output state, and carried through the
  * later blocks by LDS-tiled sweep passes.
@@ -37,10 +37,14 @@ typedef struct {
     int has_u[QGTL_MAX_QUBITS];
     qgtl_mat2 u[QGTL_MAX_QUBITS];
     int nperm;
-    int8_t perm_type[QGTL_PERM_MAX];     /* 0 CNOT(a -> b), 1 SWAP(a, b) */
+    int8_t perm_type[QGTL_PERM_MAX];     /* 0 CNOT(a -> b), 1 SWAP(a, b), 2 CZ(a, b) */
     int8_t perm_a[QGTL_PERM_MAX];
     int8_t perm_b[QGTL_PERM_MAX];
     int is_ring;                         /* M-stage is CNOT(i -> i+1 mod n), i = 0..n-1 */
+    int linear;                          /* M-stage moves indices by mstage, folded into the passes (n > 13) */
+    qgtl_mstage_t mstage;
+    int has_sign;                        /* the CZ gates' sign as a quadratic form of the input index */
+    uint32_t sgn[QGTL_MAX_QUBITS];
     int param_begin, param_end;          /* parameters created in this block */
     /* device passes that apply this block */
     int npasses;
@@ -61,7 +65,7 @@ typedef struct {
     int qubit;
     int op_index;
     qgtl_mat2 A;                         /* d_k (pre-M) = A psi_block (pre-M) */
-    uint32_t v, w;                       /* injection masks after the M-stage */
+    uint32_t v, w, z;                    /* injection masks after the M-stage */
     qgtl_mat2 B;                         /* u_q^dagger A u_q: the block's inverse applied to d_k, a 2 x 2 on
                                             the parameter's qubit acting on the block's input state */
 } qgtl_param_t;
@@ -75,6 +79,8 @@ struct qgtl_plan {
     int nops;
     int P;
     qgtl_op_t *ops;
+    int has_signs;                       /* some block's M-stage has a sign */
+    int ringless;                        /* n > 13: M-stages, but no CNOT ring among them */
     int nblocks;
     qgtl_block_t *blocks;
     int blocks_cap;

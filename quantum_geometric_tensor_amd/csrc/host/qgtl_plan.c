@@ -8,14 +8,15 @@
  * CNOT flips the target where the control bit is set (:195-210).
  *
  * Block rule: a single-qubit gate on qubit q joins the current block's
- * U-layer unless the block's M-stage has already touched q; a CNOT or SWAP
- * joins the M-stage.  CZ and CY are rewritten as H.CNOT.H and S.CNOT.Sdg.
+ * U-layer unless the block's M-stage has already touched q; a CNOT, SWAP or CZ
+ * joins the M-stage.  CY is rewritten as S.CNOT.Sdg.
  *
  * Derivative of parameter k carried by gate g on qubit q: with the block's
  * U_q = S g R (S = gates after g in the block, R = before), the derivative
  * state before the M-stage is S (-i/2 G) g R = A_k U_q, A_k = S (-i/2 G) S^H,
- * applied to the block's output.  Through the M-stage permutation pi,
- * d_k[y] = A[s][s] psi[y] + A[s][1-s] psi[y ^ pi(e_q)], s = (pi^-1 y)_q.
+ * applied to the block's output.  Through the M-stage's permutation pi and
+ * sign (-1)^{q(x)}, d_k[y] = A[s][s] psi[y] + (-1)^{q(x) + q(x ^ e_q)} A[s][1-s]
+ * psi[y ^ pi(e_q)], x = pi^-1 y, s = x_q; q(x) + q(x ^ e_q) is a constant plus a parity of y.
  */
 #include <math.h>
 #include <stdlib.h>
@@ -128,7 +129,7 @@ static uint32_t perm_apply(const qgtl_block_t *b, uint32_t x)
     for (int i = 0; i < b->nperm; i++) {
         const uint32_t ab = (x >> b->perm_a[i]) & 1u, bb = (x >> b->perm_b[i]) & 1u;
         if (b->perm_type[i] == 0) x ^= ab << b->perm_b[i];
-        else x ^= (ab ^ bb) * ((1u << b->perm_a[i]) | (1u << b->perm_b[i]));
+        else if (b->perm_type[i] == 1) x ^= (ab ^ bb) * ((1u << b->perm_a[i]) | (1u << b->perm_b[i]));
     }
     return x;
 }
@@ -138,9 +139,57 @@ static uint32_t perm_apply_inverse(const qgtl_block_t *b, uint32_t y)
     for (int i = b->nperm - 1; i >= 0; i--) {
         const uint32_t ab = (y >> b->perm_a[i]) & 1u, bb = (y >> b->perm_b[i]) & 1u;
         if (b->perm_type[i] == 0) y ^= ab << b->perm_b[i];
-        else y ^= (ab ^ bb) * ((1u << b->perm_a[i]) | (1u << b->perm_b[i]));
+        else if (b->perm_type[i] == 1) y ^= (ab ^ bb) * ((1u << b->perm_a[i]) | (1u << b->perm_b[i]));
     }
     return y;
+}
+
+static uint32_t parity32(uint32_t x)
+{
+    return (uint32_t)__builtin_popcount(x) & 1u;
+}
+
+/* The M-stage's sign as a quadratic form of its input index, q(x) = sum over i
+ * of x_i parity(sgn[i] & x) with sgn[i] within bits i..n-1 (bit i of sgn[i]:
+ * x_i itself).  Every CZ adds the product of the two qubits' current values,
+ * each a parity of the input. */
+static void find_signs(qgtl_block_t *b, int n)
+{
+    uint32_t row[QGTL_MAX_QUBITS];
+    for (int q = 0; q < n; q++) row[q] = 1u << q;
+    memset(b->sgn, 0, sizeof b->sgn);
+    b->has_sign = 0;
+    for (int g = 0; g < b->nperm; g++) {
+        const int a = b->perm_a[g], c = b->perm_b[g];
+        if (b->perm_type[g] == 0) {
+            row[c] ^= row[a];
+        } else if (b->perm_type[g] == 1) {
+            const uint32_t t = row[a];
+            row[a] = row[c];
+            row[c] = t;
+        } else {
+            for (int i = 0; i < n; i++)
+                for (int j = 0; j < n; j++)
+                    if (((row[a] >> i) & 1u) && ((row[c] >> j) & 1u)) b->sgn[i < j ? i : j] ^= 1u << (i < j ? j : i);
+        }
+    }
+    for (int q = 0; q < n; q++) b->has_sign |= b->sgn[q] != 0;
+}
+
+/* q(x) and row q of its polar form q(x) + q(y) + q(x ^ y) */
+static uint32_t sign_of(const uint32_t *sgn, uint32_t x)
+{
+    uint32_t s = 0;
+    for (int i = 0; i < QGTL_MAX_QUBITS; i++)
+        if ((x >> i) & 1u) s ^= parity32(sgn[i] & x);
+    return s;
+}
+
+static uint32_t polar_row(const uint32_t *sgn, int q)
+{
+    uint32_t r = sgn[q] & ~(1u << q);
+    for (int i = 0; i < q; i++) r |= ((sgn[i] >> q) & 1u) << i;
+    return r;
 }
 
 static void to_c64(const qgtl_mat2 *m, qgtl_c64_t out[4])
@@ -382,8 +431,8 @@ static void fold_layer(qgtl_pass_desc_t *d, qgtl_pass_desc_t *r, const rot_facto
 
 /* LDS bank of tile index j in the register kernel's swizzled tile:
  * ((j ^ (j >> 4) ^ (j >> 8) ^ (j >> 12)) & 15), a GF(2)-linear map, so tile
- * bit b lands on bank bit (b & 3).  For the ring store the written index is
- * the linear ring image of j. */
+ * bit b lands on bank bit (b & 3).  For a ring or linear store the written
+ * index is a linear image of j. */
 static uint32_t bank_vec(uint32_t j)
 {
     return (j ^ (j >> 4) ^ (j >> 8) ^ (j >> 12)) & 15u;
@@ -416,9 +465,9 @@ static int independent4(const uint32_t v[4])
 
 /* Thread-bit order of a layout with register bits rbits: the first four
  * thread bits (lanes 0..15) map to tile bits whose bank vectors are
- * independent, also through the ring map when the layout feeds a ring
+ * independent, also through the map img (the tile bits' images, or NULL) of a
  * store; phase 0 keeps ascending order (coalesced global access). */
-static void choose_thread_bits(const int32_t rbits[5], int ascending, int ring, int32_t tbits[8])
+static void choose_thread_bits(const int32_t rbits[5], int ascending, const uint32_t *img, int32_t tbits[8])
 {
     int others[QGTL_TILE_BITS_MAX], no = 0;
     for (int b = 0; b < QGTL_TILE_BITS_MAX; b++) {
@@ -436,9 +485,9 @@ static void choose_thread_bits(const int32_t rbits[5], int ascending, int ring, 
                     uint32_t v[4], w[4];
                     for (int i = 0; i < 4; i++) {
                         v[i] = bank_vec(1u << pick[i]);
-                        w[i] = bank_vec(ring_image(1u << pick[i]));
+                        w[i] = img ? bank_vec(img[pick[i]]) : v[i];
                     }
-                    if (!independent4(v) || (ring && !independent4(w))) continue;
+                    if (!independent4(v) || !independent4(w)) continue;
                     int k = 0;
                     for (int i = 0; i < 4; i++) tbits[k++] = pick[i];
                     for (int i = 0; i < no; i++)
@@ -495,9 +544,12 @@ static void plan_phases(qgtl_pass_desc_t *p)
     int32_t bits[QGTL_TILE_BITS_MAX];
     for (int i = 0; i < cnt; i++) bits[i] = p->gate_bit[order[i]];
     memcpy(p->gate_bit, bits, sizeof(int32_t) * (size_t)cnt);
-    /* thread-bit orders (the last layout also writes the ring store) */
+    /* thread-bit orders (the last layout also writes the ring or linear store) */
+    uint32_t ring[QGTL_TILE_BITS_MAX];
+    for (int i = 0; i < QGTL_TILE_BITS_MAX; i++) ring[i] = ring_image(1u << i);
+    const uint32_t *img = p->store == QGTL_STORE_RING ? ring : p->store == QGTL_STORE_LINEAR ? p->mstage.a : NULL;
     for (int ph = 0; ph < nph; ph++)
-        choose_thread_bits(p->ph_rbits[ph], ph == 0, ph == nph - 1 && p->store == QGTL_STORE_RING, p->ph_tbits[ph]);
+        choose_thread_bits(p->ph_rbits[ph], ph == 0, ph == nph - 1 ? img : NULL, p->ph_tbits[ph]);
     /* by register bit, for the kernels */
     for (int ph = 0; ph < nph; ph++) {
         p->ph_mask[ph] = 0;
@@ -539,7 +591,7 @@ static void high_passes(const qgtl_block_t *b, int n, qgtl_pass_desc_t *out, int
 
 /* The pass over tile bits 0..12 with the given load
  * and store; returns 0 when it has nothing to do. */
-static int low_pass(const qgtl_block_t *b, int n, qgtl_pass_desc_t *p, int store, int load)
+static int low_pass(const qgtl_block_t *b, int n, qgtl_pass_desc_t *p, int store, int load, int sign)
 {
     const int TB = QGTL_TILE_BITS_MAX;
     memset(p, 0, sizeof *p);
@@ -551,7 +603,78 @@ static int low_pass(const qgtl_block_t *b, int n, qgtl_pass_desc_t *p, int store
         }
     p->store = store;
     p->load = load;
-    return p->ngates > 0 || store != QGTL_STORE_INPLACE || load != QGTL_LOAD_NATURAL;
+    p->sign = sign;
+    if (store == QGTL_STORE_LINEAR) p->mstage = b->mstage;
+    memcpy(p->mstage.sgn, b->sgn, sizeof b->sgn);
+    return p->ngates > 0 || store != QGTL_STORE_INPLACE || load != QGTL_LOAD_NATURAL || sign;
+}
+
+/* The register part of a pass's M-stage for the layout with register bits rb. */
+static void mstage_registers(qgtl_pass_desc_t *p, const int32_t rb[5])
+{
+    qgtl_mstage_t *m = &p->mstage;
+    for (int i = 0; i < 5; i++) {
+        m->reg[i] = m->a[rb[i]];
+        m->sgn_bil[i] = polar_row(m->sgn, rb[i]);
+    }
+    m->sgn_reg = 0;
+    for (uint32_t r = 0; r < 32; r++) {
+        uint32_t x = 0;
+        for (int i = 0; i < 5; i++) x |= ((r >> i) & 1u) << rb[i];
+        m->sgn_reg |= sign_of(m->sgn, x) << r;
+    }
+}
+
+/* The block's M-stage as an index map of the register passes (n > 13; see
+ * qgtl_mstage_t).  0 when the map is not a bijection within the tiles (a SWAP
+ * of a low with a high qubit) or would write runs shorter than a cache line
+ * (a high qubit's parity over the lowest bits); one kernel per gate
+ * applies those. */
+static int find_mstage_map(qgtl_block_t *b, int n)
+{
+    const int TB = QGTL_TILE_BITS_MAX, nh = n - TB;
+    const uint32_t low = (1u << TB) - 1u;
+    qgtl_mstage_t *m = &b->mstage;
+    memset(m, 0, sizeof *m);
+    /* columns of a beside those of the identity, reduced together: a^-1 */
+    uint32_t col[QGTL_TILE_BITS_MAX], inv[QGTL_TILE_BITS_MAX], c[QGTL_TILE_BITS_MAX];
+    for (int q = 0; q < TB; q++) {
+        const uint32_t img = perm_apply(b, 1u << q);
+        m->a[q] = col[q] = img & low;
+        c[q] = img >> TB;
+        inv[q] = 1u << q;
+    }
+    for (int i = 0; i < TB; i++) {
+        int piv = i;
+        while (piv < TB && !((col[piv] >> i) & 1u)) piv++;
+        if (piv == TB) return 0;
+        uint32_t t = col[i]; col[i] = col[piv]; col[piv] = t;
+        t = inv[i]; inv[i] = inv[piv]; inv[piv] = t;
+        for (int j = 0; j < TB; j++)
+            if (j != i && ((col[j] >> i) & 1u)) { col[j] ^= col[i]; inv[j] ^= inv[i]; }
+    }
+    const uint32_t may = 1u << 4 | 1u << 5 | 1u << 6 | 1u << 11 | 1u << 12;
+    for (int i = 0; i < TB; i++) {
+        for (int q = 0; q < TB; q++)
+            if ((inv[i] >> q) & 1u) m->e[i] ^= c[q];
+        if (m->e[i] && !((may >> i) & 1u)) return 0;
+    }
+    for (int h = 0; h < nh; h++) {
+        const uint32_t img = perm_apply(b, 1u << (TB + h));
+        m->b[h] = img & low;
+        m->f[h] = img >> TB;
+        for (int i = 0; i < TB; i++)
+            if ((m->b[h] >> i) & 1u) m->f[h] ^= m->e[i];
+    }
+    return 1;
+}
+
+/* CNOTs and SWAPs in the M-stage that leave the index unmoved altogether (or none) */
+static int index_unmoved(const qgtl_block_t *b, int n)
+{
+    for (int q = 0; q < n; q++)
+        if (perm_apply(b, 1u << q) != 1u << q) return 0;
+    return 1;
 }
 
 /* The layouts of block b's passes (their matrices are set for given angles). */
@@ -589,13 +712,17 @@ static void build_passes(qgtl_block_t *b, int n)
         return;
     }
     high_passes(b, n, b->pass, b->pass_flips, &b->npasses);
-    if (low_pass(b, n, &b->pass[b->npasses], b->is_ring ? QGTL_STORE_RING : QGTL_STORE_INPLACE,
-                 QGTL_LOAD_NATURAL)) {
-        b->pass_flips[b->npasses] = b->is_ring;
+    b->linear = !b->is_ring && !index_unmoved(b, n);
+    b->mstage_kernels = b->linear && !find_mstage_map(b, n);
+    if (b->mstage_kernels) b->linear = 0;
+    const int store = b->is_ring ? QGTL_STORE_RING : b->linear ? QGTL_STORE_LINEAR : QGTL_STORE_INPLACE;
+    qgtl_pass_desc_t *low = &b->pass[b->npasses];
+    if (low_pass(b, n, low, store, QGTL_LOAD_NATURAL, b->has_sign && !b->mstage_kernels)) {
+        b->pass_flips[b->npasses] = store != QGTL_STORE_INPLACE;
         b->npasses++;
     }
-    if (!b->is_ring && b->nperm > 0) b->mstage_kernels = 1;
     for (int i = 0; i < b->npasses; i++) plan_phases(&b->pass[i]);
+    if (low->sign || b->linear) mstage_registers(low, low->ph_rbits[low->nphase - 1]);
 }
 
 /* The inverse of block b (n > 13): the inverse ring as a gather into the low
@@ -606,7 +733,7 @@ static void build_inverse_passes(qgtl_block_t *b, int n)
     b->ninv = 0;
     b->inv_ok = 0;
     if (n <= QGTL_TILE_BITS_MAX || (!b->is_ring && b->nperm > 0)) return;
-    if (low_pass(b, n, &b->ipass[0], QGTL_STORE_INPLACE, b->is_ring ? QGTL_LOAD_RING : QGTL_LOAD_NATURAL)) {
+    if (low_pass(b, n, &b->ipass[0], QGTL_STORE_INPLACE, b->is_ring ? QGTL_LOAD_RING : QGTL_LOAD_NATURAL, 0)) {
         b->ipass_flips[0] = b->is_ring;
         b->ninv = 1;
     }
@@ -616,7 +743,9 @@ static void build_inverse_passes(qgtl_block_t *b, int n)
     for (int i = 0; i < b->ninv; i++) {
         qgtl_pass_desc_t *p = &b->ipass[i];
         plan_phases(p);
-        if (p->load == QGTL_LOAD_RING) choose_thread_bits(p->ph_rbits[0], 0, 1, p->gather_tbits);
+        uint32_t ring[QGTL_TILE_BITS_MAX];
+        for (int j = 0; j < QGTL_TILE_BITS_MAX; j++) ring[j] = ring_image(1u << j);
+        if (p->load == QGTL_LOAD_RING) choose_thread_bits(p->ph_rbits[0], 0, ring, p->gather_tbits);
     }
     b->inv_ok = 1;
 }
@@ -635,7 +764,7 @@ typedef struct {
     double angle;
 } flat_gate_t;
 
-/* Expand CZ / CY into single-qubit gates and CNOTs. */
+/* Expand CY into single-qubit gates and a CNOT. */
 static int expand(const struct qgtl_plan *plan, flat_gate_t **out, int *count)
 {
     flat_gate_t *g = (flat_gate_t *)malloc(sizeof(flat_gate_t) * (size_t)(3 * plan->nops + 1));
@@ -644,10 +773,7 @@ static int expand(const struct qgtl_plan *plan, flat_gate_t **out, int *count)
     for (int i = 0; i < plan->nops; i++) {
         const qgtl_op_t *op = &plan->ops[i];
         flat_gate_t base = {op->type, op->q0, op->q1, op->param, i, op->angle};
-        if (op->type == GATE_TYPE_CZ) {
-            flat_gate_t h = {GATE_TYPE_H, op->q1, -1, -1, i, 0.0}, cx = {GATE_TYPE_CNOT, op->q0, op->q1, -1, i, 0.0};
-            g[k++] = h; g[k++] = cx; g[k++] = h;
-        } else if (op->type == GATE_TYPE_CY) {
+        if (op->type == GATE_TYPE_CY) {
             flat_gate_t sd = {GATE_TYPE_SDG, op->q1, -1, -1, i, 0.0}, cx = {GATE_TYPE_CNOT, op->q0, op->q1, -1, i, 0.0};
             flat_gate_t s = {GATE_TYPE_S, op->q1, -1, -1, i, 0.0};
             g[k++] = sd; g[k++] = cx; g[k++] = s;
@@ -723,6 +849,8 @@ static void set_matrices(struct qgtl_plan *plan)
             const qgtl_mat2 ub = mat_adj(&b->u[q]);
             t = mat_mul(&ub, &pp->A);
             pp->B = mat_mul(&t, &b->u[q]);
+            if ((b->sgn[q] >> q) & 1u)                           /* q(e_q) = 1: the constant of the partner's sign */
+                for (int e = 1; e <= 2; e++) pp->A.m[e] = cd(-pp->A.m[e].re, -pp->A.m[e].im);
         }
     }
     plan->tabs_dirty = 1;                                     /* new angles: phase tables to rebuild */
@@ -807,7 +935,7 @@ int qgtl_plan_build(struct qgtl_plan *plan)
 
     for (int i = 0; i < ng; i++) {
         const flat_gate_t *op = &g[i];
-        const int twoq = (op->type == GATE_TYPE_CNOT || op->type == GATE_TYPE_SWAP);
+        const int twoq = (op->type == GATE_TYPE_CNOT || op->type == GATE_TYPE_SWAP || op->type == GATE_TYPE_CZ);
         if (!twoq && touched[op->q0]) {
             /* close the block */
             cur->param_end = npar;
@@ -827,7 +955,7 @@ int qgtl_plan_build(struct qgtl_plan *plan)
                 memset(touched, 0, sizeof touched);
                 cur->param_begin = npar;
             }
-            cur->perm_type[cur->nperm] = (int8_t)(op->type == GATE_TYPE_SWAP ? 1 : 0);
+            cur->perm_type[cur->nperm] = (int8_t)(op->type == GATE_TYPE_CNOT ? 0 : op->type == GATE_TYPE_SWAP ? 1 : 2);
             cur->perm_a[cur->nperm] = (int8_t)op->q0;
             cur->perm_b[cur->nperm] = (int8_t)op->q1;
             cur->nperm++;
@@ -852,9 +980,15 @@ int qgtl_plan_build(struct qgtl_plan *plan)
     plan->nblocks = nb;
 
     /* finish blocks: ring detection, pass layouts, injection masks */
+    plan->has_signs = 0;
+    int rings = 0, stages = 0;
     for (int bi = 0; bi < nb; bi++) {
         qgtl_block_t *b = &plan->blocks[bi];
         detect_ring(b, n);
+        find_signs(b, n);
+        plan->has_signs |= b->has_sign;
+        rings += b->is_ring;
+        stages += b->nperm > 0;
         build_passes(b, n);
         if (plan->mode == QGTL_MODE_MIXED && plan->tune.sweep_schedule != 1) build_inverse_passes(b, n);
         /* images of the basis vectors under the inverse M-stage (the Z-frame masks below) */
@@ -864,14 +998,19 @@ int qgtl_plan_build(struct qgtl_plan *plan)
         for (int j = b->param_begin; j < b->param_end; j++) {
             qgtl_param_t *pp = &plan->params[order[j]];
             pp->v = perm_apply(b, 1u << pp->qubit);
-            uint32_t w = 0;
-            for (int j2 = 0; j2 < n; j2++)
+            const uint32_t bil = polar_row(b->sgn, pp->qubit);
+            uint32_t w = 0, z = 0;
+            for (int j2 = 0; j2 < n; j2++) {
                 if ((inv_img[j2] >> pp->qubit) & 1u) w |= 1u << j2;
+                z |= parity32(inv_img[j2] & bil) << j2;
+            }
             pp->w = w;
+            pp->z = z;
         }
     }
     /* D slot j holds the j-th parameter created (gate order); slot_param maps
      * slots back to the caller's parameter numbers. */
+    plan->ringless = n > QGTL_TILE_BITS_MAX && stages > 0 && rings == 0;
     free(plan->slot_param);
     plan->slot_param = order;
     free(g);
@@ -942,12 +1081,20 @@ void qgtl_resident_block(const qgtl_block_t *b, int n, qgtl_res_block_t *out, qg
     qgtl_cd pre[QGTL_RES_MAX_QUBITS][2], post[QGTL_RES_MAX_QUBITS][2];
     double scale = 1.0;
     out->has_pre = 0;
-    out->has_perm = b->nperm > 0;
+    out->has_perm = 0;
+    out->has_sign = b->has_sign;
+    if (b->has_sign) {
+        memcpy(out->sgn, b->sgn, sizeof out->sgn);
+        out->sgn_reg = 0;
+        for (uint32_t r = 0; r < 16; r++) out->sgn_reg |= sign_of(b->sgn, r << (n - 4)) << r;
+        for (int i = 0; i < 4; i++) out->sgn_bil[i] = polar_row(b->sgn, n - 4 + i);
+    }
     for (int q = 0; q < QGTL_RES_MAX_QUBITS; q++) {
         pre[q][0] = pre[q][1] = post[q][0] = post[q][1] = cd(1.0, 0.0);
         out->tan[q] = 0.f;
         out->swapped[q] = 0;
         out->img[q] = q < n ? perm_apply(b, 1u << q) : 0u;
+        if (q < n && out->img[q] != 1u << q) out->has_perm = 1;
         if (q >= n || !b->has_u[q]) continue;
         double c, s;
         factor_rotation(&b->u[q], &c, &s, pre[q], post[q]);
