@@ -30,6 +30,43 @@ __device__ __forceinline__ double2 cdiv(double2 a, double2 b) {
     return make_double2((a.x * b.x + a.y * b.y) / d, (a.y * b.x - a.x * b.y) / d);
 }
 
+// One lane of a double moved by a DPP pattern (two 32-bit DPP moves).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
+}
+
+__device__ __forceinline__ double readlane_f64(double v, int lane) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// Sum over the 64 lanes of a wave, identical in every lane and independent of timing:
+// pairs, quads (quad_perm), half rows and rows of 16 (row_half_mirror, row_mirror) by DPP,
+// each step adding two equal-shaped partial sums so every lane of a row holds the same bits;
+// then the four row sums (lanes 0, 16, 32, 48) in the order (r0 + r1) + (r2 + r3).
+__device__ __forceinline__ double wave_sum_f64(double v) {
+    v += dpp_f64<0xB1>(v);                            // quad_perm [1,0,3,2]
+    v += dpp_f64<0x4E>(v);                            // quad_perm [2,3,0,1]
+    v += dpp_f64<0x141>(v);                           // row_half_mirror
+    v += dpp_f64<0x140>(v);                           // row_mirror
+    return (readlane_f64(v, 0) + readlane_f64(v, 16)) + (readlane_f64(v, 32) + readlane_f64(v, 48));
+}
+
+// Largest of the 64 lanes, in every lane (no NaN among them).
+__device__ __forceinline__ double wave_max_f64(double v) {
+    v = fmax(v, dpp_f64<0xB1>(v));
+    v = fmax(v, dpp_f64<0x4E>(v));
+    v = fmax(v, dpp_f64<0x141>(v));
+    v = fmax(v, dpp_f64<0x140>(v));
+    return fmax(fmax(readlane_f64(v, 0), readlane_f64(v, 16)), fmax(readlane_f64(v, 32), readlane_f64(v, 48)));
+}
+
 // Block-wide sum in a fixed order (deterministic).
 __device__ double block_sum(double v, double *red) {
     red[threadIdx.x] = v;
@@ -149,6 +186,170 @@ __global__ __launch_bounds__(kT) void lu_solve_c128_kernel(double2 *Aall, const 
         for (int i = lane; i < P; i += 64) x[i] = sx[i];
         if (lane == 0) status[blockIdx.x] = 0;
     }
+}
+
+// The same for P <= 128 with the matrix in registers: lane l of wave w holds rows w + 16 s and
+// columns l + 64 c.  Rows stay where they are; pos is the position each has in the permuted order
+// (kept by every wave for the rows lane + 64 c), so the pivots, ties included, are those of the
+// kernel above.  A step: the lane with column i writes it to LDS; every wave finds
+// the pivot for itself while the pivot's wave publishes its row and two waves form
+// the multipliers and eliminate b; then each wave updates its rows.  Two barriers a step.  The rows
+// of U go to LDS by columns for the back substitution of one wave.  What bounds it: the
+// latency of the steps, about 0.7 us each (LDS, the maximum over a wave, a division).
+template <int ROWS, int COLS>
+__global__ __launch_bounds__(kT) void lu_solve_regs_kernel(const double2 *Aall, const double2 *ball, double2 *xall,
+                                                           int P, int *status) {
+    constexpr int N = 64 * COLS;
+    static_assert(16 * ROWS == N, "square");
+    __shared__ double2 col[N], mul[N], urow[N], by[N], upk[N * (N + 1) / 2];
+    const double2 *A = Aall + (size_t)blockIdx.x * P * P, *b = ball + (size_t)blockIdx.x * P;
+    double2 *x = xall + (size_t)blockIdx.x * P;
+    const int t = threadIdx.x, lane = t & 63, wave = qgtl::uniform(t >> 6);
+    double2 a[ROWS][COLS];
+    uint32_t done = 0;                       // rows of this wave that are a pivot row (or past the last)
+#pragma unroll
+    for (int s = 0; s < ROWS; s++) {
+        const int i = wave + 16 * s;
+        if (i >= P) done |= 1u << s;
+#pragma unroll
+        for (int c = 0; c < COLS; c++) {
+            const int j = lane + 64 * c;
+            a[s][c] = (i < P && j < P) ? A[(size_t)i * P + j] : make_double2(0.0, 0.0);
+        }
+    }
+    if (t < P) by[t] = b[t];
+    int pos[COLS];
+#pragma unroll
+    for (int c = 0; c < COLS; c++) pos[c] = lane + 64 * c;
+    auto pick = [](const double2 (&v)[COLS], int i) -> double2 {   // the one of index i
+        const bool up = COLS > 1 && i >= 64;
+        return make_double2(up ? v[COLS - 1].x : v[0].x, up ? v[COLS - 1].y : v[0].y);
+    };
+    auto publish = [&](int pr, int i) {      // row pr (this wave's) at position i: to urow and U
+#pragma unroll
+        for (int s = 0; s < ROWS; s++)
+            if (s == pr >> 4)
+#pragma unroll
+                for (int c = 0; c < COLS; c++) {
+                    const int j = lane + 64 * c;
+                    urow[j] = a[s][c];
+                    if (j >= i && j < P) upk[j * (j + 1) / 2 + i] = a[s][c];
+                }
+    };
+    for (int i = 0; i < P - 1; i++) {
+        if (lane == (i & 63)) {
+#pragma unroll
+            for (int s = 0; s < ROWS; s++) col[wave + 16 * s] = pick(a[s], i);
+        }
+        __syncthreads();
+        // pivot: max |a_ji|^2 over the rows at positions >= i, the first position on ties
+        double best = -1.0;
+        int brow = 0, bpos = 0;
+#pragma unroll
+        for (int c = 0; c < COLS; c++) {
+            const int row = lane + 64 * c;
+            if (row < P && pos[c] >= i) {
+                const double2 v = col[row];
+                const double m = v.x * v.x + v.y * v.y;
+                if (m > best || (m == best && pos[c] < bpos)) { best = m; brow = row; bpos = pos[c]; }
+            }
+        }
+        const double mx = wave_max_f64(best);
+        if (mx < 1e-10) {                    // the same in every wave
+            if (t == 0) status[blockIdx.x] = -1;
+            return;
+        }
+        unsigned long long cand = __ballot(best == mx);
+        int pr = 0, pp = P;
+        while (cand) {
+            const int src = __ffsll((long long)cand) - 1;
+            cand &= cand - 1;
+            const int q = __builtin_amdgcn_readlane(bpos, src);
+            if (q < pp) { pp = q; pr = __builtin_amdgcn_readlane(brow, src); }
+        }
+#pragma unroll
+        for (int c = 0; c < COLS; c++) {
+            const int row = lane + 64 * c;
+            if (row == pr) pos[c] = i;
+            else if (pos[c] == i) pos[c] = pp;
+        }
+        if (wave == (pr & 15)) {
+            publish(pr, i);
+            done |= 1u << (pr >> 4);
+        }
+        if (wave < COLS) {
+            const int mine = (COLS > 1 && wave == 1) ? pos[COLS - 1] : pos[0];
+            if (t < P && mine > i) {
+                const double2 l = cdiv(col[t], col[pr]), y = cmul(l, by[pr]);
+                mul[t] = l;
+                by[t] = make_double2(by[t].x - y.x, by[t].y - y.y);
+            }
+        }
+        __syncthreads();
+        double2 u[COLS];
+#pragma unroll
+        for (int c = 0; c < COLS; c++) u[c] = urow[lane + 64 * c];
+#pragma unroll
+        for (int s = 0; s < ROWS; s++)
+            if (!((done >> s) & 1u)) {
+                const double2 l = mul[wave + 16 * s];
+#pragma unroll
+                for (int c = 0; c < COLS; c++) {
+                    if (64 * c + 63 <= i) continue;
+                    const double2 lu = cmul(l, u[c]);
+                    a[s][c].x -= lu.x;
+                    a[s][c].y -= lu.y;
+                }
+            }
+    }
+    // the last row, and b in the permuted order
+    int last = 0;
+#pragma unroll
+    for (int c = 0; c < COLS; c++) {
+        const unsigned long long m = __ballot(pos[c] == P - 1);
+        if (m) last = 64 * c + __ffsll((long long)m) - 1;
+    }
+    __syncthreads();                         // col and urow: the last step's readers are through
+    if (wave == (last & 15)) publish(last, P - 1);
+    if (wave == 0) {
+#pragma unroll
+        for (int c = 0; c < COLS; c++)
+            if (lane + 64 * c < P) col[pos[c]] = by[lane + 64 * c];
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    double2 y[COLS], un[COLS];
+#pragma unroll
+    for (int c = 0; c < COLS; c++) y[c] = col[lane + 64 * c];
+    auto fetch = [&](int i, double2 (&u)[COLS]) -> double2 {
+#pragma unroll
+        for (int c = 0; c < COLS; c++) {
+            const int j = lane + 64 * c;
+            u[c] = upk[i * (i + 1) / 2 + (j < i ? j : i)];
+        }
+        return upk[i * (i + 1) / 2 + i];
+    };
+    double2 dn = fetch(P - 1, un);
+    for (int i = P - 1; i >= 0; i--) {
+        double2 u[COLS];
+        const double2 d = dn;
+#pragma unroll
+        for (int c = 0; c < COLS; c++) u[c] = un[c];
+        if (i > 0) dn = fetch(i - 1, un);
+        const double2 yv = pick(y, i);
+        const double2 xi = cdiv(make_double2(readlane_f64(yv.x, i & 63), readlane_f64(yv.y, i & 63)), d);
+#pragma unroll
+        for (int c = 0; c < COLS; c++) {
+            const int j = lane + 64 * c;
+            const double2 v = cmul(u[c], xi);
+            if (j < i) { y[c].x -= v.x; y[c].y -= v.y; }
+            if (j == i) y[c] = xi;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < COLS; c++)
+        if (lane + 64 * c < P) x[lane + 64 * c] = y[c];
+    if (lane == 0) status[blockIdx.x] = 0;
 }
 
 // ------------------------------------------------------- Hermitian Jacobi
@@ -505,34 +706,6 @@ constexpr int kPcgLds = 14;
 // U (P x r) is copied to LDS when P * r fits.
 constexpr int kPcgUCache = 2048;
 
-// One lane of a double moved by a DPP pattern (two 32-bit DPP moves).
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v) {
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, false);
-    return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
-}
-
-__device__ __forceinline__ double readlane_f64(double v, int lane) {
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
-// Sum over the 64 lanes of a wave, identical in every lane and independent of timing:
-// pairs, quads (quad_perm), half rows and rows of 16 (row_half_mirror, row_mirror) by DPP,
-// each step adding two equal-shaped partial sums so every lane of a row holds the same bits;
-// then the four row sums (lanes 0, 16, 32, 48) in the order (r0 + r1) + (r2 + r3).
-__device__ __forceinline__ double wave_sum_f64(double v) {
-    v += dpp_f64<0xB1>(v);                            // quad_perm [1,0,3,2]
-    v += dpp_f64<0x4E>(v);                            // quad_perm [2,3,0,1]
-    v += dpp_f64<0x141>(v);                           // row_half_mirror
-    v += dpp_f64<0x140>(v);                           // row_mirror
-    return (readlane_f64(v, 0) + readlane_f64(v, 16)) + (readlane_f64(v, 32) + readlane_f64(v, 48));
-}
-
 // W block sums with one barrier: wave sums into wp[wave][c], barrier, every thread adds the
 // 16 wave sums in wave order.  wp must not be rewritten before the next barrier, so callers
 // alternate between two buffers.
@@ -685,20 +858,15 @@ __global__ __launch_bounds__(kT) void pcg_f64_kernel(const double *Aall, const d
 // eigenvectors: Householder reduction to a real tridiagonal, then
 // multisection on the Sturm counts, 256 points at a time for each of the four.
 //
-// One workgroup; thread t owns column t % n and the rows t / n (mod nseg), in
-// registers (kExtRows per thread) where they fit, else in W (global, in L2).  A
-// step of the reduction applies the previous step's rank-2 update and forms the
+// One workgroup.  P <= 128: the matrix in registers, lane l of wave w holding rows w + 16 s and
+// columns l + 64 c, so a row's vectors are read from LDS once for two columns (and rows already reduced are
+// skipped by the whole wave); beyond, thread t owns column t % n and rows t / n (mod nseg) in W
+// (global, in L2).  A step of the reduction applies the previous step's rank-2 update and forms the
 // next matrix-vector product in one pass over the owned entries, with three
-// barriers.  What bounds it: the latency of those steps, about 6 us each.  At
-// P = 96 the condition number takes 667 us; the cyclic Jacobi iteration, which
-// did this before and still gives the eigenvectors elsewhere, 29.5 ms (8 to 10
-// sweeps of P - 1 steps, each two passes over A and one over V in global memory).
-//
+// barriers.  What bounds it: the latency of those steps.
 // Indices whose row is zero off the diagonal are set aside first: their
 // diagonal entries are exact eigenvalues (a parameter without effect leaves a
 // zero row, and its exact zero is no part of the condition number).
-constexpr int kExtRows = 16;      // register rows per thread (64 VGPRs of the 128 at 16 waves; 20 spill): n <= 128
-
 // number of eigenvalues of the tridiagonal (d, e2 = squared off-diagonals) below x
 __device__ __forceinline__ int sturm_count(const double *d, const double *e2, int n, double x, double pivmin) {
     int c = 0;
@@ -715,8 +883,86 @@ __device__ __forceinline__ int sturm_count(const double *d, const double *e2, in
     return c;
 }
 
+// The four extremes of the tridiagonal (d, e2) of order n, into the threads that searched them.
+__device__ __forceinline__ void tridiagonal_extremes(const double *sd, const double *se2, int n, double (*swv)[4],
+                                                     int *cnt, double &lo_all, double &hi_all, double &pos_all,
+                                                     double &neg_all) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    // Gershgorin bound
+    double bd = 0.0;
+    if (t < n)
+        bd = fabs(sd[t]) + (t > 0 ? sqrt(se2[t - 1]) : 0.0) + (t + 1 < n ? sqrt(se2[t]) : 0.0);
+    for (int o = 32; o > 0; o >>= 1) bd = fmax(bd, __shfl_xor(bd, o, 64));
+    if (lane == 0) swv[wave][0] = bd;
+    __syncthreads();
+    bd = 0.0;
+    for (int w = 0; w < kT / 64; w++) bd = fmax(bd, swv[w][0]);
+    // eigenvalues within 1e-30 of the bound of zero are exact zeros: rounding is at 1e-16 of it
+    const double B = bd * (1.0 + 1e-10), tiny = 1e-30 * bd, pivmin = 1e-40 * bd;
+    const int grp = t >> 8, m = t & 255;
+    const int cz = bd > 0.0 ? sturm_count(sd, se2, n, (t & 1) ? tiny : -tiny, pivmin) : 0;
+    const int n_neg = __shfl(cz, 0, 64), n_pos = __shfl(cz, 1, 64);   // below -tiny, below +tiny
+    const int idx = grp == 0 ? 0 : grp == 1 ? n - 1 : grp == 2 ? n_pos : n_neg - 1;
+    const bool want = bd > 0.0 && idx >= 0 && idx < n;
+    double lo = grp == 2 ? 0.0 : -B, hi = grp == 3 ? 0.0 : B;
+    for (int round = 0; round < 9; round++) {
+        const double h = (hi - lo) * (1.0 / 257.0);
+        int c = 0;
+        if (want) c = sturm_count(sd, se2, n, lo + h * (m + 1), pivmin) <= idx;
+        const int below = __popcll(__ballot(c != 0));
+        if (lane == 0) cnt[wave] = below;
+        __syncthreads();
+        const int k = cnt[4 * grp] + cnt[4 * grp + 1] + cnt[4 * grp + 2] + cnt[4 * grp + 3];
+        const double nl = k == 0 ? lo : lo + h * k, nh = k == 256 ? hi : lo + h * (k + 1);
+        lo = nl;
+        hi = nh;
+        __syncthreads();
+    }
+    const double v = bd > 0.0 ? 0.5 * (lo + hi) : 0.0;
+    if (grp == 0 && (want || bd == 0.0)) lo_all = fmin(lo_all, v);
+    if (grp == 1 && (want || bd == 0.0)) hi_all = fmax(hi_all, v);
+    if (grp == 2 && want) pos_all = fmin(pos_all, v);
+    if (grp == 3 && want) neg_all = fmax(neg_all, v);
+}
+
+__device__ __forceinline__ void write_extremes(double lo_all, double hi_all, double pos_all, double neg_all,
+                                               double (*swv)[4], double *out) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    for (int o = 32; o > 0; o >>= 1) {
+        lo_all = fmin(lo_all, __shfl_xor(lo_all, o, 64));
+        hi_all = fmax(hi_all, __shfl_xor(hi_all, o, 64));
+        pos_all = fmin(pos_all, __shfl_xor(pos_all, o, 64));
+        neg_all = fmax(neg_all, __shfl_xor(neg_all, o, 64));
+    }
+    __syncthreads();
+    if (lane == 0) { swv[wave][0] = lo_all; swv[wave][1] = hi_all; swv[wave][2] = pos_all; swv[wave][3] = neg_all; }
+    __syncthreads();
+    if (t == 0) {
+        for (int w = 1; w < kT / 64; w++) {
+            lo_all = fmin(lo_all, swv[w][0]);
+            hi_all = fmax(hi_all, swv[w][1]);
+            pos_all = fmin(pos_all, swv[w][2]);
+            neg_all = fmax(neg_all, swv[w][3]);
+        }
+        out[0] = lo_all; out[1] = hi_all; out[2] = pos_all; out[3] = neg_all;
+    }
+}
+
+// Householder vector of column k from x (x[i], i > k): u = x + (x_{k+1} / |x_{k+1}|) |x| e_{k+1}.  tail: the
+// sum of |x_i|^2 over i > k + 1; x0 in: x_{k+1}, out: u_{k+1}.  Returns tau = 2 / |u|^2 (0: nothing to do).
+__device__ __forceinline__ double householder(double tail, double2 &u0, double &e2) {
+    const double x0 = u0.x * u0.x + u0.y * u0.y;
+    e2 = x0;
+    if (!(tail > 0.0)) return 0.0;
+    e2 = tail + x0;
+    const double s = sqrt(e2), m = sqrt(x0);
+    const double tau = 1.0 / (s * (s + m));
+    if (m > 0.0) { u0.x += u0.x * (s / m); u0.y += u0.y * (s / m); }
+    else u0.x = s;
+    return tau;
+}
+
 // out: smallest, largest, smallest positive (+inf: none), largest negative (-inf: none)
-template <bool REG>
 __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__restrict__ A, int P, double2 *W,
                                                            double *out) {
     __shared__ double2 su[kT], sq[kT], sx[kT], part[kT];
@@ -757,7 +1003,6 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
     if (n > 0) {                                             // n >= 2: an index is live with another
         const int nseg = kT / n, seg = t / n, j = t % n;
         const int rows = (n + nseg - 1) / nseg;
-        double2 a[REG ? kExtRows : 1];
         const int oj = map[j];
         auto entry = [&](int i) -> double2 {
             const int oi = map[i];
@@ -765,16 +1010,8 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
             const double2 v = A[(size_t)oj * P + oi];
             return make_double2(v.x, -v.y);
         };
-        if constexpr (REG) {
-#pragma unroll
-            for (int r = 0; r < kExtRows; r++) {
-                const int i = seg + nseg * r;
-                a[r] = (seg < nseg && i < n) ? entry(i) : make_double2(0.0, 0.0);
-            }
-        } else {
-            if (seg < nseg)
-                for (int i = seg; i < n; i += nseg) W[(size_t)i * n + j] = entry(i);
-        }
+        if (seg < nseg)
+            for (int i = seg; i < n; i += nseg) W[(size_t)i * n + j] = entry(i);
         // x_i of column k for this thread's rows (it owns column k): the entry with the pending update
         auto pend = [&](double2 v, int i, double2 uk, double2 qk) -> double2 {
             const double2 ui = su[i], qi = sq[i];
@@ -784,24 +1021,11 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
         };
         for (int k = 0; k < n; k++) {
             const double2 uj = su[j], qj = sq[j];
-            // the row numbers formed anew at every step: hoisted out of the loop, the rows' LDS
-            // addresses take the registers the rows need (192 bytes of spills a thread: 710 against 667 us)
-            int s0 = seg;
-            __asm__ volatile("" : "+v"(s0));
-            if (j == k && seg < nseg) {
-                if constexpr (REG) {
-#pragma unroll
-                    for (int r = 0; r < kExtRows; r++) {
-                        const int i = s0 + nseg * r;
-                        if (i >= k && i < n) sx[i] = pend(a[r], i, uj, qj);
-                    }
-                } else {
-                    for (int r = 0; r < rows; r++) {
-                        const int i = seg + nseg * r;
-                        if (i >= k && i < n) sx[i] = pend(W[(size_t)i * n + j], i, uj, qj);
-                    }
+            if (j == k && seg < nseg)
+                for (int r = 0; r < rows; r++) {
+                    const int i = seg + nseg * r;
+                    if (i >= k && i < n) sx[i] = pend(W[(size_t)i * n + j], i, uj, qj);
                 }
-            }
             __syncthreads();
             if (t == 0) sd[k] = sx[k].x;
             if (k == n - 1) break;
@@ -809,15 +1033,8 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
             for (int i = k + 2 + lane; i < n; i += 64) tail += sx[i].x * sx[i].x + sx[i].y * sx[i].y;
             tail = wave_sum_f64(tail);
             double2 u0 = sx[k + 1];
-            const double x0 = u0.x * u0.x + u0.y * u0.y;
-            double tau = 0.0, e2 = x0;
-            if (tail > 0.0) {
-                e2 = tail + x0;
-                const double s = sqrt(e2), m = sqrt(x0);
-                tau = 1.0 / (s * (s + m));                   // 2 / |u|^2
-                if (m > 0.0) { u0.x += u0.x * (s / m); u0.y += u0.y * (s / m); }
-                else u0.x = s;
-            }
+            double e2;
+            const double tau = householder(tail, u0, e2);
             if (t == 0) se2[k] = e2;
             double pr = 0.0, pi = 0.0;
             if (j > k && seg < nseg) {
@@ -828,17 +1045,9 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
                     pi += v.x * ui.y - v.y * ui.x;
                     return v;
                 };
-                if constexpr (REG) {
-#pragma unroll
-                    for (int r = 0; r < kExtRows; r++) {
-                        const int i = s0 + nseg * r;
-                        if (i > k && i < n) a[r] = one(a[r], i);
-                    }
-                } else {
-                    for (int r = 0; r < rows; r++) {
-                        const int i = seg + nseg * r;
-                        if (i > k && i < n) W[(size_t)i * n + j] = one(W[(size_t)i * n + j], i);
-                    }
+                for (int r = 0; r < rows; r++) {
+                    const int i = seg + nseg * r;
+                    if (i > k && i < n) W[(size_t)i * n + j] = one(W[(size_t)i * n + j], i);
                 }
             }
             part[t] = make_double2(pr, pi);
@@ -867,60 +1076,158 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
             __syncthreads();
         }
         __syncthreads();
-        // Gershgorin bound
-        double bd = 0.0;
-        if (t < n)
-            bd = fabs(sd[t]) + (t > 0 ? sqrt(se2[t - 1]) : 0.0) + (t + 1 < n ? sqrt(se2[t]) : 0.0);
-        for (int o = 32; o > 0; o >>= 1) bd = fmax(bd, __shfl_xor(bd, o, 64));
-        if (lane == 0) swv[wave][0] = bd;
+        tridiagonal_extremes(sd, se2, n, swv, cnt, lo_all, hi_all, pos_all, neg_all);
+    }
+    write_extremes(lo_all, hi_all, pos_all, neg_all, swv, out);
+}
+
+// The same for P <= 16 ROWS = 64 COLS with the matrix in registers.
+template <int ROWS, int COLS>
+__global__ __launch_bounds__(kT) void herm_extremes_regs_kernel(const double2 *__restrict__ A, int P, double *out) {
+    constexpr int N = 64 * COLS;
+    static_assert(16 * ROWS == N, "square");
+    __shared__ double2 su[N], sq[N], sx[N], part[16][N];
+    __shared__ double sd[N], se2[N], swv[kT / 64][4], sup[kT / 64];
+    __shared__ int map[N], live[N], cnt[kT / 64];
+    const int t = threadIdx.x, lane = t & 63, wave = qgtl::uniform(t >> 6);
+    auto entry = [&](int oi, int oj) -> double2 {            // the upper triangle's
+        if (oi <= oj) { double2 v = A[(size_t)oi * P + oj]; if (oi == oj) v.y = 0.0; return v; }
+        const double2 v = A[(size_t)oj * P + oi];
+        return make_double2(v.x, -v.y);
+    };
+    double2 a[ROWS][COLS];
+#pragma unroll
+    for (int s = 0; s < ROWS; s++) {
+        const int i = wave + 16 * s;
+        bool any = false;
+#pragma unroll
+        for (int c = 0; c < COLS; c++) {
+            const int j = lane + 64 * c;
+            a[s][c] = (i < P && j < P) ? entry(i, j) : make_double2(0.0, 0.0);
+            any = any || (i != j && (a[s][c].x != 0.0 || a[s][c].y != 0.0));
+        }
+        const bool row = __ballot(any) != 0;
+        if (lane == 0) live[i] = row;
+    }
+    if (t < N) su[t] = sq[t] = make_double2(0.0, 0.0);
+    __syncthreads();
+    // live indices in order, counted by every wave
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < COLS; c++) {
+        const bool l = live[lane + 64 * c] != 0;
+        const unsigned long long b = __ballot(l);
+        if (wave == 0 && l) map[n + __popcll(b & ((1ull << lane) - 1ull))] = lane + 64 * c;
+        n += __popcll(b);
+    }
+    n = qgtl::uniform(n);
+    __syncthreads();
+    if (n < P && n > 0) {                                    // close up the isolated indices
+#pragma unroll
+        for (int s = 0; s < ROWS; s++)
+#pragma unroll
+            for (int c = 0; c < COLS; c++) {
+                const int i = wave + 16 * s, j = lane + 64 * c;
+                a[s][c] = (i < n && j < n) ? entry(map[i], map[j]) : make_double2(0.0, 0.0);
+            }
+    }
+    for (int k = 0; k < n; k++) {
+        double2 uj[COLS], qj[COLS];
+#pragma unroll
+        for (int c = 0; c < COLS; c++) { uj[c] = su[lane + 64 * c]; qj[c] = sq[lane + 64 * c]; }
+        // v - u_i conj(q_j) - q_i conj(u_j)
+        auto pend = [&](double2 v, double2 ui, double2 qi, int c) -> double2 {
+            v.x -= ui.x * qj[c].x + ui.y * qj[c].y + qi.x * uj[c].x + qi.y * uj[c].y;
+            v.y -= ui.y * qj[c].x - ui.x * qj[c].y + qi.y * uj[c].x - qi.x * uj[c].y;
+            return v;
+        };
+        if (wave == (k & 15)) {                              // column k from row k
+            const double2 uk = su[k], qk = sq[k];
+#pragma unroll
+            for (int s = 0; s < ROWS; s++)
+                if (s == k >> 4)
+#pragma unroll
+                    for (int c = 0; c < COLS; c++) {
+                        const double2 v = pend(a[s][c], uk, qk, c);
+                        sx[lane + 64 * c] = make_double2(v.x, -v.y);
+                    }
+        }
         __syncthreads();
-        bd = 0.0;
-        for (int w = 0; w < kT / 64; w++) bd = fmax(bd, swv[w][0]);
-        // eigenvalues within 1e-30 of the bound of zero are exact zeros: rounding is at 1e-16 of it
-        const double B = bd * (1.0 + 1e-10), tiny = 1e-30 * bd, pivmin = 1e-40 * bd;
-        const int grp = t >> 8, m = t & 255;
-        const int cz = bd > 0.0 ? sturm_count(sd, se2, n, (t & 1) ? tiny : -tiny, pivmin) : 0;
-        const int n_neg = __shfl(cz, 0, 64), n_pos = __shfl(cz, 1, 64);   // below -tiny, below +tiny
-        const int idx = grp == 0 ? 0 : grp == 1 ? n - 1 : grp == 2 ? n_pos : n_neg - 1;
-        const bool want = bd > 0.0 && idx >= 0 && idx < n;
-        double lo = grp == 2 ? 0.0 : -B, hi = grp == 3 ? 0.0 : B;
-        for (int round = 0; round < 9; round++) {
-            const double h = (hi - lo) * (1.0 / 257.0);
-            int c = 0;
-            if (want) c = sturm_count(sd, se2, n, lo + h * (m + 1), pivmin) <= idx;
-            const int below = __popcll(__ballot(c != 0));
-            if (lane == 0) cnt[wave] = below;
-            __syncthreads();
-            const int k = cnt[4 * grp] + cnt[4 * grp + 1] + cnt[4 * grp + 2] + cnt[4 * grp + 3];
-            const double nl = k == 0 ? lo : lo + h * k, nh = k == 256 ? hi : lo + h * (k + 1);
-            lo = nl;
-            hi = nh;
-            __syncthreads();
+        if (t == 0) sd[k] = sx[k].x;
+        if (k == n - 1) break;
+        double2 xj[COLS];
+        double tail = 0.0;
+#pragma unroll
+        for (int c = 0; c < COLS; c++) {
+            const int j = lane + 64 * c;
+            xj[c] = sx[j];
+            if (j > k + 1 && j < n) tail += xj[c].x * xj[c].x + xj[c].y * xj[c].y;
         }
-        const double v = bd > 0.0 ? 0.5 * (lo + hi) : 0.0;
-        if (grp == 0 && (want || bd == 0.0)) lo_all = fmin(lo_all, v);
-        if (grp == 1 && (want || bd == 0.0)) hi_all = fmax(hi_all, v);
-        if (grp == 2 && want) pos_all = fmin(pos_all, v);
-        if (grp == 3 && want) neg_all = fmax(neg_all, v);
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        lo_all = fmin(lo_all, __shfl_xor(lo_all, o, 64));
-        hi_all = fmax(hi_all, __shfl_xor(hi_all, o, 64));
-        pos_all = fmin(pos_all, __shfl_xor(pos_all, o, 64));
-        neg_all = fmax(neg_all, __shfl_xor(neg_all, o, 64));
+        tail = wave_sum_f64(tail);
+        double2 u0 = sx[k + 1];
+        double e2;
+        const double tau = householder(tail, u0, e2);
+        if (t == 0) se2[k] = e2;
+        double2 p[COLS];
+#pragma unroll
+        for (int c = 0; c < COLS; c++) {
+            p[c] = make_double2(0.0, 0.0);
+            if (lane + 64 * c == k + 1) xj[c] = u0;
+        }
+#pragma unroll
+        for (int s = 0; s < ROWS; s++) {
+            const int i = wave + 16 * s;
+            if (i > k && i < n) {                            // the same for the wave
+                const double2 ui = su[i], qi = sq[i], vi = i == k + 1 ? u0 : sx[i];
+#pragma unroll
+                for (int c = 0; c < COLS; c++) {
+                    if (64 * c + 63 <= k) continue;
+                    const double2 v = pend(a[s][c], ui, qi, c);
+                    a[s][c] = v;
+                    p[c].x += v.x * vi.x + v.y * vi.y;       // conj(a_ij) u_i
+                    p[c].y += v.x * vi.y - v.y * vi.x;
+                }
+            }
+        }
+        // p = tau A u; K = tau / 2 u^H p; q = p - K u
+        double up = 0.0;
+#pragma unroll
+        for (int c = 0; c < COLS; c++) {
+            const int j = lane + 64 * c;
+            part[wave][j] = p[c];
+            if (j > k && j < n) up += xj[c].x * p[c].x + xj[c].y * p[c].y;
+        }
+        up = wave_sum_f64(up);
+        if (lane == 0) sup[wave] = up;
+        __syncthreads();
+        if (wave < COLS) {
+            double2 s = part[0][t];
+            up = sup[0];
+#pragma unroll 3
+            for (int w = 1; w < 16; w++) {
+                s.x += part[w][t].x;
+                s.y += part[w][t].y;
+                up += sup[w];
+            }
+            double2 ut = make_double2(0.0, 0.0), qt = make_double2(0.0, 0.0);
+            if (t > k && t < n && tau > 0.0) {
+                ut = t == k + 1 ? u0 : sx[t];
+                const double kk = 0.5 * tau * tau * up;
+                qt = make_double2(tau * s.x - kk * ut.x, tau * s.y - kk * ut.y);
+            }
+            su[t] = ut;
+            sq[t] = qt;
+        }
+        __syncthreads();
     }
     __syncthreads();
-    if (lane == 0) { swv[wave][0] = lo_all; swv[wave][1] = hi_all; swv[wave][2] = pos_all; swv[wave][3] = neg_all; }
-    __syncthreads();
-    if (t == 0) {
-        for (int w = 1; w < kT / 64; w++) {
-            lo_all = fmin(lo_all, swv[w][0]);
-            hi_all = fmax(hi_all, swv[w][1]);
-            pos_all = fmin(pos_all, swv[w][2]);
-            neg_all = fmax(neg_all, swv[w][3]);
-        }
-        out[0] = lo_all; out[1] = hi_all; out[2] = pos_all; out[3] = neg_all;
-    }
+    const double inf = __builtin_inf();
+    const bool iso = t < P && !live[t < N ? t : 0];
+    const double isov = iso ? A[(size_t)t * P + t].x : 0.0;
+    double lo_all = iso ? isov : inf, hi_all = iso ? isov : -inf;
+    double pos_all = iso && isov > 0.0 ? isov : inf, neg_all = iso && isov < 0.0 ? isov : -inf;
+    if (n > 0) tridiagonal_extremes(sd, se2, n, swv, cnt, lo_all, hi_all, pos_all, neg_all);
+    write_extremes(lo_all, hi_all, pos_all, neg_all, swv, out);
 }
 
 // B = M^H M for the singular values of a general complex matrix
@@ -1054,8 +1361,15 @@ int qgtl_hip_pinv_apply_c128(const void *V, const double *ev, const void *g, voi
 }
 
 int qgtl_hip_lu_solve_c128(void *A, const void *b, void *x, int *piv, int P, int batch, int *status) {
-    hipLaunchKernelGGL(lu_solve_c128_kernel, dim3(batch), dim3(kT), 0, qgtl::stream(), (double2 *)A,
-                       (const double2 *)b, (double2 *)x, piv, P, status);
+    if (P <= 64)
+        hipLaunchKernelGGL((lu_solve_regs_kernel<4, 1>), dim3(batch), dim3(kT), 0, qgtl::stream(), (const double2 *)A,
+                           (const double2 *)b, (double2 *)x, P, status);
+    else if (P <= 128)
+        hipLaunchKernelGGL((lu_solve_regs_kernel<8, 2>), dim3(batch), dim3(kT), 0, qgtl::stream(), (const double2 *)A,
+                           (const double2 *)b, (double2 *)x, P, status);
+    else
+        hipLaunchKernelGGL(lu_solve_c128_kernel, dim3(batch), dim3(kT), 0, qgtl::stream(), (double2 *)A,
+                           (const double2 *)b, (double2 *)x, piv, P, status);
     QGTL_LAUNCH_CHECK("lu_solve_c128");
     return 0;
 }
@@ -1070,14 +1384,14 @@ int qgtl_hip_herm_eig_c128(void *A, void *V, double *ev, int P, int batch, int m
 
 int qgtl_hip_herm_extremes_c128(const void *A, void *W, int P, double *out4) {
     if (P < 1 || P > kT) return qgtl::set_error_msg(-118, "herm_extremes: needs 1 <= P <= 1024");
-    // every matrix of the kernel's order n <= P fits the register rows when that of order P does
-    // (n^2 entries over kT threads: rows(n) = ceil(n / floor(kT / n)) grows with n)
-    const int nseg = kT / P, rows = (P + nseg - 1) / nseg;
-    if (rows <= kExtRows)
-        hipLaunchKernelGGL(herm_extremes_kernel<true>, dim3(1), dim3(kT), 0, qgtl::stream(), (const double2 *)A, P,
-                           (double2 *)W, out4);
+    if (P <= 64)
+        hipLaunchKernelGGL((herm_extremes_regs_kernel<4, 1>), dim3(1), dim3(kT), 0, qgtl::stream(), (const double2 *)A, P,
+                           out4);
+    else if (P <= 128)
+        hipLaunchKernelGGL((herm_extremes_regs_kernel<8, 2>), dim3(1), dim3(kT), 0, qgtl::stream(), (const double2 *)A, P,
+                           out4);
     else
-        hipLaunchKernelGGL(herm_extremes_kernel<false>, dim3(1), dim3(kT), 0, qgtl::stream(), (const double2 *)A, P,
+        hipLaunchKernelGGL(herm_extremes_kernel, dim3(1), dim3(kT), 0, qgtl::stream(), (const double2 *)A, P,
                            (double2 *)W, out4);
     QGTL_LAUNCH_CHECK("herm_extremes_c128");
     return 0;
