@@ -188,77 +188,70 @@ __global__ __launch_bounds__(kT) void lu_solve_c128_kernel(double2 *Aall, const 
     }
 }
 
-// The same for P <= 128 with the matrix in registers: lane l of wave w holds rows w + 16 s and
-// columns l + 64 c.  Rows stay where they are; pos is the position each has in the permuted order
-// (kept by every wave for the rows lane + 64 c), so the pivots, ties included, are those of the
-// kernel above.  A step: the lane with column i writes it to LDS; every wave finds
-// the pivot for itself while the pivot's wave publishes its row and two waves form
-// the multipliers and eliminate b; then each wave updates its rows.  Two barriers a step.  The rows
-// of U go to LDS by columns for the back substitution of one wave.  What bounds it: the
-// latency of the steps, about 0.7 us each (LDS, the maximum over a wave, a division).
-template <int ROWS, int COLS>
+// The same for P <= 128 with the matrix in registers: wave w holds columns w + 16 s, its lane l
+// rows l + 64 c.  Rows stay where they are; pos is the position each has in the permuted order
+// (kept by every wave), so the pivots, ties included, are those of the kernel above.  The wave of
+// column i finds its pivot and the multipliers without leaving the wave and hands
+// them on through LDS; the others take the pivot row's element of a column from the lane
+// that holds it.  One barrier a step: the wave of column i + 1 updates that column first and
+// finds its pivot while the others update theirs.  b is one more column, of the last wave.  U goes
+// to LDS by columns for the back substitution of one wave.  What bounds it: the latency of that
+// chain (LDS, the maximum over a wave, a complex division).
+// P = 96: 172 us; 274 us with rows split over waves (two barriers a step, the multipliers formed
+// by two waves while the others wait), 434 us in global memory.
+template <int COLS, int ROWS>
 __global__ __launch_bounds__(kT) void lu_solve_regs_kernel(const double2 *Aall, const double2 *ball, double2 *xall,
                                                            int P, int *status) {
-    constexpr int N = 64 * COLS;
-    static_assert(16 * ROWS == N, "square");
-    __shared__ double2 col[N], mul[N], urow[N], by[N], upk[N * (N + 1) / 2];
+    constexpr int N = 64 * ROWS;
+    static_assert(16 * COLS == N, "square");
+    __shared__ double2 mul[2][N], yp[N], upk[N * (N + 1) / 2];
+    __shared__ int spiv[2];                  // pivot row | its position << 8, or -1: singular
     const double2 *A = Aall + (size_t)blockIdx.x * P * P, *b = ball + (size_t)blockIdx.x * P;
     double2 *x = xall + (size_t)blockIdx.x * P;
     const int t = threadIdx.x, lane = t & 63, wave = qgtl::uniform(t >> 6);
-    double2 a[ROWS][COLS];
-    uint32_t done = 0;                       // rows of this wave that are a pivot row (or past the last)
+    double2 a[COLS][ROWS], y[ROWS];
+    int pos[ROWS];
 #pragma unroll
-    for (int s = 0; s < ROWS; s++) {
-        const int i = wave + 16 * s;
-        if (i >= P) done |= 1u << s;
+    for (int c = 0; c < ROWS; c++) {
+        const int i = lane + 64 * c;
+        pos[c] = i;
+        y[c] = (wave == 15 && i < P) ? b[i] : make_double2(0.0, 0.0);
 #pragma unroll
-        for (int c = 0; c < COLS; c++) {
-            const int j = lane + 64 * c;
+        for (int s = 0; s < COLS; s++) {
+            const int j = wave + 16 * s;
             a[s][c] = (i < P && j < P) ? A[(size_t)i * P + j] : make_double2(0.0, 0.0);
         }
     }
-    if (t < P) by[t] = b[t];
-    int pos[COLS];
-#pragma unroll
-    for (int c = 0; c < COLS; c++) pos[c] = lane + 64 * c;
-    auto pick = [](const double2 (&v)[COLS], int i) -> double2 {   // the one of index i
-        const bool up = COLS > 1 && i >= 64;
-        return make_double2(up ? v[COLS - 1].x : v[0].x, up ? v[COLS - 1].y : v[0].y);
+    // row pr's element of a column, for every lane
+    auto of_row = [](const double2 (&v)[ROWS], int pr) __attribute__((always_inline)) -> double2 {
+        const bool up = ROWS > 1 && pr >= 64;
+        return make_double2(readlane_f64(up ? v[ROWS - 1].x : v[0].x, pr & 63),
+                            readlane_f64(up ? v[ROWS - 1].y : v[0].y, pr & 63));
     };
-    auto publish = [&](int pr, int i) {      // row pr (this wave's) at position i: to urow and U
+    auto column = [&](int j, double2 (&v)[ROWS]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int s = 0; s < ROWS; s++)
-            if (s == pr >> 4)
+        for (int c = 0; c < ROWS; c++) {
+            v[c] = a[0][c];
 #pragma unroll
-                for (int c = 0; c < COLS; c++) {
-                    const int j = lane + 64 * c;
-                    urow[j] = a[s][c];
-                    if (j >= i && j < P) upk[j * (j + 1) / 2 + i] = a[s][c];
-                }
-    };
-    for (int i = 0; i < P - 1; i++) {
-        if (lane == (i & 63)) {
-#pragma unroll
-            for (int s = 0; s < ROWS; s++) col[wave + 16 * s] = pick(a[s], i);
+            for (int s = 1; s < COLS; s++) {
+                const bool here = s == j >> 4;
+                v[c].x = here ? a[s][c].x : v[c].x;
+                v[c].y = here ? a[s][c].y : v[c].y;
+            }
         }
-        __syncthreads();
-        // pivot: max |a_ji|^2 over the rows at positions >= i, the first position on ties
+    };
+    // column i (this wave's, v): pivot and multipliers
+    auto factor = [&](int i, const double2 (&v)[ROWS]) __attribute__((always_inline)) {
+        // max |a_ji|^2 over the rows at positions >= i, the first position on ties
         double best = -1.0;
         int brow = 0, bpos = 0;
 #pragma unroll
-        for (int c = 0; c < COLS; c++) {
+        for (int c = 0; c < ROWS; c++) {
             const int row = lane + 64 * c;
-            if (row < P && pos[c] >= i) {
-                const double2 v = col[row];
-                const double m = v.x * v.x + v.y * v.y;
-                if (m > best || (m == best && pos[c] < bpos)) { best = m; brow = row; bpos = pos[c]; }
-            }
+            const double m = v[c].x * v[c].x + v[c].y * v[c].y;
+            if (row < P && pos[c] >= i && (m > best || (m == best && pos[c] < bpos))) { best = m; brow = row; bpos = pos[c]; }
         }
         const double mx = wave_max_f64(best);
-        if (mx < 1e-10) {                    // the same in every wave
-            if (t == 0) status[blockIdx.x] = -1;
-            return;
-        }
         unsigned long long cand = __ballot(best == mx);
         int pr = 0, pp = P;
         while (cand) {
@@ -267,63 +260,69 @@ __global__ __launch_bounds__(kT) void lu_solve_regs_kernel(const double2 *Aall, 
             const int q = __builtin_amdgcn_readlane(bpos, src);
             if (q < pp) { pp = q; pr = __builtin_amdgcn_readlane(brow, src); }
         }
+        const double2 d = of_row(v, pr);
 #pragma unroll
-        for (int c = 0; c < COLS; c++) {
+        for (int c = 0; c < ROWS; c++) mul[i & 1][lane + 64 * c] = cdiv(v[c], d);
+        if (lane == 0) spiv[i & 1] = mx < 1e-10 ? -1 : pr | pp << 8;
+    };
+    // v -= l u on the rows below the pivot
+    auto eliminate = [&](double2 (&v)[ROWS], const double2 (&l)[ROWS], double2 u, int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < ROWS; c++)
+            if (pos[c] > i) {
+                v[c].x = fma(l[c].y, u.y, fma(-l[c].x, u.x, v[c].x));
+                v[c].y = fma(-l[c].y, u.x, fma(-l[c].x, u.y, v[c].y));
+            }
+    };
+    if (wave == 0 && P > 1) factor(0, a[0]);
+    for (int i = 0; i < P - 1; i++) {
+        __syncthreads();
+        const int piv = qgtl::uniform(spiv[i & 1]);
+        if (piv < 0) {                       // the same for every wave
+            if (t == 0) status[blockIdx.x] = -1;
+            return;
+        }
+        const int pr = piv & 255, pp = piv >> 8;
+        double2 l[ROWS];
+#pragma unroll
+        for (int c = 0; c < ROWS; c++) {
             const int row = lane + 64 * c;
+            l[c] = mul[i & 1][row];
             if (row == pr) pos[c] = i;
             else if (pos[c] == i) pos[c] = pp;
         }
-        if (wave == (pr & 15)) {
-            publish(pr, i);
-            done |= 1u << (pr >> 4);
+        if (wave == ((i + 1) & 15)) {
+            double2 v[ROWS];
+            column(i + 1, v);
+            eliminate(v, l, of_row(v, pr), i);               // a copy: the loop below does the column itself
+            if (i + 1 < P - 1) factor(i + 1, v);
         }
-        if (wave < COLS) {
-            const int mine = (COLS > 1 && wave == 1) ? pos[COLS - 1] : pos[0];
-            if (t < P && mine > i) {
-                const double2 l = cdiv(col[t], col[pr]), y = cmul(l, by[pr]);
-                mul[t] = l;
-                by[t] = make_double2(by[t].x - y.x, by[t].y - y.y);
-            }
+#pragma unroll
+        for (int s = 0; s < COLS; s++) {
+            const int j = wave + 16 * s;
+            if (j > i && j < P) eliminate(a[s], l, of_row(a[s], pr), i);
         }
-        __syncthreads();
-        double2 u[COLS];
-#pragma unroll
-        for (int c = 0; c < COLS; c++) u[c] = urow[lane + 64 * c];
-#pragma unroll
-        for (int s = 0; s < ROWS; s++)
-            if (!((done >> s) & 1u)) {
-                const double2 l = mul[wave + 16 * s];
-#pragma unroll
-                for (int c = 0; c < COLS; c++) {
-                    if (64 * c + 63 <= i) continue;
-                    const double2 lu = cmul(l, u[c]);
-                    a[s][c].x -= lu.x;
-                    a[s][c].y -= lu.y;
-                }
-            }
+        if (wave == 15) eliminate(y, l, of_row(y, pr), i);
     }
-    // the last row, and b in the permuted order
-    int last = 0;
+    // U by columns, b in the permuted order
 #pragma unroll
-    for (int c = 0; c < COLS; c++) {
-        const unsigned long long m = __ballot(pos[c] == P - 1);
-        if (m) last = 64 * c + __ffsll((long long)m) - 1;
-    }
-    __syncthreads();                         // col and urow: the last step's readers are through
-    if (wave == (last & 15)) publish(last, P - 1);
-    if (wave == 0) {
+    for (int c = 0; c < ROWS; c++) {
+        if (lane + 64 * c >= P) continue;
+        if (wave == 15) yp[pos[c]] = y[c];
 #pragma unroll
-        for (int c = 0; c < COLS; c++)
-            if (lane + 64 * c < P) col[pos[c]] = by[lane + 64 * c];
+        for (int s = 0; s < COLS; s++) {
+            const int j = wave + 16 * s;
+            if (j < P && pos[c] <= j) upk[j * (j + 1) / 2 + pos[c]] = a[s][c];
+        }
     }
     __syncthreads();
     if (wave != 0) return;
-    double2 y[COLS], un[COLS];
 #pragma unroll
-    for (int c = 0; c < COLS; c++) y[c] = col[lane + 64 * c];
-    auto fetch = [&](int i, double2 (&u)[COLS]) -> double2 {
+    for (int c = 0; c < ROWS; c++) y[c] = yp[lane + 64 * c];
+    double2 un[ROWS];
+    auto fetch = [&](int i, double2 (&u)[ROWS]) -> double2 {
 #pragma unroll
-        for (int c = 0; c < COLS; c++) {
+        for (int c = 0; c < ROWS; c++) {
             const int j = lane + 64 * c;
             u[c] = upk[i * (i + 1) / 2 + (j < i ? j : i)];
         }
@@ -331,15 +330,14 @@ __global__ __launch_bounds__(kT) void lu_solve_regs_kernel(const double2 *Aall, 
     };
     double2 dn = fetch(P - 1, un);
     for (int i = P - 1; i >= 0; i--) {
-        double2 u[COLS];
+        double2 u[ROWS];
         const double2 d = dn;
 #pragma unroll
-        for (int c = 0; c < COLS; c++) u[c] = un[c];
+        for (int c = 0; c < ROWS; c++) u[c] = un[c];
         if (i > 0) dn = fetch(i - 1, un);
-        const double2 yv = pick(y, i);
-        const double2 xi = cdiv(make_double2(readlane_f64(yv.x, i & 63), readlane_f64(yv.y, i & 63)), d);
+        const double2 xi = cdiv(of_row(y, i), d);
 #pragma unroll
-        for (int c = 0; c < COLS; c++) {
+        for (int c = 0; c < ROWS; c++) {
             const int j = lane + 64 * c;
             const double2 v = cmul(u[c], xi);
             if (j < i) { y[c].x -= v.x; y[c].y -= v.y; }
@@ -347,7 +345,7 @@ __global__ __launch_bounds__(kT) void lu_solve_regs_kernel(const double2 *Aall, 
         }
     }
 #pragma unroll
-    for (int c = 0; c < COLS; c++)
+    for (int c = 0; c < ROWS; c++)
         if (lane + 64 * c < P) x[lane + 64 * c] = y[c];
     if (lane == 0) status[blockIdx.x] = 0;
 }
