@@ -197,7 +197,7 @@ __global__ __launch_bounds__(kT) void lu_solve_c128_kernel(double2 *Aall, const 
 // finds its pivot while the others update theirs.  b is one more column, of the last wave.  U goes
 // to LDS by columns for the back substitution of one wave.  What bounds it: the latency of that
 // chain (LDS, the maximum over a wave, a complex division).
-// P = 96: 172 us; 274 us with rows split over waves (two barriers a step, the multipliers formed
+// P = 96: 162 us; 274 us with rows split over waves (two barriers a step, the multipliers formed
 // by two waves while the others wait), 434 us in global memory.
 template <int COLS, int ROWS>
 __global__ __launch_bounds__(kT) void lu_solve_regs_kernel(const double2 *Aall, const double2 *ball, double2 *xall,
@@ -292,10 +292,12 @@ __global__ __launch_bounds__(kT) void lu_solve_regs_kernel(const double2 *Aall, 
             else if (pos[c] == i) pos[c] = pp;
         }
         if (wave == ((i + 1) & 15)) {
+            __builtin_amdgcn_s_setprio(3);                   // the chain the others wait for
             double2 v[ROWS];
             column(i + 1, v);
             eliminate(v, l, of_row(v, pr), i);               // a copy: the loop below does the column itself
             if (i + 1 < P - 1) factor(i + 1, v);
+            __builtin_amdgcn_s_setprio(0);
         }
 #pragma unroll
         for (int s = 0; s < COLS; s++) {
@@ -854,14 +856,15 @@ __global__ __launch_bounds__(kT) void pcg_f64_kernel(const double *Aall, const d
 // The eigenvalues a condition number needs -- the smallest, the largest and
 // the two next to zero -- of a Hermitian matrix (its upper triangle), without
 // eigenvectors: Householder reduction to a real tridiagonal, then
-// multisection on the Sturm counts, 256 points at a time for each of the four.
+// multisection on the Sturm counts, 128 points at a time for each of the four.
 //
-// One workgroup.  P <= 128: the matrix in registers, lane l of wave w holding rows w + 16 s and
-// columns l + 64 c, so a row's vectors are read from LDS once for two columns (and rows already reduced are
-// skipped by the whole wave); beyond, thread t owns column t % n and rows t / n (mod nseg) in W
-// (global, in L2).  A step of the reduction applies the previous step's rank-2 update and forms the
-// next matrix-vector product in one pass over the owned entries, with three
-// barriers.  What bounds it: the latency of those steps.
+// One workgroup.  P <= 128: the matrix in registers (below); beyond, thread t owns column t % n
+// and rows t / n (mod nseg) in W (global, in L2).  A step of the reduction applies the previous
+// step's rank-2 update and forms the next matrix-vector product, with three
+// barriers.  What bounds it: the latency of those steps.  P = 96: 335 us; 412 with rows split over
+// waves (their vectors broadcast from LDS row by row), 667 with the threads' columns crossing the waves, and
+// 29.5 ms by the cyclic Jacobi iteration, which still gives the eigenvectors elsewhere (8 to 10
+// sweeps of P - 1 steps, each two passes over A and one over V in global memory).
 // Indices whose row is zero off the diagonal are set aside first: their
 // diagonal entries are exact eigenvalues (a parameter without effect leaves a
 // zero row, and its exact zero is no part of the condition number).
@@ -871,8 +874,8 @@ __device__ __forceinline__ int sturm_count(const double *d, const double *e2, in
     double q = 1.0, prev = 0.0;
     for (int i = 0; i < n; i++) {
         double r = __builtin_amdgcn_rcp(q);
-        r = fma(r, fma(-q, r, 1.0), r);
-        r = fma(r, fma(-q, r, 1.0), r);
+        const double e = fma(-q, r, 1.0);                    // |e| < 2^-23: third order leaves 2^-69
+        r = fma(r, fma(e, e, e), r);
         q = (d[i] - x) - prev * r;
         if (fabs(q) < pivmin) q = -pivmin;
         c += q < 0.0;
@@ -897,21 +900,23 @@ __device__ __forceinline__ void tridiagonal_extremes(const double *sd, const dou
     for (int w = 0; w < kT / 64; w++) bd = fmax(bd, swv[w][0]);
     // eigenvalues within 1e-30 of the bound of zero are exact zeros: rounding is at 1e-16 of it
     const double B = bd * (1.0 + 1e-10), tiny = 1e-30 * bd, pivmin = 1e-40 * bd;
-    const int grp = t >> 8, m = t & 255;
-    const int cz = bd > 0.0 ? sturm_count(sd, se2, n, (t & 1) ? tiny : -tiny, pivmin) : 0;
+    // 128 points for each of the four, by the first eight waves: two waves a SIMD, whose issue then keeps
+    // pace with the recurrence's latency (n = 96: the kernel takes 335 us; with all sixteen, 256 points and 9 rounds, 359)
+    const int grp = t >> 7, m = t & 127;
+    const int cz = bd > 0.0 && grp < 4 ? sturm_count(sd, se2, n, (t & 1) ? tiny : -tiny, pivmin) : 0;
     const int n_neg = __shfl(cz, 0, 64), n_pos = __shfl(cz, 1, 64);   // below -tiny, below +tiny
     const int idx = grp == 0 ? 0 : grp == 1 ? n - 1 : grp == 2 ? n_pos : n_neg - 1;
-    const bool want = bd > 0.0 && idx >= 0 && idx < n;
+    const bool want = bd > 0.0 && grp < 4 && idx >= 0 && idx < n;
     double lo = grp == 2 ? 0.0 : -B, hi = grp == 3 ? 0.0 : B;
-    for (int round = 0; round < 9; round++) {
-        const double h = (hi - lo) * (1.0 / 257.0);
+    for (int round = 0; round < 11; round++) {
+        const double h = (hi - lo) * (1.0 / 129.0);
         int c = 0;
         if (want) c = sturm_count(sd, se2, n, lo + h * (m + 1), pivmin) <= idx;
         const int below = __popcll(__ballot(c != 0));
         if (lane == 0) cnt[wave] = below;
         __syncthreads();
-        const int k = cnt[4 * grp] + cnt[4 * grp + 1] + cnt[4 * grp + 2] + cnt[4 * grp + 3];
-        const double nl = k == 0 ? lo : lo + h * k, nh = k == 256 ? hi : lo + h * (k + 1);
+        const int k = cnt[2 * grp] + cnt[2 * grp + 1];       // (grp < 8: within cnt)
+        const double nl = k == 0 ? lo : lo + h * k, nh = k == 128 ? hi : lo + h * (k + 1);
         lo = nl;
         hi = nh;
         __syncthreads();
@@ -1079,40 +1084,42 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
     write_extremes(lo_all, hi_all, pos_all, neg_all, swv, out);
 }
 
-// The same for P <= 16 ROWS = 64 COLS with the matrix in registers.
-template <int ROWS, int COLS>
+// The same for P <= 16 COLS = 64 ROWS with the matrix in registers: wave w holds columns w + 16 s,
+// its lane l rows l + 64 c.  A step: the wave of column k brings it up to date and forms the
+// Householder vector by itself while the others apply the previous step's rank-2 update; then
+// every wave adds its columns to p = A u, and two waves add up the sixteen parts.
+template <int COLS, int ROWS>
 __global__ __launch_bounds__(kT) void herm_extremes_regs_kernel(const double2 *__restrict__ A, int P, double *out) {
-    constexpr int N = 64 * COLS;
-    static_assert(16 * ROWS == N, "square");
-    __shared__ double2 su[N], sq[N], sx[N], part[16][N];
-    __shared__ double sd[N], se2[N], swv[kT / 64][4], sup[kT / 64];
+    constexpr int N = 64 * ROWS;
+    static_assert(16 * COLS == N, "square");
+    __shared__ double2 su[N], sq[N], part[16][N];
+    __shared__ double sd[N], se2[N], swv[kT / 64][4], sup[kT / 64], stau;
     __shared__ int map[N], live[N], cnt[kT / 64];
     const int t = threadIdx.x, lane = t & 63, wave = qgtl::uniform(t >> 6);
-    auto entry = [&](int oi, int oj) -> double2 {            // the upper triangle's
+    auto entry = [&](int oi, int oj) __attribute__((always_inline)) -> double2 {   // the upper triangle's
         if (oi <= oj) { double2 v = A[(size_t)oi * P + oj]; if (oi == oj) v.y = 0.0; return v; }
         const double2 v = A[(size_t)oj * P + oi];
         return make_double2(v.x, -v.y);
     };
-    double2 a[ROWS][COLS];
+    double2 a[COLS][ROWS];
 #pragma unroll
-    for (int s = 0; s < ROWS; s++) {
-        const int i = wave + 16 * s;
+    for (int s = 0; s < COLS; s++) {
+        const int j = wave + 16 * s;
         bool any = false;
 #pragma unroll
-        for (int c = 0; c < COLS; c++) {
-            const int j = lane + 64 * c;
+        for (int c = 0; c < ROWS; c++) {
+            const int i = lane + 64 * c;
             a[s][c] = (i < P && j < P) ? entry(i, j) : make_double2(0.0, 0.0);
             any = any || (i != j && (a[s][c].x != 0.0 || a[s][c].y != 0.0));
         }
-        const bool row = __ballot(any) != 0;
-        if (lane == 0) live[i] = row;
+        const bool col = __ballot(any) != 0;
+        if (lane == 0) live[j] = col;
     }
-    if (t < N) su[t] = sq[t] = make_double2(0.0, 0.0);
     __syncthreads();
     // live indices in order, counted by every wave
     int n = 0;
 #pragma unroll
-    for (int c = 0; c < COLS; c++) {
+    for (int c = 0; c < ROWS; c++) {
         const bool l = live[lane + 64 * c] != 0;
         const unsigned long long b = __ballot(l);
         if (wave == 0 && l) map[n + __popcll(b & ((1ull << lane) - 1ull))] = lane + 64 * c;
@@ -1122,101 +1129,124 @@ __global__ __launch_bounds__(kT) void herm_extremes_regs_kernel(const double2 *_
     __syncthreads();
     if (n < P && n > 0) {                                    // close up the isolated indices
 #pragma unroll
-        for (int s = 0; s < ROWS; s++)
+        for (int s = 0; s < COLS; s++)
 #pragma unroll
-            for (int c = 0; c < COLS; c++) {
-                const int i = wave + 16 * s, j = lane + 64 * c;
+            for (int c = 0; c < ROWS; c++) {
+                const int i = lane + 64 * c, j = wave + 16 * s;
                 a[s][c] = (i < n && j < n) ? entry(map[i], map[j]) : make_double2(0.0, 0.0);
             }
     }
+    double2 u[ROWS], q[ROWS];                                // the pending update, this lane's rows
+#pragma unroll
+    for (int c = 0; c < ROWS; c++) u[c] = q[c] = make_double2(0.0, 0.0);
+    auto lane_of = [](double2 v, int l) __attribute__((always_inline)) -> double2 {
+        return make_double2(readlane_f64(v.x, l), readlane_f64(v.y, l));
+    };
+    auto at = [&](const double2 (&v)[ROWS], int i) __attribute__((always_inline)) -> double2 {   // row i
+        const bool up = ROWS > 1 && i >= 64;
+        return lane_of(make_double2(up ? v[ROWS - 1].x : v[0].x, up ? v[ROWS - 1].y : v[0].y), i & 63);
+    };
+    // v - u_i conj(q_j) - q_i conj(u_j)
+    auto pend = [&](double2 v, double2 ui, double2 qi, double2 uj, double2 qj) __attribute__((always_inline)) -> double2 {
+        v.x = fma(-ui.x, qj.x, fma(-ui.y, qj.y, fma(-qi.x, uj.x, fma(-qi.y, uj.y, v.x))));
+        v.y = fma(-ui.y, qj.x, fma(ui.x, qj.y, fma(-qi.y, uj.x, fma(qi.x, uj.y, v.y))));
+        return v;
+    };
     for (int k = 0; k < n; k++) {
-        double2 uj[COLS], qj[COLS];
+        if (wave == (k & 15)) {
+            __builtin_amdgcn_s_setprio(3);                   // the chain the others wait for
+            const double2 uk = at(u, k), qk = at(q, k);
+            double2 v[ROWS];
+            double tail = 0.0;
 #pragma unroll
-        for (int c = 0; c < COLS; c++) { uj[c] = su[lane + 64 * c]; qj[c] = sq[lane + 64 * c]; }
-        // v - u_i conj(q_j) - q_i conj(u_j)
-        auto pend = [&](double2 v, double2 ui, double2 qi, int c) -> double2 {
-            v.x -= ui.x * qj[c].x + ui.y * qj[c].y + qi.x * uj[c].x + qi.y * uj[c].y;
-            v.y -= ui.y * qj[c].x - ui.x * qj[c].y + qi.y * uj[c].x - qi.x * uj[c].y;
-            return v;
-        };
-        if (wave == (k & 15)) {                              // column k from row k
-            const double2 uk = su[k], qk = sq[k];
+            for (int c = 0; c < ROWS; c++) {
+                v[c] = a[0][c];
 #pragma unroll
-            for (int s = 0; s < ROWS; s++)
-                if (s == k >> 4)
+                for (int s = 1; s < COLS; s++) {
+                    const bool here = s == k >> 4;
+                    v[c].x = here ? a[s][c].x : v[c].x;
+                    v[c].y = here ? a[s][c].y : v[c].y;
+                }
+                v[c] = pend(v[c], u[c], q[c], uk, qk);
+                const int i = lane + 64 * c;
+                if (i > k + 1 && i < n) tail += v[c].x * v[c].x + v[c].y * v[c].y;
+            }
+            const double dk = at(v, k).x;
+            if (lane == 0) sd[k] = dk;
+            if (k < n - 1) {
+                tail = wave_sum_f64(tail);
+                double2 u0 = at(v, k + 1);
+                double e2;
+                const double tau = householder(tail, u0, e2);
+                if (lane == 0) { se2[k] = e2; stau = tau; }
 #pragma unroll
-                    for (int c = 0; c < COLS; c++) {
-                        const double2 v = pend(a[s][c], uk, qk, c);
-                        sx[lane + 64 * c] = make_double2(v.x, -v.y);
-                    }
+                for (int c = 0; c < ROWS; c++) {
+                    const int i = lane + 64 * c;
+                    double2 w = i == k + 1 ? u0 : v[c];
+                    if (i <= k || i >= n || !(tau > 0.0)) w = make_double2(0.0, 0.0);
+                    su[i] = w;
+                }
+            }
+            __builtin_amdgcn_s_setprio(0);
+        }
+        if (k == n - 1) break;
+#pragma unroll
+        for (int s = 0; s < COLS; s++) {
+            const int j = wave + 16 * s;
+            if (j > k && j < n) {                            // the same for the wave
+                const double2 uj = lane_of(u[s >> 2], j & 63), qj = lane_of(q[s >> 2], j & 63);
+#pragma unroll
+                for (int c = 0; c < ROWS; c++) a[s][c] = pend(a[s][c], u[c], q[c], uj, qj);
+            }
         }
         __syncthreads();
-        if (t == 0) sd[k] = sx[k].x;
-        if (k == n - 1) break;
-        double2 xj[COLS];
-        double tail = 0.0;
+        const double tau = stau;
+        double2 p[ROWS];
 #pragma unroll
-        for (int c = 0; c < COLS; c++) {
-            const int j = lane + 64 * c;
-            xj[c] = sx[j];
-            if (j > k + 1 && j < n) tail += xj[c].x * xj[c].x + xj[c].y * xj[c].y;
-        }
-        tail = wave_sum_f64(tail);
-        double2 u0 = sx[k + 1];
-        double e2;
-        const double tau = householder(tail, u0, e2);
-        if (t == 0) se2[k] = e2;
-        double2 p[COLS];
-#pragma unroll
-        for (int c = 0; c < COLS; c++) {
+        for (int c = 0; c < ROWS; c++) {
+            u[c] = su[lane + 64 * c];
             p[c] = make_double2(0.0, 0.0);
-            if (lane + 64 * c == k + 1) xj[c] = u0;
         }
 #pragma unroll
-        for (int s = 0; s < ROWS; s++) {
-            const int i = wave + 16 * s;
-            if (i > k && i < n) {                            // the same for the wave
-                const double2 ui = su[i], qi = sq[i], vi = i == k + 1 ? u0 : sx[i];
+        for (int s = 0; s < COLS; s++) {
+            const int j = wave + 16 * s;
+            if (j > k && j < n) {
+                const double2 uj = lane_of(u[s >> 2], j & 63);
 #pragma unroll
-                for (int c = 0; c < COLS; c++) {
-                    if (64 * c + 63 <= k) continue;
-                    const double2 v = pend(a[s][c], ui, qi, c);
-                    a[s][c] = v;
-                    p[c].x += v.x * vi.x + v.y * vi.y;       // conj(a_ij) u_i
-                    p[c].y += v.x * vi.y - v.y * vi.x;
+                for (int c = 0; c < ROWS; c++) {
+                    const double2 v = a[s][c];
+                    p[c].x = fma(v.x, uj.x, fma(-v.y, uj.y, p[c].x));
+                    p[c].y = fma(v.x, uj.y, fma(v.y, uj.x, p[c].y));
                 }
             }
         }
         // p = tau A u; K = tau / 2 u^H p; q = p - K u
         double up = 0.0;
 #pragma unroll
-        for (int c = 0; c < COLS; c++) {
-            const int j = lane + 64 * c;
-            part[wave][j] = p[c];
-            if (j > k && j < n) up += xj[c].x * p[c].x + xj[c].y * p[c].y;
+        for (int c = 0; c < ROWS; c++) {
+            part[wave][lane + 64 * c] = p[c];
+            up += u[c].x * p[c].x + u[c].y * p[c].y;         // u is zero outside k + 1 .. n - 1
         }
         up = wave_sum_f64(up);
         if (lane == 0) sup[wave] = up;
         __syncthreads();
-        if (wave < COLS) {
+        if (wave < ROWS) {
             double2 s = part[0][t];
             up = sup[0];
-#pragma unroll 3
+#pragma unroll 5
             for (int w = 1; w < 16; w++) {
                 s.x += part[w][t].x;
                 s.y += part[w][t].y;
                 up += sup[w];
             }
-            double2 ut = make_double2(0.0, 0.0), qt = make_double2(0.0, 0.0);
-            if (t > k && t < n && tau > 0.0) {
-                ut = t == k + 1 ? u0 : sx[t];
-                const double kk = 0.5 * tau * tau * up;
-                qt = make_double2(tau * s.x - kk * ut.x, tau * s.y - kk * ut.y);
-            }
-            su[t] = ut;
-            sq[t] = qt;
+            const double2 ut = su[t];
+            const double kk = 0.5 * tau * tau * up;
+            const bool in = t > k && t < n;
+            sq[t] = make_double2(in ? tau * s.x - kk * ut.x : 0.0, in ? tau * s.y - kk * ut.y : 0.0);
         }
         __syncthreads();
+#pragma unroll
+        for (int c = 0; c < ROWS; c++) q[c] = sq[lane + 64 * c];
     }
     __syncthreads();
     const double inf = __builtin_inf();
