@@ -421,11 +421,12 @@ int qgtl_hip_gram_tiles(int P);                                          /* uppe
  * rows (Re d_s, Im d_s) */
 int qgtl_hip_gram_bf16x3(const void *D, int P, size_t N, float *partials, int nchunks, int terms);
 int qgtl_hip_gram_reduce(const float *partials, int P, int nchunks, double *C);   /* C: R x R tiles, FP64 */
-/* Q = normalised G - a a^H from C and injection sums (P x 4 doubles). */
-int qgtl_hip_qgt_finalize(const double *C, const double *inj, int P, double *Q);
+/* Q = normalised G - a a^H from C and injection sums (P x 4 doubles); host: a
+ * pinned host copy written along, or NULL. */
+int qgtl_hip_qgt_finalize(const double *C, const double *inj, int P, double *Q, double *host);
 /* the same with the overlaps taken from the Gram: C is the Gram of P + 1 states,
  * state P the primal state at the derivative states' meeting point */
-int qgtl_hip_qgt_finalize_psi(const double *C, int P, double *Q);
+int qgtl_hip_qgt_finalize_psi(const double *C, int P, double *Q, double *host);
 /* one complex64 state of 2^n amplitudes (n >= 6) in split-plane form */
 int qgtl_hip_c64_to_split(const void *src, void *dst, int n);
 
@@ -443,7 +444,7 @@ int qgtl_hip_gram_cplx(const void *D, int P, size_t N, float *partials, int nchu
 int qgtl_hip_gram_cplx_reduce(const float *partials, int P, int nchunks, double *G);
 /* Q = normalised G - a a^H from the complex Gram of P + 1 states (state P the
  * primal state at the derivative states' meeting point, so a_k = G_kP) */
-int qgtl_hip_qgt_finalize_cplx(const double *G, int P, double *Q);
+int qgtl_hip_qgt_finalize_cplx(const double *G, int P, double *Q, double *host);
 /* MFMA lane-layout probe (diagnostics): 32 x 32 floats to out_dev */
 int qgtl_hip_debug_mfma_layout(float *out_dev);
 int qgtl_hip_debug_mfma16_layout(float *out_dev);   /* v_mfma_f32_16x16x32_f16 probe, 16 x 16 floats */

@@ -362,10 +362,9 @@ __global__ __launch_bounds__(kThreads) void gram_reduce_grouped_kernel(const qgt
 // ||psi|| = 1 to remove the norm drift of the complex64 sweeps.
 __device__ __forceinline__ void qgt_finalize_elem(const double *__restrict__ C, int R,
                                                   const double *__restrict__ inj, int P,
-                                                  double *__restrict__ Q, size_t idx) {
+                                                  double *__restrict__ Q, double *__restrict__ host, size_t idx) {
     {
-        const int k = (int)(idx / P), l = (int)(idx % P);
-        if (k > l) return;
+        const int r = (int)(idx / P), c = (int)(idx % P), k = min(r, c), l = max(r, c);
         const double gre = C[(size_t)(2 * k) * R + 2 * l] + C[(size_t)(2 * k + 1) * R + 2 * l + 1];
         const double gim = C[(size_t)(2 * k) * R + 2 * l + 1] - C[(size_t)(2 * k + 1) * R + 2 * l];
         const double gkk = C[(size_t)(2 * k) * R + 2 * k] + C[(size_t)(2 * k + 1) * R + 2 * k + 1];
@@ -378,12 +377,7 @@ __device__ __forceinline__ void qgt_finalize_elem(const double *__restrict__ C, 
         // a_k conj(a_l)
         const double pr = akr * alr + aki * ali, pi = aki * alr - akr * ali;
         const double qr = gre * sg - pr, qi = (k == l) ? 0.0 : gim * sg - pi;
-        Q[2 * ((size_t)k * P + l)] = qr;
-        Q[2 * ((size_t)k * P + l) + 1] = qi;
-        if (k != l) {
-            Q[2 * ((size_t)l * P + k)] = qr;
-            Q[2 * ((size_t)l * P + k) + 1] = -qi;
-        }
+        qgtl::store_q(Q, host, idx, qr, r <= c ? qi : -qi);
     }
 }
 
@@ -391,9 +385,8 @@ __device__ __forceinline__ void qgt_finalize_elem(const double *__restrict__ C, 
 // states' meeting point is Gram state P (Z rows 2P, 2P+1), so
 // <d_k|psi> = G_kP, |d_k|^2 = G_kk and |psi|^2 = G_PP.
 __device__ __forceinline__ void qgt_finalize_psi_elem(const double *__restrict__ C, int R, int P,
-                                                      double *__restrict__ Q, size_t idx) {
-    const int k = (int)(idx / P), l = (int)(idx % P);
-    if (k > l) return;
+                                                      double *__restrict__ Q, double *__restrict__ host, size_t idx) {
+    const int r = (int)(idx / P), c = (int)(idx % P), k = min(r, c), l = max(r, c);
     const int m = P;   // the primal state
     const double gre = C[(size_t)(2 * k) * R + 2 * l] + C[(size_t)(2 * k + 1) * R + 2 * l + 1];
     const double gim = C[(size_t)(2 * k) * R + 2 * l + 1] - C[(size_t)(2 * k + 1) * R + 2 * l];
@@ -409,27 +402,23 @@ __device__ __forceinline__ void qgt_finalize_psi_elem(const double *__restrict__
     const double akr = akr0 * sk, aki = aki0 * sk, alr = alr0 * sl, ali = ali0 * sl;
     const double pr = akr * alr + aki * ali, pi = aki * alr - akr * ali;
     const double qr = gre * sg - pr, qi = (k == l) ? 0.0 : gim * sg - pi;
-    Q[2 * ((size_t)k * P + l)] = qr;
-    Q[2 * ((size_t)k * P + l) + 1] = qi;
-    if (k != l) {
-        Q[2 * ((size_t)l * P + k)] = qr;
-        Q[2 * ((size_t)l * P + k) + 1] = -qi;
-    }
+    qgtl::store_q(Q, host, idx, qr, r <= c ? qi : -qi);
 }
 
 __global__ __launch_bounds__(kThreads) void qgt_finalize_psi_kernel(const double *__restrict__ C, int R, int P,
-                                                                    double *__restrict__ Q) {
+                                                                    double *__restrict__ Q,
+                                                                    double *__restrict__ host) {
     for (size_t idx = blockIdx.x * (size_t)kThreads + threadIdx.x; idx < (size_t)P * P;
          idx += (size_t)gridDim.x * kThreads)
-        qgt_finalize_psi_elem(C, R, P, Q, idx);
+        qgt_finalize_psi_elem(C, R, P, Q, host, idx);
 }
 
 __global__ __launch_bounds__(kThreads) void qgt_finalize_kernel(const double *__restrict__ C, int R,
                                                                 const double *__restrict__ inj, int P,
-                                                                double *__restrict__ Q) {
+                                                                double *__restrict__ Q, double *__restrict__ host) {
     for (size_t idx = blockIdx.x * (size_t)kThreads + threadIdx.x; idx < (size_t)P * P;
          idx += (size_t)gridDim.x * kThreads)
-        qgt_finalize_elem(C, R, inj, P, Q, idx);
+        qgt_finalize_elem(C, R, inj, P, Q, host, idx);
 }
 
 __global__ __launch_bounds__(kThreads) void finalize_grouped_kernel(const qgtl_finalize_item_t *__restrict__ items,
@@ -440,10 +429,10 @@ __global__ __launch_bounds__(kThreads) void finalize_grouped_kernel(const qgtl_f
         if (idx >= (size_t)it.P * it.P) continue;
         if (it.inj)             // overlaps and norms from FP64 injection sums
             qgt_finalize_elem(reinterpret_cast<const double *>(it.C), it.R, reinterpret_cast<const double *>(it.inj),
-                              it.P, reinterpret_cast<double *>(it.Q), idx);
+                              it.P, reinterpret_cast<double *>(it.Q), nullptr, idx);
         else                    // ... from the Gram row of the primal state (state P)
             qgt_finalize_psi_elem(reinterpret_cast<const double *>(it.C), it.R, it.P, reinterpret_cast<double *>(it.Q),
-                                  idx);
+                                  nullptr, idx);
     }
 }
 
@@ -512,22 +501,22 @@ int qgtl_hip_gram_reduce(const float *partials, int P, int nchunks, double *C) {
     return 0;
 }
 
-int qgtl_hip_qgt_finalize_psi(const double *C, int P, double *Q) {
+int qgtl_hip_qgt_finalize_psi(const double *C, int P, double *Q, double *host) {
     const int nt = (2 * (P + 1) + kTile - 1) / kTile;
     const size_t work = (size_t)P * P;
     unsigned grid = (unsigned)((work + kThreads - 1) / kThreads);
     if (grid > 4096) grid = 4096;
-    hipLaunchKernelGGL(qgt_finalize_psi_kernel, dim3(grid), dim3(kThreads), 0, qgtl::stream(), C, nt * kTile, P, Q);
+    hipLaunchKernelGGL(qgt_finalize_psi_kernel, dim3(grid), dim3(kThreads), 0, qgtl::stream(), C, nt * kTile, P, Q, host);
     QGTL_LAUNCH_CHECK("qgt_finalize_psi");
     return 0;
 }
 
-int qgtl_hip_qgt_finalize(const double *C, const double *inj, int P, double *Q) {
+int qgtl_hip_qgt_finalize(const double *C, const double *inj, int P, double *Q, double *host) {
     const int nt = (2 * P + kTile - 1) / kTile;
     const size_t work = (size_t)P * P;
     unsigned grid = (unsigned)((work + kThreads - 1) / kThreads);
     if (grid > 4096) grid = 4096;
-    hipLaunchKernelGGL(qgt_finalize_kernel, dim3(grid), dim3(kThreads), 0, qgtl::stream(), C, nt * kTile, inj, P, Q);
+    hipLaunchKernelGGL(qgt_finalize_kernel, dim3(grid), dim3(kThreads), 0, qgtl::stream(), C, nt * kTile, inj, P, Q, host);
     QGTL_LAUNCH_CHECK("qgt_finalize");
     return 0;
 }

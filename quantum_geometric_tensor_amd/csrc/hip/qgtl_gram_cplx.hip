@@ -718,9 +718,8 @@ __global__ __launch_bounds__(kThreads) void gram_cplx_reduce_grouped_kernel(
 // state P is the primal state, and the normalisation applies the exact
 // identities ||d_k psi|| = 1/2 and ||psi|| = 1 (the 2^30 scale of G cancels).
 __device__ __forceinline__ void qgt_finalize_cplx_elem(const double2 *__restrict__ G, int R, int P,
-                                                       double *__restrict__ Q, size_t idx) {
-    const int k = (int)(idx / P), l = (int)(idx % P);
-    if (k > l) return;
+                                                       double *__restrict__ Q, double *__restrict__ host, size_t idx) {
+    const int r = (int)(idx / P), c = (int)(idx % P), k = min(r, c), l = max(r, c);
     const int m = P;
     const double2 g = G[(size_t)k * R + l];
     const double gkk = G[(size_t)k * R + k].x, gll = G[(size_t)l * R + l].x, gmm = G[(size_t)m * R + m].x;
@@ -730,19 +729,14 @@ __device__ __forceinline__ void qgt_finalize_cplx_elem(const double2 *__restrict
     const double akr = ak0.x * sk, aki = ak0.y * sk, alr = al0.x * sl, ali = al0.y * sl;
     const double pr = akr * alr + aki * ali, pi = aki * alr - akr * ali;
     const double qr = g.x * sg - pr, qi = (k == l) ? 0.0 : g.y * sg - pi;
-    Q[2 * ((size_t)k * P + l)] = qr;
-    Q[2 * ((size_t)k * P + l) + 1] = qi;
-    if (k != l) {
-        Q[2 * ((size_t)l * P + k)] = qr;
-        Q[2 * ((size_t)l * P + k) + 1] = -qi;
-    }
+    qgtl::store_q(Q, host, idx, qr, r <= c ? qi : -qi);
 }
 
 __global__ __launch_bounds__(kThreads) void qgt_finalize_cplx_kernel(const double2 *__restrict__ G, int R, int P,
-                                                                     double *__restrict__ Q) {
+                                                                     double *__restrict__ Q, double *__restrict__ host) {
     for (size_t idx = blockIdx.x * (size_t)kThreads + threadIdx.x; idx < (size_t)P * P;
          idx += (size_t)gridDim.x * kThreads)
-        qgt_finalize_cplx_elem(G, R, P, Q, idx);
+        qgt_finalize_cplx_elem(G, R, P, Q, host, idx);
 }
 
 // grouped: unit = kThreads entries of an item's P x P (units per item: ceil(P^2 / kThreads))
@@ -753,7 +747,7 @@ __global__ __launch_bounds__(kThreads) void finalize_cplx_grouped_kernel(const q
         const size_t idx = (size_t)(u - it.unit_begin) * kThreads + threadIdx.x;
         if (idx < (size_t)it.P * it.P)
             qgt_finalize_cplx_elem(reinterpret_cast<const double2 *>(it.C), it.R, it.P, reinterpret_cast<double *>(it.Q),
-                                   idx);
+                                   nullptr, idx);
     }
 }
 
@@ -852,12 +846,12 @@ int qgtl_hip_debug_mfma16_layout(float *out_dev) {
     return 0;
 }
 
-int qgtl_hip_qgt_finalize_cplx(const double *G, int P, double *Q) {
+int qgtl_hip_qgt_finalize_cplx(const double *G, int P, double *Q, double *host) {
     const int nt = (P + 1 + kTileStates - 1) / kTileStates;
     unsigned grid = (unsigned)(((size_t)P * P + kThreads - 1) / kThreads);
     if (grid > 4096) grid = 4096;
     hipLaunchKernelGGL(qgt_finalize_cplx_kernel, dim3(grid), dim3(kThreads), 0, qgtl::stream(),
-                       reinterpret_cast<const double2 *>(G), nt * kTileStates, P, Q);
+                       reinterpret_cast<const double2 *>(G), nt * kTileStates, P, Q, host);
     QGTL_LAUNCH_CHECK("qgt_finalize_cplx");
     return 0;
 }

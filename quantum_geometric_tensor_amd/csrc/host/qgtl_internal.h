@@ -106,6 +106,8 @@ struct qgtl_plan {
     double *C;                           /* mixed: R x R;  plain: G (P x P complex) */
     double *Qdev;                        /* P x P complex */
     double *Qhost;                       /* pinned host copy of Qdev (download staging) */
+    double *q_to_host;                   /* Qhost when this execute's last kernel writes it, else NULL */
+    int graph_writes;                    /* the captured launches write Qhost */
     double *plain_partials;
     size_t plain_partials_len;
     uint64_t structure_hash;
