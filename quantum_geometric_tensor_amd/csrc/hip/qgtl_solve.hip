@@ -8,8 +8,9 @@
 //    compute_regularized_natural_gradient relies on
 //    (src/quantum_geometric/core/quantum_geometric_gradient.c:2887-2964).
 //  - herm_eig_c128: parallel cyclic Jacobi (round-robin pairs) for Hermitian
-//    matrices: eigenvalues ascending and eigenvectors, for the condition
-//    number and the pseudo-inverse fallback (:2733-2884).
+//    matrices: eigenvalues ascending and eigenvectors, for the pseudo-inverse
+//    fallback (:2733-2884).
+//  - herm_extremes_c128: the eigenvalues a condition number needs, without vectors.
 //  - cholesky_f64: (A + lambda I) x = b for real SPD A, the exact yardstick.
 //  - pcg_f64: preconditioned CG from x0 = 0 to ||r||/||b|| <= tol with
 //    M^-1 = diag(d) + U U^T (U = 0 gives Jacobi-PCG with d = 1/diag(A)),

@@ -5,9 +5,10 @@
  *   for each block b: apply b to the primal; create the derivative states of
  *   b's parameters from the block output (inject); carry them through the
  *   later blocks; then G = D^H D on MFMA and Q = normalised G - a a^H in FP64.
- *   When every pass is in place (states of <= 2^13 amplitudes) the derivative
- *   states advance breadth-first, one launch per pass for all of them; wider
- *   states advance depth-first in balanced chunks of up to 1 GB (a chunk's states
+ *   States of 2^4 .. 2^13 amplitudes run in one launch, every state in LDS from
+ *   start to end.  Otherwise, when every pass is in place, the derivative
+ *   states advance breadth-first, one launch per pass for all of them; else
+ *   they advance depth-first in balanced chunks of up to 1 GB (a chunk's states
  *   move together through the later blocks, so launches stay large while
  *   the ping-pong copy of a chunk is all the extra memory needed).
  * Plain FP64 mode: one complex128 kernel per gate, derivative states one at a
