@@ -16,13 +16,13 @@
 // layers at n = 13), so the call takes one circuit's latency instead of 2 L
 // dependent launches.  Kernel time of one call, before (passes, injections and
 // their reductions) and now: n = 13, L = 6 (P = 156) 579 -> 44 us; n = 10,
-// L = 4 (P = 80) 99 -> 20 us; n = 6, L = 3 (P = 36) 50 -> 12 us; the whole
-// Plan.set_angles + execute 701 -> 130, 184 -> 78 and 126 -> 59 us.
+// L = 4 (P = 80) 99 -> 18 us; n = 6, L = 3 (P = 36) 50 -> 11 us; the whole
+// Plan.set_angles + execute 701 -> 117, 184 -> 65 and 126 -> 45 us (with what else changed around it).
 //
 // Work split: 16 amplitudes per thread (four tile bits in registers, 2^(n-4)
 // threads), so a block is ceil(n / 4) LDS round trips of four gates each.
 // Below n = 10 one wave holds 2^(10-n) states.  What bounds it: the latency of
-// one wave's dependent steps (descriptor loads, LDS round trips) at n <= 10,
+// one wave's dependent steps (LDS round trips) at n <= 10,
 // LDS traffic (2 x 64 KB per round trip) and the gates' multiply-adds at n = 13.
 //
 // QGTL counterpart: the shifted-circuit evaluations of
@@ -47,6 +47,11 @@ __device__ __forceinline__ float2 cmadd(float2 acc, float2 a, float2 b) {
     acc.y = fmaf(a.x, b.y, acc.y);
     acc.y = fmaf(a.y, b.x, acc.y);
     return acc;
+}
+
+// a value every lane holds, as a scalar
+__device__ __forceinline__ float uni(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }
 
 // z with the sign (-1)^n
@@ -110,18 +115,18 @@ __device__ __forceinline__ void groups(const qgtl_res_block_t &b, float2 *tile, 
         float2 v[16];
 #pragma unroll
         for (int r = 0; r < 16; r++) v[r] = tile[l0 ^ rpad((uint32_t)r << B)];
-        if (G == 0 && b.has_pre) {
+        if (G == 0 && qgtl::uniform(b.has_pre)) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) v[r] = cmul(v[r], cmul(pre, make_float2(b.reg_pre[r].re, b.reg_pre[r].im)));
+            for (int r = 0; r < 16; r++) v[r] = cmul(v[r], cmul(pre, make_float2(uni(b.reg_pre[r].re), uni(b.reg_pre[r].im))));
         }
-        if constexpr (first <= 0) rotate<0>(v, b.tan[B], b.swapped[B]);
-        if constexpr (first <= 1) rotate<1>(v, b.tan[B + 1], b.swapped[B + 1]);
-        if constexpr (first <= 2) rotate<2>(v, b.tan[B + 2], b.swapped[B + 2]);
-        rotate<3>(v, b.tan[B + 3], b.swapped[B + 3]);
+        if constexpr (first <= 0) rotate<0>(v, uni(b.tan[B]), qgtl::uniform(b.swapped[B]));
+        if constexpr (first <= 1) rotate<1>(v, uni(b.tan[B + 1]), qgtl::uniform(b.swapped[B + 1]));
+        if constexpr (first <= 2) rotate<2>(v, uni(b.tan[B + 2]), qgtl::uniform(b.swapped[B + 2]));
+        rotate<3>(v, uni(b.tan[B + 3]), qgtl::uniform(b.swapped[B + 3]));
         if constexpr (G + 1 == S::kGroups) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) v[r] = cmul(v[r], cmul(post, make_float2(b.reg_post[r].re, b.reg_post[r].im)));
-            if (SIGN && b.has_sign) {
+            for (int r = 0; r < 16; r++) v[r] = cmul(v[r], cmul(post, make_float2(uni(b.reg_post[r].re), uni(b.reg_post[r].im))));
+            if (SIGN && qgtl::uniform(b.has_sign)) {
                 // (-1)^{q(j)}: q(j0 + r) = q(j0) + q(r) + the polar form of both
                 uint32_t acc = 0;
 #pragma unroll
@@ -133,12 +138,12 @@ __device__ __forceinline__ void groups(const qgtl_res_block_t &b, float2 *tile, 
 #pragma unroll
                 for (int r = 0; r < 16; r++) v[r] = flip_sign(v[r], neg >> r);
             }
-            if (b.has_perm) {
+            if (qgtl::uniform(b.has_perm)) {
                 // element j goes to pi(j), the XOR of the images of its bits
                 uint32_t p = j0 & ~((1u << NQ) - 1u);        // the state's number in the tile
 #pragma unroll
                 for (int i = 0; i < NQ; i++)
-                    if (i < B || i >= B + 4) p ^= (0u - ((j0 >> i) & 1u)) & b.img[i];
+                    if (i < B || i >= B + 4) p ^= (0u - ((j0 >> i) & 1u)) & qgtl::uniform(b.img[i]);
                 const uint32_t lp = rpad(p);
                 __syncthreads();
 #pragma unroll
@@ -146,7 +151,7 @@ __device__ __forceinline__ void groups(const qgtl_res_block_t &b, float2 *tile, 
                     uint32_t u = 0;
 #pragma unroll
                     for (int i = 0; i < 4; i++)
-                        if ((r >> i) & 1) u ^= b.img[B + i];
+                        if ((r >> i) & 1) u ^= qgtl::uniform(b.img[B + i]);
                     tile[lp ^ rpad(u)] = v[r];
                 }
                 __syncthreads();
@@ -172,7 +177,37 @@ __global__ __launch_bounds__(Shape<NQ>::kThreads) void resident_states_kernel(
     typedef Shape<NQ> S;
     __shared__ float2 tile[1 << S::kM];
     __shared__ double red[16][4];
+    // NQ < 13: the descriptors of this block and the next, fetched a block ahead (a wave alone on its
+    // SIMD waits several times a block for scalar loads: n = 10, L = 4 68 -> 65 us a call, n = 12, L = 6
+    // 105 -> 101; at n = 13, with two waves a SIMD and LDS the bound, 122 -> 124)
+    constexpr bool kAhead = NQ < 13;
+    __shared__ qgtl_res_block_t sb[2];
+    constexpr int kWords = sizeof(qgtl_res_block_t) / 4, kPer = (kWords + S::kThreads - 1) / S::kThreads;
     const uint32_t t = threadIdx.x;
+    uint32_t ahead[kPer];
+    auto fetch = [&](int bi) {
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const int w = (int)t + k * S::kThreads;
+            ahead[k] = (bi < nblocks && w < kWords) ? reinterpret_cast<const uint32_t *>(blocks + bi)[w] : 0u;
+        }
+    };
+    auto put = [&](int bi) {
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const int w = (int)t + k * S::kThreads;
+            if (w < kWords) reinterpret_cast<uint32_t *>(&sb[bi & 1])[w] = ahead[k];
+        }
+    };
+    if constexpr (kAhead) {
+        fetch(0);
+        put(0);
+        fetch(1);
+    }
+    auto block = [&](int bi) -> const qgtl_res_block_t & {
+        if constexpr (kAhead) return sb[bi & 1];
+        else return blocks[bi];
+    };
     const int s_first = (int)blockIdx.x * S::kStates;
     const uint32_t Nm = (1u << NQ) - 1u;
     // in the layout of group 0 (register bits 0..3) a thread's amplitudes are of one state
@@ -189,12 +224,16 @@ __global__ __launch_bounds__(Shape<NQ>::kThreads) void resident_states_kernel(
 
     const uint32_t yl = deposit<S::base(S::kGroups - 1)>(t) & Nm;   // register 0 of the last group
     for (int bi = 0; bi < nblocks; bi++) {
-        const qgtl_res_block_t &b = blocks[bi];
+        if constexpr (kAhead) {
+            put(bi + 1);                                      // block bi - 1's buffer; read after this block's barriers
+            fetch(bi + 2);
+        }
+        const qgtl_res_block_t &b = block(bi);
         const float2 *tb = tabs + (size_t)bi * QGTL_RES_TAB * 2;
         // thread parts of the phase layers (from the caches, ahead of their use)
         const float2 post = cmul(tb[yl & 127u], tb[128u + (yl >> 7)]);
         float2 pre = make_float2(1.f, 0.f);
-        if (b.has_pre) pre = cmul(tb[QGTL_RES_TAB + (y0 & 127u)], tb[QGTL_RES_TAB + 128u + (y0 >> 7)]);
+        if (qgtl::uniform(b.has_pre)) pre = cmul(tb[QGTL_RES_TAB + (y0 & 127u)], tb[QGTL_RES_TAB + 128u + (y0 >> 7)]);
         groups<NQ, 0, SIGN>(b, tile, t, pre, post);
         if (bi < blk_first || bi > blk_last) continue;        // uniform: slots are in block order
         // d[y] = M[s][s] psi[y] + (-1)^parity(y & z) M[s][1 - s] psi[y ^ v], s = parity(y & w)
