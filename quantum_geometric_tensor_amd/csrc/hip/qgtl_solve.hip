@@ -1071,7 +1071,7 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
                     double2 s = part[t];
                     for (int g = 1; g < nseg; g++) { s.x += part[g * n + t].x; s.y += part[g * n + t].y; }
                     ut = t == k + 1 ? u0 : sx[t];
-                    const double kk = 0.5 * tau * tau * up;
+                    const double kk = tau * (0.5 * tau * up);      // tau^2 alone overflows below 1e-77
                     qt = make_double2(tau * s.x - kk * ut.x, tau * s.y - kk * ut.y);
                 }
                 su[t] = ut;
@@ -1241,7 +1241,7 @@ __global__ __launch_bounds__(kT) void herm_extremes_regs_kernel(const double2 *_
                 up += sup[w];
             }
             const double2 ut = su[t];
-            const double kk = 0.5 * tau * tau * up;
+            const double kk = tau * (0.5 * tau * up);      // tau^2 alone overflows below 1e-77
             const bool in = t > k && t < n;
             sq[t] = make_double2(in ? tau * s.x - kk * ut.x : 0.0, in ? tau * s.y - kk * ut.y : 0.0);
         }

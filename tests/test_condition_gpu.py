@@ -64,3 +64,39 @@ def test_condition_number_zero_rows_and_diagonals():
     sv = np.abs(np.linalg.eigvalsh(B.astype(np.complex128)))
     assert abs(_kappa(M) - sv.max() / sv.min()) <= 1e-6 * sv.max() / sv.min()
     assert np.isinf(_kappa(np.ones((40, 40)))) or _kappa(np.ones((40, 40))) > 1e13   # rank one
+
+
+def _extremes(A):
+    """qgtl_hip_herm_extremes_c128 itself: smallest, largest, smallest positive, largest negative."""
+    L, vp = Q.lib(), ctypes.c_void_p
+    A = np.ascontiguousarray(A, np.complex128)
+    out = np.full(4, 7.0)
+    L.qgtl_hip_herm_extremes_c128.argtypes = [vp, vp, ctypes.c_int, vp]
+    for f in ("h2d", "d2h"):
+        getattr(L, "qgtl_hip_" + f).argtypes = [vp, vp, ctypes.c_size_t]
+    L.qgtl_hip_malloc.argtypes = [ctypes.POINTER(vp), ctypes.c_size_t]
+    L.qgtl_hip_free.argtypes = [vp]
+    Q.init()
+    d = [vp() for _ in range(3)]
+    for p, n in zip(d, (A.nbytes, A.nbytes, out.nbytes)):
+        assert L.qgtl_hip_malloc(ctypes.byref(p), n) == 0
+    assert L.qgtl_hip_h2d(d[0], A.ctypes.data, A.nbytes) == 0
+    assert L.qgtl_hip_herm_extremes_c128(d[0], d[1], len(A), d[2]) == 0
+    assert L.qgtl_hip_d2h(out.ctypes.data, d[2], out.nbytes) == 0 and L.qgtl_hip_sync() == 0
+    for p in d:
+        L.qgtl_hip_free(p)
+    return out
+
+
+@pytest.mark.parametrize("P", [6, 64, 100, 140])
+@pytest.mark.parametrize("scale", [1.0, 1e-62])
+def test_extremes_of_a_tiny_rank_deficient_matrix(P, scale):
+    """M^H M of entries near 1e-31, of rank 2: the columns left after two steps are rounding, 1e-78, whose
+    reflector's tau is near 1e156.  The bar is backward stability, P eps ||A|| (times 4)."""
+    rng = np.random.default_rng(P)
+    V = rng.normal(size=(P, 2)) + 1j * rng.normal(size=(P, 2))
+    A = V @ V.conj().T
+    ev = np.linalg.eigvalsh(A)
+    lo, hi = _extremes(A * scale)[:2] / scale
+    assert abs(hi - ev[-1]) <= 4 * P * np.finfo(float).eps * ev[-1]
+    assert abs(lo - ev[0]) <= 4 * P * np.finfo(float).eps * ev[-1]
