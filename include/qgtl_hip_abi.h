@@ -493,10 +493,17 @@ int qgtl_hip_kaporin(int P, int r, int B, const float *Y, const float *As_all, c
 /* ---- FP64 natural-gradient solves, one workgroup per system ---- */
 int qgtl_hip_lu_solve_c128(void *A, const void *b, void *x, int *piv, int P, int batch, int *status);
 int qgtl_hip_herm_eig_c128(void *A, void *V, double *ev, int P, int batch, int max_sweeps, int *sweeps);
-/* out4 (device): smallest, largest, smallest positive (+inf: none) and largest
- * negative (-inf: none) eigenvalue of the Hermitian A (upper triangle read);
- * W: P x P complex128 scratch */
-int qgtl_hip_herm_extremes_c128(const void *A, void *W, int P, double *out4);
+/* Extreme eigenvalues of each component of the Hermitian A (upper triangle read):
+ * comps (device): ncomps pairs (first index, order), components that no entry of A
+ * couples, each a range of adjacent indices, the largest of order `largest`; NULL:
+ * A is one.  out (device), six doubles a component: smallest, largest, smallest
+ * positive (+inf: none), largest negative (-inf: none); the smallest size of an
+ * eigenvalue other than the diagonal entries of indices that couple to none (+inf:
+ * none; 0: one is zero, or not to be told from it) and a bound B of those sizes
+ * (infinite when the entries overflow): an eigenvalue is uncertain by a few P eps B.
+ * W: P x P complex128 scratch. */
+int qgtl_hip_herm_extremes_c128(const void *A, void *W, int P, const int *comps, int ncomps, int largest,
+                                double *out);
 int qgtl_hip_cholesky_solve_f64(double *A, const double *b, double *x, int P, int batch, double lambda, int *status);
 int qgtl_hip_pcg_f64(const double *A, const double *b, double *x, int P, int batch, double lambda, const double *d,
                      const double *U, int r, double tol, int maxit, int *iters, double *relres);

@@ -859,7 +859,9 @@ __global__ __launch_bounds__(kT) void pcg_f64_kernel(const double *Aall, const d
 // eigenvectors: Householder reduction to a real tridiagonal, then
 // multisection on the Sturm counts, 128 points at a time for each of the four.
 //
-// One workgroup.  P <= 128: the matrix in registers (below); beyond, thread t owns column t % n
+// One workgroup per component (a set of indices that the matrix couples to no other, adjacent in A):
+// a small component beside a large one keeps its own accuracy and its own bounds.
+// P <= 128: the matrix in registers (below); beyond, thread t owns column t % n
 // and rows t / n (mod nseg) in W (global, in L2).  A step of the reduction applies the previous
 // step's rank-2 update and forms the next matrix-vector product, with three
 // barriers.  What bounds it: the latency of those steps.  P = 96: 335 us; 412 with rows split over
@@ -885,21 +887,23 @@ __device__ __forceinline__ int sturm_count(const double *d, const double *e2, in
     return c;
 }
 
-// The four extremes of the tridiagonal (d, e2) of order n, into the threads that searched them.
-__device__ __forceinline__ void tridiagonal_extremes(const double *sd, const double *se2, int n, double (*swv)[4],
+// The four extremes of the tridiagonal (d, e2) of order n, into the threads that searched them, and a
+// bound of its eigenvalues' sizes, which every thread receives; near: the smallest size of an
+// eigenvalue, zero when one is within 1e-30 of the bound of zero.
+__device__ __forceinline__ void tridiagonal_extremes(const double *sd, const double *se2, int n, double (*swv)[6],
                                                      int *cnt, double &lo_all, double &hi_all, double &pos_all,
-                                                     double &neg_all) {
+                                                     double &neg_all, double &near, double &bd) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     // Gershgorin bound
-    double bd = 0.0;
+    bd = 0.0;
     if (t < n)
         bd = fabs(sd[t]) + (t > 0 ? sqrt(se2[t - 1]) : 0.0) + (t + 1 < n ? sqrt(se2[t]) : 0.0);
+    if (!(bd < __builtin_inf())) bd = __builtin_inf();       // NaN too: the caller sees the bound
     for (int o = 32; o > 0; o >>= 1) bd = fmax(bd, __shfl_xor(bd, o, 64));
     if (lane == 0) swv[wave][0] = bd;
     __syncthreads();
     bd = 0.0;
     for (int w = 0; w < kT / 64; w++) bd = fmax(bd, swv[w][0]);
-    // eigenvalues within 1e-30 of the bound of zero are exact zeros: rounding is at 1e-16 of it
     const double B = bd * (1.0 + 1e-10), tiny = 1e-30 * bd, pivmin = 1e-40 * bd;
     // 128 points for each of the four, by the first eight waves: two waves a SIMD, whose issue then keeps
     // pace with the recurrence's latency (n = 96: the kernel takes 335 us; with all sixteen, 256 points and 9 rounds, 359)
@@ -927,19 +931,25 @@ __device__ __forceinline__ void tridiagonal_extremes(const double *sd, const dou
     if (grp == 1 && (want || bd == 0.0)) hi_all = fmax(hi_all, v);
     if (grp == 2 && want) pos_all = fmin(pos_all, v);
     if (grp == 3 && want) neg_all = fmax(neg_all, v);
+    if (grp >= 2 && want) near = fmin(near, fabs(v));
+    if (t < 128 && (n_pos != n_neg || !(bd > 0.0))) near = 0.0;
 }
 
 __device__ __forceinline__ void write_extremes(double lo_all, double hi_all, double pos_all, double neg_all,
-                                               double (*swv)[4], double *out) {
+                                               double near, double bd, double (*swv)[6], double *out) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     for (int o = 32; o > 0; o >>= 1) {
         lo_all = fmin(lo_all, __shfl_xor(lo_all, o, 64));
         hi_all = fmax(hi_all, __shfl_xor(hi_all, o, 64));
         pos_all = fmin(pos_all, __shfl_xor(pos_all, o, 64));
         neg_all = fmax(neg_all, __shfl_xor(neg_all, o, 64));
+        near = fmin(near, __shfl_xor(near, o, 64));
     }
     __syncthreads();
-    if (lane == 0) { swv[wave][0] = lo_all; swv[wave][1] = hi_all; swv[wave][2] = pos_all; swv[wave][3] = neg_all; }
+    if (lane == 0) {
+        swv[wave][0] = lo_all; swv[wave][1] = hi_all; swv[wave][2] = pos_all; swv[wave][3] = neg_all;
+        swv[wave][4] = near;
+    }
     __syncthreads();
     if (t == 0) {
         for (int w = 1; w < kT / 64; w++) {
@@ -947,8 +957,10 @@ __device__ __forceinline__ void write_extremes(double lo_all, double hi_all, dou
             hi_all = fmax(hi_all, swv[w][1]);
             pos_all = fmin(pos_all, swv[w][2]);
             neg_all = fmax(neg_all, swv[w][3]);
+            near = fmin(near, swv[w][4]);
         }
         out[0] = lo_all; out[1] = hi_all; out[2] = pos_all; out[3] = neg_all;
+        out[4] = near; out[5] = bd;
     }
 }
 
@@ -966,11 +978,28 @@ __device__ __forceinline__ double householder(double tail, double2 &u0, double &
     return tau;
 }
 
-// out: smallest, largest, smallest positive (+inf: none), largest negative (-inf: none)
-__global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__restrict__ A, int P, double2 *W,
-                                                           double *out) {
+// The component of this workgroup in A (rows of ld): its first entry, its order in P.
+__device__ __forceinline__ const double2 *component(const double2 *A, int ld, const int2 *comps, int &P) {
+    P = ld;
+    if (!comps) return A;
+    const int2 c = comps[blockIdx.x];
+    P = qgtl::uniform(c.y);
+    return A + (size_t)qgtl::uniform(c.x) * (ld + 1);
+}
+
+// out, six values a component: smallest, largest, smallest positive (+inf: none), largest negative
+// (-inf: none) eigenvalue; the smallest size of an eigenvalue that the reduction found (indices set
+// aside left out; +inf: none) and a bound of the reduced part's eigenvalues, of which it is a
+// few P eps uncertain
+__global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__restrict__ Aall, int ld,
+                                                           const int2 *__restrict__ comps, double2 *Wall,
+                                                           double *outs) {
+    int P;
+    const double2 *A = component(Aall, ld, comps, P);
+    double2 *W = Wall + (A - Aall) / (ld + 1) * (size_t)ld;   // n^2 of ld n: apart for all components
+    double *out = outs + 6 * blockIdx.x;
     __shared__ double2 su[kT], sq[kT], sx[kT], part[kT];
-    __shared__ double sd[kT], se2[kT], swv[kT / 64][4];
+    __shared__ double sd[kT], se2[kT], swv[kT / 64][6];
     __shared__ int map[kT];
     __shared__ unsigned long long bal[kT / 64];
     __shared__ int cnt[kT / 64];
@@ -982,10 +1011,10 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
         iso = true;
         for (int i = 0; i < P; i++) {
             if (i == t) continue;
-            const double2 a = i < t ? A[(size_t)i * P + t] : A[(size_t)t * P + i];
+            const double2 a = i < t ? A[(size_t)i * ld + t] : A[(size_t)t * ld + i];
             if (a.x != 0.0 || a.y != 0.0) iso = false;
         }
-        isov = A[(size_t)t * P + t].x;
+        isov = A[(size_t)t * ld + t].x;
     }
     const bool live = t < P && !iso;
     const unsigned long long b = __ballot(live);
@@ -1004,14 +1033,15 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
     const double inf = __builtin_inf();
     double lo_all = iso ? isov : inf, hi_all = iso ? isov : -inf;
     double pos_all = iso && isov > 0.0 ? isov : inf, neg_all = iso && isov < 0.0 ? isov : -inf;
+    double near = inf, bd = 0.0;
     if (n > 0) {                                             // n >= 2: an index is live with another
         const int nseg = kT / n, seg = t / n, j = t % n;
         const int rows = (n + nseg - 1) / nseg;
         const int oj = map[j];
         auto entry = [&](int i) -> double2 {
             const int oi = map[i];
-            if (oi <= oj) { double2 v = A[(size_t)oi * P + oj]; if (oi == oj) v.y = 0.0; return v; }
-            const double2 v = A[(size_t)oj * P + oi];
+            if (oi <= oj) { double2 v = A[(size_t)oi * ld + oj]; if (oi == oj) v.y = 0.0; return v; }
+            const double2 v = A[(size_t)oj * ld + oi];
             return make_double2(v.x, -v.y);
         };
         if (seg < nseg)
@@ -1080,9 +1110,9 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
             __syncthreads();
         }
         __syncthreads();
-        tridiagonal_extremes(sd, se2, n, swv, cnt, lo_all, hi_all, pos_all, neg_all);
+        tridiagonal_extremes(sd, se2, n, swv, cnt, lo_all, hi_all, pos_all, neg_all, near, bd);
     }
-    write_extremes(lo_all, hi_all, pos_all, neg_all, swv, out);
+    write_extremes(lo_all, hi_all, pos_all, neg_all, near, bd, swv, out);
 }
 
 // The same for P <= 16 COLS = 64 ROWS with the matrix in registers: wave w holds columns w + 16 s,
@@ -1090,16 +1120,20 @@ __global__ __launch_bounds__(kT) void herm_extremes_kernel(const double2 *__rest
 // Householder vector by itself while the others apply the previous step's rank-2 update; then
 // every wave adds its columns to p = A u, and two waves add up the sixteen parts.
 template <int COLS, int ROWS>
-__global__ __launch_bounds__(kT) void herm_extremes_regs_kernel(const double2 *__restrict__ A, int P, double *out) {
+__global__ __launch_bounds__(kT) void herm_extremes_regs_kernel(const double2 *__restrict__ Aall, int ld,
+                                                                const int2 *__restrict__ comps, double *outs) {
     constexpr int N = 64 * ROWS;
+    int P;
+    const double2 *A = component(Aall, ld, comps, P);
+    double *out = outs + 6 * blockIdx.x;
     static_assert(16 * COLS == N, "square");
     __shared__ double2 su[N], sq[N], part[16][N];
-    __shared__ double sd[N], se2[N], swv[kT / 64][4], sup[kT / 64], stau;
+    __shared__ double sd[N], se2[N], swv[kT / 64][6], sup[kT / 64], stau;
     __shared__ int map[N], live[N], cnt[kT / 64];
     const int t = threadIdx.x, lane = t & 63, wave = qgtl::uniform(t >> 6);
     auto entry = [&](int oi, int oj) __attribute__((always_inline)) -> double2 {   // the upper triangle's
-        if (oi <= oj) { double2 v = A[(size_t)oi * P + oj]; if (oi == oj) v.y = 0.0; return v; }
-        const double2 v = A[(size_t)oj * P + oi];
+        if (oi <= oj) { double2 v = A[(size_t)oi * ld + oj]; if (oi == oj) v.y = 0.0; return v; }
+        const double2 v = A[(size_t)oj * ld + oi];
         return make_double2(v.x, -v.y);
     };
     double2 a[COLS][ROWS];
@@ -1252,11 +1286,12 @@ __global__ __launch_bounds__(kT) void herm_extremes_regs_kernel(const double2 *_
     __syncthreads();
     const double inf = __builtin_inf();
     const bool iso = t < P && !live[t < N ? t : 0];
-    const double isov = iso ? A[(size_t)t * P + t].x : 0.0;
+    const double isov = iso ? A[(size_t)t * ld + t].x : 0.0;
     double lo_all = iso ? isov : inf, hi_all = iso ? isov : -inf;
     double pos_all = iso && isov > 0.0 ? isov : inf, neg_all = iso && isov < 0.0 ? isov : -inf;
-    if (n > 0) tridiagonal_extremes(sd, se2, n, swv, cnt, lo_all, hi_all, pos_all, neg_all);
-    write_extremes(lo_all, hi_all, pos_all, neg_all, swv, out);
+    double near = inf, bd = 0.0;
+    if (n > 0) tridiagonal_extremes(sd, se2, n, swv, cnt, lo_all, hi_all, pos_all, neg_all, near, bd);
+    write_extremes(lo_all, hi_all, pos_all, neg_all, near, bd, swv, out);
 }
 
 // B = M^H M for the singular values of a general complex matrix
@@ -1411,17 +1446,21 @@ int qgtl_hip_herm_eig_c128(void *A, void *V, double *ev, int P, int batch, int m
     return 0;
 }
 
-int qgtl_hip_herm_extremes_c128(const void *A, void *W, int P, double *out4) {
-    if (P < 1 || P > kT) return qgtl::set_error_msg(-118, "herm_extremes: needs 1 <= P <= 1024");
-    if (P <= 64)
-        hipLaunchKernelGGL((herm_extremes_regs_kernel<4, 1>), dim3(1), dim3(kT), 0, qgtl::stream(), (const double2 *)A, P,
-                           out4);
-    else if (P <= 128)
-        hipLaunchKernelGGL((herm_extremes_regs_kernel<8, 2>), dim3(1), dim3(kT), 0, qgtl::stream(), (const double2 *)A, P,
-                           out4);
+int qgtl_hip_herm_extremes_c128(const void *A, void *W, int P, const int *comps, int ncomps, int largest,
+                                double *out) {
+    if (P < 1 || P > kT || ncomps < 1 || ncomps > P || largest < 1 || largest > P || (!comps && largest != P))
+        return qgtl::set_error_msg(-118, "herm_extremes: needs 1 <= P <= 1024 and components of 1 .. P indices");
+    const dim3 grid((unsigned)(comps ? ncomps : 1));
+    const int2 *c = (const int2 *)comps;
+    if (largest <= 64)
+        hipLaunchKernelGGL((herm_extremes_regs_kernel<4, 1>), grid, dim3(kT), 0, qgtl::stream(), (const double2 *)A, P, c,
+                           out);
+    else if (largest <= 128)
+        hipLaunchKernelGGL((herm_extremes_regs_kernel<8, 2>), grid, dim3(kT), 0, qgtl::stream(), (const double2 *)A, P, c,
+                           out);
     else
-        hipLaunchKernelGGL(herm_extremes_kernel, dim3(1), dim3(kT), 0, qgtl::stream(), (const double2 *)A, P,
-                           (double2 *)W, out4);
+        hipLaunchKernelGGL(herm_extremes_kernel, grid, dim3(kT), 0, qgtl::stream(), (const double2 *)A, P, c,
+                           (double2 *)W, out);
     QGTL_LAUNCH_CHECK("herm_extremes_c128");
     return 0;
 }

@@ -301,51 +301,158 @@ static int singular_values(const double *M, size_t P, double *sv, int *hermitian
     return 0;
 }
 
+/* The components of M's indices: two indices are in one when a chain of nonzero
+ * entries joins them (by a common row, for the columns of a general M: the
+ * entries of M^H M).  label[i]: the component of index i, numbered by smallest
+ * index; returns their count, 0 without memory. */
+static int find_components(const double *M, int P, int herm, int *label)
+{
+    int *queue = (int *)malloc(2 * (size_t)P * sizeof(int)), *row_seen = queue + P;
+    if (!queue) return 0;
+    int count = 0, left = P;
+#define NONZERO(i, j) (M[2 * ((size_t)(i) * P + (j))] != 0.0 || M[2 * ((size_t)(i) * P + (j)) + 1] != 0.0)
+    for (int i = 0; i < P; i++) label[i] = -1, row_seen[i] = 0;
+    for (int first = 0; first < P; first++) {
+        if (label[first] >= 0) continue;
+        int head = 0, tail = 0;
+        queue[tail++] = first;
+        label[first] = count;
+        left--;
+        while (head < tail && left > 0) {
+            const int i = queue[head++];
+            for (int r = herm ? i : 0; r < (herm ? i + 1 : P) && left > 0; r++) {
+                if (!herm && (row_seen[r] || !NONZERO(r, i))) continue;
+                row_seen[r] = 1;
+                for (int j = 0; j < P; j++)
+                    if (label[j] < 0 && (NONZERO(r, j) || (herm && NONZERO(j, r)))) {
+                        label[j] = count;
+                        queue[tail++] = j;
+                        left--;
+                    }
+            }
+        }
+        count++;
+    }
+#undef NONZERO
+    free(queue);
+    return count;
+}
+
+/* The extreme eigenvalues of M (herm) or of M^H M, component by component: lo,
+ * hi, the smallest positive and the largest negative one over all of them.
+ * *sure = 0 when an eigenvalue of some component is not well above that
+ * component's rounding. */
+static int extreme_eigenvalues(const double *M, int P, int herm, double e[4], int *sure)
+{
+    const size_t PP = (size_t)P * P;
+    int *label = (int *)malloc(4 * (size_t)P * sizeof(int));
+    if (!label) return QGT_ERROR_NO_MEMORY;
+    int *order = label + P, *comps = order + P;              /* comps: P pairs */
+    int rc = QGT_ERROR_NO_MEMORY;
+    double *moved = NULL, *out = NULL;
+    void *dA, *dV, *dout, *dB, *dcomps = NULL;
+    int nc = find_components(M, P, herm, label), largest = P;
+    if (nc == 0) goto done;
+    const double *src = M;
+    if (nc > 1) {
+        /* indices in component order: rows and columns of M, or columns for M^H M */
+        int k = 0;
+        largest = 0;
+        for (int c = 0; c < nc; c++) comps[2 * c + 1] = 0;
+        for (int i = 0; i < P; i++) comps[2 * label[i] + 1]++;
+        for (int c = 0; c < nc; c++) {
+            comps[2 * c] = k;
+            k += comps[2 * c + 1];
+            if (comps[2 * c + 1] > largest) largest = comps[2 * c + 1];
+            comps[2 * c + 1] = 0;
+        }
+        for (int i = 0; i < P; i++) {
+            const int c = label[i];
+            order[comps[2 * c] + comps[2 * c + 1]++] = i;
+        }
+        moved = (double *)malloc(PP * 16);
+        if (!moved) goto done;
+        for (int i = 0; i < P; i++)
+            for (int j = 0; j < P; j++)
+                memcpy(moved + 2 * ((size_t)i * P + j),
+                       M + 2 * ((size_t)(herm ? order[i] : i) * P + order[j]), 16);
+        src = moved;
+    }
+    out = (double *)malloc((size_t)nc * 6 * sizeof(double));
+    if (!out) goto done;
+#define CTRY(call) do { rc = (call); if (rc) goto done; } while (0)
+    CTRY(scratch(S_A, PP * 16, &dA));
+    CTRY(scratch(S_V, PP * 16, &dV));
+    CTRY(scratch(S_EV, (size_t)nc * 6 * sizeof(double), &dout));
+    if (nc > 1) {
+        CTRY(scratch(S_U, (size_t)nc * 2 * sizeof(int), &dcomps));
+        CTRY(qgtl_hip_h2d(dcomps, comps, (size_t)nc * 2 * sizeof(int)));
+    }
+    if (herm) {
+        CTRY(qgtl_hip_h2d(dA, src, PP * 16));
+    } else {
+        CTRY(scratch(S_B, PP * 16, &dB));
+        CTRY(qgtl_hip_h2d(dB, src, PP * 16));
+        CTRY(qgtl_hip_gram_small_c128(dB, dA, P));
+    }
+    CTRY(qgtl_hip_herm_extremes_c128(dA, dV, P, (const int *)dcomps, nc, largest, (double *)dout));
+    CTRY(qgtl_hip_d2h(out, dout, (size_t)nc * 6 * sizeof(double)));
+    CTRY(qgtl_hip_sync());
+#undef CTRY
+    e[0] = INFINITY, e[1] = -INFINITY, e[2] = INFINITY, e[3] = -INFINITY;
+    *sure = 1;
+    for (int c = 0; c < nc; c++) {
+        const double *o = out + 6 * (size_t)c;
+        e[0] = fmin(e[0], o[0]);
+        e[1] = fmax(e[1], o[1]);
+        e[2] = fmin(e[2], o[2]);
+        e[3] = fmax(e[3], o[3]);
+        /* 2^-44 P of the bound: 256 times the rounding of an eigenvalue, P eps */
+        if (!(o[4] > 0x1p-44 * (nc > 1 ? comps[2 * c + 1] : P) * o[5])) *sure = 0;
+    }
+done:
+    if (rc) qgtl_hip_sync();                                  /* no copy may still read the buffers below */
+    free(label);
+    free(moved);
+    free(out);
+    return rc;
+}
+
 /* The largest and the smallest nonzero singular value of M (smallest: +inf when
- * M has none), as singular_values would list them, without the eigenvectors. */
+ * M has none), as singular_values would list them.  Without eigenvectors where
+ * every eigenvalue of every component stands clear of the rounding; a matrix
+ * with infinities or NaN, or one that is singular or nearly so, whose smallest
+ * values are rounding or exact zeros as the iteration leaves them, takes the full
+ * decomposition. */
 static int extreme_singular_values(const double *M, size_t P, double *smax, double *smin)
 {
-    const size_t PP = P * P;
-    int finite = 1;
-    for (size_t i = 0; i < 2 * PP; i++) finite &= isfinite(M[i]) != 0;
-    if (!finite) {                             /* infinities and NaN: whatever the full decomposition lists */
-        double *sv = (double *)malloc(P * sizeof(double));
-        int h = 0;
-        if (!sv) return QGT_ERROR_NO_MEMORY;
-        const int rc = singular_values(M, P, sv, &h);
-        *smax = 0.0;
-        *smin = INFINITY;
-        for (size_t i = 0; !rc && i < P; i++) {
-            if (sv[i] > *smax) *smax = sv[i];
-            if (sv[i] > 0.0 && sv[i] < *smin) *smin = sv[i];
+    int finite = 1, sure = 0;
+    for (size_t i = 0; i < 2 * P * P; i++) finite &= isfinite(M[i]) != 0;
+    if (finite) {
+        const int herm = is_hermitian(M, P);
+        double e[4];
+        TRY(extreme_eigenvalues(M, (int)P, herm, e, &sure));
+        if (sure && herm) {
+            *smax = fmax(fabs(e[0]), fabs(e[1]));
+            *smin = fmin(e[2], -e[3]);
+        } else if (sure) {                     /* eigenvalues of M^H M */
+            *smax = sqrt(fmax(e[1], 0.0));
+            *smin = sqrt(e[2]);
         }
-        free(sv);
-        return rc;
+        if (sure) return 0;
     }
-    void *dA, *dV, *dev, *dB;
-    double e[4];
-    TRY(scratch(S_A, PP * 16, &dA));
-    TRY(scratch(S_V, PP * 16, &dV));
-    TRY(scratch(S_EV, P * 8 > sizeof e ? P * 8 : sizeof e, &dev));
-    const int herm = is_hermitian(M, P);
-    if (herm) {
-        TRY(qgtl_hip_h2d(dA, M, PP * 16));
-    } else {
-        TRY(scratch(S_B, PP * 16, &dB));
-        TRY(qgtl_hip_h2d(dB, M, PP * 16));
-        TRY(qgtl_hip_gram_small_c128(dB, dA, (int)P));
+    double *sv = (double *)malloc(P * sizeof(double));
+    int h = 0;
+    if (!sv) return QGT_ERROR_NO_MEMORY;
+    const int rc = singular_values(M, P, sv, &h);
+    *smax = 0.0;
+    *smin = INFINITY;
+    for (size_t i = 0; !rc && i < P; i++) {
+        if (sv[i] > *smax) *smax = sv[i];
+        if (sv[i] > 0.0 && sv[i] < *smin) *smin = sv[i];
     }
-    TRY(qgtl_hip_herm_extremes_c128(dA, dV, (int)P, (double *)dev));
-    TRY(qgtl_hip_d2h(e, dev, sizeof e));
-    TRY(qgtl_hip_sync());
-    if (herm) {
-        *smax = fmax(fabs(e[0]), fabs(e[1]));
-        *smin = fmin(e[2], -e[3]);
-    } else {                                   /* eigenvalues of M^H M: rounding below zero counts as zero */
-        *smax = sqrt(fmax(e[1], 0.0));
-        *smin = sqrt(e[2]);
-    }
-    return 0;
+    free(sv);
+    return rc;
 }
 
 bool compute_complex_matrix_condition_number(const ComplexFloat *matrix, size_t dimension, float *condition_number)

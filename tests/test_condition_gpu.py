@@ -67,11 +67,12 @@ def test_condition_number_zero_rows_and_diagonals():
 
 
 def _extremes(A):
-    """qgtl_hip_herm_extremes_c128 itself: smallest, largest, smallest positive, largest negative."""
-    L, vp = Q.lib(), ctypes.c_void_p
+    """qgtl_hip_herm_extremes_c128 itself, A one component: smallest, largest, smallest positive, largest
+    negative; smallest size, bound."""
+    L, vp, ip = Q.lib(), ctypes.c_void_p, ctypes.c_int
     A = np.ascontiguousarray(A, np.complex128)
-    out = np.full(4, 7.0)
-    L.qgtl_hip_herm_extremes_c128.argtypes = [vp, vp, ctypes.c_int, vp]
+    out = np.full(6, 7.0)
+    L.qgtl_hip_herm_extremes_c128.argtypes = [vp, vp, ip, vp, ip, ip, vp]
     for f in ("h2d", "d2h"):
         getattr(L, "qgtl_hip_" + f).argtypes = [vp, vp, ctypes.c_size_t]
     L.qgtl_hip_malloc.argtypes = [ctypes.POINTER(vp), ctypes.c_size_t]
@@ -81,7 +82,7 @@ def _extremes(A):
     for p, n in zip(d, (A.nbytes, A.nbytes, out.nbytes)):
         assert L.qgtl_hip_malloc(ctypes.byref(p), n) == 0
     assert L.qgtl_hip_h2d(d[0], A.ctypes.data, A.nbytes) == 0
-    assert L.qgtl_hip_herm_extremes_c128(d[0], d[1], len(A), d[2]) == 0
+    assert L.qgtl_hip_herm_extremes_c128(d[0], d[1], len(A), None, 1, len(A), d[2]) == 0
     assert L.qgtl_hip_d2h(out.ctypes.data, d[2], out.nbytes) == 0 and L.qgtl_hip_sync() == 0
     for p in d:
         L.qgtl_hip_free(p)
@@ -100,3 +101,58 @@ def test_extremes_of_a_tiny_rank_deficient_matrix(P, scale):
     lo, hi = _extremes(A * scale)[:2] / scale
     assert abs(hi - ev[-1]) <= 4 * P * np.finfo(float).eps * ev[-1]
     assert abs(lo - ev[0]) <= 4 * P * np.finfo(float).eps * ev[-1]
+
+
+def _coupled(P, rng, general):
+    """A P x P block all of whose indices are coupled, condition number about 100."""
+    U, _ = np.linalg.qr(rng.normal(size=(P, P)) + 1j * rng.normal(size=(P, P)))
+    V = U
+    if general:
+        V, _ = np.linalg.qr(rng.normal(size=(P, P)) + 1j * rng.normal(size=(P, P)))
+    B = (U * np.logspace(-2, 0, P)) @ V.conj().T
+    return B if general else 0.5 * (B + B.conj().T)
+
+
+# sizes of the blocks: all within one kernel form, and across its limits of 64 and 128
+@pytest.mark.parametrize("sizes", [(2, 2), (5, 3, 4), (50, 40), (90, 33, 20), (140, 20)])
+@pytest.mark.parametrize("general", [False, True])
+@pytest.mark.parametrize("scales", [(1e5, 1e-11), (1.0, 1e-31), (1.0, 1e-7), (1e5, 1e-6)])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_condition_number_of_decoupled_blocks(sizes, general, scales, mixed):
+    """Blocks that no entry couples keep their own accuracy however small they are beside the others
+    (and wherever their indices stand): the extremes are those of each block by itself."""
+    rng = np.random.default_rng(sum(sizes))
+    blocks = [_coupled(n, rng, general) * scales[i % 2] for i, n in enumerate(sizes)]
+    blocks = [b.astype(np.complex64) for b in blocks]
+    if not general:
+        blocks = [np.tril(b, -1) + np.tril(b, -1).conj().T + np.diag(b.diagonal().real) for b in blocks]
+    P = sum(sizes) + 1                                          # and a row and column of zeros
+    M = np.zeros((P, P), np.complex64)
+    at = np.arange(P)
+    if mixed:
+        at = rng.permutation(P)
+    o = 0
+    for b in blocks:
+        i = at[o:o + len(b)]
+        M[np.ix_(i, i)] = b
+        o += len(b)
+    sv = np.concatenate([np.linalg.svd(b.astype(np.complex128), compute_uv=False) for b in blocks])
+    ref = sv.max() / sv.min() if sv.min() > 1e-15 else np.inf   # QGTL's rule: 1e-15 is zero
+    k = _kappa(M)
+    assert k == ref if np.isinf(ref) else abs(k - ref) <= 2e-6 * ref
+
+
+@pytest.mark.parametrize("P,rank", [(2, 1), (3, 2), (40, 1), (64, 40), (70, 69), (131, 100)])
+@pytest.mark.parametrize("scale", [1.0, 1e5])
+def test_condition_number_of_coupled_singular_matrices(P, rank, scale):
+    """Singular matrices: the smallest nonzero value is rounding, or an exact zero is left out, as the
+    eigenvalues of the full decomposition have it."""
+    rng = np.random.default_rng(P)
+    V = rng.integers(-3, 4, size=(P, rank)) * (1.0 + 0j)
+    V[0] = 1.0
+    if rank == 1:
+        V[:] = 1.0                                              # all entries equal
+    M = ((V @ V.conj().T) * scale).astype(np.complex64)
+    sv = np.abs(Q.hermitian_eig(M.astype(np.complex128))[0])
+    smin = sv[sv > 0].min()
+    assert _kappa(M) == (np.float32(sv.max() / smin) if smin > 1e-15 else np.inf)
