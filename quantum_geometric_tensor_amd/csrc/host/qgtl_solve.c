@@ -262,7 +262,8 @@ static double *to_c128(const ComplexFloat *m, size_t count)
     return o;
 }
 
-static int is_hermitian(const double *M, size_t P)
+/* Hermitian within 1e-6 of the largest entry; *exact (may be NULL): to the last bit. */
+static int is_hermitian(const double *M, size_t P, int *exact)
 {
     /* squared magnitudes of float-range values: no overflow in FP64 */
     double mx = 0.0, dev = 0.0;
@@ -273,6 +274,7 @@ static int is_hermitian(const double *M, size_t P)
             mx = fmax(mx, fmax(ar * ar + ai * ai, br * br + bi * bi));
             dev = fmax(dev, (ar - br) * (ar - br) + (ai + bi) * (ai + bi));
         }
+    if (exact) *exact = dev == 0.0;
     return dev <= 1e-12 * (mx > 0 ? mx : 1.0);
 }
 
@@ -286,7 +288,7 @@ static int singular_values(const double *M, size_t P, double *sv, int *hermitian
     TRY(scratch(S_V, PP * 16, &dV));
     TRY(scratch(S_EV, P * 8, &dev));
     TRY(scratch(S_INT, sizeof(int), &dsw));
-    *hermitian = is_hermitian(M, P);
+    *hermitian = is_hermitian(M, P, NULL);
     if (*hermitian) {
         TRY(qgtl_hip_h2d(dA, M, PP * 16));
     } else {
@@ -338,11 +340,13 @@ static int find_components(const double *M, int P, int herm, int *label)
     return count;
 }
 
-/* The extreme eigenvalues of M (herm) or of M^H M, component by component: lo,
- * hi, the smallest positive and the largest negative one over all of them.
+/* The extreme eigenvalues of M (herm; unless exact of its Hermitian part, whose
+ * eigenvalues differ from M's singular values by squares of what the triangles
+ * differ by, where those of one triangle differ by as much) or of M^H M, component by
+ * component: lo, hi, the smallest positive and the largest negative one over all of them.
  * *sure = 0 when an eigenvalue of some component is not well above that
  * component's rounding. */
-static int extreme_eigenvalues(const double *M, int P, int herm, double e[4], int *sure)
+static int extreme_eigenvalues(const double *M, int P, int herm, int exact, double e[4], int *sure)
 {
     const size_t PP = (size_t)P * P;
     int *label = (int *)malloc(4 * (size_t)P * sizeof(int));
@@ -370,12 +374,20 @@ static int extreme_eigenvalues(const double *M, int P, int herm, double e[4], in
             const int c = label[i];
             order[comps[2 * c] + comps[2 * c + 1]++] = i;
         }
+    } else {
+        for (int i = 0; i < P; i++) order[i] = i;
+    }
+    if (nc > 1 || (herm && !exact)) {
         moved = (double *)malloc(PP * 16);
         if (!moved) goto done;
         for (int i = 0; i < P; i++)
-            for (int j = 0; j < P; j++)
-                memcpy(moved + 2 * ((size_t)i * P + j),
-                       M + 2 * ((size_t)(herm ? order[i] : i) * P + order[j]), 16);
+            for (int j = 0; j < P; j++) {
+                const size_t oi = (size_t)(herm ? order[i] : i), oj = (size_t)order[j];
+                const double *a = M + 2 * (oi * P + oj), *b = M + 2 * (oj * P + oi);
+                double *o = moved + 2 * ((size_t)i * P + j);
+                o[0] = herm ? 0.5 * (a[0] + b[0]) : a[0];
+                o[1] = herm ? 0.5 * (a[1] - b[1]) : a[1];
+            }
         src = moved;
     }
     out = (double *)malloc((size_t)nc * 6 * sizeof(double));
@@ -429,9 +441,10 @@ static int extreme_singular_values(const double *M, size_t P, double *smax, doub
     int finite = 1, sure = 0;
     for (size_t i = 0; i < 2 * P * P; i++) finite &= isfinite(M[i]) != 0;
     if (finite) {
-        const int herm = is_hermitian(M, P);
+        int exact;
+        const int herm = is_hermitian(M, P, &exact);
         double e[4];
-        TRY(extreme_eigenvalues(M, (int)P, herm, e, &sure));
+        TRY(extreme_eigenvalues(M, (int)P, herm, exact, e, &sure));
         if (sure && herm) {
             *smax = fmax(fabs(e[0]), fabs(e[1]));
             *smin = fmin(e[2], -e[3]);

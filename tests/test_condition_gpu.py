@@ -156,3 +156,16 @@ def test_condition_number_of_coupled_singular_matrices(P, rank, scale):
     sv = np.abs(Q.hermitian_eig(M.astype(np.complex128))[0])
     smin = sv[sv > 0].min()
     assert _kappa(M) == (np.float32(sv.max() / smin) if smin > 1e-15 else np.inf)
+
+
+@pytest.mark.parametrize("P", [2, 40, 64, 100, 140])
+def test_condition_number_of_a_nearly_hermitian_matrix(P):
+    """Triangles that differ by rounding (here 5e-7 of the largest entry; up to 1e-6 counts as Hermitian):
+    the singular values are those of the Hermitian part up to squares, not those of one triangle."""
+    rng = np.random.default_rng(P)
+    M = _hermitian(P, 0.25 * np.logspace(-3, 0, P), P)
+    E = 5e-7 * np.abs(M).max() * rng.choice([-1.0, 1.0], size=(P, P))
+    M = (M + np.tril(E, -1)).astype(np.complex64).astype(np.complex128)
+    ev = np.linalg.eigvalsh(0.5 * (M + M.conj().T))
+    ref = np.abs(ev).max() / np.abs(ev).min()
+    assert abs(_kappa(M) - ref) <= ref * (1e-6 + P * np.finfo(np.float64).eps * ref)
