@@ -74,7 +74,7 @@ typedef struct {
     int32_t hi_pos[QGTL_TILE_BITS_MAX];        /* physical bit of tile bit nlow+i */
     int32_t rest_pos[QGTL_MAX_QUBITS];         /* physical bit of tile-index bit i */
     int32_t gate_bit[QGTL_TILE_BITS_MAX];      /* tile bit of matrix g */
-    int32_t sign;                              /* mstage's sign, applied before the store */
+    int32_t sign;                              /* mstage's sign, applied before the store; QGTL_STORE_PERM: a CZ in the list */
     union {
         struct {                               /* QGTL_STORE_PERM */
             int32_t perm_type[QGTL_PERM_MAX];  /* 0 = CNOT(a -> b), 1 = SWAP(a, b), 2 = CZ(a, b) */
@@ -252,9 +252,11 @@ typedef struct {
     uint32_t tiles;         /* ceil(2^n / 2048) */
     uint32_t K;
     uint32_t unit_begin;    /* units: tiles * K */
-    uint32_t pad;           /* QGTL_INJECT_ITEM_SPLIT: write the states in split-plane form (no sums) */
+    uint32_t pad;           /* QGTL_INJECT_ITEM_SPLIT: write the states in split-plane form (no sums);
+                               QGTL_INJECT_ITEM_SIGN: some z of the descriptor is not 0 */
 } qgtl_inject_item_t;
 #define QGTL_INJECT_ITEM_SPLIT 1u
+#define QGTL_INJECT_ITEM_SIGN 2u
 
 typedef struct {
     uint64_t partials;      /* [K][tiles][4] */

@@ -468,7 +468,7 @@ static int build_schedule(struct qgtl_batch *B)
                     it[k].tiles = (uint32_t)in->tiles;
                     it[k].K = (uint32_t)c;
                     it[k].unit_begin = (uint32_t)u;
-                    it[k].pad = final_split;
+                    it[k].pad = final_split | (p->has_signs ? QGTL_INJECT_ITEM_SIGN : 0u);
                     u += (uint64_t)it[k].tiles * (uint64_t)c;
                     k++;
                 }

@@ -700,6 +700,7 @@ static void build_passes(qgtl_block_t *b, int n)
                     p->perm_type[i] = b->perm_type[i];
                     p->perm_a[i] = b->perm_a[i];
                     p->perm_b[i] = b->perm_b[i];
+                    p->sign |= b->perm_type[i] == 2;
                 }
             } else {
                 b->mstage_kernels = 1;
