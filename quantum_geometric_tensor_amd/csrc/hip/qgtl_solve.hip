@@ -479,9 +479,10 @@ __global__ __launch_bounds__(kT) void herm_eig_c128_kernel(double2 *Aall, double
 // rank-1 update of the whole trailing matrix per column in global memory and
 // one reduction over a wave per row of the substitutions.
 //
-// NB = 32 while the panel fits LDS beside the rest (P <= 512), 16 above;
-// up to 256 the panel buffer is sized so that two workgroups share a CU.
-constexpr int kCT = 512;          // 8 waves: the register rows of 32 doubles need more than 128 VGPRs
+// NB = 32 while the panel fits LDS beside the rest (P <= 512), 16 above: one workgroup of eight
+// waves a CU (the register rows of 32 doubles take 232 VGPRs).  Small systems, of which a batch
+// has many, take narrower blocks and fewer waves, so that a short column is not padded to 32 and
+// several workgroups share a CU: 1024 systems of P = 8 14 us, of P = 33 32 us (82 and 169 us with NB = 32).
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ double readlane_f64(double v, int lane);
@@ -519,14 +520,14 @@ __device__ __forceinline__ int factor_diag(double (*dg)[NB + 2], double *inv, in
     return bad;
 }
 
-template <int NB, int ROWS>
-__global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const double *ball, double *xall, int P,
+template <int NB, int ROWS, int CT>
+__global__ __launch_bounds__(CT) void cholesky_f64_kernel(double *Lall, const double *ball, double *xall, int P,
                                                           double lambda, int *status) {
     constexpr int LD = ROWS + 1;                     // odd: the transposing writes hit all banks
     constexpr int kOwn = NB == 32 ? 3 : 1;           // 16 x 16 tiles of a diagonal block
     __shared__ double lp[NB * LD];                   // panel, column c of row i at c * LD + i
     __shared__ __attribute__((aligned(16))) double dgs[2][NB][NB + 2];
-    __shared__ double y[1024], invs[2][NB];
+    __shared__ double y[ROWS + NB], invs[2][NB];
     __shared__ int s_fail;
     double *L = Lall + (size_t)blockIdx.x * P * P;   // holds A on entry (row-major, symmetric)
     const double *b = ball + (size_t)blockIdx.x * P;
@@ -534,12 +535,12 @@ __global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const d
     const int t = threadIdx.x, lane = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     if (t == 0) s_fail = 0;
-    for (int i = t; i < P; i += kCT) {
+    for (int i = t; i < P; i += CT) {
         y[i] = b[i];
         L[(size_t)i * P + i] += lambda;
     }
     __syncthreads();
-    for (int e = t; e < NB * NB; e += kCT) {
+    for (int e = t; e < NB * NB; e += CT) {
         const int r = e / NB, c = e % NB;
         dgs[0][r][c] = (r < P && c <= r) ? L[(size_t)r * P + c] : (r == c ? 1.0 : 0.0);
     }
@@ -553,7 +554,7 @@ __global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const d
         const int m = P - kb - nb + 1;               // rows below the block and the row of b
         const int m16 = (m + 15) / 16 * 16;
 #pragma unroll 4
-        for (int e = t; e < m16 * NB; e += kCT) {
+        for (int e = t; e < m16 * NB; e += CT) {
             const int r = e / NB, c = e % NB;
             const bool in = c < nb && r < m - 1;
             double v = L[in ? (size_t)(kb + nb + r) * P + kb + c : (size_t)0];
@@ -562,7 +563,7 @@ __global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const d
         }
         __syncthreads();
         if (s_fail) break;                           // uniform
-        for (int r = t; r < m; r += kCT) {
+        for (int r = t; r < m; r += CT) {
             double v[NB];
 #pragma unroll
             for (int c = 0; c < NB; c++) v[c] = lp[c * LD + r];
@@ -618,20 +619,20 @@ __global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const d
             }
         };
         if (w == 0) {
-            if (nn > 0) {
+            if (NB >= 16 && nn > 0) {                            // NB = 4: P <= 4, one block
                 for (int e = lane; e < NB * NB; e += 64)         // identity past a short last block
                     if (e / NB >= nn) dgs[cur ^ 1][e / NB][e % NB] = e / NB == e % NB ? 1.0 : 0.0;
                 for (int u = 0; u < kOwn && u < nt * (nt + 1) / 2; u++) tile(u, true);
                 if (factor_diag<NB>(dgs[cur ^ 1], invs[cur ^ 1], lane) && lane == 0) s_fail = 1;
             }
         } else {
-            for (int u = kOwn + w - 1; u < nt * (nt + 1) / 2; u += kCT / 64 - 1) tile(u, false);
+            for (int u = kOwn + w - 1; u < nt * (nt + 1) / 2; u += CT / 64 - 1) tile(u, false);
             // the factor's columns, for the back substitution (the diagonal inverted; b's row: y)
-            for (int e = t - 64; e < NB * NB; e += kCT - 64) {
+            for (int e = t - 64; e < NB * NB; e += CT - 64) {
                 const int r = e / NB, c = e % NB;
                 if (c <= r && r < nb) L[(size_t)(kb + r) * P + kb + c] = c == r ? inv[r] : dg[c][r];
             }
-            for (int e = t - 64; e < m * NB; e += kCT - 64) {
+            for (int e = t - 64; e < m * NB; e += CT - 64) {
                 const int r = e / NB, c = e % NB;
                 if (c >= nb) continue;
                 if (r < m - 1) L[(size_t)(kb + nb + r) * P + kb + c] = lp[c * LD + r];
@@ -685,7 +686,7 @@ __global__ __launch_bounds__(kCT) void cholesky_f64_kernel(double *Lall, const d
                 for (int j = 0; j < NB; j++) s = fma(-lc[j], j < nb ? y[kb + j] : 0.0, s);
                 y[t - 64] = s;
             }
-            for (int i = t - 64 + kCT - 64; i < kb; i += kCT - 64) {
+            for (int i = t - 64 + CT - 64; i < kb; i += CT - 64) {
                 double s = y[i];
 #pragma unroll 4
                 for (int j = 0; j < nb; j++) s = fma(-L[(size_t)(kb + j) * P + i], y[kb + j], s);
@@ -1467,12 +1468,17 @@ int qgtl_hip_herm_extremes_c128(const void *A, void *W, int P, const int *comps,
 
 int qgtl_hip_cholesky_solve_f64(double *A, const double *b, double *x, int P, int batch, double lambda, int *status) {
     if (P < 1 || P > 1024) return qgtl::set_error_msg(-118, "cholesky: needs 1 <= P <= 1024");
-#define QGTL_CHOL(NB, ROWS)                                                                                       \
-    hipLaunchKernelGGL((cholesky_f64_kernel<NB, ROWS>), dim3(batch), dim3(kCT), 0, qgtl::stream(), A, b, x, P, lambda, \
+#define QGTL_CHOL(NB, ROWS, CT)                                                                                   \
+    hipLaunchKernelGGL((cholesky_f64_kernel<NB, ROWS, CT>), dim3(batch), dim3(CT), 0, qgtl::stream(), A, b, x, P, lambda, \
                        status)
-    if (P <= 256) QGTL_CHOL(32, 240);                // ROWS >= round16(P - NB + 1)
-    else if (P <= 512) QGTL_CHOL(32, 496);
-    else QGTL_CHOL(16, 1024);
+    // ROWS >= round16(P - NB + 1).  Device time of one system, this line / the next one's form: P = 4 7 / 12 us,
+    // P = 32 20 / 25, P = 64 34 / 49
+    if (P <= 4) QGTL_CHOL(4, 16, 128);
+    else if (P <= 32) QGTL_CHOL(16, 32, 128);
+    else if (P <= 64) QGTL_CHOL(16, 64, 256);
+    else if (P <= 256) QGTL_CHOL(32, 240, 512);      // P = 192: 145 us, 147 with the next line's panel
+    else if (P <= 512) QGTL_CHOL(32, 496, 512);
+    else QGTL_CHOL(16, 1024, 512);
 #undef QGTL_CHOL
     QGTL_LAUNCH_CHECK("cholesky_f64");
     return 0;

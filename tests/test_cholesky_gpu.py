@@ -20,7 +20,7 @@ def _residual_ok(A, x, b):
     assert r <= 8 * len(b) * np.finfo(np.float64).eps * np.linalg.norm(A, 2) * np.linalg.norm(x), r
 
 
-@pytest.mark.parametrize("P", [1, 2, 15, 16, 31, 32, 33, 47, 48, 63, 64, 65, 192, 255, 256, 257, 511, 512, 513, 1023, 1024])
+@pytest.mark.parametrize("P", [1, 2, 4, 5, 15, 16, 17, 31, 32, 33, 47, 48, 63, 64, 65, 192, 255, 256, 257, 511, 512, 513, 1023, 1024])
 @pytest.mark.parametrize("noalloc", [False, True])
 def test_cholesky_sizes(P, noalloc):
     A, b = _spd(P, P)
@@ -42,7 +42,7 @@ def test_cholesky_sizes(P, noalloc):
     _residual_ok(A + lam * np.eye(P), x, b)
 
 
-@pytest.mark.parametrize("P,batch", [(20, 300), (100, 7), (300, 3)])
+@pytest.mark.parametrize("P,batch", [(3, 50), (20, 300), (40, 60), (100, 7), (300, 3)])
 def test_cholesky_batch_with_one_indefinite(P, batch):
     """Each system has its own workgroup and status: the one that is not positive definite (a
     negative last pivot, found in the last column block) fails alone."""
