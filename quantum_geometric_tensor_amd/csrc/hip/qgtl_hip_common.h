@@ -23,6 +23,15 @@ __device__ __forceinline__ int find_item(const Item *__restrict__ items, int nit
     return lo;
 }
 
+// Orders the LDS accesses of one wave's lanes: what a lane stored before is what the
+// others load after (the hardware keeps a wave's LDS accesses in order; this
+// keeps the compiler from moving or forwarding them).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // A value every lane of the wave holds (e.g. loaded from a grouped launch's item
 // table) moved into scalar registers, so the code using it stays scalar.
 // Entry idx of Q; host: the caller's pinned copy (consecutive threads write consecutive

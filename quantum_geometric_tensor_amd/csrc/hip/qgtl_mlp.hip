@@ -445,7 +445,7 @@ __global__ __launch_bounds__(kThreads) void kaporin_kernel(int P, int r, const f
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) ld += __shfl_xor(ld, o, 64);
         if (lane == 0) sh_logdet = ld;
-        __builtin_amdgcn_wave_barrier();
+        qgtl::wave_sync();                                     // inv and W's rows, by other lanes
         if constexpr (RT == 1) {
             double x[R];
 #pragma unroll
@@ -467,7 +467,7 @@ __global__ __launch_bounds__(kThreads) void kaporin_kernel(int P, int r, const f
             if (lane < R)
 #pragma unroll
                 for (int i = 0; i < R; i++) Wi[lane * (R + 1) + i] = x[i];
-        } else {
+        } else if (lane < R) {
             // 32 unknowns and their rows do not fit the registers: the column lives in LDS
             double *x = Wi + row * (R + 1);
             for (int i = 0; i < R; i++) {

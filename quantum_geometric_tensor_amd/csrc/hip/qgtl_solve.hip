@@ -152,14 +152,12 @@ __global__ __launch_bounds__(kT) void lu_solve_c128_kernel(double2 *Aall, const 
         if (threadIdx.x == 0) status[blockIdx.x] = -1;
         return;
     }
-    // forward (unit lower) and back substitution by one wave through LDS (an
-    // LDS write by lane 0 is seen by the wave's later LDS reads: in order)
+    // forward (unit lower) and back substitution by one wave through LDS
     __shared__ double2 sx[1024];
     if (threadIdx.x < 64) {
         const int lane = threadIdx.x;
         for (int i = lane; i < P; i += 64) sx[i] = b[piv[i]];
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
+        qgtl::wave_sync();
         for (int i = 0; i < P; i++) {
             double sr = 0.0, si = 0.0;
             for (int j = lane; j < i; j += 64) {
@@ -169,8 +167,7 @@ __global__ __launch_bounds__(kT) void lu_solve_c128_kernel(double2 *Aall, const 
             }
             for (int o = 32; o > 0; o >>= 1) { sr += __shfl_xor(sr, o, 64); si += __shfl_xor(si, o, 64); }
             if (lane == 0) sx[i] = make_double2(sx[i].x - sr, sx[i].y - si);
-            __builtin_amdgcn_s_waitcnt(0);
-            __builtin_amdgcn_wave_barrier();
+            qgtl::wave_sync();
         }
         for (int i = P - 1; i >= 0; i--) {
             double sr = 0.0, si = 0.0;
@@ -181,8 +178,7 @@ __global__ __launch_bounds__(kT) void lu_solve_c128_kernel(double2 *Aall, const 
             }
             for (int o = 32; o > 0; o >>= 1) { sr += __shfl_xor(sr, o, 64); si += __shfl_xor(si, o, 64); }
             if (lane == 0) sx[i] = cdiv(make_double2(sx[i].x - sr, sx[i].y - si), A[(size_t)i * P + i]);
-            __builtin_amdgcn_s_waitcnt(0);
-            __builtin_amdgcn_wave_barrier();
+            qgtl::wave_sync();
         }
         for (int i = lane; i < P; i += 64) x[i] = sx[i];
         if (lane == 0) status[blockIdx.x] = 0;
@@ -623,6 +619,7 @@ __global__ __launch_bounds__(CT) void cholesky_f64_kernel(double *Lall, const do
                 for (int e = lane; e < NB * NB; e += 64)         // identity past a short last block
                     if (e / NB >= nn) dgs[cur ^ 1][e / NB][e % NB] = e / NB == e % NB ? 1.0 : 0.0;
                 for (int u = 0; u < kOwn && u < nt * (nt + 1) / 2; u++) tile(u, true);
+                qgtl::wave_sync();                   // the lanes' tile elements are read by rows
                 if (factor_diag<NB>(dgs[cur ^ 1], invs[cur ^ 1], lane) && lane == 0) s_fail = 1;
             }
         } else {
