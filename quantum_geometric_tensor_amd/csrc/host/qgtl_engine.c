@@ -250,13 +250,29 @@ static void free_chain(struct qgtl_plan *p)
     p->nchain = 0;
 }
 
-static void plan_free_device(struct qgtl_plan *p)
+/* What alloc_mixed and alloc_plain made. */
+static void free_states(struct qgtl_plan *p)
 {
     free_chain(p);
     qgtl_hip_free(p->psi[0]);
     qgtl_hip_free(p->psi[1]);
     qgtl_hip_free(p->D);
     qgtl_hip_free(p->tmp);
+    qgtl_hip_free(p->inj_partials);
+    qgtl_hip_free(p->inj_sums);
+    qgtl_hip_free(p->gram_partials);
+    qgtl_hip_free(p->C);
+    qgtl_hip_free(p->Qdev);
+    qgtl_hip_host_free(p->Qhost);
+    qgtl_hip_free(p->plain_partials);
+    p->psi[0] = p->psi[1] = p->D = p->tmp = NULL;
+    p->inj_partials = p->inj_sums = p->C = p->Qdev = p->Qhost = p->plain_partials = NULL;
+    p->gram_partials = NULL;
+}
+
+static void plan_free_device(struct qgtl_plan *p)
+{
+    free_states(p);
     qgtl_hip_free(p->tabs_dev);                          /* the injection slots are part of it */
     qgtl_hip_host_free(p->tabs_host);
     p->tabs_dev = p->inj_slots_dev = NULL;
@@ -266,14 +282,6 @@ static void plan_free_device(struct qgtl_plan *p)
     qgtl_hip_free(p->res_dev);
     qgtl_hip_host_free(p->res_host);
     p->res_dev = p->res_host = NULL;
-    qgtl_hip_free(p->inj_partials);
-    qgtl_hip_free(p->inj_sums);
-    qgtl_hip_free(p->gram_partials);
-    qgtl_hip_free(p->C);
-    qgtl_hip_free(p->Qdev);
-    qgtl_hip_host_free(p->Qhost);
-    p->Qhost = NULL;
-    qgtl_hip_free(p->plain_partials);
     qgtl_hip_free(p->terms_dev);
     qgtl_hip_free(p->hpsi);
     qgtl_hip_free(p->eg_partials);
@@ -295,9 +303,6 @@ static void plan_free_device(struct qgtl_plan *p)
     p->terms_dev = p->hpsi = NULL;
     p->eg_partials = p->eg_sums = p->eg_out = NULL;
     p->psi_final = NULL;
-    p->psi[0] = p->psi[1] = p->D = p->tmp = NULL;
-    p->inj_partials = p->inj_sums = p->C = p->Qdev = p->plain_partials = NULL;
-    p->gram_partials = NULL;
 }
 
 qgtl_plan_t *qgtl_plan_create(int n, int nops, const qgtl_op_t *ops, int mode, const qgtl_tune_t *tune)
@@ -475,9 +480,8 @@ static void alloc_chain(struct qgtl_plan *p)
         p->tmp_side = NULL;
 }
 
-static int alloc_mixed(struct qgtl_plan *p)
+static int alloc_mixed_states(struct qgtl_plan *p)
 {
-    if (p->psi[0]) return 0;
     const size_t N = p->N, P = (size_t)p->P;
     HIPCALL(qgtl_hip_malloc(&p->psi[0], N * 8));
     HIPCALL(qgtl_hip_malloc(&p->psi[1], N * 8));
@@ -513,9 +517,18 @@ static int alloc_mixed(struct qgtl_plan *p)
     return 0;
 }
 
-static int alloc_plain(struct qgtl_plan *p)
+/* All of a plan's buffers or none: a plan that did not fit keeps nothing, and
+ * its next execute tries (and reports) again. */
+static int alloc_mixed(struct qgtl_plan *p)
 {
     if (p->psi[0]) return 0;
+    const int rc = alloc_mixed_states(p);
+    if (rc) free_states(p);
+    return rc;
+}
+
+static int alloc_plain_states(struct qgtl_plan *p)
+{
     const size_t N = p->N, P = (size_t)p->P;
     HIPCALL(qgtl_hip_malloc(&p->psi[0], N * 16));
     if (P > 0) {
@@ -531,6 +544,14 @@ static int alloc_plain(struct qgtl_plan *p)
     }
     alloc_chain(p);
     return 0;
+}
+
+static int alloc_plain(struct qgtl_plan *p)
+{
+    if (p->psi[0]) return 0;
+    const int rc = alloc_plain_states(p);
+    if (rc) free_states(p);
+    return rc;
 }
 
 /* device phase tables of pass i of block b (inv: of its inverse), NULL before they exist */
