@@ -268,6 +268,7 @@ static void free_states(struct qgtl_plan *p)
     p->psi[0] = p->psi[1] = p->D = p->tmp = NULL;
     p->inj_partials = p->inj_sums = p->C = p->Qdev = p->Qhost = p->plain_partials = NULL;
     p->gram_partials = NULL;
+    p->chain_tried = 0;
 }
 
 static void plan_free_device(struct qgtl_plan *p)
@@ -513,7 +514,6 @@ static int alloc_mixed_states(struct qgtl_plan *p)
         HIPCALL(qgtl_hip_malloc((void **)&p->Qdev, P * P * 2 * sizeof(double)));
         HIPCALL(qgtl_hip_host_alloc((void **)&p->Qhost, P * P * 2 * sizeof(double)));
     }
-    alloc_chain(p);
     return 0;
 }
 
@@ -1115,16 +1115,33 @@ static int run_mixed_lanes(struct qgtl_plan *p, qgtl_stats_t *st, int lanes)
     return 0;
 }
 
-/* Everything before the launches of a mixed execute: device buffers, phase
- * tables and injection slots uploaded, the schedule chosen, the events of the
- * two lanes made (none of it may happen under graph capture). */
-static int prepare_mixed(struct qgtl_plan *p)
+/* Device buffers, phase tables and injection slots uploaded. */
+static int prepare_buffers(struct qgtl_plan *p)
 {
-    int rc = alloc_mixed(p);
+    const int rc = alloc_mixed(p);
     if (rc) return rc;
     p->resident = resident_ok(p);
-    rc = p->resident ? upload_resident(p) : upload_tabs(p);
+    return p->resident ? upload_resident(p) : upload_tabs(p);
+}
+
+/* Everything before the launches of a mixed execute: the buffers, the schedule
+ * chosen, the events of the two lanes made (none of it may happen under graph
+ * capture). */
+static int prepare_mixed(struct qgtl_plan *p)
+{
+    int rc = prepare_buffers(p);
+    if (rc && p->ringless && !p->inplace && any_flip(p)) {
+        /* no room for the chunk buffer that folded stages need: the stages' gates one by one, in place */
+        free_states(p);
+        p->inplace = 1;
+        rc = qgtl_plan_build(p);
+        if (!rc) rc = prepare_buffers(p);
+    }
     if (rc) return rc;
+    if (!p->chain_tried) {                                   /* optional, so after all that is not */
+        p->chain_tried = 1;
+        alloc_chain(p);
+    }
     const int depth_first = any_flip(p);
     p->meet = choose_meet(p, depth_first);
     p->presplit = presplit_ok(p, depth_first, gram_terms(p));

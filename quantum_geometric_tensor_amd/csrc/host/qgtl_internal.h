@@ -81,6 +81,7 @@ struct qgtl_plan {
     qgtl_op_t *ops;
     int has_signs;                       /* some block's M-stage has a sign */
     int ringless;                        /* n > 13: M-stages, but no CNOT ring among them */
+    int inplace;                         /* M-stages that move indices by per-gate kernels, in place (n > 13) */
     int nblocks;
     qgtl_block_t *blocks;
     int blocks_cap;
@@ -119,6 +120,7 @@ struct qgtl_plan {
      * on the second stream and each chunk waits only for the state it reads */
     void **chain;
     int nchain;                          /* nblocks + 1, or 0 (two-buffer chain) */
+    int chain_tried;                     /* allocated, or there was no room for it */
     void *chain_tmp;
     void *tmp_side;                      /* chunk buffer of the chain's stream (backward chunks), or NULL */
     int capturing;                       /* the launches being issued are captured into the plan's graph */

@@ -677,8 +677,9 @@ static int index_unmoved(const qgtl_block_t *b, int n)
     return 1;
 }
 
-/* The layouts of block b's passes (their matrices are set for given angles). */
-static void build_passes(qgtl_block_t *b, int n)
+/* The layouts of block b's passes (their matrices are set for given angles).
+ * inplace: no index map is folded into them (n > 13). */
+static void build_passes(qgtl_block_t *b, int n, int inplace)
 {
     const int TB = QGTL_TILE_BITS_MAX;
     b->npasses = 0;
@@ -714,7 +715,7 @@ static void build_passes(qgtl_block_t *b, int n)
     }
     high_passes(b, n, b->pass, b->pass_flips, &b->npasses);
     b->linear = !b->is_ring && !index_unmoved(b, n);
-    b->mstage_kernels = b->linear && !find_mstage_map(b, n);
+    b->mstage_kernels = b->linear && (inplace || !find_mstage_map(b, n));
     if (b->mstage_kernels) b->linear = 0;
     const int store = b->is_ring ? QGTL_STORE_RING : b->linear ? QGTL_STORE_LINEAR : QGTL_STORE_INPLACE;
     qgtl_pass_desc_t *low = &b->pass[b->npasses];
@@ -990,7 +991,7 @@ int qgtl_plan_build(struct qgtl_plan *plan)
         plan->has_signs |= b->has_sign;
         rings += b->is_ring;
         stages += b->nperm > 0;
-        build_passes(b, n);
+        build_passes(b, n, plan->inplace);
         if (plan->mode == QGTL_MODE_MIXED && plan->tune.sweep_schedule != 1) build_inverse_passes(b, n);
         /* images of the basis vectors under the inverse M-stage (the Z-frame masks below) */
         uint32_t inv_img[QGTL_MAX_QUBITS];

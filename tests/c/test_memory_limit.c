@@ -260,6 +260,30 @@ int main(void)
         qgtl_plan_destroy(p);
         if (used) return fail("a destroyed plan keeps memory");
     }
+    /* 2. CNOT lines within the memory that CZ lines take, whose passes stay in place */
+    size_t need = 0;
+    for (int kind = 0; kind < 3; kind++) {
+        const int k = circuit(kind ? GATE_TYPE_CNOT : GATE_TYPE_CZ, 0, ops);
+        limit = kind == 2 ? need : SIZE_MAX;
+        peak = used;
+        linear_passes = gate_kernels = 0;
+        qgtl_plan_t *p = qgtl_plan_create(N_QUBITS, k, ops, QGTL_MODE_MIXED, &tune);
+        if (!p || qgtl_plan_execute(p, Q, NULL) || bad) return fail("a circuit without a ring does not run in place");
+        if (kind == 0) need = peak;
+        if (kind == 1 && (!linear_passes || gate_kernels)) return fail("a CNOT line is not folded where memory allows it");
+        if (kind == 2 && (linear_passes || !gate_kernels)) return fail("passes that move indices without their buffer");
+        double th[LAYERS * N_QUBITS * 3] = {0.0};
+        if (qgtl_plan_set_angles(p, k, th) || qgtl_plan_execute(p, Q, NULL) || bad) return fail("new angles in place");
+        qgtl_plan_destroy(p);
+        if (used) return fail("a destroyed plan keeps memory");
+    }
+    /* and within any more */
+    const int k = circuit(GATE_TYPE_CNOT, 0, ops);
+    for (limit = need; limit < 4 * need; limit += 20000) {
+        qgtl_plan_t *p = qgtl_plan_create(N_QUBITS, k, ops, QGTL_MODE_MIXED, &tune);
+        if (!p || qgtl_plan_execute(p, Q, NULL) || bad) return fail("more memory than in place, and it does not fit");
+        qgtl_plan_destroy(p);
+    }
     puts("ok");
     return 0;
 }
