@@ -64,12 +64,23 @@ int qgtl_plan_set_hamiltonian(qgtl_plan_t *p, int nterms, const qgtl_pauli_term_
     if (nterms > p->nterms) {
         qgtl_hip_free(p->terms_dev);
         p->terms_dev = NULL;
+        p->nterms = 0;
         TRYH(qgtl_hip_malloc(&p->terms_dev, sizeof(qgtl_pauli_term_t) * (size_t)nterms));
     }
     TRYH(qgtl_hip_h2d(p->terms_dev, terms, sizeof(qgtl_pauli_term_t) * (size_t)nterms));
     TRYH(qgtl_hip_sync());
     p->nterms = nterms;
     return 0;
+}
+
+void qgtl_energy_free(struct qgtl_plan *p)
+{
+    qgtl_hip_free(p->hpsi);
+    qgtl_hip_free(p->eg_partials);
+    qgtl_hip_free(p->eg_sums);
+    qgtl_hip_free(p->eg_out);
+    p->hpsi = NULL;
+    p->eg_partials = p->eg_sums = p->eg_out = NULL;
 }
 
 int qgtl_energy_gradient_device(qgtl_plan_t *p)
@@ -79,11 +90,16 @@ int qgtl_energy_gradient_device(qgtl_plan_t *p)
     if (p->nterms < 1) return qgtl_set_error(QGT_ERROR_INVALID_STATE, "no Hamiltonian set");
     const size_t N = p->N, P = (size_t)p->P;
     const size_t tiles = (N + 2047) / 2048;
-    if (!p->hpsi) {
-        TRYH(qgtl_hip_malloc(&p->hpsi, N * 8));
-        TRYH(qgtl_hip_malloc((void **)&p->eg_partials, (P + 1) * tiles * 4 * sizeof(double)));
-        TRYH(qgtl_hip_malloc((void **)&p->eg_sums, (P + 1) * 4 * sizeof(double)));
-        TRYH(qgtl_hip_malloc((void **)&p->eg_out, (P + 1) * sizeof(double)));
+    if (!p->hpsi) {                                          /* all of them or none */
+        int rc = qgtl_hip_malloc(&p->hpsi, N * 8);
+        if (!rc) rc = qgtl_hip_malloc((void **)&p->eg_partials, (P + 1) * tiles * 4 * sizeof(double));
+        if (!rc) rc = qgtl_hip_malloc((void **)&p->eg_sums, (P + 1) * 4 * sizeof(double));
+        if (!rc) rc = qgtl_hip_malloc((void **)&p->eg_out, (P + 1) * sizeof(double));
+        if (rc) {
+            qgtl_set_error(rc, "energy buffers: %s", qgtl_hip_last_error());
+            qgtl_energy_free(p);
+            return rc;
+        }
     }
     int t1 = 0, t2 = 0;
     TRYH(qgtl_hip_pauli_apply_c64(p->psi_final, p->hpsi, p->n, p->nterms, p->terms_dev));

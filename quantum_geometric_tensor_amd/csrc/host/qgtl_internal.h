@@ -209,6 +209,8 @@ void qgtl_mlp_shape(const qgtl_mlp_t *m, int *in_dim, int *P, int *rank);
 void qgtl_pass_phase_tables(const qgtl_pass_desc_t *p, float *out);
 void qgtl_resident_block(const qgtl_block_t *b, int n, qgtl_res_block_t *out, qgtl_c64_t *tabs);
 int qgtl_carry_to_meet(struct qgtl_plan *p, void **state, void **scratch);
+void qgtl_energy_free(struct qgtl_plan *p);              /* buffers of the energy and gradient (qgtl_hamiltonian.c) */
+void qgtl_ng_free(struct qgtl_plan *p);                  /* buffers of the natural-gradient step (qgtl_ngvqe.c) */
 
 /* file container of qgtl_io.c (prefix, kind header, payload, FNV-1a 64 checksum) */
 uint64_t qgtl_fnv1a(uint64_t h, const void *data, size_t n);

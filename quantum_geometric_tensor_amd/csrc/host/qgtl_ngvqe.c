@@ -36,6 +36,23 @@ static double wall_ms(void)
     return ts.tv_sec * 1e3 + ts.tv_nsec * 1e-6;
 }
 
+void qgtl_ng_free(struct qgtl_plan *p)
+{
+    qgtl_hip_free(p->ng_slot);
+    qgtl_hip_free(p->ng_A);
+    qgtl_hip_free(p->ng_D);
+    qgtl_hip_free(p->ng_g);
+    qgtl_hip_free(p->ng_x);
+    qgtl_hip_free(p->ng_d);
+    qgtl_hip_free(p->ng_U);
+    qgtl_hip_free(p->ng_theta);
+    qgtl_hip_free(p->ng_res);
+    qgtl_hip_free(p->ng_it);
+    p->ng_slot = p->ng_it = NULL;
+    p->ng_A = p->ng_D = p->ng_g = p->ng_x = p->ng_d = p->ng_U = p->ng_theta = p->ng_res = NULL;
+    p->ng_rank = 0;
+}
+
 static int ensure_ng_buffers(qgtl_plan_t *p, int rank)
 {
     const size_t P = (size_t)p->P;
@@ -57,7 +74,10 @@ static int ensure_ng_buffers(qgtl_plan_t *p, int rank)
         NTRY(qgtl_hip_sync());
     out:
         free(slot);
-        if (rc) return rc;
+        if (rc) {                                            /* all of them or none */
+            qgtl_ng_free(p);
+            return rc;
+        }
     }
     if (rank > p->ng_rank) {
         qgtl_hip_free(p->ng_U);

@@ -211,6 +211,53 @@ EXPORT int qgtl_hip_qgt_finalize_plain(const double *G, const double *a, int P, 
     return finalize(G, P, Q);
 }
 
+EXPORT int qgtl_hip_fill_f32(void *d, size_t count, float v) { (void)v; touch(d, 4 * count, "fill"); return 0; }
+EXPORT int qgtl_hip_pauli_apply_c64(const void *psi, void *out, int n, int nterms, const void *terms)
+{
+    touch(psi, (size_t)8 << n, "H psi");
+    touch(out, (size_t)8 << n, "H psi");
+    touch(terms, sizeof(qgtl_pauli_term_t) * (size_t)nterms, "H psi");
+    return 0;
+}
+EXPORT int qgtl_hip_dot_states_c64(const void *D, size_t stride, int K, const void *v, int n, double *part, int *tiles,
+                                   int planes)
+{
+    (void)planes;
+    states(D, stride, K, n, "dot");
+    touch(v, (size_t)8 << n, "dot");
+    touch(part, (size_t)K * 32, "dot");
+    *tiles = 1;
+    return 0;
+}
+EXPORT int qgtl_hip_energy_gradient_finalize(const double *dk, const double *psi, int P, double *out)
+{
+    touch(dk, (size_t)P * 32, "energy");
+    touch(psi, 32, "energy");
+    touch(out, (size_t)(P + 1) * 8, "energy");
+    return 0;
+}
+EXPORT int qgtl_hip_ng_assemble(const double *Q, const int *slot, int P, double lambda, const double *eg, double *A,
+                                double *D, double *g)
+{
+    (void)lambda;
+    touch(Q, (size_t)P * P * 16, "assemble");
+    touch(slot, (size_t)P * 4, "assemble");
+    touch(eg, (size_t)(P + 1) * 8, "assemble");
+    touch(A, (size_t)P * P * 8, "assemble");
+    touch(D, (size_t)P * 8, "assemble");
+    touch(g, (size_t)P * 8, "assemble");
+    return 0;
+}
+EXPORT int qgtl_hip_cholesky_solve_f64(double *A, const double *b, double *x, int P, int batch, double lambda, int *status)
+{
+    (void)batch, (void)lambda;
+    touch(A, (size_t)P * P * 8, "solve");
+    touch(b, (size_t)P * 8, "solve");
+    touch(x, (size_t)P * 8, "solve");
+    touch(status, 4, "solve");
+    return 0;
+}
+
 /* ---- circuits: L layers of RY, RZ on every qubit and a line or ring of two-qubit gates */
 enum { N_QUBITS = 14, LAYERS = 4 };
 static int circuit(int two, int ring, qgtl_op_t *ops)
@@ -260,6 +307,40 @@ int main(void)
         qgtl_plan_destroy(p);
         if (used) return fail("a destroyed plan keeps memory");
     }
+    /* ... and to a Hamiltonian's, the energy's and the natural gradient's buffers */
+    {
+        const int k = circuit(GATE_TYPE_CNOT, 1, ops);
+        qgtl_pauli_term_t terms[2 * N_QUBITS];
+        const int nt = qgtl_tfim_terms(N_QUBITS, 1.0, 0.5, terms);
+        const qgtl_ng_config_t cfg = {.lambda = 1e-3, .eta = 0.1, .method = QGTL_SOLVE_CHOLESKY};
+        double th[LAYERS * N_QUBITS * 3] = {0.0};
+        for (int grow = 0; grow < 2; grow++) {
+            limit = SIZE_MAX;
+            qgtl_plan_t *p = qgtl_plan_create(N_QUBITS, k, ops, QGTL_MODE_MIXED, &tune);
+            if (!p || qgtl_plan_set_hamiltonian(p, 1, terms) || (grow && qgtl_plan_execute(p, Q, NULL)))
+                return fail("a plan with room enough fails");
+            const size_t base = used;
+            int ok = 0;
+            for (size_t l = 0; !ok && l < (size_t)64 << 20; l += 100000) {
+                limit = base + l;
+                const int r1 = qgtl_ng_step(p, th, &cfg, NULL, 0.5, NULL), r2 = qgtl_ng_step(p, th, &cfg, NULL, 0.5, NULL);
+                if (bad) return 1;
+                if (!r1 != !r2) return fail("a second step at the same limit ends otherwise");
+                ok = !r1;
+            }
+            if (!ok) return fail("no step with room enough");
+            /* more terms than there is room for: an error, and the step says that there are none */
+            limit = used;
+            if (!qgtl_plan_set_hamiltonian(p, nt, terms) || !qgtl_ng_step(p, th, &cfg, NULL, 0.5, NULL) || bad)
+                return fail("a Hamiltonian that did not fit is used");
+            limit = SIZE_MAX;
+            if (qgtl_plan_set_hamiltonian(p, nt, terms) || qgtl_ng_step(p, th, &cfg, NULL, 0.5, NULL) || bad)
+                return fail("a Hamiltonian that fits is not used");
+            qgtl_plan_destroy(p);
+            if (used) return fail("a destroyed plan keeps memory");
+        }
+    }
+
     /* 2. CNOT lines within the memory that CZ lines take, whose passes stay in place */
     size_t need = 0;
     for (int kind = 0; kind < 3; kind++) {
