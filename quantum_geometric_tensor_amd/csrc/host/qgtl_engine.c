@@ -263,26 +263,22 @@ static void free_states(struct qgtl_plan *p)
     qgtl_hip_free(p->gram_partials);
     qgtl_hip_free(p->C);
     qgtl_hip_free(p->Qdev);
-    qgtl_hip_host_free(p->Qhost);
+    qgtl_hip_host_free(p->Qhost);                        /* the tables' host copy is part of it */
+    qgtl_hip_free(p->tabs_dev);
+    qgtl_hip_free(p->res_dev);
     qgtl_hip_free(p->plain_partials);
     p->psi[0] = p->psi[1] = p->D = p->tmp = NULL;
     p->inj_partials = p->inj_sums = p->C = p->Qdev = p->Qhost = p->plain_partials = NULL;
     p->gram_partials = NULL;
+    p->tabs_dev = p->inj_slots_dev = p->res_dev = NULL;
+    p->tabs_host = NULL;
     p->chain_tried = 0;
+    p->tabs_dirty = 1;
 }
 
 static void plan_free_device(struct qgtl_plan *p)
 {
     free_states(p);
-    qgtl_hip_free(p->tabs_dev);                          /* the injection slots are part of it */
-    qgtl_hip_host_free(p->tabs_host);
-    p->tabs_dev = p->inj_slots_dev = NULL;
-    p->tabs_host = NULL;
-    p->inj_slots_host = NULL;
-    p->tabs_passes = 0;
-    qgtl_hip_free(p->res_dev);
-    qgtl_hip_host_free(p->res_host);
-    p->res_dev = p->res_host = NULL;
     qgtl_hip_free(p->terms_dev);
     p->terms_dev = NULL;
     qgtl_energy_free(p);
@@ -465,6 +461,35 @@ static void alloc_chain(struct qgtl_plan *p)
         p->tmp_side = NULL;
 }
 
+/* Circuits whose states one workgroup holds in LDS from start to end; the
+ * general-matrix sweep form and the one- to three-qubit circuits keep the
+ * breadth-first passes. */
+static int resident_ok(const struct qgtl_plan *p)
+{
+    return p->P > 0 && p->n >= QGTL_RES_MIN_QUBITS && p->n <= QGTL_RES_MAX_QUBITS && p->tune.sweep_form != 1;
+}
+
+/* Layout of the tables that new angles rebuild, uploaded in one copy; its size
+ * in bytes.  Resident plans: blocks, phase tables, slots; others: the phase
+ * tables of every pass, then the injection slots (forward, backward). */
+static size_t table_layout(struct qgtl_plan *p)
+{
+    const size_t nb = (size_t)p->nblocks, P = (size_t)p->P;
+    if (resident_ok(p)) {
+        p->tab_first = nb * sizeof(qgtl_res_block_t);
+        p->tab_slots = p->tab_first + nb * 2 * QGTL_RES_TAB * sizeof(qgtl_c64_t);
+        return p->tab_slots + (P + 1) * sizeof(qgtl_res_slot_t);
+    }
+    int total = 0;
+    for (int bi = 0; bi < p->nblocks; bi++) {
+        p->blocks[bi].tab0 = total;
+        total += p->blocks[bi].npasses + p->blocks[bi].ninv;
+    }
+    p->tab_first = 0;
+    p->tab_slots = 2 * QGTL_PHASE_TAB * sizeof(qgtl_c64_t) * (size_t)total;
+    return total ? p->tab_slots + 2 * P * sizeof(qgtl_inject_slot_t) : 0;
+}
+
 static int alloc_mixed_states(struct qgtl_plan *p)
 {
     const size_t N = p->N, P = (size_t)p->P;
@@ -496,8 +521,13 @@ static int alloc_mixed_states(struct qgtl_plan *p)
         const size_t ntc = (P + 1 + 127) / 128, Rc = ntc * 128;
         HIPCALL(qgtl_hip_malloc((void **)&p->C, (R * R > 2 * Rc * Rc ? R * R : 2 * Rc * Rc) * sizeof(double)));
         HIPCALL(qgtl_hip_malloc((void **)&p->Qdev, P * P * 2 * sizeof(double)));
-        HIPCALL(qgtl_hip_host_alloc((void **)&p->Qhost, P * P * 2 * sizeof(double)));
     }
+    /* one page-locked buffer for Q and the tables: page-locking takes 27 us and up, however little */
+    p->tab_bytes = table_layout(p);
+    const size_t qbytes = (P * P * 2 * sizeof(double) + 255) / 256 * 256;
+    HIPCALL(qgtl_hip_host_alloc((void **)&p->Qhost, qbytes + p->tab_bytes));
+    p->tabs_host = (char *)p->Qhost + qbytes;
+    HIPCALL(qgtl_hip_malloc(resident_ok(p) ? &p->res_dev : &p->tabs_dev, p->tab_bytes));
     return 0;
 }
 
@@ -571,40 +601,23 @@ static void slot_matrix(qgtl_inject_slot_t *q, const qgtl_mat2 *M)
 /* Build and upload the phase tables of every pass after the angles changed. */
 static int upload_tabs(struct qgtl_plan *p)
 {
-    if (!p->tabs_dirty && p->tabs_dev) return 0;
-    int total = 0;
-    for (int bi = 0; bi < p->nblocks; bi++) {
-        p->blocks[bi].tab0 = total;
-        total += p->blocks[bi].npasses + p->blocks[bi].ninv;
-    }
-    if (total == 0) { p->tabs_dirty = 0; return 0; }
+    if (!p->tabs_dirty) return 0;
+    if (p->tab_bytes == 0) { p->tabs_dirty = 0; return 0; }
     const size_t per = 2 * QGTL_PHASE_TAB * 2;                /* floats per pass */
     const size_t P = (size_t)p->P;
-    /* tables and slots in one pinned buffer: one asynchronous copy */
-    const size_t tab_bytes = sizeof(float) * per * (size_t)total;
-    const size_t bytes = tab_bytes + 2 * P * sizeof(qgtl_inject_slot_t);
-    if (total != p->tabs_passes) {
-        qgtl_hip_free(p->tabs_dev);
-        qgtl_hip_host_free(p->tabs_host);
-        p->tabs_dev = p->inj_slots_dev = NULL;
-        p->tabs_host = NULL;
-        p->tabs_passes = 0;
-        HIPCALL(qgtl_hip_host_alloc((void **)&p->tabs_host, bytes));
-        HIPCALL(qgtl_hip_malloc(&p->tabs_dev, bytes));
-        p->inj_slots_host = (qgtl_inject_slot_t *)((char *)p->tabs_host + tab_bytes);
-        p->inj_slots_dev = P > 0 ? (char *)p->tabs_dev + tab_bytes : NULL;
-        p->tabs_passes = total;
-    }
+    float *tabs = (float *)p->tabs_host;
+    qgtl_inject_slot_t *slots = (qgtl_inject_slot_t *)(p->tabs_host + p->tab_slots);
+    p->inj_slots_dev = P > 0 ? (char *)p->tabs_dev + p->tab_slots : NULL;
     int k = 0;
     for (int bi = 0; bi < p->nblocks; bi++) {
         for (int i = 0; i < p->blocks[bi].npasses; i++, k++)
-            qgtl_pass_phase_tables(&p->blocks[bi].pass[i], p->tabs_host + per * (size_t)k);
+            qgtl_pass_phase_tables(&p->blocks[bi].pass[i], tabs + per * (size_t)k);
         for (int i = 0; i < p->blocks[bi].ninv; i++, k++)
-            qgtl_pass_phase_tables(&p->blocks[bi].ipass[i], p->tabs_host + per * (size_t)k);
+            qgtl_pass_phase_tables(&p->blocks[bi].ipass[i], tabs + per * (size_t)k);
     }
     for (size_t s = 0; s < P; s++) {
         const qgtl_param_t *pp = &p->params[p->slot_param[s]];
-        qgtl_inject_slot_t *f = &p->inj_slots_host[s], *bk = &p->inj_slots_host[P + s];
+        qgtl_inject_slot_t *f = &slots[s], *bk = &slots[P + s];
         f->v = pp->v;
         f->w = pp->w;
         f->z = pp->z;
@@ -613,38 +626,22 @@ static int upload_tabs(struct qgtl_plan *p)
         slot_matrix(f, &pp->A);
         slot_matrix(bk, &pp->B);
     }
-    HIPCALL(qgtl_hip_h2d(p->tabs_dev, p->tabs_host, bytes));
+    HIPCALL(qgtl_hip_h2d(p->tabs_dev, p->tabs_host, p->tab_bytes));
     p->tabs_dirty = 0;
     return 0;
-}
-
-/* Circuits whose states one workgroup holds in LDS from start to end; the
- * general-matrix sweep form and the one- to three-qubit circuits keep the
- * breadth-first passes. */
-static int resident_ok(const struct qgtl_plan *p)
-{
-    return p->P > 0 && p->n >= QGTL_RES_MIN_QUBITS && p->n <= QGTL_RES_MAX_QUBITS && p->tune.sweep_form != 1;
 }
 
 /* Build and upload the resident kernel's blocks, phase tables and slots after
  * the angles changed. */
 static int upload_resident(struct qgtl_plan *p)
 {
+    if (!p->tabs_dirty) return 0;
     const size_t nb = (size_t)p->nblocks, P = (size_t)p->P;
-    if (!p->res_dev) {
-        p->res_tabs = nb * sizeof(qgtl_res_block_t);
-        p->res_slots = p->res_tabs + nb * 2 * QGTL_RES_TAB * sizeof(qgtl_c64_t);
-        p->res_bytes = p->res_slots + (P + 1) * sizeof(qgtl_res_slot_t);
-        if (!p->res_host) HIPCALL(qgtl_hip_host_alloc(&p->res_host, p->res_bytes));
-        HIPCALL(qgtl_hip_malloc(&p->res_dev, p->res_bytes));
-    } else if (!p->tabs_dirty) {
-        return 0;
-    }
-    char *h = (char *)p->res_host;
-    qgtl_res_slot_t *slots = (qgtl_res_slot_t *)(h + p->res_slots);
+    char *h = p->tabs_host;
+    qgtl_res_slot_t *slots = (qgtl_res_slot_t *)(h + p->tab_slots);
     for (size_t b = 0; b < nb; b++)
         qgtl_resident_block(&p->blocks[b], p->n, (qgtl_res_block_t *)h + b,
-                            (qgtl_c64_t *)(h + p->res_tabs) + b * 2 * QGTL_RES_TAB);
+                            (qgtl_c64_t *)(h + p->tab_first) + b * 2 * QGTL_RES_TAB);
     for (size_t s = 0; s < P; s++) {
         const qgtl_param_t *pp = &p->params[p->slot_param[s]];
         qgtl_inject_slot_t q;
@@ -655,7 +652,7 @@ static int upload_resident(struct qgtl_plan *p)
     }
     memset(&slots[P], 0, sizeof slots[P]);
     slots[P].block = p->nblocks;
-    HIPCALL(qgtl_hip_h2d(p->res_dev, p->res_host, p->res_bytes));
+    HIPCALL(qgtl_hip_h2d(p->res_dev, p->tabs_host, p->tab_bytes));
     p->tabs_dirty = 0;
     return 0;
 }
@@ -1152,7 +1149,7 @@ static int prepare_mixed(struct qgtl_plan *p)
 static int run_resident(struct qgtl_plan *p, qgtl_stats_t *st)
 {
     const char *d = (const char *)p->res_dev;
-    LAUNCH(K_SWEEP, qgtl_hip_resident_states(p->n, d, p->nblocks, d + p->res_tabs, d + p->res_slots, p->P,
+    LAUNCH(K_SWEEP, qgtl_hip_resident_states(p->n, d, p->nblocks, d + p->tab_first, d + p->tab_slots, p->P,
                                              p->has_signs, p->D, p->psi[0], p->inj_sums));
     p->psi_final = p->psi[0];
     if (st) {

@@ -133,19 +133,17 @@ struct qgtl_plan {
                                             later blocks' states are carried backwards); nblocks - 1: the end */
     /* rotation-form phase tables of every pass (block order), built on the host */
     int tabs_dirty;                      /* angles changed since the last upload */
-    int tabs_passes;
-    float *tabs_host;                    /* tabs_passes x 2 x QGTL_PHASE_TAB complex64, then the slots; pinned */
+    char *tabs_host;                     /* behind Q in the pinned buffer at Qhost */
+    size_t tab_first, tab_slots, tab_bytes;   /* byte offsets of the phase tables and the slots; size */
     void *tabs_dev;
     /* per D slot: the injection as a load-time formula, forward (slots 0..P-1)
      * and backward (P..2P-1), rebuilt with the tables */
-    qgtl_inject_slot_t *inj_slots_host;
     void *inj_slots_dev;
     /* small circuits evolved in LDS by one launch (qgtl_hip_resident_states): the
      * blocks' descriptors, their phase tables and the injection slots, in one
-     * buffer rebuilt with the tables (pinned host copy beside it) */
+     * buffer, as the tables of the others are */
     int resident;
-    void *res_dev, *res_host;
-    size_t res_tabs, res_slots, res_bytes;   /* byte offsets of the tables and the slots; size */
+    void *res_dev;
     /* Hamiltonian for energy / gradient */
     int nterms;
     void *terms_dev;
