@@ -756,10 +756,13 @@ static long meet_cost(const struct qgtl_plan *p, int c)
 
 /* The last block for circuits whose entanglers are never the ring: their
  * states are carried to the end in complex64 and the overlaps and norms are FP64
- * sums.  The two-sided schedule with split-plane states is faster by 0.9 to 1.5
- * (n = 15, four layers of mixed gates and CNOT / CZ lines 297 us against 357) but the Gram of half-evolved,
- * nearly product states is less accurate (mean error against FP64 over six
- * circuits at n = 16: 2.3e-7 of max |Q|, 0.9e-7 at the end of the circuit). */
+ * sums, as such circuits always ran.  The two-sided schedule with split-plane
+ * states would be 10% faster (three layers of mixed gates with CNOT and CZ lines,
+ * n = 15, 16, 17: 224, 252, 337 us against 248, 282, 374) but less accurate (30
+ * circuits, n = 14 .. 18: mean error 1.31e-7 of max |Q| against 1.03e-7).  It is a
+ * rule on the gate list and a heuristic: what makes the difference is how
+ * entangled the states are where they meet.  Circuits with a ring in some
+ * block always met there, and do still (1.3e-7 over the same kinds with one ring). */
 static int choose_meet(const struct qgtl_plan *p, int depth_first)
 {
     const int last = p->nblocks - 1;

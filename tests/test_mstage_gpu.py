@@ -87,3 +87,37 @@ def test_statevector_and_batch(n):
     else:
         with pytest.raises(Q.QGTLError):
             Q.Batch([(n, Q.make_ops(gates))])
+
+
+def _layers(n, kinds, seed):
+    """One layer of random rotations and fixed gates per kind ("r" ring, "n" CNOT line, "z" CZ line)."""
+    rng = np.random.default_rng(seed)
+    gates, k = [], 0
+    for kind in kinds:
+        for q in range(n):
+            if rng.integers(2):
+                gates.append((str(rng.choice(["H", "S", "T", "SX", "X"])), q, -1, -1, 0.0))
+            for _ in range(2):
+                gates.append((str(rng.choice(["RX", "RY", "RZ"])), q, -1, k, rng.uniform(0.0, 2 * np.pi)))
+                k += 1
+        if kind == "r":
+            gates += [("CNOT", q, (q + 1) % n, -1, 0.0) for q in range(n)]
+        else:
+            gates += [("CNOT" if kind == "n" else "CZ", q, q + 1, -1, 0.0) for q in range(n - 1)]
+    return Q.make_ops(gates)
+
+
+@pytest.mark.parametrize("n", [16, 17, 18])
+@pytest.mark.parametrize("kinds", ["rnz", "rzz", "znr", "zzr", "nrz", "zrn", "nzn"])
+def test_accuracy_of_rings_among_lines(n, kinds):
+    """Circuits with a ring in some layer meet half way, on 22-bit Gram operands; those without one go to
+    the end in complex64.  The rule looks at the gate list, not at how entangled the states are where
+    they meet, so the accuracy is held here: the operands' rounding (2^-23) and the sweeps' (about 2^-24
+    a gate on a qubit, seven gates, randomly signed: 1.6e-7) add to 2e-7 of an element of the largest size; a
+    maximum over P^2 of them lies within twice that, of the mean over three circuits."""
+    err = []
+    for seed in range(3):
+        ops = _layers(n, kinds, seed)
+        ref = Q.qgt(n, ops, Q.MODE_FP64_PLAIN)
+        err.append(Q.rel_err(Q.qgt(n, ops), ref))
+    assert np.mean(err) <= 4e-7, err
