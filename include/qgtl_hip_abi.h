@@ -493,6 +493,8 @@ int qgtl_hip_kaporin(int P, int r, int B, const float *Y, const float *As_all, c
                      float *dY, float scale);
 
 /* ---- FP64 natural-gradient solves, one workgroup per system ---- */
+/* A x = b with partial pivoting; status -1: singular by QGTL's rule (qgtl_solve.hip).
+ * A (P x P each) and piv (P each) are working space: unspecified after the call */
 int qgtl_hip_lu_solve_c128(void *A, const void *b, void *x, int *piv, int P, int batch, int *status);
 int qgtl_hip_herm_eig_c128(void *A, void *V, double *ev, int P, int batch, int max_sweeps, int *sweeps);
 /* Extreme eigenvalues of each component of the Hermitian A (upper triangle read):

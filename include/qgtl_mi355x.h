@@ -135,7 +135,7 @@ void qgtl_release_cache(void);
  *
  * ops: the instances' gate lists one after another (nops[i] each); every
  * instance needs n in 1..30, at least one parameter, and M-stages that are
- * CNOT rings when n > 13 (any CNOT/SWAP list when n <= 13).  Q output: the
+ * CNOT rings when n > 13 (any CNOT/SWAP/CZ list when n <= 13).  Q output: the
  * instances' P_i x P_i complex128 matrices one after another (parameter
  * order), at complex offset qgtl_batch_q_offset(b, i). */
 typedef struct qgtl_batch qgtl_batch_t;

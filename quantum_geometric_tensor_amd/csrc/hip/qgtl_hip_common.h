@@ -32,8 +32,6 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// A value every lane of the wave holds (e.g. loaded from a grouped launch's item
-// table) moved into scalar registers, so the code using it stays scalar.
 // Entry idx of Q; host: the caller's pinned copy (consecutive threads write consecutive
 // entries of a row: whole lines cross the bus) or nullptr.
 __device__ __forceinline__ void store_q(double *Q, double *host, size_t idx, double re, double im) {
@@ -42,6 +40,8 @@ __device__ __forceinline__ void store_q(double *Q, double *host, size_t idx, dou
     if (host) reinterpret_cast<double2 *>(host)[idx] = q;
 }
 
+// A value every lane of the wave holds (e.g. loaded from a grouped launch's item
+// table) moved into scalar registers, so the code using it stays scalar.
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 __device__ __forceinline__ int32_t uniform(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ uint64_t uniform(uint64_t v) {

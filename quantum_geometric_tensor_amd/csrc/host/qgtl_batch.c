@@ -773,7 +773,7 @@ qgtl_batch_t *qgtl_batch_create(int count, const int *n, const int *nops, const 
         for (int b = 0; b < p->nblocks; b++) {
             if (n[i] > QGTL_TILE_BITS_MAX && p->blocks[b].nperm > 0 && !p->blocks[b].is_ring) {
                 qgtl_set_error(QGT_ERROR_NOT_IMPLEMENTED,
-                               "instance %d: a CNOT/SWAP stage that is not a ring on more than 13 qubits "
+                               "instance %d: a CNOT/SWAP/CZ stage that is not a ring on more than 13 qubits "
                                "(batched sweeps fold M-stages into passes)", i);
                 return fail_create(B);
             }

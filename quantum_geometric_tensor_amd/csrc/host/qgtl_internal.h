@@ -70,7 +70,7 @@ typedef struct {
                                             the parameter's qubit acting on the block's input state */
 } qgtl_param_t;
 
-/* a single-qubit gate of the expanded gate list (CZ and CY rewritten) */
+/* a single-qubit gate of the expanded gate list (CY rewritten) */
 typedef struct { int type, q, param, op_index, block; } qgtl_gate1_t;
 
 struct qgtl_plan {
