@@ -240,13 +240,10 @@ int qgtl_num_params(int nops, const qgtl_op_t *ops)
 /* ------------------------------------------------------------------ plans */
 static void free_chain(struct qgtl_plan *p)
 {
-    for (int k = 0; k < p->nchain; k++) qgtl_hip_free(p->chain[k]);
-    qgtl_hip_free(p->chain_tmp);
-    qgtl_hip_free(p->tmp_side);
+    qgtl_hip_free(p->chain_mem);
     free(p->chain);
     p->chain = NULL;
-    p->chain_tmp = NULL;
-    p->tmp_side = NULL;
+    p->chain_mem = p->chain_tmp = p->tmp_side = NULL;
     p->nchain = 0;
 }
 
@@ -445,20 +442,25 @@ static void alloc_chain(struct qgtl_plan *p)
 {
     const size_t bytes = p->N * 8, nchain = (size_t)p->nblocks + 1;
     if (p->chain || !any_flip(p) || (nchain + 1) * bytes > ((size_t)2 << 30)) return;
+    const size_t side = p->tmp_states * bytes <= ((size_t)1 << 30) ? p->tmp_states : 0;
     p->chain = (void **)calloc(nchain, sizeof(void *));
     if (!p->chain) return;
-    int ok = qgtl_hip_malloc(&p->chain_tmp, bytes) == 0;
-    for (size_t k = 0; ok && k < nchain; k++) {
-        ok = qgtl_hip_malloc(&p->chain[k], bytes) == 0;
-        if (ok) p->nchain = (int)k + 1;
+    /* one allocation: each may take the driver 270 us */
+    int with_side = side > 0;
+    int rc = qgtl_hip_malloc(&p->chain_mem, (nchain + 1 + side) * bytes);
+    if (rc && with_side) {
+        with_side = 0;
+        rc = qgtl_hip_malloc(&p->chain_mem, (nchain + 1) * bytes);
     }
-    if (!ok) {
+    if (rc) {
         free_chain(p);
         return;
     }
-    if (p->tmp_states > 0 && p->tmp_states * bytes <= ((size_t)1 << 30) &&
-        qgtl_hip_malloc(&p->tmp_side, p->tmp_states * bytes) != 0)
-        p->tmp_side = NULL;
+    char *mem = (char *)p->chain_mem;
+    for (size_t k = 0; k < nchain; k++, mem += bytes) p->chain[k] = mem;
+    p->nchain = (int)nchain;
+    p->chain_tmp = mem;
+    if (with_side) p->tmp_side = mem + bytes;
 }
 
 /* Circuits whose states one workgroup holds in LDS from start to end; the

@@ -121,6 +121,7 @@ struct qgtl_plan {
     void **chain;
     int nchain;                          /* nblocks + 1, or 0 (two-buffer chain) */
     int chain_tried;                     /* allocated, or there was no room for it */
+    void *chain_mem;                     /* chain[], chain_tmp and tmp_side */
     void *chain_tmp;
     void *tmp_side;                      /* chunk buffer of the chain's stream (backward chunks), or NULL */
     int capturing;                       /* the launches being issued are captured into the plan's graph */
