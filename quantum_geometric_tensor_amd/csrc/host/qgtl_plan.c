@@ -993,18 +993,22 @@ int qgtl_plan_build(struct qgtl_plan *plan)
         stages += b->nperm > 0;
         build_passes(b, n, plan->inplace);
         if (plan->mode == QGTL_MODE_MIXED && plan->tune.sweep_schedule != 1) build_inverse_passes(b, n);
-        /* images of the basis vectors under the inverse M-stage (the Z-frame masks below) */
-        uint32_t inv_img[QGTL_MAX_QUBITS];
+        /* images of the basis vectors under the M-stage and its inverse (the masks below) */
+        uint32_t img[QGTL_MAX_QUBITS], inv_img[QGTL_MAX_QUBITS];
         if (b->param_end > b->param_begin)
-            for (int j2 = 0; j2 < n; j2++) inv_img[j2] = perm_apply_inverse(b, 1u << j2);
+            for (int j2 = 0; j2 < n; j2++) {
+                img[j2] = perm_apply(b, 1u << j2);
+                inv_img[j2] = perm_apply_inverse(b, 1u << j2);
+            }
         for (int j = b->param_begin; j < b->param_end; j++) {
             qgtl_param_t *pp = &plan->params[order[j]];
-            pp->v = perm_apply(b, 1u << pp->qubit);
-            const uint32_t bil = polar_row(b->sgn, pp->qubit);
+            pp->v = img[pp->qubit];
             uint32_t w = 0, z = 0;
-            for (int j2 = 0; j2 < n; j2++) {
+            for (int j2 = 0; j2 < n; j2++)
                 if ((inv_img[j2] >> pp->qubit) & 1u) w |= 1u << j2;
-                z |= parity32(inv_img[j2] & bil) << j2;
+            if (b->has_sign) {
+                const uint32_t bil = polar_row(b->sgn, pp->qubit);
+                for (int j2 = 0; j2 < n; j2++) z |= parity32(inv_img[j2] & bil) << j2;
             }
             pp->w = w;
             pp->z = z;
