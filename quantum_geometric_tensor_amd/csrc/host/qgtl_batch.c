@@ -110,6 +110,7 @@ struct qgtl_batch {
     size_t items_bytes, items_cap;
     launch_t *launches;
     int nlaunch, launch_cap;
+    int ready;                 /* the launch sequence and its buffers are those of the tune */
     qgtl_hip_graph_t graph;
     double *qhost;
     double sweep_bytes, gram_flops;
@@ -660,6 +661,7 @@ static int rebuild(struct qgtl_batch *B)
 {
     qgtl_hip_graph_destroy(B->graph);
     B->graph = NULL;
+    B->ready = 0;
     size_t gp = 0;
     for (int i = 0; i < B->count; i++) {
         inst_t *in = &B->inst[i];
@@ -692,6 +694,7 @@ static int rebuild(struct qgtl_batch *B)
         if (rc2) return qgtl_set_error(rc2, "graph capture: %s", qgtl_hip_last_error());
         B->graph = g;
     }
+    B->ready = 1;
     return 0;
 }
 
@@ -906,6 +909,7 @@ int qgtl_batch_get_tune(const qgtl_batch_t *B, qgtl_batch_tune_t *tune)
 /* Run the sequence; device time (HIP events) to *device_ms. */
 static int run_device(struct qgtl_batch *B, double *device_ms)
 {
+    if (!B->ready) return qgtl_set_error(QGT_ERROR_INVALID_STATE, "the batch's tune did not fit: set another");
     if (B->descs_dirty) {
         BTRY(qgtl_hip_h2d(B->pass_d, B->pass_h, B->npass * sizeof(qgtl_pass_desc_t)));
         BTRY(qgtl_hip_h2d(B->inj_d, B->inj_h, B->ninj * sizeof(qgtl_inject_desc_t)));

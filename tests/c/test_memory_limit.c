@@ -258,6 +258,32 @@ EXPORT int qgtl_hip_cholesky_solve_f64(double *A, const double *b, double *x, in
     return 0;
 }
 
+/* grouped launches: the items are host structures that the copy to the device left behind */
+EXPORT int qgtl_hip_cu_count(void) { return 256; }
+EXPORT int qgtl_hip_event_elapsed_ms(qgtl_hip_event_t a, qgtl_hip_event_t b, float *ms) { (void)a, (void)b; *ms = 0.f; return 0; }
+EXPORT int qgtl_hip_phase_tables_grouped(const qgtl_pass_desc_t *d, int n, void *tabs)
+{
+    touch(d, sizeof *d * (size_t)n, "phase tables");
+    touch(tabs, 2 * QGTL_PHASE_TAB * 8 * (size_t)n, "phase tables");
+    return 0;
+}
+#define GROUPED(name, item, ...)                                                       \
+    EXPORT int name(const item *items, int n, uint32_t units, int grid, ##__VA_ARGS__) \
+    {                                                                                  \
+        (void)units, (void)grid;                                                       \
+        touch(items, sizeof *items * (size_t)n, #name);                                \
+        return 0;                                                                      \
+    }
+GROUPED(qgtl_hip_fill_grouped, qgtl_fill_item_t)
+GROUPED(qgtl_hip_pass_grouped, qgtl_pass_item_t, int variant __attribute__((unused)))
+GROUPED(qgtl_hip_inject_grouped, qgtl_inject_item_t)
+GROUPED(qgtl_hip_gram_grouped, qgtl_gram_item_t, int terms __attribute__((unused)))
+GROUPED(qgtl_hip_gram_reduce_grouped, qgtl_gram_reduce_item_t)
+GROUPED(qgtl_hip_finalize_grouped, qgtl_finalize_item_t)
+GROUPED(qgtl_hip_gram_cplx_grouped, qgtl_gram_item_t, int products __attribute__((unused)))
+GROUPED(qgtl_hip_gram_cplx_reduce_grouped, qgtl_gram_reduce_item_t)
+GROUPED(qgtl_hip_finalize_cplx_grouped, qgtl_finalize_item_t)
+
 /* ---- circuits: L layers of RY, RZ on every qubit and a line or ring of two-qubit gates */
 enum { N_QUBITS = 14, LAYERS = 4 };
 static int circuit(int two, int ring, qgtl_op_t *ops)
@@ -339,6 +365,30 @@ int main(void)
             qgtl_plan_destroy(p);
             if (used) return fail("a destroyed plan keeps memory");
         }
+    }
+
+    /* ... and to a batch that is tuned to more than there is room for */
+    {
+        const int n[2] = {N_QUBITS, N_QUBITS};
+        const int k = circuit(GATE_TYPE_CNOT, 1, ops), nops[2] = {k, k};
+        qgtl_op_t *two = malloc(2 * sizeof(qgtl_op_t) * (size_t)k);
+        memcpy(two, ops, sizeof(qgtl_op_t) * (size_t)k);
+        memcpy(two + k, ops, sizeof(qgtl_op_t) * (size_t)k);
+        qgtl_batch_tune_t bt = {.no_graph = 1, .gram_chunk_len = 1 << N_QUBITS};
+        limit = SIZE_MAX;
+        qgtl_batch_t *b = qgtl_batch_create(2, n, nops, two, &bt);
+        double *Qb = malloc(sizeof(double) * 4 * (size_t)P * P);
+        if (!b || qgtl_batch_execute(b, Qb, NULL) || bad) return fail("a batch with room enough fails");
+        const qgtl_batch_tune_t fine = {.no_graph = 1, .gram_chunk_len = 256};
+        limit = used + 1000;
+        if (!qgtl_batch_set_tune(b, &fine) || !qgtl_batch_execute(b, Qb, NULL) || !qgtl_batch_execute(b, Qb, NULL) || bad)
+            return fail("a tune that did not fit is used");
+        limit = SIZE_MAX;
+        if (qgtl_batch_set_tune(b, &fine) || qgtl_batch_execute(b, Qb, NULL) || bad) return fail("a tune that fits is not used");
+        qgtl_batch_destroy(b);
+        free(two);
+        free(Qb);
+        if (used) return fail("a destroyed batch keeps memory");
     }
 
     /* 2. CNOT lines within the memory that CZ lines take, whose passes stay in place */
